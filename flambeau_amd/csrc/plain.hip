@@ -12,6 +12,7 @@
 //   SiLU gate crates/kernels-hip/src/kernels/swiglu_f32_to_f16.cu:21-23
 #include "common.h"
 #include "api.h"
+#include "gemm_float.h"
 #include "recordable.h"
 
 // ------------------------------------------------------------------ embedding
@@ -189,7 +190,8 @@ FL_RECORDABLE(fl_add_inplace)
 // how many rows the call has.  The 16 products of a step are added in a chain of their own and the
 // steps' sums with a compensated (Kahan) addition, still all in float: over K = 14336 a single
 // chain loses about sqrt(K) roundings, which is what showed in the 32-bit path's logits (6.6e-5 at
-// 7B layer sizes against a float64 reference, against a bound of 1e-4).
+// 7B layer sizes against a float64 reference, against a bound of 1e-4).  Floats whose rows are whole 16-byte
+// pieces go to gemm_float.hip, which forms the same sums on the matrix cores; this kernel takes the rest.
 template <typename TIn, typename TOut>
 __global__ __launch_bounds__(256) void gemm_plain_kernel(const TIn* __restrict__ x,
                                                          const TIn* __restrict__ w,
@@ -258,7 +260,9 @@ extern "C" int fl_gemm_plain(const void* x, const void* w, void* out, int in_dty
     FL_CHECK(M >= 0 && N > 0 && K > 0, "gemm: bad sizes M=%d N=%d K=%d", M, N, K);
     if (M == 0) return 0;
     dim3 grid(ceil_div(N, 64), ceil_div(M, 64));
-    if (in_dtype == FL_F32 && out_dtype == FL_F32)
+    if (in_dtype == FL_F32 && out_dtype == FL_F32 && gemm_float_takes(x, w, out, M, N, K))
+        gemm_float_launch((const float*)x, (const float*)w, (float*)out, M, N, K, stream);
+    else if (in_dtype == FL_F32 && out_dtype == FL_F32)
         gemm_plain_kernel<float, float><<<grid, 256, 0, stream>>>((const float*)x, (const float*)w, (float*)out, M, N, K, N);
     else if (in_dtype == FL_BF16 && out_dtype == FL_F32)
         gemm_plain_kernel<bf16_t, float><<<grid, 256, 0, stream>>>((const bf16_t*)x, (const bf16_t*)w, (float*)out, M, N, K, N);

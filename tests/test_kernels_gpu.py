@@ -1178,3 +1178,20 @@ def test_gemm_swiglu_epilogue(out_dtype, M, I, K):
         mid = torch.full((M, I), float("nan"), dtype=out_dtype, device=DEV)
         tuned().gemm_mid(x, W.packed, mid, swiglu_rows=W.packed_rows)
         assert (mid.double() - ref).abs().max() < tol * ref.abs().max()
+
+
+# ---------------------------------------------------------------- the 32-bit product on the matrix cores
+@pytest.mark.parametrize("M", [1, 4, 5, 16, 17, 32, 33, 48, 65, 97])
+@pytest.mark.parametrize("N,K", [(1, 4), (15, 16), (17, 20), (64, 36), (65, 256), (130, 260), (192, 516), (31, 1040)])
+def test_gemm_float_gives_the_plain_kernel_s_bits(M, N, K):
+    """Rows that do not begin at 16 bytes go to the plain kernel, whose sums these are: equal to the last bit."""
+    def at(offset, rows, seed):
+        buf = torch.empty(rows * K + 4, dtype=torch.float32, device=DEV)
+        view = buf[offset:offset + rows * K].view(rows, K)
+        view.copy_(rnd(rows, K, seed=seed))
+        return view
+    want = torch.empty(M, N, dtype=torch.float32, device=DEV)
+    ops().gemm_plain(at(1, M, 31), at(0, N, 32), want)
+    got = torch.full((M, N), float("nan"), dtype=torch.float32, device=DEV)
+    ops().gemm_plain(at(0, M, 31), at(0, N, 32), got)
+    assert torch.equal(got, want)
