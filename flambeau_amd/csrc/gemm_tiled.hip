@@ -10,10 +10,10 @@
 //  * LDS is a ring of NS stages of one k-step (32 values of k); one bare s_barrier per stage;
 //  * the w tile is the A operand and the x tile the B operand: C[feature][token] leaves each
 //    lane with four consecutive features of one token, one 16-byte store;
-//  * two shapes: 256 features x 128 tokens per block (four waves, a wave computes 8 x 4 tiles: 12
-//    operand reads feed 32 products; ring of 3; two blocks per compute unit) when that grid fills
-//    the chip, else 128 x 256 (eight waves of 4 x 4 tiles, ring of 4, one block per unit); blocks
-//    are handed to the eight dies in turn, each die working on a compact patch of tiles;
+//  * blocks of four waves (256, 192 or 128 features x 128 tokens, a wave computes 8 x 4 tiles: 12 operand
+//    reads feed 32 products; ring of 3; two blocks per compute unit) and of eight (256, 224 or 192 features x
+//    256 tokens; ring of 4, one block per unit, the two waves of a SIMD taking turns at the matrix cores);
+//    blocks are handed to the eight dies in turn, each die working on a compact patch of tiles;
 //  * with few rows and a narrow matrix even that grid is small: K is then split over
 //    blockIdx.z, the parts are written as float partial sums and a second kernel adds them in
 //    a fixed order;
@@ -21,11 +21,10 @@
 //    cache rows (rope_store.h); add to the residual stream and leave the next norm in factors.
 //    Every one can scale a token's results by the factor of a norm left that way (TiledFusion).
 //
-// Measured on the 7B shapes: 0.78 to 1.09 PFLOP/s at 2,048 rows, 1.1 to 1.2 at 4,096.  What bounds
-// it is the delivery of operand tiles into LDS: for 28672 x 4096 x 4096 the matrix cores alone take
-// 555 us, with the operand reads 583, with the barrier 637, the whole kernel 871, and the stream
-// of copies alone 700 (about 14 TB/s out of the L2s, whatever the tile shape, ring depth, order of
-// issue or row stride).
+// Measured on the 7B shapes, weights from HBM: 1.0 to 1.2 PFLOP/s at 2,048 rows (28672 x 4096 392 us, 448 before the
+// waves of eight took turns), 1.3 at 4,096, 1.4 at 4,001 rows of 4096 x 14336 (338 us).  What bounds the blocks of
+// four waves is the delivery of operand tiles into LDS (about 57 GB/s per unit); the blocks of eight wait for
+// weights and matrix cores (the loop of gemm_async_kernel says how much for which).
 //
 // The reference's nearest kernel multiplies a 64 x 8 tile per 64-thread block without matrix
 // cores (crates/kernels-hip/src/kernels/mmq_f16_tile.cu:33-107).
@@ -84,8 +83,11 @@ __global__ __launch_bounds__(128 * WT, OCC) void gemm_async_kernel(const bf16_t*
     constexpr int NW = 2 * WT;                        // waves: 2 along the features, WT along the tokens
     constexpr int NTF = 2 * FT, NTT = WT * TT;        // operand tiles of the block: features, tokens
     constexpr int TILES = NTF + NTT;                  // 1 KB tiles per stage
-    constexpr int LPS = TILES / NW;                   // load instructions per wave and stage
-    static_assert(TILES % NW == 0, "tiles must divide among the waves");
+    constexpr int LW = (NTF + NW - 1) / NW, LX = NTT / NW;     // tiles of w and of x that a wave copies per stage (where NTF
+                                                               // does not divide, the last waves copy the last tile too)
+    constexpr int LPS = LW + LX;                      // load instructions per wave and stage
+    constexpr bool PAIRED = NW == 8;                  // two waves per SIMD, half a period apart (below)
+    static_assert(NTT % NW == 0, "tiles of x must divide among the waves");
     extern __shared__ __attribute__((aligned(16))) bf16_t ring[];      // [NS][TILES][512]
     __shared__ float s_scale[NTT * 16];                               // row scale of the block's tokens
 
@@ -117,13 +119,12 @@ __global__ __launch_bounds__(128 * WT, OCC) void gemm_async_kernel(const bf16_t*
 
     // per-lane source addresses of this wave's tiles at the next stage to load; a wave copies LW
     // tiles of w and LX tiles of x per stage
-    constexpr int LW = NTF / NW, LX = NTT / NW;
-    static_assert(NTF % NW == 0 && NTT % NW == 0, "tiles must divide among the waves");
     const bf16_t* wsrc[LW];
     const bf16_t* xsrc[LX];
+    auto w_tile = [&](int u) { return NTF % NW == 0 ? wave * LW + u : min(wave * LW + u, NTF - 1); };
 #pragma unroll
     for (int u = 0; u < LW; ++u) {
-        const int gg = min((n0 >> 4) + wave * LW + u, n_groups - 1);
+        const int gg = min((n0 >> 4) + w_tile(u), n_groups - 1);
         wsrc[u] = wp + (((size_t)gg * n_steps + s_begin) * 64 + lane) * 8;
     }
     // x: the four lanes of a quad read 64 consecutive bytes of one row (a quad that spreads over four
@@ -147,7 +148,7 @@ __global__ __launch_bounds__(128 * WT, OCC) void gemm_async_kernel(const bf16_t*
         bf16_t* slot = ring + (size_t)(i % NS) * TILES * 512;
         if constexpr (c < LW) {
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)wsrc[c],
-                                             (__attribute__((address_space(3))) void*)(slot + (wave * LW + c) * 512), 16, 0, 0);
+                                             (__attribute__((address_space(3))) void*)(slot + w_tile(c) * 512), 16, 0, 0);
             wsrc[c] += 512;
         } else {
             constexpr int u = c - LW;
@@ -232,7 +233,41 @@ __global__ __launch_bounds__(128 * WT, OCC) void gemm_async_kernel(const bf16_t*
         asm volatile("s_barrier" ::: "memory");
     };
     using Behind1 = std::integral_constant<int, NS - 2>;       // reads follow the loads NS - 1 stages behind
-    {
+    if constexpr (PAIRED) {
+        // Waves v and v + 4 share a SIMD, and the second four run half a period behind (one barrier more at the
+        // start, one fewer at the end): while one of a SIMD's waves has the matrix cores, the other reads its
+        // operands and sends its copies on their way.  A period is two barriers, one behind each half.
+        //  - stage i is read by the first four in period i's first half, by the others in its second.  Whoever reads
+        //    it finds it landed: every wave has waited for its own copies of stage i at the end of its reads of i - 1.
+        //  - stage i + NS - 1 goes into the slot of stage i - 1: the reads of that one had arrived in registers before
+        //    their wave's barrier (lgkmcnt(0)), a half period or more ago.
+        // Without it both waves read, then both multiplied: 28672 x 4096 x 4096 803 us, with it 728 (1.19 to 1.32
+        // PFLOP/s).  What is left: the matrix cores alone take 0.52 us a step of 256 x 256, with the operand reads
+        // 0.57, with the copies 0.68 (weights in the caches) to 0.78 (from HBM).  Measured and no faster: copies
+        // among the products, copies of w and x by different waves through rings of their own (w 5 or 6 deep), x
+        // copied in whole lines of 128 bytes (the copies alone 20 to 45 % faster, the kernel 2 % slower).
+        const bool trails = wave >= NW / 2;
+        wait_stage(0, Behind1{});
+        if (trails) asm volatile("s_barrier" ::: "memory");
+        for (int i = 0; i < n_iter; ++i) {
+            bf16x8 a[FT], b[TT];
+            read_operands(a, b, i);
+            __builtin_amdgcn_sched_barrier(0);
+            if (i + NS - 1 < n_iter) issue(i + NS - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            constexpr int N_LATER = LPS * (NS - 2);
+            if (i + NS - 1 < n_iter) __builtin_amdgcn_s_waitcnt(0x070 | (N_LATER & 0xF) | (((N_LATER >> 4) & 3) << 14));
+            else __builtin_amdgcn_s_waitcnt(0x070);
+            asm volatile("s_barrier" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(1);
+            products(a, b);
+            __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_barrier" ::: "memory");
+        }
+        if (!trails) asm volatile("s_barrier" ::: "memory");
+    } else {
         for (int i = 0; i < n_iter; ++i) {
             wait_stage(i, Behind1{});
             // the operand reads of this stage go first (x, then w in the order the products want
@@ -414,28 +449,25 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 
 // Shape of the block: 3 = 256 features x 128 tokens (4 waves, ring of 3, two blocks per compute unit),
 // 7 = 192 x 128 and 8 = 128 x 128 (the same with fewer features), 10 = 256 x 256 (8 waves, ring of 4, one
-// block per compute unit), 6 = 128 x 256 (the same with fewer features); 0 = chosen here, together
-// with the number of K-splits.  The entry points whose names end in _ex take either from the caller, for
-// tests and measurements.
+// block per compute unit), 11 = 224 x 256, 12 = 192 x 256 and 6 = 128 x 256 (the same with fewer features; 6 on
+// request only); 0 = chosen here, together with the number of K-splits.  The entry points whose names end in
+// _ex take either from the caller, for tests and measurements.
 //
-// What a shape costs follows from what bounds the kernel, the copies into LDS: a compute unit takes
-// about 0.1 us per k-step and round of resident blocks plus 17.5 ns per KB that its blocks copy
-// (57 GB/s per unit, whatever the shape and however many blocks share the unit).  So the time of a
-// product is that of the units' load, taken half from the mean and half from the unit with the
-// most blocks; splitting K adds the parts' way to memory and back and the kernel that sums them.
-// A 256 x 256 block copies a third less per product and is bound by the matrix cores as much as by
-// the copies: 0.80 us per k-step, and 8 us per block that nothing overlaps (0.73 and 2 where K is
-// split and the grid gives no unit a second block: such blocks store plain partial sums; with K whole
-// the epilogue is a rotation, an addition to the residual stream or an activation, and the same
-// price for it made the joined q/k/v product of 2,048 rows 130 us instead of 118).  It wins where its few blocks still load the units evenly (large
-// products: 10 to 20 % at the 24B feed-forward, 12 to 15 % at 7B o/down and 4,096 rows, the 7B down
-// product at 300 to 2,048 rows with K in parts).
-// Against every shape and number of parts measured (7B and 24B q/k/v, o, gate/up and down at 14 row
-// counts from 128 to 4,096, cold weights, parts of K 1 to 6 and 8) the formula's picks take 1.1 % more time
-// than the best in total, 2.4 % per product on average and 38 % at worst (o at 384, 768 and 1,536 rows, where
-// a split or a smaller block would do better than it predicts).
+// What a shape costs.  Four waves, two blocks per unit: bound by the copies into LDS, 0.056 us per k-step and
+// round of resident blocks plus 17.7 ns per KB that a unit's blocks copy, 0.6 of it from the mean and 0.4
+// from the unit with the most blocks.  Eight waves, one block after the other: bound by the matrix cores and
+// by the wait for weights from HBM, 0.25 us + 1.6 ns per feature and k-step, and 3.7 us per block that nothing
+// overlaps.  Splitting K adds the parts' way to memory and back and the kernel that sums them.  What decides
+// between 256, 224 and 192 features is how evenly the blocks fill the rounds: gate/up of 2,048 rows, 28672
+// features, is 3.5 rounds of 256 (422 us with its activation) and 4 of 224 (408; 512 with 4 waves before those
+// of a pair took turns), q/k/v of 2,048 rows, 6144 features, 0.75 rounds of 256 (108 us with its rotation) and 1
+// of 192 (102; 115 with 256 x 128).
+// Against every shape and number of parts measured (products of 7B, 12B and 24B sizes at 11 row counts from 128
+// to 4,001, cold weights, parts of K 1 to 4 and 6; 110 products, 2,400 timings) the formula's picks take 2.0 % more
+// time than the best on average and 22 % at worst (5120 x 4096 at 384 rows, 44 us against 37); against the
+// shapes with their real epilogues (42 products) 1.2 % and 17 %.
 struct TileShape { int variant, features, tokens, per_unit; };
-static const TileShape g_shapes[] = {{3, 256, 128, 2}, {7, 192, 128, 2}, {8, 128, 128, 2}, {10, 256, 256, 1}, {6, 128, 256, 1}};
+static const TileShape g_shapes[] = {{3, 256, 128, 2}, {7, 192, 128, 2}, {8, 128, 128, 2}, {10, 256, 256, 1}, {11, 224, 256, 1}, {12, 192, 256, 1}, {6, 128, 256, 1}};
 static const TileShape& tile_shape(int variant) {
     for (const TileShape& t : g_shapes)
         if (t.variant == variant) return t;
@@ -452,10 +484,8 @@ static float tiled_cost(const TileShape& t, int splits, int M, int N, int K) {
     const float mean = blocks > units ? (float)blocks / units : 1.f;
     const float kb = (t.features + t.tokens) * 64 / 1024.f;            // copied per block and k-step
     float us;
-    // eight waves, a unit to itself, one block after the other; a grid of parts of K that gives no
-    // unit a second block measures shorter (the long K of a down product at 300 to 1,500 rows)
-    if (t.variant == 10) us = most == 1 && splits > 1 ? steps * 0.73f + 2.f + 3.f : most * (steps * 0.80f + 8.f) + 3.f;
-    else us = steps * (0.10f * rounds + 0.0175f * kb * 0.5f * (mean + most)) + 3.f;
+    if (t.per_unit == 1) us = most * (steps * (0.247f + 0.0016f * t.features) + 3.65f) + (most == 1 && splits > 1 ? -0.2f : 0.57f);
+    else us = steps * (0.056f * rounds + 0.0177f * kb * (0.6f * mean + 0.4f * most)) + 2.33f;
     if (splits > 1) us += 3.f + (float)M * N * 4.f * (2 * splits + 1) / 4.5e6f;
     return us;
 }
@@ -471,7 +501,7 @@ static TilePlan tiled_plan(int M, int N, int K, bool may_split, int forced_varia
     } else if (may_split) {
         float best_us = 0.f;
         for (const TileShape& t : g_shapes) {
-            if (t.variant == 6) continue;                              // (128 x 256 only on request)
+            if (t.variant == 6) continue;                              // (128 x 256 only on request: never the fastest by more than 4 %)
             // (any number of parts up to 6, or 8: three fill two rounds where four start a third; 7 and more
             // than 8 measured worse than the formula says, their partial sums no longer stay in the caches)
             for (int s = 1; s <= 8 && (s == 1 || steps / s >= 8); s += (s == 6 ? 2 : 1)) {
@@ -505,6 +535,8 @@ static void launch_tiled(int variant, int splits, hipStream_t stream, const bf16
         case 6: launch_async<4, 4, 4, 4, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
         case 7: launch_async<6, 4, 2, 3, 2, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
         case 8: launch_async<4, 4, 2, 3, 2, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
+        case 11: launch_async<7, 4, 4, 4, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
+        case 12: launch_async<6, 4, 4, 4, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
         case 10: launch_async<8, 4, 4, 4, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
         default: launch_async<8, 4, 2, 3, 2, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
     }
@@ -538,7 +570,7 @@ static int tiled_entry(const void* x, const void* w_packed, void* out, float* wo
     FL_CHECK(!in_ssq || in_parts > 0, "gemm_tiled: a row scale over %d parts", in_parts);
     if (M == 0) return 0;
     const int n_steps = ceil_div(K, 32);
-    FL_CHECK(tiled_known(variant), "gemm_tiled: block shape %d (0, 3, 6, 7, 8 or 10)", variant);
+    FL_CHECK(tiled_known(variant), "gemm_tiled: block shape %d (0, 3, 6, 7, 8, 10, 11 or 12)", variant);
     const TilePlan plan = tiled_plan(M, N, K, !epilogue, variant, epilogue ? 1 : forced_splits);
     const int splits = plan.splits, v = plan.variant;
     FL_CHECK(splits == 1 || workspace, "gemm_tiled: this shape splits K %d ways and needs a workspace", splits);
@@ -608,7 +640,7 @@ FL_RECORDABLE(fl_gemm_tiled)
 extern "C" int fl_gemm_tiled_residual_ex(const void* x, const void* w_packed, float* workspace, int M, int N, int K,
                                          float* resid, const float* g, void* xg, float* out_ssq, int variant,
                                          hipStream_t stream) {
-    FL_CHECK(tiled_known(variant), "gemm_tiled_residual: block shape %d (0, 3, 6, 7, 8 or 10)", variant);
+    FL_CHECK(tiled_known(variant), "gemm_tiled_residual: block shape %d (0, 3, 6, 7, 8, 10, 11 or 12)", variant);
     FL_CHECK(M >= 0 && N > 0 && K > 0, "gemm_tiled_residual: bad sizes M=%d N=%d K=%d", M, N, K);
     FL_CHECK(K % 8 == 0, "gemm_tiled_residual: K=%d is no multiple of 8 (16-byte loads)", K);
     FL_CHECK(N % 4 == 0, "gemm_tiled_residual: N=%d is no multiple of 4 (16-byte accesses to the residual rows)", N);
@@ -699,7 +731,7 @@ extern "C" int fl_gemm_tiled_rope_ex(const void* x, const void* w_packed, int M,
                                      const int* block_table, int max_blocks, const float* cs, void* q_out,
                                      void* cache_base, int nh, int nkv, int hd, int page_size, int n_pages, int rot,
                                      int write_cache, int variant, hipStream_t stream) {
-    FL_CHECK(tiled_known(variant), "gemm_tiled_rope: block shape %d (0, 3, 6, 7, 8 or 10)", variant);
+    FL_CHECK(tiled_known(variant), "gemm_tiled_rope: block shape %d (0, 3, 6, 7, 8, 10, 11 or 12)", variant);
     FL_CHECK(M >= 0 && N > 0 && K > 0, "gemm_tiled_rope: bad sizes M=%d N=%d K=%d", M, N, K);
     FL_CHECK(K % 8 == 0, "gemm_tiled_rope: K=%d is no multiple of 8 (16-byte loads)", K);
     FL_CHECK(positions && tok_seq && block_table && cs && q_out && cache_base,

@@ -1195,3 +1195,19 @@ def test_gemm_float_gives_the_plain_kernel_s_bits(M, N, K):
     got = torch.full((M, N), float("nan"), dtype=torch.float32, device=DEV)
     ops().gemm_plain(at(0, M, 31), at(0, N, 32), got)
     assert torch.equal(got, want)
+
+
+# ---------------------------------------------------------------- the tiled product's blocks of eight waves
+@pytest.mark.parametrize("variant", [10, 11, 12])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 8), (255, 223, 32), (257, 449, 40), (256, 192, 128), (300, 1000, 104), (512, 700, 4096)])
+def test_gemm_tiled_eight_waves_equal_four(variant, M, N, K):
+    """256, 224 and 192 features x 256 tokens against 256 x 128: every output is the same chain over K, so the same
+    bits; one stage, fewer and more stages than the ring, K's and the tiles' remainders."""
+    from flambeau_amd.kernels.packing import pack_weight
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=41), rnd(N, K, dtype=torch.bfloat16, seed=42, scale=0.05)
+    packed, got = pack_weight(w), []
+    for v in (3, variant):
+        out = torch.full((M, N), float("nan"), dtype=torch.float32, device=DEV)
+        tuned().gemm_tiled(x, packed, out, variant=v, splits=1)
+        got.append(out)
+    assert torch.equal(*got)
