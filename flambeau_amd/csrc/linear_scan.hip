@@ -35,12 +35,24 @@
 // The step's tokens come through LDS a run of RUN tokens at a time, rows 16 * RPT wide and zero behind D;
 // the next run's values are asked for (into registers) before the walk over this run begins and put into
 // LDS after it, so that the trip to memory hides behind the walk.
+//
+// What bounds it are the vector operations of a token, 25 to 45 of them and their addressing at four clocks each (a
+// wave has its SIMD to itself; sixteen waves with a column each, the sums over 64 lanes, took as long: 285 us fixed,
+// 580 delta).  So a token's values are read from LDS into registers while the token before is worked on, the sums over
+// lanes of four tokens' outputs are formed together, and the 16 lanes of a column, which all hold a token's sum,
+// keep one of 16 tokens' outputs each and store them at once.  WHOLE: 16 RPT key dims, a multiple of 16 columns, rows
+// and records in whole 16-byte pieces: loads without conditions, four values at a time (rows behind the request's
+// last are its last again).
+// 2,048 tokens, heads of 128 x 128 (in brackets a token's reads, chain and store one after the other): delta rule, 32
+// heads, 409 us (527); fixed decay, 16 heads, 307 (422); gated, 32 heads, 337 (509); forget gates, 32 heads, 342 (510);
+// delta rule with a decay per key dim 417 (601); written, 32 heads of 128 x 64, 340 (438).  The bits are the same.
+//
 // MODE 0: a decay per head or per token and head, u = v; 1: the delta rule; 2: a decay per token, head AND key dim
 // (`k` holds the forget gates f; the key is 1 - f: what is forgotten makes room for what is written); 3: the delta rule
 // with a decay per token, head and key dim (`chan_decay`, rows ldc wide, heads x D: S <- diag(g) S before the correction);
 // 4: such a decay without the correction (gated linear attention: u = v); 5: a decay and a write strength per token and
 // head without the correction (u = beta v), and skip[head] v added to what is read out
-template <int RPT, int MODE>
+template <int RPT, int MODE, bool WHOLE>
 __global__ __launch_bounds__(LS_GROUP * LS_COLS) void linear_scan_kernel(
     const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk, const float* __restrict__ v, int ldv,
     const float* __restrict__ head_decay, const float* __restrict__ tok_decay, const float* __restrict__ beta, int ldg,
@@ -51,44 +63,64 @@ __global__ __launch_bounds__(LS_GROUP * LS_COLS) void linear_scan_kernel(
     constexpr int NT = LS_GROUP * LS_COLS;
     constexpr int DP = LS_GROUP * RPT;                                // a row of q or k in LDS
     constexpr int RUN = RPT <= 8 ? 32 : RPT <= 16 ? 16 : 8;          // tokens per run
-    constexpr int PRE = RUN * DP / NT;                                // q (and k) values of a run per thread
+    constexpr int VEC = WHOLE ? 4 : 1;                               // values per load
+    constexpr int PRE = RUN * DP / NT / VEC;                          // loads of q (and k) of a run per thread
     constexpr int PRE_V = (RUN * LS_COLS + NT - 1) / NT;
+    using V = std::conditional_t<WHOLE, f32x4, float>;
     const int g = threadIdx.x & (LS_GROUP - 1), c = threadIdx.x / LS_GROUP;
     const int j = blockIdx.x * LS_COLS + c, head = blockIdx.y, s = blockIdx.z;
     const int qk_head = head / (H / G);
-    const bool live = j < Dv;
+    const bool live = WHOLE || j < Dv;
     const int start = seq_q_start[s], len = seq_q_len[s];
     float* st = state + (size_t)seq_slots[s] * slot_stride + (size_t)head * D * Dv;
     float S[RPT];
+    if constexpr (WHOLE) {
 #pragma unroll
-    for (int u = 0; u < RPT; ++u) {
-        const int d = g * RPT + u;
-        S[u] = (live && d < D) ? st[(size_t)j * D + d] : 0.f;
+        for (int u = 0; u < RPT; u += 4) {
+            const f32x4 four = *(const f32x4*)(st + (size_t)j * D + g * RPT + u);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[u + r] = four[r];
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            const int d = g * RPT + u;
+            S[u] = (live && d < D) ? st[(size_t)j * D + d] : 0.f;
+        }
     }
     const float fixed = head_decay ? head_decay[head] : 1.f;
     const float skip_h = MODE == 5 && skip ? skip[head] : 0.f;
     __shared__ __attribute__((aligned(16))) float qs[RUN * DP];
     __shared__ __attribute__((aligned(16))) float ks[RUN * DP];
-    __shared__ float vs[RUN * LS_COLS], fs[RUN * 2];
+    __shared__ __attribute__((aligned(16))) float vs[RUN * LS_COLS], fs[RUN * 2];
     __shared__ __attribute__((aligned(16))) float gs[CHAN ? RUN * DP : 4];
-    float pq[PRE], pk[PRE], pd[CHAN ? PRE : 1], pv[PRE_V], pf0 = 0.f, pf1 = 0.f;
+    V pq[PRE], pk[PRE], pd[CHAN ? PRE : 1];
+    float pv[PRE_V], pf0 = 0.f, pf1 = 0.f;
     auto fetch = [&](int t0) {                     // the values of the run that starts at token t0, into registers
         const int cnt = min(RUN, len - t0);
 #pragma unroll
         for (int i = 0; i < PRE; ++i) {
-            const int e = threadIdx.x + NT * i;
+            const int e = (threadIdx.x + NT * i) * VEC;
             const int tt = e / DP, d = e % DP;
-            const bool in = tt < cnt && d < D;
-            const size_t row = (size_t)(start + t0 + (in ? tt : 0));
-            pq[i] = in ? q[row * ldq + qk_head * D + d] : 0.f;
-            pk[i] = in ? k[row * ldk + qk_head * D + d] : (MODE == 2 ? 1.f : 0.f);
-            if (CHAN) pd[i] = in ? chan_decay[row * ldc + head * D + d] : 1.f;
+            if constexpr (WHOLE) {
+                const size_t row = (size_t)(start + t0 + min(tt, cnt - 1));
+                pq[i] = *(const f32x4*)(q + row * ldq + qk_head * D + d);
+                pk[i] = *(const f32x4*)(k + row * ldk + qk_head * D + d);
+                if (CHAN) pd[i] = *(const f32x4*)(chan_decay + row * ldc + head * D + d);
+            } else {
+                const bool in = tt < cnt && d < D;
+                const size_t row = (size_t)(start + t0 + (in ? tt : 0));
+                pq[i] = in ? q[row * ldq + qk_head * D + d] : 0.f;
+                pk[i] = in ? k[row * ldk + qk_head * D + d] : (MODE == 2 ? 1.f : 0.f);
+                if (CHAN) pd[i] = in ? chan_decay[row * ldc + head * D + d] : 1.f;
+            }
         }
 #pragma unroll
         for (int i = 0; i < PRE_V; ++i) {
             const int e = threadIdx.x + NT * i;
             const int tt = e / LS_COLS, jj = blockIdx.x * LS_COLS + (e - tt * LS_COLS);
-            pv[i] = (tt < cnt && jj < Dv) ? v[(size_t)(start + t0 + tt) * ldv + head * Dv + jj] : 0.f;
+            if constexpr (WHOLE) pv[i] = v[(size_t)(start + t0 + min(tt, cnt - 1)) * ldv + head * Dv + jj];
+            else pv[i] = (tt < cnt && jj < Dv) ? v[(size_t)(start + t0 + tt) * ldv + head * Dv + jj] : 0.f;
         }
         if (threadIdx.x < cnt) {
             const size_t row = (size_t)(start + t0 + threadIdx.x);
@@ -96,15 +128,76 @@ __global__ __launch_bounds__(LS_GROUP * LS_COLS) void linear_scan_kernel(
             pf1 = (MODE == 1 || MODE == 3 || MODE == 5) ? beta[row * ldg + head] : 1.f;
         }
     };
+    // Where a thread's row u lies in an LDS row: its pieces of four 16 threads apart, so that the 16 threads of a
+    // column read 256 neighbouring bytes at a time (a thread's rows side by side: two threads on every bank, and LDS,
+    // which the four waves of a block keep busy half of the time, decides)
+    auto place = [](int thread, int u) { return RPT % 4 == 0 ? (u >> 2) * (4 * LS_GROUP) + 4 * thread + (u & 3) : thread * RPT + u; };
+    struct Token {                                 // what a thread needs of a token
+        float k[RPT], q[RPT], g[CHAN ? RPT : 1], decay, beta, v;
+    };
+    auto read = [&](int tt, Token& t) {
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            t.k[u] = ks[tt * DP + place(g, u)];
+            t.q[u] = qs[tt * DP + place(g, u)];
+            if (CHAN) t.g[u] = gs[tt * DP + place(g, u)];
+        }
+        t.v = vs[tt * LS_COLS + c];
+        t.decay = fs[2 * tt];
+        t.beta = fs[2 * tt + 1];
+    };
+    auto advance = [&](Token& t) {                 // one token of the recurrence; returns this lane's share of what is read out
+        float uv = t.v;
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            if (MODE == 2) {
+                S[u] *= t.k[u];
+                t.k[u] = 1.0f - t.k[u];
+            } else if (CHAN) {
+                S[u] *= t.g[u];
+            } else {
+                S[u] *= t.decay;
+            }
+        }
+        if (MODE == 1 || MODE == 3) {
+            float seen0 = 0.f, seen1 = 0.f;                       // two chains of half the length
+#pragma unroll
+            for (int u = 0; u < RPT; u += 2) {
+                seen0 = fmaf(S[u], t.k[u], seen0);
+                if (u + 1 < RPT) seen1 = fmaf(S[u + 1], t.k[u + 1], seen1);
+            }
+            uv = t.beta * (uv - row_sum16(seen0 + seen1));
+        }
+        if (MODE == 5) uv *= t.beta;
+        float num0 = 0.f, num1 = 0.f;
+#pragma unroll
+        for (int u = 0; u < RPT; u += 2) {
+            S[u] = fmaf(t.k[u], uv, S[u]);
+            num0 = fmaf(S[u], t.q[u], num0);
+            if (u + 1 < RPT) {
+                S[u + 1] = fmaf(t.k[u + 1], uv, S[u + 1]);
+                num1 = fmaf(S[u + 1], t.q[u + 1], num1);
+            }
+        }
+        return num0 + num1;
+    };
+    auto finish = [&](float share, float v) {      // the 16 threads of a column are a row of lanes
+        float num = row_sum16(share);
+        if (MODE == 4) num *= o_scale;
+        if (MODE == 5 && skip) num = fmaf(skip_h, v, num);
+        return num;
+    };
     if (len > 0) fetch(0);
     for (int t0 = 0; t0 < len; t0 += RUN) {
         const int cnt = min(RUN, len - t0);
         __syncthreads();                           // the walk over the run before has read its last value
 #pragma unroll
         for (int i = 0; i < PRE; ++i) {
-            qs[threadIdx.x + NT * i] = pq[i];
-            ks[threadIdx.x + NT * i] = pk[i];
-            if (CHAN) gs[threadIdx.x + NT * i] = pd[i];
+            const int e = (threadIdx.x + NT * i) * VEC, d = e % DP;
+            const int at = e - d + place(d / RPT, d % RPT);
+            *(V*)&qs[at] = pq[i];
+            *(V*)&ks[at] = pk[i];
+            if (CHAN) *(V*)&gs[at] = pd[i];
         }
 #pragma unroll
         for (int i = 0; i < PRE_V; ++i)
@@ -112,54 +205,49 @@ __global__ __launch_bounds__(LS_GROUP * LS_COLS) void linear_scan_kernel(
         if (threadIdx.x < RUN) { fs[2 * threadIdx.x] = pf0; fs[2 * threadIdx.x + 1] = pf1; }
         __syncthreads();
         if (t0 + RUN < len) fetch(t0 + RUN);
-#pragma unroll 2
-        for (int tt = 0; tt < cnt; ++tt) {
-            const float decay = fs[2 * tt];
-            float uv = vs[tt * LS_COLS + c];
-            float kr[RPT], qr[RPT];
-#pragma unroll
-            for (int u = 0; u < RPT; ++u) {
-                kr[u] = ks[tt * DP + g * RPT + u];
-                qr[u] = qs[tt * DP + g * RPT + u];
-                if (MODE == 2) {
-                    S[u] *= kr[u];
-                    kr[u] = 1.0f - kr[u];
-                } else if (CHAN) {
-                    S[u] *= gs[tt * DP + g * RPT + u];
-                } else {
-                    S[u] *= decay;
-                }
+        Token even, odd;
+        if (RPT <= 16) read(0, even);
+        float kept = 0.f;                          // the output of this lane's token of the 16
+        float* orow = out + ((size_t)(start + t0 + g) * H + head) * Dv + j;
+        // (reads stay where they are written, ahead of the token before; the sums over lanes of four tokens go together)
+        int tt = 0;
+        for (; RPT <= 16 && tt + 4 <= cnt; tt += 4) {
+            read(tt + 1, odd);
+            __builtin_amdgcn_sched_barrier(1);
+            const float v0 = even.v, v1 = odd.v, s0 = advance(even);
+            read(tt + 2, even);
+            __builtin_amdgcn_sched_barrier(1);
+            const float s1 = advance(odd);
+            read(tt + 3, odd);
+            __builtin_amdgcn_sched_barrier(1);
+            const float v2 = even.v, v3 = odd.v, s2 = advance(even);
+            read(min(tt + 4, RUN - 1), even);
+            __builtin_amdgcn_sched_barrier(1);
+            const float s3 = advance(odd);
+            const float n0 = finish(s0, v0), n1 = finish(s1, v1), n2 = finish(s2, v2), n3 = finish(s3, v3);
+            const int mine = g - (tt & 15);
+            kept = mine == 0 ? n0 : mine == 1 ? n1 : mine == 2 ? n2 : mine == 3 ? n3 : kept;
+            if ((tt & 15) == 12 || tt + 8 > cnt) {                    // 16 tokens, or the run's last four
+                const int t16 = tt & ~15;
+                if (live && t16 + g < tt + 4) orow[(size_t)t16 * H * Dv] = kept;
             }
-            if (MODE == 1 || MODE == 3) {
-                float seen0 = 0.f, seen1 = 0.f;                   // two chains of half the length
-#pragma unroll
-                for (int u = 0; u < RPT; u += 2) {
-                    seen0 = fmaf(S[u], kr[u], seen0);
-                    if (u + 1 < RPT) seen1 = fmaf(S[u + 1], kr[u + 1], seen1);
-                }
-                uv = fs[2 * tt + 1] * (uv - row_sum16(seen0 + seen1));
-            }
-            if (MODE == 5) uv *= fs[2 * tt + 1];
-            float num0 = 0.f, num1 = 0.f;
-#pragma unroll
-            for (int u = 0; u < RPT; u += 2) {
-                S[u] = fmaf(kr[u], uv, S[u]);
-                num0 = fmaf(S[u], qr[u], num0);
-                if (u + 1 < RPT) {
-                    S[u + 1] = fmaf(kr[u + 1], uv, S[u + 1]);
-                    num1 = fmaf(S[u + 1], qr[u + 1], num1);
-                }
-            }
-            float num = row_sum16(num0 + num1);                   // the 16 threads of a column are a row of lanes
-            if (MODE == 4) num *= o_scale;
-            if (MODE == 5 && skip) num = fmaf(skip_h, vs[tt * LS_COLS + c], num);
-            if (live && g == 0) out[((size_t)(start + t0 + tt) * H + head) * Dv + j] = num;
+        }
+        for (; tt < cnt; ++tt) {                   // the last one to three of a request (heads beyond 256: all, two tokens of them do not fit the registers)
+            if (RPT > 16) read(tt, even);
+            const float v = even.v, num = finish(advance(even), v);
+            if (live && g == 0) orow[(size_t)tt * H * Dv] = num;
+            if (RPT <= 16) read(min(tt + 1, RUN - 1), even);
         }
     }
+    if constexpr (WHOLE) {
 #pragma unroll
-    for (int u = 0; u < RPT; ++u) {
-        const int d = g * RPT + u;
-        if (live && d < D) st[(size_t)j * D + d] = S[u];
+        for (int u = 0; u < RPT; u += 4) *(f32x4*)(st + (size_t)j * D + g * RPT + u) = (f32x4){S[u], S[u + 1], S[u + 2], S[u + 3]};
+    } else {
+#pragma unroll
+        for (int u = 0; u < RPT; ++u) {
+            const int d = g * RPT + u;
+            if (live && d < D) st[(size_t)j * D + d] = S[u];
+        }
     }
 }
 
@@ -184,10 +272,21 @@ static int linear_scan_launch(const float* q, int ldq, const float* k, int ldk, 
     FL_CHECK(n_seqs <= 65535 && H <= 65535, "linear_scan: %d requests of %d heads are more than one grid takes", n_seqs, H);
     dim3 grid(ceil_div(Dv, LS_COLS), H, n_seqs);
     const int rpt = ceil_div(D, LS_GROUP);
-#define FL_LS2(R, MODE)                                                                                               \
-    linear_scan_kernel<R, MODE><<<grid, LS_GROUP * LS_COLS, 0, stream>>>(q, ldq, k, ldk, v, ldv, head_decay, tok_decay, beta, \
+    // rows of q, k and decays, and every head's state, in whole 16-byte pieces that fill a thread's rows
+    const auto pieces = [](const float* p, int ld) { return (uintptr_t)p % 16 == 0 && ld % 4 == 0; };
+    const bool whole = (D == 64 || D == 128 || D == 256) && Dv % LS_COLS == 0 && pieces(q, ldq) && pieces(k, ldk) &&
+                       (!chan_decay || pieces(chan_decay, ldc)) && (uintptr_t)state % 16 == 0 && slot_stride % 4 == 0;
+#define FL_LS3(R, MODE, W)                                                                                             \
+    linear_scan_kernel<R, MODE, W><<<grid, LS_GROUP * LS_COLS, 0, stream>>>(q, ldq, k, ldk, v, ldv, head_decay, tok_decay, beta, \
                                                                           ldg, state, (size_t)slot_stride, seq_q_start,        \
                                                                           seq_q_len, seq_slots, out, H, G, D, Dv, chan_decay, ldc, o_scale, skip)
+#define FL_LS2(R, MODE)                                  \
+    do {                                                 \
+        if constexpr (R == 4 || R == 8 || R == 16) {     \
+            if (whole) { FL_LS3(R, MODE, true); break; } \
+        }                                                \
+        FL_LS3(R, MODE, false);                          \
+    } while (0)
 #define FL_LS(R)             \
     do {                     \
         if (chan_decay && corrects) FL_LS2(R, 3); \
@@ -205,6 +304,7 @@ static int linear_scan_launch(const float* q, int ldq, const float* k, int ldk, 
     else FL_LS(LS_MAX_ROWS);
 #undef FL_LS
 #undef FL_LS2
+#undef FL_LS3
     FL_LAUNCH_CHECK();
     return 0;
 }

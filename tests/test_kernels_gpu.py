@@ -1211,3 +1211,41 @@ def test_gemm_tiled_eight_waves_equal_four(variant, M, N, K):
         tuned().gemm_tiled(x, packed, out, variant=v, splits=1)
         got.append(out)
     assert torch.equal(*got)
+
+
+# ---------------------------------------------------------------- the walk of the linear recurrences
+@pytest.mark.parametrize("mode", ["fixed", "delta", "forget", "delta_per_dim", "gated", "written"])
+@pytest.mark.parametrize("D,Dv", [(64, 16), (128, 48), (256, 32)])
+def test_linear_scan_in_whole_pieces_gives_the_same_bits(mode, D, Dv):
+    """Rows that are no whole 16-byte pieces go the general way, one value at a time: equal outputs and states, for
+    requests whose tokens end anywhere in a group of four, of 16 and in a run."""
+    from types import SimpleNamespace
+    H, lens = 2, [1, 3, 4, 7, 16, 18, 31, 32, 33, 70]
+    G = 2 if mode == "forget" else 1
+    n, S = sum(lens), len(lens)
+    ints = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    starts, slots = ints([sum(lens[:i]) for i in range(S)]), ints(list(range(S))[::-1])
+    step = SimpleNamespace(seq_q_start=starts, seq_q_len=ints(lens), seq_slots=slots)
+    v, gates, decay = rnd(n, H * Dv, seed=52), torch.sigmoid(rnd(n, 2 * H, seed=53)), torch.sigmoid(rnd(n, H * D, seed=54) + 2)
+    first, got = rnd(S, H * D * Dv, seed=55), []
+    for pad in (4, 3):                             # rows a multiple of four floats apart, and not
+        q, k = (torch.empty(n, G * D + pad, dtype=torch.float32, device=DEV)[:, :G * D] for _ in range(2))
+        q.copy_(rnd(n, G * D, seed=50))
+        k.copy_(torch.sigmoid(rnd(n, G * D, seed=51)) if mode == "forget" else torch.nn.functional.normalize(rnd(n, G * D, seed=51), dim=1))
+        state, out = first.clone(), torch.full((n, H * Dv), float("nan"), dtype=torch.float32, device=DEV)
+        where = (state, starts, step.seq_q_len, slots, out, H, G, D, Dv)
+        if mode == "fixed":
+            ops().linear_scan(q, k, v, *where, head_decay=torch.tensor([0.97, 0.5], device=DEV))
+        elif mode == "delta":
+            ops().linear_scan(q, k, v, *where, token_gates=gates)
+        elif mode == "forget":
+            ops().linear_scan(q, k, v, *where, channel_decay=True)
+        elif mode == "delta_per_dim":
+            ops().linear_scan(q, k, v, *where, token_gates=gates, key_decay=decay)
+        elif mode == "gated":
+            ops().linear_scan_gated(q, k, v, decay, state, step, out, H, G, D, Dv, out_scale=0.3)
+        else:
+            ops().linear_scan_written(q, k, v, gates, torch.tensor([0.7, -1.5], device=DEV), state, step, out, H, G, D, Dv)
+        got.append((out, state))
+    assert not got[0][0].isnan().any()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
