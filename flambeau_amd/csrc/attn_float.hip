@@ -1,0 +1,210 @@
+// Attention over the paged cache for the 32-bit path: floats in, floats out, every product on the matrix cores
+// (v_mfma_f32_16x16x4_f32), precise expf.  The same result, to the bit, whatever tokens run beside a token.
+//
+// What a (token, query head) is: its keys in blocks of 64 counted from position 0.  A block's scores (four sums of a
+// quarter of the head dims each, added in pairs), their maximum m, the weights e^(score - m), their sum l and the
+// weighted sum of the values in rising order of the keys; then (M, L, A) over the blocks in rising order,
+//     M' = max(M, m),  L <- L e^(M - M') + l e^(m - M'),  A <- A e^(M - M') + a e^(m - M').
+// Keys outside the row's range weigh nothing (their scores are not looked at), and a block without a key of the row
+// leaves (M, L, A) as it is.  So neither the rows of a tile, nor how a prompt is cut, nor who forms a block shows.
+//
+// Block of threads = a tile of up to 16 rows (token, query head) that read one key/value head: T tokens by its query
+// heads (T = 1 in steps of few tokens, where the heads alone have to fill the chip).  Eight waves form eight blocks of
+// keys at a time and leave (m, l, a) in LDS, where all threads add them in order, four head dims of a row each.  A tile
+// whose tokens belong to several requests takes them one after the other.
+// No operand passes through LDS.  Scores are computed transposed, S^T = K Q^T, so that a lane holds scores of one row:
+// instruction (c, e) takes head dims 16 c + 4 g + e of lane group g = lane / 16, four neighbouring dims of a row being one
+// 16-byte load for four instructions.  S^T leaves lane (g, row) with keys 16 t + 4 g + r, which is just what it has to
+// give as an operand of O^T = V^T P^T if instruction (t, r) takes those keys, and the values of four neighbouring keys
+// are 16 bytes of the transposed page.
+//
+// Bound by the chain look-up of the page, loads, 256 matrix instructions of 32 clocks, adding up.  32 heads of 128 over 8:
+// a prompt of 333 tokens 59 us (553 with attn_plain_kernel, a block per token and head that goes through its keys one by
+// one), one token behind 340 24 us (161).
+#include "attn_float.h"
+
+#define AF_WAVES 8
+#define AF_ROWS 16
+#define AF_KEYS 64
+
+template <int HD>
+__global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const float* __restrict__ q, float* __restrict__ out,
+                                                                      PagedCache cache, const int* __restrict__ positions,
+                                                                      const int* __restrict__ tok_seq,
+                                                                      const int* __restrict__ block_table, int max_blocks, int n,
+                                                                      int nh, int tokens, int heads, int head_tiles, float scale,
+                                                                      int window, float softcap, const float* __restrict__ sink) {
+    constexpr int NC = HD / 16, LD = HD + 4, FOURS = HD / 4;
+    constexpr int MINE = AF_ROWS * FOURS / (64 * AF_WAVES);           // groups of four dims a thread adds up
+    static_assert(AF_ROWS * FOURS % (64 * AF_WAVES) == 0 || AF_ROWS * FOURS < 64 * AF_WAVES, "rows must divide among the threads");
+    constexpr int SUMS = MINE > 0 ? MINE : 1;
+    __shared__ __attribute__((aligned(16))) float part_a[AF_WAVES][AF_ROWS][LD];
+    __shared__ float part_m[AF_WAVES][AF_ROWS], part_l[AF_WAVES][AF_ROWS];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, g = lane >> 4;
+    const int kvh = blockIdx.y / head_tiles, group = nh / cache.n_kv_heads;
+    const int h0 = (blockIdx.y % head_tiles) * heads;                 // first query head of the tile within the group
+    const int tok0 = blockIdx.x * tokens, n_tok = min(tokens, n - tok0);
+    const int n_heads = min(heads, group - h0);
+    // row j: token j / heads, query head j % heads of the tile
+    const int my_tok = j / heads, my_head = j % heads;
+    const bool my_row = my_tok < n_tok && my_head < n_heads;
+    const int at_tok = tok0 + min(my_tok, n_tok - 1), at_head = kvh * group + h0 + min(my_head, n_heads - 1);
+    const int my_p = positions[at_tok], my_lo = window > 0 ? max(0, my_p - window + 1) : 0;
+    f32x4 qv[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) qv[c] = *(const f32x4*)(q + ((size_t)at_tok * nh + at_head) * HD + 16 * c + 4 * g);
+    // what this thread adds up: row a_row[u], head dims a_d[u] ..+ 3
+    float M[SUMS], L[SUMS];
+    f32x4 A[SUMS];
+#pragma unroll
+    for (int u = 0; u < SUMS; ++u) {
+        M[u] = -INFINITY;
+        L[u] = 0.f;
+        A[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+    const size_t block = (size_t)cache.page_size * HD;                // floats of a (page, K or V, head)
+    for (int from = 0; from < n_tok;) {                               // the tile's tokens, request by request
+        const int seq = tok_seq[tok0 + from];
+        int to = from, p_max = -1, lo_min = 0x7fffffff;
+        for (; to < n_tok && tok_seq[tok0 + to] == seq; ++to) {
+            const int p = positions[tok0 + to];
+            p_max = max(p_max, p);
+            lo_min = min(lo_min, window > 0 ? max(0, p - window + 1) : 0);
+        }
+        const int* table = block_table + (size_t)seq * max_blocks;
+        const bool in_turn = my_row && my_tok >= from && my_tok < to;
+        const int last = p_max / AF_KEYS;
+        for (int b0 = lo_min / AF_KEYS; b0 <= last; b0 += AF_WAVES) {
+            const int b = b0 + wave;
+            if (b <= last) {
+                const int key0 = b * AF_KEYS;
+                // S^T: lane (g, row j) gets the scores of keys key0 + 16 t + 4 g + r
+                f32x4 S[4];
+                bool there[4];                                        // keys 16 t + 4 g .. + 3 have a page (all four or none)
+                const float* vals[4];                                 // their values of head dim 0
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const int key = min(key0 + 16 * t + j, p_max);    // (beyond the last key: that one again, not looked at)
+                    const int page = table[key / cache.page_size];
+                    const int held = page >= 0 && page < cache.n_pages ? page : 0;
+                    const float* kr = (const float*)cache.base + ((size_t)held * 2 * cache.n_kv_heads + kvh) * block +
+                                      (size_t)(key % cache.page_size) * HD;
+                    f32x4 kf[NC];
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) kf[c] = *(const f32x4*)(kr + 16 * c + 4 * g);
+                    const int key4 = key0 + 16 * t + 4 * g;           // (pages hold a multiple of four tokens)
+                    const int page4 = key4 <= p_max ? table[key4 / cache.page_size] : -1;
+                    there[t] = page4 >= 0 && page4 < cache.n_pages;
+                    vals[t] = (const float*)cache.base + ((size_t)(there[t] ? page4 : 0) * 2 * cache.n_kv_heads + cache.n_kv_heads + kvh) * block +
+                              (there[t] ? key4 % cache.page_size : 0);
+                    f32x4 sum[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) sum[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int c = 0; c < NC; ++c)
+                            sum[c & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c][e], qv[c][e], sum[c & 3], 0, 0, 0);
+                    S[t] = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+                }
+                float m = -INFINITY;
+                bool seen[4][4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int key = key0 + 16 * t + 4 * g + r;
+                        seen[t][r] = in_turn && there[t] && key >= my_lo && key <= my_p;
+                        float s = S[t][r] * scale;
+                        if (softcap > 0.f) s = softcap * tanhf(s / softcap);          // scores capped smoothly at +-softcap
+                        S[t][r] = s;
+                        if (seen[t][r]) m = fmaxf(m, s);
+                    }
+                m = fmaxf(m, __shfl_xor(m, 16, 64));
+                m = fmaxf(m, __shfl_xor(m, 32, 64));
+                float l = 0.f;
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        S[t][r] = seen[t][r] ? expf(S[t][r] - m) : 0.f;
+                        l += S[t][r];
+                    }
+                l += __shfl_xor(l, 16, 64);
+                l += __shfl_xor(l, 32, 64);
+                // O^T: keys in rising order of (t, r), values of keys that are not the request's set to zero
+#pragma unroll
+                for (int d0 = 0; d0 < HD; d0 += 16) {
+                    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+                    f32x4 vf[4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) vf[t] = *(const f32x4*)(vals[t] + (size_t)(d0 + j) * cache.page_size);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const int key = key0 + 16 * t + 4 * g + r;
+                            const float val = there[t] && key >= lo_min && key <= p_max ? vf[t][r] : 0.f;
+                            o = __builtin_amdgcn_mfma_f32_16x16x4f32(val, S[t][r], o, 0, 0, 0);
+                        }
+                    *(f32x4*)&part_a[wave][j][d0 + 4 * g] = o;
+                }
+                if (g == 0) {
+                    part_m[wave][j] = m;
+                    part_l[wave][j] = l;
+                }
+            }
+            __syncthreads();
+            const int blocks = min(AF_WAVES, last - b0 + 1);
+#pragma unroll
+            for (int u = 0; u < SUMS; ++u) {
+                const int e = threadIdx.x + 64 * AF_WAVES * u, row = e / FOURS, d = 4 * (e % FOURS);
+                if (row < AF_ROWS && row / heads >= from && row / heads < to) {
+                    for (int w = 0; w < blocks; ++w) {
+                        const float m = part_m[w][row];
+                        if (m == -INFINITY) continue;                 // no key of this row in the block
+                        const float top = fmaxf(M[u], m), old = expf(M[u] - top), now = expf(m - top);
+                        const f32x4 a = *(const f32x4*)&part_a[w][row][d];
+                        L[u] = L[u] * old + part_l[w][row] * now;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) A[u][r] = A[u][r] * old + a[r] * now;
+                        M[u] = top;
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        from = to;
+    }
+#pragma unroll
+    for (int u = 0; u < SUMS; ++u) {
+        const int e = threadIdx.x + 64 * AF_WAVES * u, row = e / FOURS, d = 4 * (e % FOURS);
+        const int tok = row / heads, hh = row % heads;
+        if (row >= AF_ROWS || tok >= n_tok || hh >= n_heads) continue;
+        const int head = kvh * group + h0 + hh;
+        const float inv = sink ? softmax_factor_with_sink(M[u], L[u], sink[head]) : L[u] > 0.f ? 1.0f / L[u] : 0.f;
+        f32x4 o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = A[u][r] * inv;
+        *(f32x4*)(out + ((size_t)(tok0 + tok) * nh + head) * HD + d) = o;
+    }
+}
+
+bool attn_float_takes(const void* q, const void* out, const void* cache_base, int hd, int page_size) {
+    return (hd == 64 || hd == 128) && page_size % 4 == 0 && (((uintptr_t)q | (uintptr_t)out | (uintptr_t)cache_base) % 16) == 0;
+}
+
+void attn_float_launch(const float* q, float* out, const PagedCache& cache, const int* positions, const int* tok_seq,
+                       const int* block_table, int max_blocks, int n, int nh, float scale, int window, float softcap,
+                       const float* sink, hipStream_t stream) {
+    const int group = nh / cache.n_kv_heads, heads = min(group, AF_ROWS), head_tiles = ceil_div(group, heads);
+    // as many tokens as fill the rows, unless a tile per token is at most two per unit (few tokens, most often of as many requests)
+    const int tokens = (long)n * cache.n_kv_heads * head_tiles <= 2 * fl_units() ? 1 : AF_ROWS / heads;
+    const dim3 grid(ceil_div(n, tokens), cache.n_kv_heads * head_tiles);
+    if (cache.head_dim == 64)
+        attn_float_kernel<64><<<grid, 64 * AF_WAVES, 0, stream>>>(q, out, cache, positions, tok_seq, block_table, max_blocks, n, nh,
+                                                                  tokens, heads, head_tiles, scale, window, softcap, sink);
+    else
+        attn_float_kernel<128><<<grid, 64 * AF_WAVES, 0, stream>>>(q, out, cache, positions, tok_seq, block_table, max_blocks, n, nh,
+                                                                   tokens, heads, head_tiles, scale, window, softcap, sink);
+}

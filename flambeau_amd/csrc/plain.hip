@@ -12,6 +12,7 @@
 //   SiLU gate crates/kernels-hip/src/kernels/swiglu_f32_to_f16.cu:21-23
 #include "common.h"
 #include "api.h"
+#include "attn_float.h"
 #include "gemm_float.h"
 #include "recordable.h"
 
@@ -427,6 +428,7 @@ FL_RECORDABLE(fl_rope_kv_write)
 // t in [max(0, p - window + 1), p] of its own request (window 0: from 0), all read from the
 // paged cache (this step's keys were written before).  Four waves take every fourth key with
 // an online softmax each; lanes own the head dims; the four states are merged at the end.
+// (Float heads of 64 and 128 go to attn_float.hip.)
 #define FL_PLAIN_MAX_HD 256
 template <typename T>
 __global__ __launch_bounds__(256) void attn_plain_kernel(
@@ -520,7 +522,9 @@ static int attn_plain_launch(const void* q, void* out, const void* cache_base, i
     if (n == 0) return 0;
     PagedCache c{(void*)cache_base, nkv, page_size, hd, n_pages};
     dim3 grid(n, nh);
-    if (dtype == FL_F32)
+    if (dtype == FL_F32 && attn_float_takes(q, out, cache_base, hd, page_size) && nkv * ceil_div(nh / nkv, 16) <= 65535)
+        attn_float_launch((const float*)q, (float*)out, c, positions, tok_seq, block_table, max_blocks, n, nh, scale, window, softcap, sink, stream);
+    else if (dtype == FL_F32)
         attn_plain_kernel<float><<<grid, 256, 0, stream>>>((const float*)q, (float*)out, c, positions, tok_seq, block_table, max_blocks, nh, scale, window, softcap, sink);
     else if (dtype == FL_BF16)
         attn_plain_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)q, (bf16_t*)out, c, positions, tok_seq, block_table, max_blocks, nh, scale, window, softcap, sink);

@@ -1249,3 +1249,52 @@ def test_linear_scan_in_whole_pieces_gives_the_same_bits(mode, D, Dv):
         got.append((out, state))
     assert not got[0][0].isnan().any()
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+# ---------------------------------------------------------------- the 32-bit attention on the matrix cores
+@pytest.mark.parametrize("cap,sinks", [(0.0, False), (3.0, True)])
+@pytest.mark.parametrize("nh,nkv,hd,ps,window", [(8, 2, 128, 16, 0), (4, 4, 64, 8, 0), (40, 2, 64, 4, 37), (3, 1, 128, 32, 100), (6, 2, 64, 64, 64)])
+def test_attn_float_rows_do_not_depend_on_their_neighbours(nh, nkv, hd, ps, window, cap, sinks):
+    """Requests of one token to several blocks of 64 keys, many rows (tiles of several tokens and requests) against each
+    row alone, bit for bit, and against the formula in 64 bits; pages in front of the window given back, what lies behind a
+    request's last token and in pages of nobody NaN."""
+    seqs = [(300, 300), (70, 70), (33, 1), (200, 9), (1, 1), (640, 3), (64, 64), (65, 1), (449, 130)]
+    case = build_attention_case(torch.float32, nh, nkv, hd, ps, seqs, seed=4)
+    pool, table = case["cache"].pool, case["table"].cpu()
+    held = set()
+    for s, (c, ql) in enumerate(seqs):
+        if window:
+            table[s, :max(0, c - ql - window + 1) // ps] = -1
+        held |= {int(p) for p in table[s] if p >= 0}
+        if c % ps:
+            last = int(table[s, c // ps])
+            pool[last, 0].reshape(nkv, ps, hd)[:, c % ps:] = float("nan")
+            pool[last, 1].reshape(nkv, hd, ps)[:, :, c % ps:] = float("nan")
+    for p in set(range(pool.shape[0])) - held:
+        pool[p] = float("nan")
+    scale, n = 1 / math.sqrt(hd), case["n"]
+    sink = rnd(nh, seed=8) if sinks else None
+    q, dev_table = case["q"].reshape(n, nh * hd), table.to(DEV)
+
+    def run(rows):
+        out = torch.full((len(rows), nh * hd), float("nan"), dtype=torch.float32, device=DEV)
+        ops().attn_plain(q[rows].contiguous(), out, case["cache"], case["pos_d"][rows].contiguous(), case["seq_d"][rows].contiguous(),
+                         dev_table, nh, scale, window, softcap=cap, sink=sink)
+        return out
+    everything = run(list(range(n)))
+    for i in list(range(0, n, 37)) + [299, 300, n - 1]:
+        assert torch.equal(run([i])[0], everything[i]), i
+    some = sorted(torch.randperm(n, generator=torch.Generator().manual_seed(1))[:40].tolist())
+    assert torch.equal(run(some), everything[some])
+    for i in range(0, n, 7):
+        s, p = case["tok_seq"][i], case["pos"][i]
+        lo = max(0, p - window + 1) if window else 0
+        for h in range(nh):
+            kv = h // (nh // nkv)
+            score = (case["K"][s][lo:p + 1, kv] @ case["q"][i, h].double()) * scale
+            score = cap * torch.tanh(score / cap) if cap else score
+            if sinks:
+                score = torch.cat([score, sink[h:h + 1].double()])
+            want = torch.softmax(score, 0)[:p + 1 - lo] @ case["V"][s][lo:p + 1, kv]
+            # weights and values sum in float over up to 640 keys: a few roundings of values up to 4
+            assert (everything[i, h * hd:(h + 1) * hd].double() - want).abs().max() < 4e-6
