@@ -36,16 +36,19 @@
 // the next run's values are asked for (into registers) before the walk over this run begins and put into
 // LDS after it, so that the trip to memory hides behind the walk.
 //
-// What bounds it are the vector operations of a token, 25 to 45 of them and their addressing at four clocks each (a
+// What bounds it are the vector operations of a token, 25 to 55 of them and their addressing at four clocks each (a
 // wave has its SIMD to itself; sixteen waves with a column each, the sums over 64 lanes, took as long: 285 us fixed,
-// 580 delta).  So a token's values are read from LDS into registers while the token before is worked on, the sums over
+// 580 delta), and the trips to LDS.  So a token's values are read from LDS into registers AHEAD tokens before their
+// turn (four; two where a token of eight rows brings a decay per key dim, or has sixteen rows: four of them left the
+// compiler moving registers, 357 us gated; none beyond 256 key dims), the sums over
 // lanes of four tokens' outputs are formed together, and the 16 lanes of a column, which all hold a token's sum,
 // keep one of 16 tokens' outputs each and store them at once.  WHOLE: 16 RPT key dims, a multiple of 16 columns, rows
 // and records in whole 16-byte pieces: loads without conditions, four values at a time (rows behind the request's
 // last are its last again).
-// 2,048 tokens, heads of 128 x 128 (in brackets a token's reads, chain and store one after the other): delta rule, 32
-// heads, 409 us (527); fixed decay, 16 heads, 307 (422); gated, 32 heads, 337 (509); forget gates, 32 heads, 342 (510);
-// delta rule with a decay per key dim 417 (601); written, 32 heads of 128 x 64, 340 (438).  The bits are the same.
+// 2,048 tokens, heads of 128 x 128 (in brackets a token's values read one token before their turn; and a token's reads,
+// chain and store one after the other): delta rule, 32 heads, 371 us (409, 527); fixed decay, 16 heads, 309 (307, 422);
+// gated, 32 heads, 323 (337, 509); forget gates, 32 heads, 335 (342, 510); delta rule with a decay per key dim 393 (417,
+// 601); written, 32 heads of 128 x 64, 319 (340, 438); delta, heads of 64 x 48, 240 (285, 421).  The bits are the same.
 //
 // MODE 0: a decay per head or per token and head, u = v; 1: the delta rule; 2: a decay per token, head AND key dim
 // (`k` holds the forget gates f; the key is 1 - f: what is forgotten makes room for what is written); 3: the delta rule
@@ -63,6 +66,7 @@ __global__ __launch_bounds__(LS_GROUP * LS_COLS) void linear_scan_kernel(
     constexpr int NT = LS_GROUP * LS_COLS;
     constexpr int DP = LS_GROUP * RPT;                                // a row of q or k in LDS
     constexpr int RUN = RPT <= 8 ? 32 : RPT <= 16 ? 16 : 8;          // tokens per run
+    constexpr int AHEAD = RPT > 16 ? 0 : RPT > 8 || (CHAN && RPT == 8) ? 2 : 4;   // tokens whose values wait in registers (as many as fit)
     constexpr int VEC = WHOLE ? 4 : 1;                               // values per load
     constexpr int PRE = RUN * DP / NT / VEC;                          // loads of q (and k) of a run per thread
     constexpr int PRE_V = (RUN * LS_COLS + NT - 1) / NT;
@@ -205,38 +209,50 @@ __global__ __launch_bounds__(LS_GROUP * LS_COLS) void linear_scan_kernel(
         if (threadIdx.x < RUN) { fs[2 * threadIdx.x] = pf0; fs[2 * threadIdx.x + 1] = pf1; }
         __syncthreads();
         if (t0 + RUN < len) fetch(t0 + RUN);
-        Token even, odd;
-        if (RPT <= 16) read(0, even);
         float kept = 0.f;                          // the output of this lane's token of the 16
         float* orow = out + ((size_t)(start + t0 + g) * H + head) * Dv + j;
-        // (reads stay where they are written, ahead of the token before; the sums over lanes of four tokens go together)
         int tt = 0;
-        for (; RPT <= 16 && tt + 4 <= cnt; tt += 4) {
-            read(tt + 1, odd);
-            __builtin_amdgcn_sched_barrier(1);
-            const float v0 = even.v, v1 = odd.v, s0 = advance(even);
-            read(tt + 2, even);
-            __builtin_amdgcn_sched_barrier(1);
-            const float s1 = advance(odd);
-            read(tt + 3, odd);
-            __builtin_amdgcn_sched_barrier(1);
-            const float v2 = even.v, v3 = odd.v, s2 = advance(even);
-            read(min(tt + 4, RUN - 1), even);
-            __builtin_amdgcn_sched_barrier(1);
-            const float s3 = advance(odd);
-            const float n0 = finish(s0, v0), n1 = finish(s1, v1), n2 = finish(s2, v2), n3 = finish(s3, v3);
-            const int mine = g - (tt & 15);
-            kept = mine == 0 ? n0 : mine == 1 ? n1 : mine == 2 ? n2 : mine == 3 ? n3 : kept;
-            if ((tt & 15) == 12 || tt + 8 > cnt) {                    // 16 tokens, or the run's last four
-                const int t16 = tt & ~15;
-                if (live && t16 + g < tt + 4) orow[(size_t)t16 * H * Dv] = kept;
+        if constexpr (AHEAD > 0) {
+            Token ahead[AHEAD];
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i) read(i, ahead[i]);
+            for (; tt + 4 <= cnt; tt += 4) {
+                float sums[4], values[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    Token& t = ahead[i % AHEAD];
+                    values[i] = t.v;
+                    sums[i] = advance(t);
+                    read(min(tt + i + AHEAD, RUN - 1), t);            // (the row exists, whatever it holds)
+                    __builtin_amdgcn_sched_barrier(1);                // reads stay where they are written
+                }
+                const int mine = g - (tt & 15);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {                         // (together: the moves of one sum hide the waits of another)
+                    const float num = finish(sums[i], values[i]);
+                    kept = mine == i ? num : kept;
+                }
+                if ((tt & 15) == 12 || tt + 8 > cnt) {                // 16 tokens, or the run's last four
+                    const int t16 = tt & ~15;
+                    if (live && t16 + g < tt + 4) orow[(size_t)t16 * H * Dv] = kept;
+                }
             }
-        }
-        for (; tt < cnt; ++tt) {                   // the last one to three of a request (heads beyond 256: all, two tokens of them do not fit the registers)
-            if (RPT > 16) read(tt, even);
-            const float v = even.v, num = finish(advance(even), v);
-            if (live && g == 0) orow[(size_t)tt * H * Dv] = num;
-            if (RPT <= 16) read(min(tt + 1, RUN - 1), even);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {                             // the last one to three of a request
+                if (tt + i < cnt) {
+                    Token& t = ahead[i % AHEAD];
+                    const float v = t.v, num = finish(advance(t), v);
+                    if (live && g == 0) orow[(size_t)(tt + i) * H * Dv] = num;
+                    read(min(tt + i + AHEAD, RUN - 1), t);
+                }
+            }
+        } else {
+            for (; tt < cnt; ++tt) {
+                Token t;
+                read(tt, t);
+                const float num = finish(advance(t), t.v);
+                if (live && g == 0) orow[(size_t)tt * H * Dv] = num;
+            }
         }
     }
     if constexpr (WHOLE) {
