@@ -142,3 +142,26 @@ def test_random_orders_keep_the_books(seed):
     for rid in list(m.live):
         m.release(rid)
     assert m.free_pages() == [12] * len(windows) and m.n_free_slots == 4
+
+
+@pytest.mark.parametrize("slots", [[], [0], [6], [2, 3, 4], [4, 2, 3, 2], [0, 1, 5, 6], [0, 2, 4], [6, 1, 3, 0], list(range(7))])
+def test_claimed_slots_start_from_zero_whatever_their_order(slots):
+    import torch
+    from flambeau_amd.cache.storage import CacheStorage
+    store = CacheStorage([], [], torch.device("cpu"), torch.float32, n_pages=1, page_size=8, max_slots=7)
+    store.states = {0: torch.full((7, 6), 3.0), 1: torch.full((7, 2), 5, dtype=torch.int32)}
+    store.records = {0: {"window": torch.full((7, 2, 3), 4.0)}}
+    store.zero_slots(slots)
+    for t, kept in ((store.states[0], 3), (store.states[1], 5), (store.records[0]["window"], 4)):
+        for slot in range(7):
+            assert (t[slot] == (0 if slot in slots else kept)).all(), (slot, slots)
+
+
+@pytest.mark.parametrize("slots", [[7], [0, 9]])
+def test_a_slot_that_does_not_exist_is_refused(slots):
+    import torch
+    from flambeau_amd.cache.storage import CacheStorage
+    store = CacheStorage([], [], torch.device("cpu"), torch.float32, n_pages=1, page_size=8, max_slots=7)
+    store.states = {0: torch.full((7, 6), 3.0)}
+    with pytest.raises(IndexError):
+        store.zero_slots(slots)
