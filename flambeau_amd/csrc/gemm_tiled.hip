@@ -11,8 +11,9 @@
 //  * the w tile is the A operand and the x tile the B operand: C[feature][token] leaves each
 //    lane with four consecutive features of one token, one 16-byte store;
 //  * blocks of four waves (256, 192 or 128 features x 128 tokens, a wave computes 8 x 4 tiles: 12 operand
-//    reads feed 32 products; ring of 3; two blocks per compute unit) and of eight (256, 224 or 192 features x
-//    256 tokens; ring of 4, one block per unit, the two waves of a SIMD taking turns at the matrix cores);
+//    reads feed 32 products; ring of 3; two blocks per compute unit; with 128 features also a ring of 8 and one
+//    block per unit) and of eight (256, 224 or 192 features x 256 tokens, 224 x 192; ring of 4 or 5, one block per
+//    unit, the two waves of a SIMD taking turns at the matrix cores);
 //    blocks are handed to the eight dies in turn, each die working on a compact patch of tiles;
 //  * with few rows and a narrow matrix even that grid is small: K is then split over
 //    blockIdx.z, the parts are written as float partial sums and a second kernel adds them in
@@ -83,11 +84,10 @@ __global__ __launch_bounds__(128 * WT, OCC) void gemm_async_kernel(const bf16_t*
     constexpr int NW = 2 * WT;                        // waves: 2 along the features, WT along the tokens
     constexpr int NTF = 2 * FT, NTT = WT * TT;        // operand tiles of the block: features, tokens
     constexpr int TILES = NTF + NTT;                  // 1 KB tiles per stage
-    constexpr int LW = (NTF + NW - 1) / NW, LX = NTT / NW;     // tiles of w and of x that a wave copies per stage (where NTF
+    constexpr int LW = (NTF + NW - 1) / NW, LX = (NTT + NW - 1) / NW;     // tiles of w and of x that a wave copies per stage (where NTF
                                                                // does not divide, the last waves copy the last tile too)
     constexpr int LPS = LW + LX;                      // load instructions per wave and stage
     constexpr bool PAIRED = NW == 8;                  // two waves per SIMD, half a period apart (below)
-    static_assert(NTT % NW == 0, "tiles of x must divide among the waves");
     extern __shared__ __attribute__((aligned(16))) bf16_t ring[];      // [NS][TILES][512]
     __shared__ float s_scale[NTT * 16];                               // row scale of the block's tokens
 
@@ -122,6 +122,7 @@ __global__ __launch_bounds__(128 * WT, OCC) void gemm_async_kernel(const bf16_t*
     const bf16_t* wsrc[LW];
     const bf16_t* xsrc[LX];
     auto w_tile = [&](int u) { return NTF % NW == 0 ? wave * LW + u : min(wave * LW + u, NTF - 1); };
+    auto x_tile = [&](int u) { return NTT % NW == 0 ? wave * LX + u : min(wave * LX + u, NTT - 1); };
 #pragma unroll
     for (int u = 0; u < LW; ++u) {
         const int gg = min((n0 >> 4) + w_tile(u), n_groups - 1);
@@ -135,7 +136,7 @@ __global__ __launch_bounds__(128 * WT, OCC) void gemm_async_kernel(const bf16_t*
     const int x_piece = 8 * ((lane & 3) ^ ((lane >> 3) & 3));
 #pragma unroll
     for (int u = 0; u < LX; ++u) {
-        const int row = min(m0 + (wave * LX + u) * 16 + (lane >> 2), M - 1);
+        const int row = min(m0 + x_tile(u) * 16 + (lane >> 2), M - 1);
         xsrc[u] = x + (size_t)row * K + (size_t)s_begin * 32 + x_piece;
     }
     const int x_kmax = K - 8;                         // last whole 16-byte chunk of a row of x
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(128 * WT, OCC) void gemm_async_kernel(const bf16_t*
                 if (k > x_kmax) g -= (k - x_kmax);
             }
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
-                                             (__attribute__((address_space(3))) void*)(slot + (NTF + wave * LX + u) * 512), 16, 0, 0);
+                                             (__attribute__((address_space(3))) void*)(slot + (NTF + x_tile(u)) * 512), 16, 0, 0);
             xsrc[u] += 32;
         }
     };
@@ -448,26 +449,34 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 }
 
 // Shape of the block: 3 = 256 features x 128 tokens (4 waves, ring of 3, two blocks per compute unit),
-// 7 = 192 x 128 and 8 = 128 x 128 (the same with fewer features), 10 = 256 x 256 (8 waves, ring of 4, one
-// block per compute unit), 11 = 224 x 256, 12 = 192 x 256 and 6 = 128 x 256 (the same with fewer features; 6 on
-// request only); 0 = chosen here, together with the number of K-splits.  The entry points whose names end in
-// _ex take either from the caller, for tests and measurements.
+// 7 = 192 x 128 and 8 = 128 x 128 (the same with fewer features), 13 = 128 x 128 (4 waves, ring of 8, one block per
+// unit), 10 = 256 x 256 (8 waves, ring of 4, one block per compute unit), 11 = 224 x 256, 12 = 192 x 256 and
+// 6 = 128 x 256 (the same with fewer features; 6 on request only), 14 = 224 x 192 (8 waves, ring of 5); 0 = chosen
+// here, together with the number of K-splits.  The entry points whose names end in _ex take either from the caller,
+// for tests and measurements.
 //
-// What a shape costs.  Four waves, two blocks per unit: bound by the copies into LDS, 0.056 us per k-step and
-// round of resident blocks plus 17.7 ns per KB that a unit's blocks copy, 0.6 of it from the mean and 0.4
-// from the unit with the most blocks.  Eight waves, one block after the other: bound by the matrix cores and
-// by the wait for weights from HBM, 0.25 us + 1.6 ns per feature and k-step, and 3.7 us per block that nothing
-// overlaps.  Splitting K adds the parts' way to memory and back and the kernel that sums them.  What decides
+// What a shape costs.  Four waves, two blocks per unit: bound by the copies into LDS, 0.061 us per k-step and
+// round of resident blocks plus 16.4 ns per KB that a unit's blocks copy, about half of it from the mean and half
+// from the unit with the most blocks.  Four waves alone on their unit have the whole LDS for stages on their way:
+// 0.30 us per k-step, weights from HBM at 4 TB/s where three stages reach 3.5 (28672 x 4096 at 64 rows 50.9 us
+// against 57.2, at 128 60.6 against 63.7, 28672 x 5120 at 64 rows 63.8 against 74.3; no good where a unit gets a
+// second block: 207 rows 91.5 against 77.9 with 256 features).  Eight waves, one block after the other: bound by the
+// matrix cores and by the wait for weights from HBM, 0.22 us + 1.6 ns per feature and k-step (with 192 tokens 0.18 us
+// + 1.5 ns), and 3.7 us per block that nothing overlaps.  Splitting K adds the parts' way to memory and back and the
+// kernel that sums them.  What decides
 // between 256, 224 and 192 features is how evenly the blocks fill the rounds: gate/up of 2,048 rows, 28672
 // features, is 3.5 rounds of 256 (422 us with its activation) and 4 of 224 (408; 512 with 4 waves before those
 // of a pair took turns), q/k/v of 2,048 rows, 6144 features, 0.75 rounds of 256 (108 us with its rotation) and 1
-// of 192 (102; 115 with 256 x 128).
-// Against every shape and number of parts measured (products of 7B, 12B and 24B sizes at 11 row counts from 128
-// to 4,001, cold weights, parts of K 1 to 4 and 6; 110 products, 2,400 timings) the formula's picks take 2.0 % more
-// time than the best on average and 22 % at worst (5120 x 4096 at 384 rows, 44 us against 37); against the
-// shapes with their real epilogues (42 products) 1.2 % and 17 %.
+// of 192 (102; 115 with 256 x 128).  192 tokens are for rows that end soon behind a multiple of 256: 28672 x 4096
+// at 333 rows 90 us (96.6 with 256 tokens), 528 rows 157 (160; 167 with the 192 features chosen without it), 1,040
+// rows 252 (257); 28672 x 5120 at 1,040 rows 318 (329).  224 x 224 does not divide among the waves, 192 x 192 and
+// 256 x 192 gained nothing beside it (528 rows 161.8 and 168).
+// Against every shape and number of parts measured (products of 7B, 12B and 24B sizes at 14 row counts from 64
+// to 4,001, cold weights, parts of K 1 to 4 and 6; 140 products, 3,000 timings) the formula's picks take 1.2 % more
+// time than the best on average and 14 % at worst (5120 x 14336 at 384 rows, 91 us against 80), 2.6 % less
+// than the picks among the shapes without 13 and 14.
 struct TileShape { int variant, features, tokens, per_unit; };
-static const TileShape g_shapes[] = {{3, 256, 128, 2}, {7, 192, 128, 2}, {8, 128, 128, 2}, {10, 256, 256, 1}, {11, 224, 256, 1}, {12, 192, 256, 1}, {6, 128, 256, 1}};
+static const TileShape g_shapes[] = {{3, 256, 128, 2}, {7, 192, 128, 2}, {8, 128, 128, 2}, {10, 256, 256, 1}, {11, 224, 256, 1}, {12, 192, 256, 1}, {6, 128, 256, 1}, {13, 128, 128, 1}, {14, 224, 192, 1}};
 static const TileShape& tile_shape(int variant) {
     for (const TileShape& t : g_shapes)
         if (t.variant == variant) return t;
@@ -484,8 +493,10 @@ static float tiled_cost(const TileShape& t, int splits, int M, int N, int K) {
     const float mean = blocks > units ? (float)blocks / units : 1.f;
     const float kb = (t.features + t.tokens) * 64 / 1024.f;            // copied per block and k-step
     float us;
-    if (t.per_unit == 1) us = most * (steps * (0.247f + 0.0016f * t.features) + 3.65f) + (most == 1 && splits > 1 ? -0.2f : 0.57f);
-    else us = steps * (0.056f * rounds + 0.0177f * kb * (0.6f * mean + 0.4f * most)) + 2.33f;
+    if (t.variant == 13) us = most * (steps * 0.30f + 3.2f);
+    else if (t.per_unit == 1) us = most * (steps * (0.217f + 0.00163f * t.features - (1.f - t.tokens / 256.f) * (0.137f + 0.00036f * t.features)) + 3.7f)
+                                 + (most == 1 && splits > 1 ? -0.4f : 0.86f);
+    else us = steps * (0.061f * rounds + 0.0164f * kb * (0.456f * mean + 0.544f * most)) + 4.3f;
     if (splits > 1) us += 3.f + (float)M * N * 4.f * (2 * splits + 1) / 4.5e6f;
     return us;
 }
@@ -537,6 +548,8 @@ static void launch_tiled(int variant, int splits, hipStream_t stream, const bf16
         case 8: launch_async<4, 4, 2, 3, 2, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
         case 11: launch_async<7, 4, 4, 4, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
         case 12: launch_async<6, 4, 4, 4, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
+        case 13: launch_async<4, 4, 2, 8, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
+        case 14: launch_async<7, 3, 4, 5, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
         case 10: launch_async<8, 4, 4, 4, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
         default: launch_async<8, 4, 2, 3, 2, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
     }
@@ -570,7 +583,7 @@ static int tiled_entry(const void* x, const void* w_packed, void* out, float* wo
     FL_CHECK(!in_ssq || in_parts > 0, "gemm_tiled: a row scale over %d parts", in_parts);
     if (M == 0) return 0;
     const int n_steps = ceil_div(K, 32);
-    FL_CHECK(tiled_known(variant), "gemm_tiled: block shape %d (0, 3, 6, 7, 8, 10, 11 or 12)", variant);
+    FL_CHECK(tiled_known(variant), "gemm_tiled: block shape %d (0, 3, 6, 7, 8 or 10 to 14)", variant);
     const TilePlan plan = tiled_plan(M, N, K, !epilogue, variant, epilogue ? 1 : forced_splits);
     const int splits = plan.splits, v = plan.variant;
     FL_CHECK(splits == 1 || workspace, "gemm_tiled: this shape splits K %d ways and needs a workspace", splits);
@@ -640,7 +653,7 @@ FL_RECORDABLE(fl_gemm_tiled)
 extern "C" int fl_gemm_tiled_residual_ex(const void* x, const void* w_packed, float* workspace, int M, int N, int K,
                                          float* resid, const float* g, void* xg, float* out_ssq, int variant,
                                          hipStream_t stream) {
-    FL_CHECK(tiled_known(variant), "gemm_tiled_residual: block shape %d (0, 3, 6, 7, 8, 10, 11 or 12)", variant);
+    FL_CHECK(tiled_known(variant), "gemm_tiled_residual: block shape %d (0, 3, 6, 7, 8 or 10 to 14)", variant);
     FL_CHECK(M >= 0 && N > 0 && K > 0, "gemm_tiled_residual: bad sizes M=%d N=%d K=%d", M, N, K);
     FL_CHECK(K % 8 == 0, "gemm_tiled_residual: K=%d is no multiple of 8 (16-byte loads)", K);
     FL_CHECK(N % 4 == 0, "gemm_tiled_residual: N=%d is no multiple of 4 (16-byte accesses to the residual rows)", N);
@@ -731,7 +744,7 @@ extern "C" int fl_gemm_tiled_rope_ex(const void* x, const void* w_packed, int M,
                                      const int* block_table, int max_blocks, const float* cs, void* q_out,
                                      void* cache_base, int nh, int nkv, int hd, int page_size, int n_pages, int rot,
                                      int write_cache, int variant, hipStream_t stream) {
-    FL_CHECK(tiled_known(variant), "gemm_tiled_rope: block shape %d (0, 3, 6, 7, 8, 10, 11 or 12)", variant);
+    FL_CHECK(tiled_known(variant), "gemm_tiled_rope: block shape %d (0, 3, 6, 7, 8 or 10 to 14)", variant);
     FL_CHECK(M >= 0 && N > 0 && K > 0, "gemm_tiled_rope: bad sizes M=%d N=%d K=%d", M, N, K);
     FL_CHECK(K % 8 == 0, "gemm_tiled_rope: K=%d is no multiple of 8 (16-byte loads)", K);
     FL_CHECK(positions && tok_seq && block_table && cs && q_out && cache_base,

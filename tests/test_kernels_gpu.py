@@ -1197,12 +1197,13 @@ def test_gemm_float_gives_the_plain_kernel_s_bits(M, N, K):
     assert torch.equal(got, want)
 
 
-# ---------------------------------------------------------------- the tiled product's blocks of eight waves
-@pytest.mark.parametrize("variant", [10, 11, 12])
-@pytest.mark.parametrize("M,N,K", [(1, 16, 8), (255, 223, 32), (257, 449, 40), (256, 192, 128), (300, 1000, 104), (512, 700, 4096)])
+# ---------------------------------------------------------------- the tiled product's blocks
+@pytest.mark.parametrize("variant", [10, 11, 12, 13, 14])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 8), (255, 223, 32), (257, 449, 40), (256, 192, 128), (193, 225, 160), (128, 129, 256), (300, 1000, 104),
+                                   (512, 700, 4096)])
 def test_gemm_tiled_eight_waves_equal_four(variant, M, N, K):
-    """256, 224 and 192 features x 256 tokens against 256 x 128: every output is the same chain over K, so the same
-    bits; one stage, fewer and more stages than the ring, K's and the tiles' remainders."""
+    """256, 224 and 192 features x 256 tokens, 224 x 192 and 128 x 128 in a deep ring against 256 x 128: every output is
+    the same chain over K, so the same bits; one stage, fewer and more stages than the ring, K's and the tiles' remainders."""
     from flambeau_amd.kernels.packing import pack_weight
     x, w = rnd(M, K, dtype=torch.bfloat16, seed=41), rnd(N, K, dtype=torch.bfloat16, seed=42, scale=0.05)
     packed, got = pack_weight(w), []
