@@ -455,12 +455,12 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 // here, together with the number of K-splits.  The entry points whose names end in _ex take either from the caller,
 // for tests and measurements.
 //
-// What a shape costs.  Four waves, two blocks per unit: bound by the copies into LDS, 0.061 us per k-step and
-// round of resident blocks plus 16.4 ns per KB that a unit's blocks copy, about half of it from the mean and half
+// What a shape costs.  Four waves, two blocks per unit: bound by the copies into LDS, 0.056 us per k-step and
+// round of resident blocks plus 17.7 ns per KB that a unit's blocks copy, 0.6 of it from the mean and 0.4
 // from the unit with the most blocks.  Four waves alone on their unit have the whole LDS for stages on their way:
 // 0.30 us per k-step, weights from HBM at 4 TB/s where three stages reach 3.5 (28672 x 4096 at 64 rows 50.9 us
-// against 57.2, at 128 60.6 against 63.7, 28672 x 5120 at 64 rows 63.8 against 74.3; no good where a unit gets a
-// second block: 207 rows 91.5 against 77.9 with 256 features).  Eight waves, one block after the other: bound by the
+// against 57.2, at 128 60.6 against 63.7, 28672 x 5120 at 64 rows 63.8 against 74.3; only where
+// more than three quarters of the units get a block and none gets a second: 207 rows 91.5 against 77.9 with 256 features).  Eight waves, one block after the other: bound by the
 // matrix cores and by the wait for weights from HBM, 0.22 us + 1.6 ns per feature and k-step (with 192 tokens 0.18 us
 // + 1.5 ns), and 3.7 us per block that nothing overlaps.  Splitting K adds the parts' way to memory and back and the
 // kernel that sums them.  What decides
@@ -472,8 +472,8 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 // rows 252 (257); 28672 x 5120 at 1,040 rows 318 (329).  224 x 224 does not divide among the waves, 192 x 192 and
 // 256 x 192 gained nothing beside it (528 rows 161.8 and 168).
 // Against every shape and number of parts measured (products of 7B, 12B and 24B sizes at 14 row counts from 64
-// to 4,001, cold weights, parts of K 1 to 4 and 6; 140 products, 3,000 timings) the formula's picks take 1.2 % more
-// time than the best on average and 14 % at worst (5120 x 14336 at 384 rows, 91 us against 80), 2.6 % less
+// to 4,001, cold weights, parts of K 1 to 4 and 6; 140 products, 3,000 timings) the formula's picks take 1.3 % more
+// time than the best on average and 14 % at worst (5120 x 14336 at 384 rows, 91 us against 80), 2.5 % less
 // than the picks among the shapes without 13 and 14.
 struct TileShape { int variant, features, tokens, per_unit; };
 static const TileShape g_shapes[] = {{3, 256, 128, 2}, {7, 192, 128, 2}, {8, 128, 128, 2}, {10, 256, 256, 1}, {11, 224, 256, 1}, {12, 192, 256, 1}, {6, 128, 256, 1}, {13, 128, 128, 1}, {14, 224, 192, 1}};
@@ -493,10 +493,9 @@ static float tiled_cost(const TileShape& t, int splits, int M, int N, int K) {
     const float mean = blocks > units ? (float)blocks / units : 1.f;
     const float kb = (t.features + t.tokens) * 64 / 1024.f;            // copied per block and k-step
     float us;
-    if (t.variant == 13) us = most * (steps * 0.30f + 3.2f);
-    else if (t.per_unit == 1) us = most * (steps * (0.217f + 0.00163f * t.features - (1.f - t.tokens / 256.f) * (0.137f + 0.00036f * t.features)) + 3.7f)
-                                 + (most == 1 && splits > 1 ? -0.4f : 0.86f);
-    else us = steps * (0.061f * rounds + 0.0164f * kb * (0.456f * mean + 0.544f * most)) + 4.3f;
+    if (t.variant == 13) us = blocks > units || 4 * blocks <= 3 * units ? 1e9f : steps * 0.30f + 3.2f;
+    else if (t.per_unit == 1) us = most * (steps * (0.217f + 0.00163f * t.features - (1.f - t.tokens / 256.f) * (0.137f + 0.00036f * t.features)) + 3.7f) + 0.86f;
+    else us = steps * (0.056f * rounds + 0.0177f * kb * (0.6f * mean + 0.4f * most)) + 2.33f;
     if (splits > 1) us += 3.f + (float)M * N * 4.f * (2 * splits + 1) / 4.5e6f;
     return us;
 }
