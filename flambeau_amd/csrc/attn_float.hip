@@ -7,6 +7,9 @@
 //     M' = max(M, m),  L <- L e^(M - M') + l e^(m - M'),  A <- A e^(M - M') + a e^(m - M').
 // Keys outside the row's range weigh nothing (their scores are not looked at), and a block without a key of the row
 // leaves (M, L, A) as it is.  So neither the rows of a tile, nor how a prompt is cut, nor who forms a block shows.
+// A block's weights add up to at least 1 where it has a score above minus infinity, and to NaN where a score is NaN (or
+// plus infinity), which a maximum would pass by: the sum tells whether a block counts, never the maximum.  A row
+// whose scores are all minus infinity is NaN, as the formula has it.
 //
 // Block of threads = a tile of up to 16 rows (token, query head) that read one key/value head: T tokens by its query
 // heads (T = 1 in steps of few tokens, where the heads alone have to fill the chip).  Eight waves form eight blocks of
@@ -56,10 +59,12 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
     // what this thread adds up: row a_row[u], head dims a_d[u] ..+ 3
     float M[SUMS], L[SUMS];
     f32x4 A[SUMS];
+    bool low[SUMS];                                                   // a block of the row had keys, all at minus infinity
 #pragma unroll
     for (int u = 0; u < SUMS; ++u) {
         M[u] = -INFINITY;
         L[u] = 0.f;
+        low[u] = false;
         A[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
     const size_t block = (size_t)cache.page_size * HD;                // floats of a (page, K or V, head)
@@ -122,16 +127,21 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
                     }
                 m = fmaxf(m, __shfl_xor(m, 16, 64));
                 m = fmaxf(m, __shfl_xor(m, 32, 64));
+                const float base = m == -INFINITY ? 0.f : m;
                 float l = 0.f;
+                bool any = false;
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        S[t][r] = seen[t][r] ? expf(S[t][r] - m) : 0.f;
+                        S[t][r] = seen[t][r] ? expf(S[t][r] - base) : 0.f;
                         l += S[t][r];
+                        any = any || seen[t][r];
                     }
                 l += __shfl_xor(l, 16, 64);
                 l += __shfl_xor(l, 32, 64);
+                // lanes j, j + 16, j + 32, j + 48 hold row j's keys; -1: there are some, and every score is minus infinity
+                if (l == 0.f && ((__ballot(any) >> j) & 0x0001000100010001ull)) l = -1.f;
                 // O^T: keys in rising order of (t, r), values of keys that are not the request's set to zero
 #pragma unroll
                 for (int d0 = 0; d0 < HD; d0 += 16) {
@@ -161,11 +171,15 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
                 const int e = threadIdx.x + 64 * AF_WAVES * u, row = e / FOURS, d = 4 * (e % FOURS);
                 if (row < AF_ROWS && row / heads >= from && row / heads < to) {
                     for (int w = 0; w < blocks; ++w) {
-                        const float m = part_m[w][row];
-                        if (m == -INFINITY) continue;                 // no key of this row in the block
+                        const float m = part_m[w][row], l = part_l[w][row];
+                        if (l == 0.f) continue;                       // no key of this row in the block
+                        if (l < 0.f) {
+                            low[u] = true;
+                            continue;
+                        }
                         const float top = fmaxf(M[u], m), old = expf(M[u] - top), now = expf(m - top);
                         const f32x4 a = *(const f32x4*)&part_a[w][row][d];
-                        L[u] = L[u] * old + part_l[w][row] * now;
+                        L[u] = L[u] * old + l * now;
 #pragma unroll
                         for (int r = 0; r < 4; ++r) A[u][r] = A[u][r] * old + a[r] * now;
                         M[u] = top;
@@ -182,7 +196,8 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
         const int tok = row / heads, hh = row % heads;
         if (row >= AF_ROWS || tok >= n_tok || hh >= n_heads) continue;
         const int head = kvh * group + h0 + hh;
-        const float inv = sink ? softmax_factor_with_sink(M[u], L[u], sink[head]) : L[u] > 0.f ? 1.0f / L[u] : 0.f;
+        const float none = low[u] ? NAN : 0.f;                        // (NaN, or no key at all)
+        const float inv = sink ? softmax_factor_with_sink(M[u], L[u], sink[head]) : L[u] == 0.f ? none : 1.0f / L[u];
         f32x4 o;
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[r] = A[u][r] * inv;

@@ -1299,3 +1299,43 @@ def test_attn_float_rows_do_not_depend_on_their_neighbours(nh, nkv, hd, ps, wind
             want = torch.softmax(score, 0)[:p + 1 - lo] @ case["V"][s][lo:p + 1, kv]
             # weights and values sum in float over up to 640 keys: a few roundings of values up to 4
             assert (everything[i, h * hd:(h + 1) * hd].double() - want).abs().max() < 4e-6
+
+
+def attn_float_case(nh, nkv, hd, ps, seqs, window, edit=None):
+    """A 32-bit case after ``edit(case, put_key, put_value)``, its outputs ``[n, nh, hd]`` and the formula's in 64 bits."""
+    case = build_attention_case(torch.float32, nh, nkv, hd, ps, seqs, seed=6)
+    pool, table = case["cache"].pool, case["table"].cpu()
+
+    def put(kind):
+        def into(s, t, kv, d, value):
+            page, r = int(table[s, t // ps]), t % ps
+            case["KV"[kind]][s][t, kv, d] = value
+            (pool[page, 0].reshape(nkv, ps, hd)[kv, r] if kind == 0 else pool[page, 1].reshape(nkv, hd, ps)[kv, :, r])[d] = value
+        return into
+    if edit:
+        edit(case, put(0), put(1))
+    n, scale = case["n"], 1 / math.sqrt(hd)
+    out = torch.full((n, nh * hd), 7.0, dtype=torch.float32, device=DEV)
+    ops().attn_plain(case["q"].reshape(n, nh * hd), out, case["cache"], case["pos_d"], case["seq_d"], case["table"], nh, scale, window)
+    return case, out.reshape(n, nh, hd), attention_case_ref(case, scale, window)
+
+
+@pytest.mark.parametrize("what", ["query", "block", "key", "low block", "low request"])
+def test_attn_float_keeps_a_nan(what):
+    """A NaN in a query, in all 64 keys of a block or in a row's only key of one: NaN in the rows that see it and nowhere
+    else.  Scores of minus infinity weigh nothing; a row that has no other is NaN."""
+    seqs = [(200, 200), (65, 65), (130, 1), (300, 2)]
+
+    def edit(case, put_key, put_value):
+        case["q"][:, :, 0] = case["q"][:, :, 0].abs() + 0.1
+        if what == "query":
+            case["q"][77, 3, 40] = float("nan")
+        elif what == "key":
+            put_key(1, 64, 1, 9, float("nan"))
+        for s, keys in {"block": [(0, range(64, 128))], "low block": [(0, range(64, 128)), (3, [256])], "low request": [(1, range(65))]}.get(what, []):
+            for t in keys:
+                put_key(s, t, 1, 0, float("nan" if what == "block" else "-inf"))
+    _, out, ref = attn_float_case(8, 2, 128, 16, seqs, 0, edit)
+    assert torch.equal(out.isnan(), ref.isnan()) and ref.isnan().any() == (what != "low block")
+    good = ~ref.isnan()
+    assert (out.double() - ref)[good].abs().max() < 4e-6         # as for finite inputs: float sums of up to 300 keys
