@@ -30,6 +30,22 @@
 #define AF_ROWS 16
 #define AF_KEYS 64
 
+// o[e], the sum of lane (g, row j) for dim 4 g + e, plus weight times value for the values of `v` that are no finite
+// numbers: v of lane (g, d) belongs to dim d and to the key whose weights for the rows (g, 0) .. (g, 15) are in `weight`
+// of those lanes; `sees`: whether the row's range holds that key.
+__device__ __forceinline__ void add_unbounded(f32x4& o, float v, float weight, bool sees) {
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    for (unsigned long long rest = __ballot(!isfinite(v)); rest; rest &= rest - 1) {
+        const int from = __ffsll(rest) - 1, d = from & 15;
+        const float value = __shfl(v, from, 64), p = __shfl(weight, (from & 48) + j, 64);
+        if (__shfl((int)sees, (from & 48) + j, 64) && g == d >> 2) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (e == (d & 3)) o[e] += p * value;
+        }
+    }
+}
+
 template <int HD>
 __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const float* __restrict__ q, float* __restrict__ out,
                                                                       PagedCache cache, const int* __restrict__ positions,
@@ -143,6 +159,7 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
                 // lanes j, j + 16, j + 32, j + 48 hold row j's keys; -1: there are some, and every score is minus infinity
                 if (l == 0.f && ((__ballot(any) >> j) & 0x0001000100010001ull)) l = -1.f;
                 // O^T: keys in rising order of (t, r), values of keys that are not the request's set to zero
+                bool finite = true;
 #pragma unroll
                 for (int d0 = 0; d0 < HD; d0 += 16) {
                     f32x4 o = {0.f, 0.f, 0.f, 0.f};
@@ -157,7 +174,31 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
                             const float val = there[t] && key >= lo_min && key <= p_max ? vf[t][r] : 0.f;
                             o = __builtin_amdgcn_mfma_f32_16x16x4f32(val, S[t][r], o, 0, 0, 0);
                         }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) finite = finite && isfinite(o[r]);
                     *(f32x4*)&part_a[wave][j][d0 + 4 * g] = o;
+                }
+                if (__any(!finite)) {
+#pragma unroll 1
+                    for (int d0 = 0; d0 < HD; d0 += 16) {
+                        f32x4 o = {0.f, 0.f, 0.f, 0.f};
+                        f32x4 val[4];
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) {
+                            const f32x4 vf = *(const f32x4*)(vals[t] + (size_t)(d0 + j) * cache.page_size);
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                const int key = key0 + 16 * t + 4 * g + r;
+                                val[t][r] = there[t] && key >= lo_min && key <= p_max ? vf[r] : 0.f;
+                                o = __builtin_amdgcn_mfma_f32_16x16x4f32(isfinite(val[t][r]) ? val[t][r] : 0.f, S[t][r], o, 0, 0, 0);
+                            }
+                        }
+#pragma unroll
+                        for (int t = 0; t < 4; ++t)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) add_unbounded(o, val[t][r], S[t][r], seen[t][r]);
+                        *(f32x4*)&part_a[wave][j][d0 + 4 * g] = o;
+                    }
                 }
                 if (g == 0) {
                     part_m[wave][j] = m;

@@ -1339,3 +1339,25 @@ def test_attn_float_keeps_a_nan(what):
     assert torch.equal(out.isnan(), ref.isnan()) and ref.isnan().any() == (what != "low block")
     good = ~ref.isnan()
     assert (out.double() - ref)[good].abs().max() < 4e-6         # as for finite inputs: float sums of up to 300 keys
+
+
+@pytest.mark.parametrize("window", [0, 37])
+@pytest.mark.parametrize("nh,nkv,hd,ps", [(16, 4, 128, 16), (6, 6, 64, 8)])
+def test_attn_float_values_reach_the_rows_that_see_them(nh, nkv, hd, ps, window):
+    """Infinities and NaN among the values, of later tokens of the same tile and in front of a window: the rows
+    that see them as the formula has it, every other row to the last bit what it is without them."""
+    seqs = [(200, 200), (70, 9), (90, 30)]
+
+    def edit(case, put_key, put_value):
+        put_value(0, 70, 1, 5, float("inf"))
+        put_value(0, 101, 0, hd - 1, float("nan"))
+        put_value(0, 103, 0, hd - 1, float("-inf"))
+        put_value(1, 69, 1, 17, float("nan"))
+        for d in range(hd):
+            put_value(2, 62, 1, d, float("-inf"))
+    _, clean, _ = attn_float_case(nh, nkv, hd, ps, seqs, window)
+    case, out, ref = attn_float_case(nh, nkv, hd, ps, seqs, window, edit)
+    finite = ref.isfinite()
+    assert 0 < (~finite).sum() < finite.numel() / 4
+    assert torch.equal(out[finite], clean[finite])
+    assert torch.equal(out.nan_to_num(7, 8, 9)[~finite], ref.nan_to_num(7, 8, 9).float()[~finite])
