@@ -1,9 +1,9 @@
 // Attention over the paged cache for the 32-bit path: floats in, floats out, every product on the matrix cores
 // (v_mfma_f32_16x16x4_f32), precise expf.  The same result, to the bit, whatever tokens run beside a token.
 //
-// What a (token, query head) is: its keys in blocks of 64 counted from position 0.  A block's scores (four sums of a
-// quarter of the head dims each, added in pairs), their maximum m, the weights e^(score - m), their sum l and the
-// weighted sum of the values in rising order of the keys; then (M, L, A) over the blocks in rising order,
+// What a (token, query head) is: its keys in blocks of 64 counted from position 0.  A block's scores (chains of 8
+// head dims, added in a tree), their maximum m, the weights e^(score - m), their sum l and the weighted sum a of the
+// values (chains of 16 keys, added in pairs); then (M, L, A) over the blocks in rising order,
 //     M' = max(M, m),  L <- L e^(M - M') + l e^(m - M'),  A <- A e^(M - M') + a e^(m - M').
 // Keys outside the row's range weigh nothing (their scores are not looked at), and a block without a key of the row
 // leaves (M, L, A) as it is.  So neither the rows of a tile, nor how a prompt is cut, nor who forms a block shows.
@@ -30,6 +30,34 @@
 #define AF_ROWS 16
 #define AF_KEYS 64
 
+// The scores of 16 keys: chains of two instructions from zero, their results added in a tree.  Longer chains lose
+// more: the error against 64 bits, beside the plain kernel's, is 0.98, 0.92, 0.72 and 0.56 times at 64, 100, 340 and
+// 1,000 keys, with chains of 16 products 1.05, 1.03, 0.89, 0.63, with chains of 32 (and the values of a block in one
+// chain) 1.41, 1.30, 1.11, 0.76.  A result is added two chains after its own, so that no addition waits for the
+// matrix unit.
+template <int NC>
+__device__ __forceinline__ f32x4 scores(const f32x4 (&kf)[NC], const f32x4 (&qv)[NC]) {
+    constexpr int N = 2 * NC, LATE = 2;
+    f32x4 sum[N];
+#pragma unroll
+    for (int n = 0; n < N + LATE; ++n) {
+        if (n < N) {
+            sum[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 2 * (n & 1); e < 2 * (n & 1) + 2; ++e)
+                sum[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[n / 2][e], qv[n / 2][e], sum[n], 0, 0, 0);
+        }
+        const int d = n - LATE;                       // (a binary counter: d's trailing ones are complete pairs)
+#pragma unroll
+        for (int w = 1; w < N; w *= 2) {
+            if (d < 0 || !(d & w)) break;
+            sum[d & ~(2 * w - 1)] += sum[(d & ~(2 * w - 1)) + w];
+        }
+        __builtin_amdgcn_sched_barrier(0);            // (in this order: all chains first would hold all their results)
+    }
+    return sum[0];
+}
+
 // o[e], the sum of lane (g, row j) for dim 4 g + e, plus weight times value for the values of `v` that are no finite
 // numbers: v of lane (g, d) belongs to dim d and to the key whose weights for the rows (g, 0) .. (g, 15) are in `weight`
 // of those lanes; `sees`: whether the row's range holds that key.
@@ -53,7 +81,7 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
                                                                       const int* __restrict__ block_table, int max_blocks, int n,
                                                                       int nh, int tokens, int heads, int head_tiles, float scale,
                                                                       int window, float softcap, const float* __restrict__ sink) {
-    constexpr int NC = HD / 16, LD = HD + 4, FOURS = HD / 4;
+    constexpr int NC = HD / 16, LD = HD + 4, FOURS = HD / 4, AHEAD = 2;
     constexpr int MINE = AF_ROWS * FOURS / (64 * AF_WAVES);           // groups of four dims a thread adds up
     static_assert(AF_ROWS * FOURS % (64 * AF_WAVES) == 0 || AF_ROWS * FOURS < 64 * AF_WAVES, "rows must divide among the threads");
     constexpr int SUMS = MINE > 0 ? MINE : 1;
@@ -103,100 +131,115 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
                 f32x4 S[4];
                 bool there[4];                                        // keys 16 t + 4 g .. + 3 have a page (all four or none)
                 const float* vals[4];                                 // their values of head dim 0
+                const float* keys[4];
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const int key = min(key0 + 16 * t + j, p_max);    // (beyond the last key: that one again, not looked at)
                     const int page = table[key / cache.page_size];
                     const int held = page >= 0 && page < cache.n_pages ? page : 0;
-                    const float* kr = (const float*)cache.base + ((size_t)held * 2 * cache.n_kv_heads + kvh) * block +
-                                      (size_t)(key % cache.page_size) * HD;
-                    f32x4 kf[NC];
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) kf[c] = *(const f32x4*)(kr + 16 * c + 4 * g);
+                    keys[t] = (const float*)cache.base + ((size_t)held * 2 * cache.n_kv_heads + kvh) * block +
+                              (size_t)(key % cache.page_size) * HD + 4 * g;
                     const int key4 = key0 + 16 * t + 4 * g;           // (pages hold a multiple of four tokens)
                     const int page4 = key4 <= p_max ? table[key4 / cache.page_size] : -1;
                     there[t] = page4 >= 0 && page4 < cache.n_pages;
                     vals[t] = (const float*)cache.base + ((size_t)(there[t] ? page4 : 0) * 2 * cache.n_kv_heads + cache.n_kv_heads + kvh) * block +
-                              (there[t] ? key4 % cache.page_size : 0);
-                    f32x4 sum[4];
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) sum[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-#pragma unroll
-                        for (int c = 0; c < NC; ++c)
-                            sum[c & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c][e], qv[c][e], sum[c & 3], 0, 0, 0);
-                    S[t] = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+                              (there[t] ? key4 % cache.page_size : 0) + (size_t)j * cache.page_size;
                 }
+                // 16 keys at a time, the next 16 on their way (a wait for all of them at once would take the registers of 64)
+                f32x4 kf[2][NC];
+#pragma unroll
+                for (int c = 0; c < NC; ++c) kf[0][c] = *(const f32x4*)(keys[0] + 16 * c);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    if (t < 3) {
+#pragma unroll
+                        for (int c = 0; c < NC; ++c) kf[(t + 1) & 1][c] = *(const f32x4*)(keys[t + 1] + 16 * c);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    S[t] = scores<NC>(kf[t & 1], qv);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                f32x4 vf[AHEAD][4];                                   // values of 16 head dims, AHEAD times 16 on their way
+                auto fetch = [&](int d0, f32x4* to) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) to[t] = *(const f32x4*)(vals[t] + (size_t)d0 * cache.page_size);
+                };
+#pragma unroll
+                for (int a = 0; a < AHEAD; ++a) fetch(16 * a, vf[a]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) S[t] *= scale;
+                if (softcap > 0.f) {                                  // scores capped smoothly at +-softcap
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) S[t][r] = softcap * tanhf(S[t][r] / softcap);
+                }
+                auto sees = [&](int t, int r) {                       // whether the row looks at key 16 t + 4 g + r
+                    const int key = key0 + 16 * t + 4 * g + r;
+                    return in_turn && there[t] && key >= my_lo && key <= my_p;
+                };
                 float m = -INFINITY;
-                bool seen[4][4];
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int key = key0 + 16 * t + 4 * g + r;
-                        seen[t][r] = in_turn && there[t] && key >= my_lo && key <= my_p;
-                        float s = S[t][r] * scale;
-                        if (softcap > 0.f) s = softcap * tanhf(s / softcap);          // scores capped smoothly at +-softcap
-                        S[t][r] = s;
-                        if (seen[t][r]) m = fmaxf(m, s);
-                    }
+                    for (int r = 0; r < 4; ++r)
+                        if (sees(t, r)) m = fmaxf(m, S[t][r]);
                 m = fmaxf(m, __shfl_xor(m, 16, 64));
                 m = fmaxf(m, __shfl_xor(m, 32, 64));
                 const float base = m == -INFINITY ? 0.f : m;
-                float l = 0.f;
                 bool any = false;
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        S[t][r] = seen[t][r] ? expf(S[t][r] - base) : 0.f;
-                        l += S[t][r];
-                        any = any || seen[t][r];
+                        const bool seen = sees(t, r);
+                        S[t][r] = seen ? expf(S[t][r] - base) : 0.f;
+                        any = any || seen;
                     }
+                const f32x4 four = (S[0] + S[1]) + (S[2] + S[3]);
+                float l = (four[0] + four[1]) + (four[2] + four[3]);
                 l += __shfl_xor(l, 16, 64);
                 l += __shfl_xor(l, 32, 64);
                 // lanes j, j + 16, j + 32, j + 48 hold row j's keys; -1: there are some, and every score is minus infinity
                 if (l == 0.f && ((__ballot(any) >> j) & 0x0001000100010001ull)) l = -1.f;
-                // O^T: keys in rising order of (t, r), values of keys that are not the request's set to zero
+                // O^T: four chains of 16 keys, instruction (t, r) the keys 16 t + 4 g + r; whatever lies behind a weight of zero
+                // counts only if it is no finite number, and then it shows in the sums
                 bool finite = true;
 #pragma unroll
                 for (int d0 = 0; d0 < HD; d0 += 16) {
-                    f32x4 o = {0.f, 0.f, 0.f, 0.f};
-                    f32x4 vf[4];
+                    f32x4 part[4];
+                    f32x4* now = vf[d0 / 16 % AHEAD];
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) vf[t] = *(const f32x4*)(vals[t] + (size_t)(d0 + j) * cache.page_size);
+                    for (int t = 0; t < 4; ++t) part[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int t = 0; t < 4; ++t)
+                    for (int r = 0; r < 4; ++r)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int key = key0 + 16 * t + 4 * g + r;
-                            const float val = there[t] && key >= lo_min && key <= p_max ? vf[t][r] : 0.f;
-                            o = __builtin_amdgcn_mfma_f32_16x16x4f32(val, S[t][r], o, 0, 0, 0);
-                        }
+                        for (int t = 0; t < 4; ++t) part[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(now[t][r], S[t][r], part[t], 0, 0, 0);
+                    if (d0 + 16 * AHEAD < HD) fetch(d0 + 16 * AHEAD, now);
+                    const f32x4 o = (part[0] + part[1]) + (part[2] + part[3]);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) finite = finite && isfinite(o[r]);
                     *(f32x4*)&part_a[wave][j][d0 + 4 * g] = o;
+                    __builtin_amdgcn_sched_barrier(0);
                 }
                 if (__any(!finite)) {
 #pragma unroll 1
                     for (int d0 = 0; d0 < HD; d0 += 16) {
-                        f32x4 o = {0.f, 0.f, 0.f, 0.f};
-                        f32x4 val[4];
+                        f32x4 val[4], part[4];
+                        fetch(d0, val);
 #pragma unroll
                         for (int t = 0; t < 4; ++t) {
-                            const f32x4 vf = *(const f32x4*)(vals[t] + (size_t)(d0 + j) * cache.page_size);
+                            part[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                            for (int r = 0; r < 4; ++r) {
-                                const int key = key0 + 16 * t + 4 * g + r;
-                                val[t][r] = there[t] && key >= lo_min && key <= p_max ? vf[r] : 0.f;
-                                o = __builtin_amdgcn_mfma_f32_16x16x4f32(isfinite(val[t][r]) ? val[t][r] : 0.f, S[t][r], o, 0, 0, 0);
-                            }
+                            for (int r = 0; r < 4; ++r)
+                                part[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(isfinite(val[t][r]) ? val[t][r] : 0.f, S[t][r], part[t], 0, 0, 0);
                         }
+                        f32x4 o = (part[0] + part[1]) + (part[2] + part[3]);
 #pragma unroll
                         for (int t = 0; t < 4; ++t)
 #pragma unroll
-                            for (int r = 0; r < 4; ++r) add_unbounded(o, val[t][r], S[t][r], seen[t][r]);
+                            for (int r = 0; r < 4; ++r) add_unbounded(o, val[t][r], S[t][r], sees(t, r));
                         *(f32x4*)&part_a[wave][j][d0 + 4 * g] = o;
                     }
                 }
