@@ -13,8 +13,8 @@
 //
 // Block of threads = a tile of up to 16 rows (token, query head) that read one key/value head: T tokens by its query
 // heads (T = 1 in steps of few tokens, where the heads alone have to fill the chip).  Eight waves form eight blocks of
-// keys at a time and leave (m, l, a) in LDS, where all threads add them in order, four head dims of a row each.  A tile
-// whose tokens belong to several requests takes them one after the other.
+// keys at a time and leave (m, l, a) in LDS, where all threads add them in order, four head dims of a row each.  The
+// tokens of a tile may belong to several requests: their blocks of keys are one list that the waves share.
 // No operand passes through LDS.  Scores are computed transposed, S^T = K Q^T, so that a lane holds scores of one row:
 // instruction (c, e) takes head dims 16 c + 4 g + e of lane group g = lane / 16, four neighbouring dims of a row being one
 // 16-byte load for four instructions.  S^T leaves lane (g, row) with keys 16 t + 4 g + r, which is just what it has to
@@ -112,167 +112,185 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
         A[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
     const size_t block = (size_t)cache.page_size * HD;                // floats of a (page, K or V, head)
-    for (int from = 0; from < n_tok;) {                               // the tile's tokens, request by request
-        const int seq = tok_seq[tok0 + from];
-        int to = from, p_max = -1, lo_min = 0x7fffffff;
-        for (; to < n_tok && tok_seq[tok0 + to] == seq; ++to) {
-            const int p = positions[tok0 + to];
+    // The tile's requests, one after the other, each from the first to the last block of keys that its tokens see: lane r
+    // keeps the r-th of them, and every wave takes the next block of the whole list (not of one request: 16 requests of
+    // one token are two rounds instead of 16).
+    const int last_tok = min(lane & (AF_ROWS - 1), n_tok - 1);
+    const int lane_seq = tok_seq[tok0 + last_tok], lane_p = positions[tok0 + last_tok];
+    int blocks = 0, requests = 0, r_seq = 0, r_max = 0, r_min = 0, r_from = 0, r_to = 0, r_end = 0;
+    for (int from = 0, to; from < n_tok; from = to) {
+        const int seq = __builtin_amdgcn_readlane(lane_seq, from);
+        int p_max = -1, p_min = 0x7fffffff;
+        for (to = from; to < n_tok && __builtin_amdgcn_readlane(lane_seq, to) == seq; ++to) {
+            const int p = __builtin_amdgcn_readlane(lane_p, to);
             p_max = max(p_max, p);
-            lo_min = min(lo_min, window > 0 ? max(0, p - window + 1) : 0);
+            p_min = min(p_min, p);
         }
-        const int* table = block_table + (size_t)seq * max_blocks;
-        const bool in_turn = my_row && my_tok >= from && my_tok < to;
-        const int last = p_max / AF_KEYS;
-        for (int b0 = lo_min / AF_KEYS; b0 <= last; b0 += AF_WAVES) {
-            const int b = b0 + wave;
-            if (b <= last) {
-                const int key0 = b * AF_KEYS;
-                // S^T: lane (g, row j) gets the scores of keys key0 + 16 t + 4 g + r
-                f32x4 S[4];
-                bool there[4];                                        // keys 16 t + 4 g .. + 3 have a page (all four or none)
-                const float* vals[4];                                 // their values of head dim 0
-                const float* keys[4];
+        if (p_max < 0) continue;
+        const int lo_min = window > 0 ? max(0, p_min - window + 1) : 0;
+        blocks += p_max / AF_KEYS - lo_min / AF_KEYS + 1;
+        if (lane == requests) {
+            r_seq = seq;
+            r_max = p_max;
+            r_min = lo_min;
+            r_from = from;
+            r_to = to;
+            r_end = blocks;
+        }
+        ++requests;
+    }
+    for (int b0 = 0; b0 < blocks; b0 += AF_WAVES) {
+        const int b = b0 + wave;
+        if (b < blocks) {
+            const int r = __ffsll(__ballot(lane < requests && r_end > b)) - 1;
+            const int p_max = __builtin_amdgcn_readlane(r_max, r), lo_min = __builtin_amdgcn_readlane(r_min, r);
+            const int* table = block_table + (size_t)__builtin_amdgcn_readlane(r_seq, r) * max_blocks;
+            const bool in_turn = my_row && my_tok >= __builtin_amdgcn_readlane(r_from, r) && my_tok < __builtin_amdgcn_readlane(r_to, r);
+            const int key0 = (p_max / AF_KEYS - (__builtin_amdgcn_readlane(r_end, r) - 1 - b)) * AF_KEYS;
+            // S^T: lane (g, row j) gets the scores of keys key0 + 16 t + 4 g + r
+            f32x4 S[4];
+            bool there[4];                                        // keys 16 t + 4 g .. + 3 have a page (all four or none)
+            const float* vals[4];                                 // their values of head dim 0
+            const float* keys[4];
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const int key = min(key0 + 16 * t + j, p_max);    // (beyond the last key: that one again, not looked at)
-                    const int page = table[key / cache.page_size];
-                    const int held = page >= 0 && page < cache.n_pages ? page : 0;
-                    keys[t] = (const float*)cache.base + ((size_t)held * 2 * cache.n_kv_heads + kvh) * block +
-                              (size_t)(key % cache.page_size) * HD + 4 * g;
-                    const int key4 = key0 + 16 * t + 4 * g;           // (pages hold a multiple of four tokens)
-                    const int page4 = key4 <= p_max ? table[key4 / cache.page_size] : -1;
-                    there[t] = page4 >= 0 && page4 < cache.n_pages;
-                    vals[t] = (const float*)cache.base + ((size_t)(there[t] ? page4 : 0) * 2 * cache.n_kv_heads + cache.n_kv_heads + kvh) * block +
-                              (there[t] ? key4 % cache.page_size : 0) + (size_t)j * cache.page_size;
+            for (int t = 0; t < 4; ++t) {
+                const int key = min(key0 + 16 * t + j, p_max);    // (beyond the last key: that one again, not looked at)
+                const int page = table[key / cache.page_size];
+                const int held = page >= 0 && page < cache.n_pages ? page : 0;
+                keys[t] = (const float*)cache.base + ((size_t)held * 2 * cache.n_kv_heads + kvh) * block +
+                          (size_t)(key % cache.page_size) * HD + 4 * g;
+                const int key4 = key0 + 16 * t + 4 * g;           // (pages hold a multiple of four tokens)
+                const int page4 = key4 <= p_max ? table[key4 / cache.page_size] : -1;
+                there[t] = page4 >= 0 && page4 < cache.n_pages;
+                vals[t] = (const float*)cache.base + ((size_t)(there[t] ? page4 : 0) * 2 * cache.n_kv_heads + cache.n_kv_heads + kvh) * block +
+                          (there[t] ? key4 % cache.page_size : 0) + (size_t)j * cache.page_size;
+            }
+            // 16 keys at a time, the next 16 on their way (a wait for all of them at once would take the registers of 64)
+            f32x4 kf[2][NC];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) kf[0][c] = *(const f32x4*)(keys[0] + 16 * c);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                if (t < 3) {
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) kf[(t + 1) & 1][c] = *(const f32x4*)(keys[t + 1] + 16 * c);
                 }
-                // 16 keys at a time, the next 16 on their way (a wait for all of them at once would take the registers of 64)
-                f32x4 kf[2][NC];
-#pragma unroll
-                for (int c = 0; c < NC; ++c) kf[0][c] = *(const f32x4*)(keys[0] + 16 * c);
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    if (t < 3) {
-#pragma unroll
-                        for (int c = 0; c < NC; ++c) kf[(t + 1) & 1][c] = *(const f32x4*)(keys[t + 1] + 16 * c);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                    S[t] = scores<NC>(kf[t & 1], qv);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                f32x4 vf[AHEAD][4];                                   // values of 16 head dims, AHEAD times 16 on their way
-                auto fetch = [&](int d0, f32x4* to) {
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) to[t] = *(const f32x4*)(vals[t] + (size_t)d0 * cache.page_size);
-                };
-#pragma unroll
-                for (int a = 0; a < AHEAD; ++a) fetch(16 * a, vf[a]);
                 __builtin_amdgcn_sched_barrier(0);
+                S[t] = scores<NC>(kf[t & 1], qv);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            f32x4 vf[AHEAD][4];                                   // values of 16 head dims, AHEAD times 16 on their way
+            auto fetch = [&](int d0, f32x4* to) {
 #pragma unroll
-                for (int t = 0; t < 4; ++t) S[t] *= scale;
-                if (softcap > 0.f) {                                  // scores capped smoothly at +-softcap
+                for (int t = 0; t < 4; ++t) to[t] = *(const f32x4*)(vals[t] + (size_t)d0 * cache.page_size);
+            };
+#pragma unroll
+            for (int a = 0; a < AHEAD; ++a) fetch(16 * a, vf[a]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) S[t] *= scale;
+            if (softcap > 0.f) {                                  // scores capped smoothly at +-softcap
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) S[t][r] = softcap * tanhf(S[t][r] / softcap);
+            }
+            auto sees = [&](int t, int r) {                       // whether the row looks at key 16 t + 4 g + r
+                const int key = key0 + 16 * t + 4 * g + r;
+                return in_turn && there[t] && key >= my_lo && key <= my_p;
+            };
+            float m = -INFINITY;
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (sees(t, r)) m = fmaxf(m, S[t][r]);
+            m = fmaxf(m, __shfl_xor(m, 16, 64));
+            m = fmaxf(m, __shfl_xor(m, 32, 64));
+            const float base = m == -INFINITY ? 0.f : m;
+            bool any = false;
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const bool seen = sees(t, r);
+                    S[t][r] = seen ? expf(S[t][r] - base) : 0.f;
+                    any = any || seen;
+                }
+            const f32x4 four = (S[0] + S[1]) + (S[2] + S[3]);
+            float l = (four[0] + four[1]) + (four[2] + four[3]);
+            l += __shfl_xor(l, 16, 64);
+            l += __shfl_xor(l, 32, 64);
+            // lanes j, j + 16, j + 32, j + 48 hold row j's keys; -1: there are some, and every score is minus infinity
+            if (l == 0.f && ((__ballot(any) >> j) & 0x0001000100010001ull)) l = -1.f;
+            // O^T: four chains of 16 keys, instruction (t, r) the keys 16 t + 4 g + r; whatever lies behind a weight of zero
+            // counts only if it is no finite number, and then it shows in the sums
+            bool finite = true;
+#pragma unroll
+            for (int d0 = 0; d0 < HD; d0 += 16) {
+                f32x4 part[4];
+                f32x4* now = vf[d0 / 16 % AHEAD];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) part[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) part[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(now[t][r], S[t][r], part[t], 0, 0, 0);
+                if (d0 + 16 * AHEAD < HD) fetch(d0 + 16 * AHEAD, now);
+                const f32x4 o = (part[0] + part[1]) + (part[2] + part[3]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) finite = finite && isfinite(o[r]);
+                *(f32x4*)&part_a[wave][j][d0 + 4 * g] = o;
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (__any(!finite)) {
+#pragma unroll 1
+                for (int d0 = 0; d0 < HD; d0 += 16) {
+                    f32x4 val[4], part[4];
+                    fetch(d0, val);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        part[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            part[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(isfinite(val[t][r]) ? val[t][r] : 0.f, S[t][r], part[t], 0, 0, 0);
+                    }
+                    f32x4 o = (part[0] + part[1]) + (part[2] + part[3]);
 #pragma unroll
                     for (int t = 0; t < 4; ++t)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) S[t][r] = softcap * tanhf(S[t][r] / softcap);
-                }
-                auto sees = [&](int t, int r) {                       // whether the row looks at key 16 t + 4 g + r
-                    const int key = key0 + 16 * t + 4 * g + r;
-                    return in_turn && there[t] && key >= my_lo && key <= my_p;
-                };
-                float m = -INFINITY;
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (sees(t, r)) m = fmaxf(m, S[t][r]);
-                m = fmaxf(m, __shfl_xor(m, 16, 64));
-                m = fmaxf(m, __shfl_xor(m, 32, 64));
-                const float base = m == -INFINITY ? 0.f : m;
-                bool any = false;
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const bool seen = sees(t, r);
-                        S[t][r] = seen ? expf(S[t][r] - base) : 0.f;
-                        any = any || seen;
-                    }
-                const f32x4 four = (S[0] + S[1]) + (S[2] + S[3]);
-                float l = (four[0] + four[1]) + (four[2] + four[3]);
-                l += __shfl_xor(l, 16, 64);
-                l += __shfl_xor(l, 32, 64);
-                // lanes j, j + 16, j + 32, j + 48 hold row j's keys; -1: there are some, and every score is minus infinity
-                if (l == 0.f && ((__ballot(any) >> j) & 0x0001000100010001ull)) l = -1.f;
-                // O^T: four chains of 16 keys, instruction (t, r) the keys 16 t + 4 g + r; whatever lies behind a weight of zero
-                // counts only if it is no finite number, and then it shows in the sums
-                bool finite = true;
-#pragma unroll
-                for (int d0 = 0; d0 < HD; d0 += 16) {
-                    f32x4 part[4];
-                    f32x4* now = vf[d0 / 16 % AHEAD];
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) part[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-#pragma unroll
-                        for (int t = 0; t < 4; ++t) part[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(now[t][r], S[t][r], part[t], 0, 0, 0);
-                    if (d0 + 16 * AHEAD < HD) fetch(d0 + 16 * AHEAD, now);
-                    const f32x4 o = (part[0] + part[1]) + (part[2] + part[3]);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) finite = finite && isfinite(o[r]);
+                        for (int r = 0; r < 4; ++r) add_unbounded(o, val[t][r], S[t][r], sees(t, r));
                     *(f32x4*)&part_a[wave][j][d0 + 4 * g] = o;
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                if (__any(!finite)) {
-#pragma unroll 1
-                    for (int d0 = 0; d0 < HD; d0 += 16) {
-                        f32x4 val[4], part[4];
-                        fetch(d0, val);
-#pragma unroll
-                        for (int t = 0; t < 4; ++t) {
-                            part[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                            for (int r = 0; r < 4; ++r)
-                                part[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(isfinite(val[t][r]) ? val[t][r] : 0.f, S[t][r], part[t], 0, 0, 0);
-                        }
-                        f32x4 o = (part[0] + part[1]) + (part[2] + part[3]);
-#pragma unroll
-                        for (int t = 0; t < 4; ++t)
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) add_unbounded(o, val[t][r], S[t][r], sees(t, r));
-                        *(f32x4*)&part_a[wave][j][d0 + 4 * g] = o;
-                    }
-                }
-                if (g == 0) {
-                    part_m[wave][j] = m;
-                    part_l[wave][j] = l;
                 }
             }
-            __syncthreads();
-            const int blocks = min(AF_WAVES, last - b0 + 1);
-#pragma unroll
-            for (int u = 0; u < SUMS; ++u) {
-                const int e = threadIdx.x + 64 * AF_WAVES * u, row = e / FOURS, d = 4 * (e % FOURS);
-                if (row < AF_ROWS && row / heads >= from && row / heads < to) {
-                    for (int w = 0; w < blocks; ++w) {
-                        const float m = part_m[w][row], l = part_l[w][row];
-                        if (l == 0.f) continue;                       // no key of this row in the block
-                        if (l < 0.f) {
-                            low[u] = true;
-                            continue;
-                        }
-                        const float top = fmaxf(M[u], m), old = expf(M[u] - top), now = expf(m - top);
-                        const f32x4 a = *(const f32x4*)&part_a[w][row][d];
-                        L[u] = L[u] * old + l * now;
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) A[u][r] = A[u][r] * old + a[r] * now;
-                        M[u] = top;
-                    }
-                }
+            if (g == 0) {
+                part_m[wave][j] = m;
+                part_l[wave][j] = l;
             }
-            __syncthreads();
         }
-        from = to;
+        __syncthreads();
+        const int formed = min(AF_WAVES, blocks - b0);
+#pragma unroll
+        for (int u = 0; u < SUMS; ++u) {
+            const int e = threadIdx.x + 64 * AF_WAVES * u, row = e / FOURS, d = 4 * (e % FOURS);
+            if (row < AF_ROWS) {
+                for (int w = 0; w < formed; ++w) {
+                    const float m = part_m[w][row], l = part_l[w][row];
+                    if (l == 0.f) continue;                           // no key of this row in the block
+                    if (l < 0.f) {
+                        low[u] = true;
+                        continue;
+                    }
+                    const float top = fmaxf(M[u], m), old = expf(M[u] - top), now = expf(m - top);
+                    const f32x4 a = *(const f32x4*)&part_a[w][row][d];
+                    L[u] = L[u] * old + l * now;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) A[u][r] = A[u][r] * old + a[r] * now;
+                    M[u] = top;
+                }
+            }
+        }
+        __syncthreads();
     }
 #pragma unroll
     for (int u = 0; u < SUMS; ++u) {
@@ -297,8 +315,10 @@ void attn_float_launch(const float* q, float* out, const PagedCache& cache, cons
                        const int* block_table, int max_blocks, int n, int nh, float scale, int window, float softcap,
                        const float* sink, hipStream_t stream) {
     const int group = nh / cache.n_kv_heads, heads = min(group, AF_ROWS), head_tiles = ceil_div(group, heads);
-    // as many tokens as fill the rows, unless a tile per token is at most two per unit (few tokens, most often of as many requests)
-    const int tokens = (long)n * cache.n_kv_heads * head_tiles <= 2 * fl_units() ? 1 : AF_ROWS / heads;
+    // A unit holds one thread block at a time: as few tokens per tile as still give every unit at most one, up to what
+    // fills the rows.
+    const int per_head = fl_units() / (cache.n_kv_heads * head_tiles);
+    const int tokens = per_head > 0 ? min(AF_ROWS / heads, ceil_div(n, per_head)) : AF_ROWS / heads;
     const dim3 grid(ceil_div(n, tokens), cache.n_kv_heads * head_tiles);
     if (cache.head_dim == 64)
         attn_float_kernel<64><<<grid, 64 * AF_WAVES, 0, stream>>>(q, out, cache, positions, tok_seq, block_table, max_blocks, n, nh,
