@@ -9,7 +9,11 @@
 // leaves (M, L, A) as it is.  So neither the rows of a tile, nor how a prompt is cut, nor who forms a block shows.
 // A block's weights add up to at least 1 where it has a score above minus infinity, and to NaN where a score is NaN (or
 // plus infinity), which a maximum would pass by: the sum tells whether a block counts, never the maximum.  A row
-// whose scores are all minus infinity is NaN, as the formula has it.
+// whose scores are all minus infinity is NaN, as the formula has it.  A value that is no finite number reaches the rows
+// that see its key and no other, although a tile's rows share the values: where a block's sums are not all finite
+// they are formed again, such values as zero and then row by row (add_unbounded).
+// A row whose keys fit into AF_FEW positions (from a multiple of four on) is a wave's own work instead
+// (attn_float_few): whether it is one, the row's position and the window alone decide.
 //
 // Block of threads = a tile of up to 16 rows (token, query head) that read one key/value head: T tokens by its query
 // heads (T = 1 in steps of few tokens, where the heads alone have to fill the chip).  Eight waves form eight blocks of
@@ -21,17 +25,25 @@
 // give as an operand of O^T = V^T P^T if instruction (t, r) takes those keys, and the values of four neighbouring keys
 // are 16 bytes of the transposed page.
 //
-// Bound by the chain look-up of the page, loads, 256 matrix instructions of 32 clocks, adding up.  32 heads of 128 over 8:
-// a prompt of 333 tokens 59 us (553 with attn_plain_kernel, a block per token and head that goes through its keys one by
-// one), one token behind 340 24 us (161).
+// Bound by the chain look-up of the page, loads, 256 matrix instructions of 32 clocks, adding up.  Microseconds with 32
+// heads of 128 over 8 (attn_plain_kernel, a block per token and head that goes through its keys one by one): a prompt of
+// 333 tokens 48.6 (527), of 100 14.8 (67); one token behind 340 19.7 (88), behind 4,000 137 (1,526); 64 tokens behind 340
+// 36 (213), behind 17 6.8 (15.7), behind 1 5.3 (4.8).  With a key head for each of the 32 heads, 64 tokens behind 100
+// 44 (72).  Error against 64 bits beside that kernel's: 0.96 to 1.0 up to 64 keys, 0.92, 0.72, 0.56, 0.43 at 100, 340,
+// 1,000, 4,000.
 #include "attn_float.h"
+#include "lanes.h"
 
 #define AF_WAVES 8
 #define AF_ROWS 16
 #define AF_KEYS 64
+// Rows of 33 to 48 keys: 6.1 us against 11.7 on the matrix cores (eight tokens, as above), and 0.97 against 1.07 times the
+// plain kernel's error; with 64 a prompt of 100 tokens took 16.9 us instead of 14.8 (a tile's rows share matrix
+// instructions, here a wave has one or two rows after the other).
+#define AF_FEW 48
 
 // The scores of 16 keys: chains of two instructions from zero, their results added in a tree.  Longer chains lose
-// more: the error against 64 bits, beside the plain kernel's, is 0.98, 0.92, 0.72 and 0.56 times at 64, 100, 340 and
+// more: the error against 64 bits, beside the plain kernel's, was 0.98, 0.92, 0.72 and 0.56 times at 64, 100, 340 and
 // 1,000 keys, with chains of 16 products 1.05, 1.03, 0.89, 0.63, with chains of 32 (and the values of a block in one
 // chain) 1.41, 1.30, 1.11, 0.76.  A result is added two chains after its own, so that no addition waits for the
 // matrix unit.
@@ -74,6 +86,91 @@ __device__ __forceinline__ void add_unbounded(f32x4& o, float v, float weight, b
     }
 }
 
+// The result of one row with at most AF_FEW keys from position lo4 on (lo rounded down to a multiple of four), by one
+// wave on the vector unit: 256 matrix instructions for a handful of keys, most of them for nothing, take 7 us.  Lane
+// (g, j) forms a share of four dims in 64 of the scores of keys 4 i + g, i = 0 .. 15, keeps that of i = j, and holds two
+// (one) of the head dims when the values are added, in four chains of every fourth key.
+template <int HD>
+__device__ __forceinline__ void attn_float_few(const float* __restrict__ q, float* __restrict__ out, const PagedCache& cache,
+                                               const int* __restrict__ table, int kvh, int lo, int p, float scale, float softcap,
+                                               const float* __restrict__ sink) {
+    constexpr int NV = HD / 64;                                       // pieces of four dims of a key, and dims of a value, per lane
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    const int lo4 = lo & ~3, groups = (p - lo4 + 4) >> 2;             // groups of four keys, which share a page
+    const size_t block = (size_t)cache.page_size * HD;
+    const int at = lo4 + 4 * min(j, groups - 1);
+    const int page = table[at / cache.page_size], row = at % cache.page_size;
+    const bool there = page >= 0 && page < cache.n_pages;
+    const int held = there ? page : 0;                                // (lane i knows group i's page and row)
+    const bool seen = there && j < groups && lo4 + 4 * j + g >= lo && lo4 + 4 * j + g <= p;
+    f32x4 qv[NV];
+#pragma unroll
+    for (int c = 0; c < NV; ++c) qv[c] = *(const f32x4*)(q + 64 * c + 4 * j);
+    auto base_of = [&](int i, int is_v) {
+        return (const float*)cache.base + (((size_t)__builtin_amdgcn_readlane(held, i) * 2 + is_v) * cache.n_kv_heads + kvh) * block;
+    };
+    f32x4 vf[4][NV];
+    auto values = [&](int i0) {                                       // of four groups (behind the last one it is that one again)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const int i = min(i0 + a, groups - 1);
+            const float* v = base_of(i, 1) + __builtin_amdgcn_readlane(row, i);
+#pragma unroll
+            for (int d = 0; d < NV; ++d) vf[a][d] = *(const f32x4*)(v + (size_t)(64 * d + lane) * cache.page_size);
+        }
+    };
+    float s = 0.f;
+    for (int i0 = 0; i0 < groups; i0 += 4) {
+        f32x4 kf[4][NV];
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const int i = min(i0 + a, groups - 1);
+            const float* k = base_of(i, 0) + (size_t)(__builtin_amdgcn_readlane(row, i) + g) * HD;
+#pragma unroll
+            for (int d = 0; d < NV; ++d) kf[a][d] = *(const f32x4*)(k + 64 * d + 4 * j);
+        }
+        if (i0 == 0) values(0);
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            float part[NV];
+#pragma unroll
+            for (int d = 0; d < NV; ++d) {
+                part[d] = kf[a][d][0] * qv[d][0];
+#pragma unroll
+                for (int r = 1; r < 4; ++r) part[d] = fmaf(kf[a][d][r], qv[d][r], part[d]);
+            }
+            const float sum = row_sum16(NV == 2 ? part[0] + part[NV - 1] : part[0]);
+            if (i0 + a == j) s = sum;
+        }
+    }
+    s *= scale;
+    if (softcap > 0.f) s = softcap * tanhf(s / softcap);              // scores capped smoothly at +-softcap
+    const float m = wave_max(seen ? s : -INFINITY), base = m == -INFINITY ? 0.f : m;
+    const float weight = seen ? expf(s - base) : 0.f;
+    const float l = wave_sum(weight);
+    const unsigned long long sees = __ballot(seen);
+    f32x4 acc[NV];
+#pragma unroll
+    for (int c = 0; c < NV; ++c) acc[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int i0 = 0; i0 < groups; i0 += 4) {
+        if (i0) values(i0);
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int from = 16 * e + i0 + a;                     // (behind the last group: seen by nobody)
+                const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), from));
+                const bool counts = (sees >> from) & 1;
+#pragma unroll
+                for (int d = 0; d < NV; ++d) acc[d][e] = fmaf(w, counts ? vf[a][d][e] : 0.f, acc[d][e]);
+            }
+    }
+    const float none = sees ? NAN : 0.f;                              // every score minus infinity, or no key at all
+    const float inv = sink ? softmax_factor_with_sink(m, l, *sink) : l == 0.f ? none : 1.0f / l;
+#pragma unroll
+    for (int c = 0; c < NV; ++c) out[64 * c + lane] = ((acc[c][0] + acc[c][1]) + (acc[c][2] + acc[c][3])) * inv;
+}
+
 template <int HD>
 __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const float* __restrict__ q, float* __restrict__ out,
                                                                       PagedCache cache, const int* __restrict__ positions,
@@ -94,9 +191,21 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
     const int n_heads = min(heads, group - h0);
     // row j: token j / heads, query head j % heads of the tile
     const int my_tok = j / heads, my_head = j % heads;
-    const bool my_row = my_tok < n_tok && my_head < n_heads;
     const int at_tok = tok0 + min(my_tok, n_tok - 1), at_head = kvh * group + h0 + min(my_head, n_heads - 1);
     const int my_p = positions[at_tok], my_lo = window > 0 ? max(0, my_p - window + 1) : 0;
+    const bool my_row = my_tok < n_tok && my_head < n_heads && my_p - (my_lo & ~3) >= AF_FEW;
+    // Rows of few keys, a wave each.  (Lane `row` knows whether that row is one.)
+    const unsigned few = (unsigned)__ballot(g == 0 && my_tok < n_tok && my_head < n_heads && my_p - (my_lo & ~3) < AF_FEW);
+    int dealt = 0;
+    for (unsigned rest = few; rest; rest &= rest - 1, ++dealt) {
+        if (dealt % AF_WAVES != wave) continue;
+        const int row = __ffs(rest) - 1, tok = tok0 + row / heads, head = kvh * group + h0 + row % heads;
+        const int p = __builtin_amdgcn_readlane(my_p, row), lo = __builtin_amdgcn_readlane(my_lo, row);
+        const size_t at = ((size_t)tok * nh + head) * HD;
+        attn_float_few<HD>(q + at, out + at, cache, block_table + (size_t)tok_seq[tok] * max_blocks, kvh, lo, p, scale, softcap,
+                           sink ? sink + head : nullptr);
+    }
+    if (!__any(my_row)) return;                                       // (the same in every wave)
     f32x4 qv[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) qv[c] = *(const f32x4*)(q + ((size_t)at_tok * nh + at_head) * HD + 16 * c + 4 * g);
@@ -123,6 +232,7 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
         int p_max = -1, p_min = 0x7fffffff;
         for (to = from; to < n_tok && __builtin_amdgcn_readlane(lane_seq, to) == seq; ++to) {
             const int p = __builtin_amdgcn_readlane(lane_p, to);
+            if (p - ((window > 0 ? max(0, p - window + 1) : 0) & ~3) < AF_FEW) continue;
             p_max = max(p_max, p);
             p_min = min(p_min, p);
         }
@@ -139,8 +249,9 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
         }
         ++requests;
     }
+    const int slot = (wave + AF_WAVES - dealt % AF_WAVES) % AF_WAVES;  // (first the waves that had a row of few keys less)
     for (int b0 = 0; b0 < blocks; b0 += AF_WAVES) {
-        const int b = b0 + wave;
+        const int b = b0 + slot;
         if (b < blocks) {
             const int r = __ffsll(__ballot(lane < requests && r_end > b)) - 1;
             const int p_max = __builtin_amdgcn_readlane(r_max, r), lo_min = __builtin_amdgcn_readlane(r_min, r);
@@ -240,7 +351,7 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
                 const f32x4 o = (part[0] + part[1]) + (part[2] + part[3]);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) finite = finite && isfinite(o[r]);
-                *(f32x4*)&part_a[wave][j][d0 + 4 * g] = o;
+                *(f32x4*)&part_a[slot][j][d0 + 4 * g] = o;
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (__any(!finite)) {
@@ -260,12 +371,12 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
                     for (int t = 0; t < 4; ++t)
 #pragma unroll
                         for (int r = 0; r < 4; ++r) add_unbounded(o, val[t][r], S[t][r], sees(t, r));
-                    *(f32x4*)&part_a[wave][j][d0 + 4 * g] = o;
+                    *(f32x4*)&part_a[slot][j][d0 + 4 * g] = o;
                 }
             }
             if (g == 0) {
-                part_m[wave][j] = m;
-                part_l[wave][j] = l;
+                part_m[slot][j] = m;
+                part_l[slot][j] = l;
             }
         }
         __syncthreads();
@@ -296,7 +407,7 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void attn_float_kernel(const floa
     for (int u = 0; u < SUMS; ++u) {
         const int e = threadIdx.x + 64 * AF_WAVES * u, row = e / FOURS, d = 4 * (e % FOURS);
         const int tok = row / heads, hh = row % heads;
-        if (row >= AF_ROWS || tok >= n_tok || hh >= n_heads) continue;
+        if (row >= AF_ROWS || tok >= n_tok || hh >= n_heads || ((few >> row) & 1)) continue;
         const int head = kvh * group + h0 + hh;
         const float none = low[u] ? NAN : 0.f;                        // (NaN, or no key at all)
         const float inv = sink ? softmax_factor_with_sink(M[u], L[u], sink[head]) : L[u] == 0.f ? none : 1.0f / L[u];
