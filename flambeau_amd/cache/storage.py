@@ -83,13 +83,13 @@ class CacheStorage:
                 runs[-1][1] += 1
             else:
                 runs.append([slot, slot + 1])
-        # A fill per run needs nothing from the host but its launch; a list of slots has to be copied to the device, and
-        # that copy waits for all work before it (300 to 500 us between two prompts of 2,048 tokens).  With more
-        # than two runs the launches, one per table and run, would cost more than the wait.
-        if len(runs) <= 2 and runs[0][0] >= 0 and runs[-1][1] <= min(len(t) for t in tables):
-            for t in tables:
-                for first, end in runs:
-                    t[first:end].zero_()
+        # Fills need nothing from the host but their launch, one for all tables of a type; a list of slots has to be copied
+        # to the device, and that copy waits for all work before it (300 to 500 us between two prompts of 2,048 tokens).
+        # Microseconds with nothing to wait for, 16 / 64 / 128 tables: the list 142 / 370 / 692 for any slots, fills 35 / 83 /
+        # 155 with one run, 48 / 153 / 288 with two, 79 / 274 / 532 with four, which is where they end.
+        if len(runs) <= 4 and runs[0][0] >= 0 and runs[-1][1] <= min(len(t) for t in tables):
+            for dtype in {t.dtype for t in tables}:
+                torch._foreach_zero_([t[first:end] for t in tables if t.dtype == dtype for first, end in runs])
             return
         idx = torch.tensor([s for first, end in runs for s in range(first, end)], dtype=torch.long, device=tables[0].device)
         for t in tables:

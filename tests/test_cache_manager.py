@@ -144,7 +144,7 @@ def test_random_orders_keep_the_books(seed):
     assert m.free_pages() == [12] * len(windows) and m.n_free_slots == 4
 
 
-@pytest.mark.parametrize("slots", [[], [0], [6], [2, 3, 4], [4, 2, 3, 2], [0, 1, 5, 6], [0, 2, 4], [6, 1, 3, 0], list(range(7))])
+@pytest.mark.parametrize("slots", [[], [0], [6], [2, 3, 4], [4, 2, 3, 2], [0, 1, 5, 6], [0, 2, 4], [6, 1, 3, 0], [0, 2, 4, 6], list(range(7))])
 def test_claimed_slots_start_from_zero_whatever_their_order(slots):
     import torch
     from flambeau_amd.cache.storage import CacheStorage
@@ -165,3 +165,24 @@ def test_a_slot_that_does_not_exist_is_refused(slots):
     store.states = {0: torch.full((7, 6), 3.0)}
     with pytest.raises(IndexError):
         store.zero_slots(slots)
+
+
+@pytest.mark.parametrize("slots", [[3], [0, 5], [1, 2, 6]])
+def test_claimed_slots_are_cleared_by_one_fill_per_type(slots):
+    """Not by one per table and run: with two runs of 128 tables that took twice as long as the list of slots before."""
+    import torch
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from flambeau_amd.cache.storage import CacheStorage
+    store = CacheStorage([], [], torch.device("cpu"), torch.float32, n_pages=1, page_size=8, max_slots=7)
+    store.states = {i: torch.full((7, 6), 3.0) for i in range(5)}
+    store.records = {0: {"window": torch.full((7, 3), 4, dtype=torch.int32)}}
+    writes = []
+
+    class Writes(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if func.overloadpacket.__name__.endswith("_"):
+                writes.append(func)
+            return func(*args, **(kwargs or {}))
+    with Writes():
+        store.zero_slots(slots)
+    assert len(writes) == 2 and not any(t[slots].any() for t in [*store.states.values(), store.records[0]["window"]])
