@@ -40,7 +40,9 @@
 // wave has its SIMD to itself; sixteen waves with a column each, the sums over 64 lanes, took as long: 285 us fixed,
 // 580 delta), and the trips to LDS.  So a token's values are read from LDS into registers AHEAD tokens before their
 // turn (four; two where a token of eight rows brings a decay per key dim, or has sixteen rows: four of them left the
-// compiler moving registers, 357 us gated; none beyond 256 key dims), the sums over
+// compiler moving registers, 357 us gated; none beyond 256 key dims; with 129 to 255 dims as many as leave registers for
+// three blocks on a unit, because a step of one token per request waits for states: 64 of 8 heads of 160 x 64 36 us
+// with three, 40 with two, 35 in the kernel that read no token ahead), the sums over
 // lanes of four tokens' outputs are formed together, and the 16 lanes of a column, which all hold a token's sum,
 // keep one of 16 tokens' outputs each and store them at once.  WHOLE: 16 RPT key dims, a multiple of 16 columns, rows
 // and records in whole 16-byte pieces: loads without conditions, four values at a time (rows behind the request's
@@ -56,7 +58,7 @@
 // 4: such a decay without the correction (gated linear attention: u = v); 5: a decay and a write strength per token and
 // head without the correction (u = beta v), and skip[head] v added to what is read out
 template <int RPT, int MODE, bool WHOLE>
-__global__ __launch_bounds__(LS_GROUP * LS_COLS) void linear_scan_kernel(
+__global__ __launch_bounds__(LS_GROUP * LS_COLS, RPT == 16 && !WHOLE ? 3 : 1) void linear_scan_kernel(
     const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk, const float* __restrict__ v, int ldv,
     const float* __restrict__ head_decay, const float* __restrict__ tok_decay, const float* __restrict__ beta, int ldg,
     float* __restrict__ state, size_t slot_stride, const int* __restrict__ seq_q_start, const int* __restrict__ seq_q_len,
@@ -66,7 +68,7 @@ __global__ __launch_bounds__(LS_GROUP * LS_COLS) void linear_scan_kernel(
     constexpr int NT = LS_GROUP * LS_COLS;
     constexpr int DP = LS_GROUP * RPT;                                // a row of q or k in LDS
     constexpr int RUN = RPT <= 8 ? 32 : RPT <= 16 ? 16 : 8;          // tokens per run
-    constexpr int AHEAD = RPT > 16 ? 0 : RPT > 8 || (CHAN && RPT == 8) ? 2 : 4;   // tokens whose values wait in registers (as many as fit)
+    constexpr int AHEAD = RPT > 16 ? 0 : CHAN && RPT == 16 && !WHOLE ? 1 : RPT > 8 || (CHAN && RPT == 8) ? 2 : 4;   // tokens whose values wait in registers (as many as fit)
     constexpr int VEC = WHOLE ? 4 : 1;                               // values per load
     constexpr int PRE = RUN * DP / NT / VEC;                          // loads of q (and k) of a run per thread
     constexpr int PRE_V = (RUN * LS_COLS + NT - 1) / NT;
