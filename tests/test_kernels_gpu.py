@@ -694,11 +694,11 @@ def test_gemm_tiled_against_plain(out_dtype, M, N, K):
     assert (got.double() - ref).abs().max() < tol * scale
 
 
-@pytest.mark.parametrize("variant", [3, 6, 7, 8, 10])
-@pytest.mark.parametrize("M,N,K", [(300, 520, 72), (129, 264, 96), (1100, 640, 256)])
+@pytest.mark.parametrize("variant", [3, 6, 7, 8, 10, 11, 12, 13, 14])
+@pytest.mark.parametrize("M,N,K", [(300, 520, 72), (129, 264, 96), (1100, 640, 256), (400, 452, 1032)])
 def test_gemm_tiled_block_shapes(variant, M, N, K):
-    """Every block shape of the tiled product (256 x 128, 192 x 128, 128 x 128, 256 x 256 and 128 x 256
-    features x tokens), whichever the sizes would choose, through the plain epilogue, SwiGLU, the row scale and
+    """Every block shape of the tiled product (features x tokens: 256, 192 or 128 x 128; 256, 224, 192 or 128 x 256;
+    128 x 128 alone on its unit; 224 x 192), whichever the sizes would choose, through the plain epilogue, SwiGLU, the row scale and
     the add-to-the-stream epilogue."""
     from flambeau_amd.kernels.library import load
     from flambeau_amd.kernels.packing import pack_weight
@@ -900,7 +900,7 @@ def test_gemm_with_rotation_and_stores_in_its_kernel(M, nh, nkv, hd, rot, ps, H)
         assert torch.equal(q_a, q_b) and torch.equal(cache_a.pool, cache_b.pool)      # the same sums in the same order
     elif M > 64:
         # every block shape of the tiled product writes the same
-        for variant in (3, 6, 7, 8, 10):
+        for variant in (3, 6, 7, 8, 10, 11, 12, 13, 14):
             cache_v = make_cache(n_pages, nkv, ps, hd, torch.bfloat16)
             q_v = torch.full((M, nh * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
             store_v = tuned().RopeStore(pos_d, seq_d, table, angles, q_v, cache_v, nh, rot, True)
@@ -1181,10 +1181,12 @@ def test_gemm_swiglu_epilogue(out_dtype, M, I, K):
 
 
 # ---------------------------------------------------------------- the 32-bit product on the matrix cores
-@pytest.mark.parametrize("M", [1, 4, 5, 16, 17, 32, 33, 48, 65, 97])
-@pytest.mark.parametrize("N,K", [(1, 4), (15, 16), (17, 20), (64, 36), (65, 256), (130, 260), (192, 516), (31, 1040)])
+@pytest.mark.parametrize("M,N,K", [(M, N, K) for N, K in [(1, 4), (15, 16), (17, 20), (64, 36), (65, 256), (130, 260), (192, 516), (31, 1040)]
+                                   for M in [1, 4, 5, 16, 17, 32, 33, 48, 49, 64, 65, 97, 150]] +
+                         [(40, 8192, 36), (40, 8196, 36), (64, 8192, 68), (64, 8260, 516), (33, 4096, 14336)])
 def test_gemm_float_gives_the_plain_kernel_s_bits(M, N, K):
-    """Rows that do not begin at 16 bytes go to the plain kernel, whose sums these are: equal to the last bit."""
+    """Every kernel for few rows (to 4, 16, 32, 48, 64) and for many (32, 48 and 64 a block), both sides of each rule between
+    them.  Rows that do not begin at 16 bytes go to the plain kernel, whose sums these are: equal to the last bit."""
     def at(offset, rows, seed):
         buf = torch.empty(rows * K + 4, dtype=torch.float32, device=DEV)
         view = buf[offset:offset + rows * K].view(rows, K)
