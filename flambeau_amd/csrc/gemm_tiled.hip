@@ -455,26 +455,27 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 // here, together with the number of K-splits.  The entry points whose names end in _ex take either from the caller,
 // for tests and measurements.
 //
-// What a shape costs.  Four waves, two blocks per unit: bound by the copies into LDS, 0.056 us per k-step and
-// round of resident blocks plus 17.7 ns per KB that a unit's blocks copy, 0.6 of it from the mean and 0.4
-// from the unit with the most blocks.  Four waves alone on their unit have the whole LDS for stages on their way:
-// 0.30 us per k-step, weights from HBM at 4 TB/s where three stages reach 3.5 (28672 x 4096 at 64 rows 50.9 us
-// against 57.2, at 128 60.6 against 63.7, 28672 x 5120 at 64 rows 63.8 against 74.3; only where
-// more than three quarters of the units get a block and none gets a second: 207 rows 91.5 against 77.9 with 256 features).  Eight waves, one block after the other: bound by the
-// matrix cores and by the wait for weights from HBM, 0.22 us + 1.6 ns per feature and k-step (with 192 tokens 0.18 us
-// + 1.5 ns), and 3.7 us per block that nothing overlaps.  Splitting K adds the parts' way to memory and back and the
-// kernel that sums them.  What decides
-// between 256, 224 and 192 features is how evenly the blocks fill the rounds: gate/up of 2,048 rows, 28672
+// What a shape costs, in us.  Four waves, two blocks per unit: bound by the copies into LDS, per k-step 0.115 a round of
+// resident blocks and 0.0193 per KB that a unit's blocks copy, 0.8 of it from the mean and 0.2 from the unit with the most
+// blocks; a tile of w that few tiles of tokens share comes from HBM more often (a quarter more with one of them), and
+// blocks of 128 features copy 9 % faster.  Four waves alone on their unit have the whole LDS for stages on their way:
+// 0.377 per k-step, less where the tile's rows are few (28672 x 4096 at 65 rows 55.5 against 64 with three stages, at 97
+// 59.5 against 63).  Eight waves, one block after the other: bound by the matrix cores and by the wait for weights,
+// 0.69, 0.66, 0.60 per k-step with 256, 224, 192 features and 0.56 with 224 x 192, less where a tile's rows are few,
+// more where a unit gets a second block of another part of K, and 6 per block that nothing overlaps.  Splitting K adds the
+// parts' way to memory and back and the kernel that sums them: 2.38 us per million values and part.
+// What decides between 256, 224 and 192 features is how evenly the blocks fill the rounds: gate/up of 2,048 rows, 28672
 // features, is 3.5 rounds of 256 (422 us with its activation) and 4 of 224 (408; 512 with 4 waves before those
 // of a pair took turns), q/k/v of 2,048 rows, 6144 features, 0.75 rounds of 256 (108 us with its rotation) and 1
-// of 192 (102; 115 with 256 x 128).  192 tokens are for rows that end soon behind a multiple of 256: 28672 x 4096
-// at 333 rows 90 us (96.6 with 256 tokens), 528 rows 157 (160; 167 with the 192 features chosen without it), 1,040
-// rows 252 (257); 28672 x 5120 at 1,040 rows 318 (329).  224 x 224 does not divide among the waves, 192 x 192 and
-// 256 x 192 gained nothing beside it (528 rows 161.8 and 168).
-// Against every shape and number of parts measured (products of 7B, 12B and 24B sizes at 14 row counts from 64
-// to 4,001, cold weights, parts of K 1 to 4 and 6; 140 products, 3,000 timings) the formula's picks take 1.3 % more
-// time than the best on average and 14 % at worst (5120 x 14336 at 384 rows, 91 us against 80), 2.5 % less
-// than the picks among the shapes without 13 and 14.
+// of 192 (102; 115 with 256 x 128).  192 tokens are mostly for rows that end soon behind a multiple of 256: 28672 x 4096
+// at 333 rows 90 us (96.6 with 256 tokens), 528 rows 157 (160), 1,040 rows 252 (257).  224 x 224 does not divide among
+// the waves, 192 x 192 and 256 x 192 gained nothing beside it (528 rows 161.8 and 168).
+// The constants are those that pick best among all that may be picked: 14 products (7B, 12B and 24B sizes and layers of
+// width 2,048, each with the epilogue that it runs with: rotation and stores, sum into the stream, activation, none; where
+// K is split with the kernel that adds the parts) at 50 row counts from 65 to 4,001, weights from HBM, every shape with 1
+// to 6 and 8 parts, 26,000 timings.  Picks take 0.9 % more time than the best on average and 16 % at worst (4096 x 4096
+// at 768 rows, 53.7 against 46.2).  A formula fitted to plain products and fewer numbers of parts, with no sharing of w
+// and no rows per tile in it, was 1.9 % off and 44 % at worst (6144 x 5120 at 700 rows; 5120 x 32768 at 1,040 473 us against 358).
 struct TileShape { int variant, features, tokens, per_unit; };
 static const TileShape g_shapes[] = {{3, 256, 128, 2}, {7, 192, 128, 2}, {8, 128, 128, 2}, {10, 256, 256, 1}, {11, 224, 256, 1}, {12, 192, 256, 1}, {6, 128, 256, 1}, {13, 128, 128, 1}, {14, 224, 192, 1}};
 static const TileShape& tile_shape(int variant) {
@@ -491,12 +492,20 @@ static float tiled_cost(const TileShape& t, int splits, int M, int N, int K) {
     const long most = (blocks + units - 1) / units;                    // blocks of the unit with the most
     const long rounds = (most + t.per_unit - 1) / t.per_unit;
     const float mean = blocks > units ? (float)blocks / units : 1.f;
-    const float kb = (t.features + t.tokens) * 64 / 1024.f;            // copied per block and k-step
+    const int m_tiles = ceil_div(M, t.tokens);
+    const float empty = 1.f - (float)M / ((long)m_tiles * t.tokens);   // share of the tiles' rows that are none
     float us;
-    if (t.variant == 13) us = blocks > units || 4 * blocks <= 3 * units ? 1e9f : steps * 0.30f + 3.2f;
-    else if (t.per_unit == 1) us = most * (steps * (0.217f + 0.00163f * t.features - (1.f - t.tokens / 256.f) * (0.137f + 0.00036f * t.features)) + 3.7f) + 0.86f;
-    else us = steps * (0.056f * rounds + 0.0177f * kb * (0.6f * mean + 0.4f * most)) + 2.33f;
-    if (splits > 1) us += 3.f + (float)M * N * 4.f * (2 * splits + 1) / 4.5e6f;
+    if (t.variant == 14 && empty > 0.375f) return 1e9f;                // (tiles with so few rows: 28672 x 5120 at 207 rows 112.8 us, 106.4 with 256 x 128)
+    if (t.variant == 13) {
+        us = most * steps * (0.377f - 0.104f * empty) + 1.72f;
+    } else if (t.per_unit == 1) {
+        const float step = t.variant == 14 ? 0.563f : t.features == 256 ? 0.689f : t.features == 224 ? 0.662f : 0.601f;
+        us = most * (steps * (step * (1.f + 0.0864f / m_tiles + (splits > 1 && most > 1 ? 0.0543f : 0.f)) - 0.0736f * empty * t.tokens / 256.f) + 6.06f);
+    } else {
+        const float kb = (t.features * (1.f + 0.276f / m_tiles) + t.tokens) * 64 / 1024.f;      // copied per block and k-step
+        us = steps * (0.115f * rounds + (t.features == 128 ? 0.0175f : 0.0193f) * kb * (0.8f * mean + 0.2f * most));
+    }
+    if (splits > 1) us += 2.38e-6f * M * N * splits;
     return us;
 }
 

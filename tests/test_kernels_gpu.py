@@ -743,6 +743,22 @@ def test_gemm_tiled_block_shapes(variant, M, N, K):
         assert (out2.double() - ref2).abs().max() < 1e-2 * ref2.abs().max()
 
 
+@pytest.mark.parametrize("M,N,K,gate,variant,splits", [(1040, 5120, 32768, False, 11, 2), (384, 16384, 2048, True, 8, 1)])
+def test_gemm_tiled_plan_knows_what_is_faster(M, N, K, gate, variant, splits):
+    """Block shapes and parts that are a fifth faster than what the plan once picked for these sizes (473 and 50 us against
+    358 and 40): what it picks now is within a tenth of them.  Weights from memory: enough copies that none stays in a
+    cache."""
+    copies = max(2, -(-600_000_000 // (2 * N * K)))
+    w = [rnd(N * K, dtype=torch.bfloat16, seed=22, scale=0.05) for _ in range(copies)]       # (N, K multiples of a tile: any values are a packed matrix)
+    x, out = rnd(M, K, dtype=torch.bfloat16, seed=21), torch.empty(M, N // 2 if gate else N, dtype=torch.bfloat16, device=DEV)
+    ws = torch.empty(8 * M * N, dtype=torch.float32, device=DEV)
+    times = []
+    for v, s in ((variant, splits), (0, 0)):
+        turn = iter(range(1 << 30))
+        times.append(time_of(lambda: tuned().gemm_tiled(x, w[next(turn) % copies], out, ws, swiglu_rows=N if gate else 0, variant=v, splits=s)))
+    assert times[1] < 1.1 * times[0], times
+
+
 def test_gemm_tiled_splits_k_for_small_grids():
     assert tuned().gemm_tiled_splits(2048, 4096, 4096) == 1
     assert tuned().gemm_tiled_splits(128, 4096, 4096) > 1
