@@ -9,8 +9,8 @@
 // are independent of one another; only the compensated addition, four operations per chunk, is serial.
 //
 // Operand of the instruction for the chunk's k = 4 s .. 4 s + 3 (s = 0 .. 3): lane l gives row l % 16 at
-// k = 4 s + l / 16.  Rows lie in LDS as in memory, 4 floats apart more than a multiple of 64 banks, so that the
-// 16 rows x 4 neighbours of a read meet no bank twice.
+// k = 4 s + l / 16.  Rows lie in LDS as in memory, an odd multiple of 4 floats apart (68 or 36): 16 such rows
+// begin at 16 different multiples of 4 of the 64 banks, so that the 16 rows x 4 neighbours of a read meet no bank twice.
 //
 // Two kernels: `few` streams w for a few rows of x (bound by HBM), `many` tiles both (bound by the matrix and the
 // vector unit, which 32-bit matrix instructions share: 128 clocks of products and 64 of compensated additions per
