@@ -255,10 +255,21 @@ __global__ __launch_bounds__(256, 2) void gemm_float_many_kernel(const float* __
     }
 }
 
+// Which of the two kernels takes a product (gemm_float_launch says why).
+static bool gf_few(int M, int N) { return M <= 32 || (M <= 64 && N <= 8192); }
+
 bool gemm_float_takes(const void* x, const void* w, const void* out, int M, int N, int K) {
     // 16-byte pieces of rows; a grid of fewer than 2^31 blocks, and 64 rows within a 32-bit offset
-    return K % 4 == 0 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 == 0 && K < (1 << 24) &&
-           (long)(N / 64 + 1) * (M / 32 + 1) < (1l << 30);
+    const bool fits = K % 4 == 0 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 == 0 && K < (1 << 24) &&
+                      (long)(N / 64 + 1) * (M / 32 + 1) < (1l << 30);
+    if (!fits) return false;
+    // A block's beginning and end take as long as some hundred k, so a K that is short beside the number of blocks is left to
+    // gemm_plain_kernel, the same bits.  Microseconds here / there, one row: 32768 x 4 15.0 / 4.3, x 32 14.8 / 6.5, x 64 14.9 / 10.9, x 128
+    // 15 / 20; 16384 x 32 1.27 times as long, x 64 0.73; 131072 x 128 1.5 times; 64 rows: 8192 x 32 1.5 times, x 64 0.93, 4096 x 20
+    // 0.89; 1,000 rows: 4096 x 16 1.13 times, 1024 x 16 0.95, 4096 x 20 0.96.
+    if (K <= 16) return !gf_few(M, N) && (long)M * N <= (1l << 20);
+    if (!gf_few(M, N)) return true;
+    return M <= 32 ? 256l * K >= N : N <= 4096 || K >= 64;
 }
 
 void gemm_float_launch(const float* x, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
@@ -277,8 +288,8 @@ void gemm_float_launch(const float* x, const float* w, float* out, int M, int N,
     if (M <= 4) GF_FEW(1, 4, 1);
     else if (M <= 16) GF_FEW(1, 4, 4);
     else if (M <= 32) GF_FEW(2, 2, 4);
-    else if (M <= 48 && N <= 8192) GF_FEW(3, 2, 6);
-    else if (M <= 64 && N <= 8192) GF_FEW(4, 2, 8);
+    else if (gf_few(M, N) && M <= 48) GF_FEW(3, 2, 6);
+    else if (gf_few(M, N)) GF_FEW(4, 2, 8);
     else if (best == 4) GF_MANY(4);
     else if (best == 3) GF_MANY(3);
     else GF_MANY(2);
