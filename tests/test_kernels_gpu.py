@@ -1244,6 +1244,26 @@ def test_gemm_tiled_eight_waves_equal_four(variant, M, N, K):
     assert torch.equal(*got)
 
 
+@pytest.mark.parametrize("variant", [3, 7, 11, 12, 14])
+@pytest.mark.parametrize("M,inter", [(1, 8), (130, 113), (257, 132), (300, 264), (193, 226)])
+def test_gemm_tiled_activation_for_rows_of_any_width(variant, M, inter):
+    """Rows of results that are whole multiples of eight, of four and of neither, in tiles of features with four, six,
+    seven and eight groups of 16: float results against the formula, bfloat16 results their rounding to the bit."""
+    x, w = rnd(M, 72, dtype=torch.bfloat16, seed=43), rnd(2 * inter, 72, dtype=torch.bfloat16, seed=44, scale=0.3)
+    W = tuned().prepare_gate_up(w[:inter].contiguous(), w[inter:].contiguous())
+    ref = x.double() @ w.double().T
+    for gate, f in (("silu", torch.nn.functional.silu), ("gelu_tanh", lambda z: torch.nn.functional.gelu(z, approximate="tanh"))):
+        got = []
+        for dtype in (torch.float32, torch.bfloat16):
+            out = torch.full((M + 1, inter), float("nan"), dtype=dtype, device=DEV)           # (a row behind the last: not written)
+            tuned().gemm_tiled(x, W.packed, out[:M], swiglu_rows=W.packed_rows, gate=gate, variant=variant)
+            assert torch.isnan(out[M]).all()
+            got.append(out[:M])
+        want = f(ref[:, :inter]) * ref[:, inter:]
+        assert (got[0].double() - want).abs().max() < 2e-5 * want.abs().max()         # (sums of 72 products, the activation at unit slope)
+        assert torch.equal(got[0].bfloat16(), got[1])
+
+
 # ---------------------------------------------------------------- the walk of the linear recurrences
 @pytest.mark.parametrize("mode", ["fixed", "delta", "forget", "delta_per_dim", "gated", "written"])
 @pytest.mark.parametrize("D,Dv", [(64, 16), (128, 48), (256, 32)])
