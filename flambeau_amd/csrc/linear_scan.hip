@@ -22,6 +22,7 @@
 #include "api.h"
 #include "recordable.h"
 #include "lanes.h"
+#include "scan_chunks.h"
 
 #define LS_GROUP 16          // threads that share a column of S; they own the rows d = g, g + 16, ...
 #define LS_COLS 16           // columns of S per block
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(LS_GROUP * LS_COLS, RPT == 16 && !WHOLE ? 3 : 1) vo
     const float* __restrict__ head_decay, const float* __restrict__ tok_decay, const float* __restrict__ beta, int ldg,
     float* __restrict__ state, size_t slot_stride, const int* __restrict__ seq_q_start, const int* __restrict__ seq_q_len,
     const int* __restrict__ seq_slots, float* __restrict__ out, int H, int G, int D, int Dv,
-    const float* __restrict__ chan_decay = nullptr, int ldc = 0, float o_scale = 1.f, const float* __restrict__ skip = nullptr) {
+    const float* __restrict__ chan_decay = nullptr, int ldc = 0, float o_scale = 1.f, const float* __restrict__ skip = nullptr, int below = INT_MAX) {
     constexpr bool CHAN = MODE == 3 || MODE == 4;
     constexpr int NT = LS_GROUP * LS_COLS;
     constexpr int DP = LS_GROUP * RPT;                                // a row of q or k in LDS
@@ -78,6 +79,7 @@ __global__ __launch_bounds__(LS_GROUP * LS_COLS, RPT == 16 && !WHOLE ? 3 : 1) vo
     const int qk_head = head / (H / G);
     const bool live = WHOLE || j < Dv;
     const int start = seq_q_start[s], len = seq_q_len[s];
+    if (len >= below) return;                      // (a request that goes chunk by chunk)
     float* st = state + (size_t)seq_slots[s] * slot_stride + (size_t)head * D * Dv;
     float S[RPT];
     if constexpr (WHOLE) {
@@ -276,7 +278,7 @@ static int linear_scan_launch(const float* q, int ldq, const float* k, int ldk, 
                               long slot_stride, const int* seq_q_start, const int* seq_q_len, const int* seq_slots,
                               float* out, int n_seqs, int H, int G, int D, int Dv, bool channel_decay, hipStream_t stream,
                               const float* chan_decay = nullptr, int ldc = 0, bool corrects = true, float o_scale = 1.f,
-                              const float* skip = nullptr) {
+                              const float* skip = nullptr, int below = INT_MAX) {
     FL_CHECK(!chan_decay || (!beta == !corrects && !head_decay && !tok_decay && !channel_decay && ldc >= H * D),
              "linear_scan: a decay per key dim comes without another decay, and under the delta rule with write strengths");
     FL_CHECK(n_seqs >= 0 && H > 0 && G > 0 && H % G == 0 && D > 0 && Dv > 0, "linear_scan: bad sizes");
@@ -297,7 +299,7 @@ static int linear_scan_launch(const float* q, int ldq, const float* k, int ldk, 
 #define FL_LS3(R, MODE, W)                                                                                             \
     linear_scan_kernel<R, MODE, W><<<grid, LS_GROUP * LS_COLS, 0, stream>>>(q, ldq, k, ldk, v, ldv, head_decay, tok_decay, beta, \
                                                                           ldg, state, (size_t)slot_stride, seq_q_start,        \
-                                                                          seq_q_len, seq_slots, out, H, G, D, Dv, chan_decay, ldc, o_scale, skip)
+                                                                          seq_q_len, seq_slots, out, H, G, D, Dv, chan_decay, ldc, o_scale, skip, below)
 #define FL_LS2(R, MODE)                                  \
     do {                                                 \
         if constexpr (R == 4 || R == 8 || R == 16) {     \
@@ -381,6 +383,42 @@ extern "C" int fl_linear_scan_written(const float* q, int ldq, const float* k, i
                               seq_slots, out, n_seqs, H, G, D, Dv, false, stream, nullptr, 0, false, 1.f, skip);
 }
 FL_RECORDABLE(fl_linear_scan_written)
+
+// The recurrences without a correction in their chunked form: for requests of at least min_len tokens, and the walk for the others
+// (walk_short), or for all requests (walk_short = 0).
+// a decay per head (head_decay), per token and head (tok_decay, with write strengths or without: rows ldg wide) or per token, head
+// and key dim (chan_decay, rows ldc wide); o = o_scale S^T q (with chan_decay; 1 otherwise) + skip v (skip: per head or null; with
+// write strengths).  records:
+// fl_linear_scan_records(n, n_seqs) x fl_linear_scan_record_floats(H, D, chan_decay != null) floats, n = the step's tokens.
+extern "C" int fl_linear_scan_chunked_takes(int D, int Dv) { return scan_chunks_takes(D, Dv); }
+extern "C" int fl_linear_scan_record_floats(int H, int D, int per_dim) { return H * (per_dim ? SC_CHANNEL_RECORD(D) : SC_RECORD); }
+extern "C" int fl_linear_scan_records(int n, int n_seqs) { return scan_chunks_records(n, n_seqs); }
+extern "C" int fl_linear_scan_chunked(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* head_decay,
+                                      const float* tok_decay, const float* write, int ldg, const float* chan_decay, int ldc, float o_scale,
+                                      const float* skip, float* state, long slot_stride, const int* seq_q_start, const int* seq_q_len,
+                                      const int* seq_slots, float* out, float* records, int n, int n_seqs, int min_len, int walk_short, int H, int G,
+                                      int D, int Dv, hipStream_t stream) {
+    FL_CHECK(n >= 0 && n_seqs >= 0 && H > 0 && G > 0 && H % G == 0 && min_len >= 1, "linear_scan_chunked: bad sizes");
+    FL_CHECK(scan_chunks_takes(D, Dv), "linear_scan_chunked: heads of %d x %d", D, Dv);
+    FL_CHECK(!!head_decay + !!tok_decay + !!chan_decay == 1 && (!write == !tok_decay) && (!skip || write) && (chan_decay || o_scale == 1.f),
+             "linear_scan_chunked: one decay per head, or one per token and head with write strengths, or one per token, head and key dim");
+    FL_CHECK(ldq >= G * D && ldk >= G * D && ldv >= H * Dv && (!tok_decay || ldg >= H) && (!chan_decay || ldc >= H * D), "linear_scan_chunked: rows narrower than their heads");
+    const auto pieces = [](const float* p, int ld) { return (uintptr_t)p % 16 == 0 && ld % 4 == 0; };
+    FL_CHECK(pieces(q, ldq) && pieces(k, ldk) && (!chan_decay || pieces(chan_decay, ldc)) && (uintptr_t)state % 16 == 0 && slot_stride % 4 == 0 &&
+             (uintptr_t)records % 16 == 0, "linear_scan_chunked: rows and states must be whole 16-byte pieces");
+    FL_CHECK(slot_stride >= (long)H * D * Dv, "linear_scan_chunked: a slot of %ld floats does not hold %d heads", slot_stride, H);
+    FL_CHECK((long)SC_CHUNK * max(max(ldq, ldk), ldv) < (1l << 28), "linear_scan_chunked: rows of %d, %d and %d floats", ldq, ldk, ldv);
+    if (n == 0 || n_seqs == 0) return 0;
+    FL_CHECK(n_seqs <= 65535 && H <= 65535, "linear_scan_chunked: %d requests of %d heads are more than one grid takes", n_seqs, H);
+    const ScanChunks a = {q, k, v, ldq, ldk, ldv, head_decay, tok_decay, write, ldg, state, (size_t)slot_stride, seq_q_start, seq_q_len,
+                          seq_slots, out, records, n_seqs, walk_short ? min_len : 1, H, G, Dv, o_scale, skip, chan_decay, ldc};
+    scan_chunks_launch(a, D, n, stream);
+    FL_LAUNCH_CHECK();
+    if (!walk_short) return 0;
+    return linear_scan_launch(q, ldq, k, ldk, v, ldv, head_decay, tok_decay, write, ldg, state, slot_stride, seq_q_start, seq_q_len,
+                              seq_slots, out, n_seqs, H, G, D, Dv, false, stream, chan_decay, ldc, false, o_scale, skip, min_len);
+}
+FL_RECORDABLE(fl_linear_scan_chunked)
 
 // g[t][h][d] = exp(-exp(A_log[h]) * softplus(a[t][col + h * D + d] + dt_bias[h * D + d])): the decays of a recurrence
 // that forgets per head and key dim

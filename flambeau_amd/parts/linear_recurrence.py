@@ -36,6 +36,7 @@ from __future__ import annotations
 import torch
 
 from ..config.base import ConfigError
+from ..kernels import linear_scan as _kernels  # noqa: F401  (registers these mixers' kernel set)
 from ..kernels import ops
 from .base import MIXERS, POSITION_ENCODINGS, Mixer, PartSpec, Product, StateSpec, TensorSpec
 
@@ -69,7 +70,8 @@ class Retention(Mixer):
         return ("retention",)
 
     def step_signature(self, batch):
-        return ()
+        """Which requests go in chunks: all that this mixer decides from their lengths."""
+        return self.kernels.signature(batch)
 
     def tensors(self):
         W, H, D, Dv = self.hidden_size, self.n_heads, self.head_dim, self.value_dim
@@ -85,6 +87,7 @@ class Retention(Mixer):
         joined = [weights["q.weight"], weights["k.weight"], weights["v.weight"]] + ([weights["g.weight"]] if self.gate else [])
         self.w_in = rt.prepare_weight(torch.cat(joined, dim=0).contiguous())
         self.col_k, self.col_v, self.col_g = H * D, 2 * H * D, 2 * H * D + H * Dv
+        self.kernels = rt.kernels("linear_scan")
         self.decay_dev = torch.tensor(self.decay, dtype=torch.float32, device=rt.device)
         self.w_o = rt.prepare_weight(weights["o.weight"])
         self.position.bind({}, rt)
@@ -101,8 +104,7 @@ class Retention(Mixer):
         k = rt.buffer("ret_k", n, H * D, torch.float32)
         ops.rotate_scale(proj, 0, self.col_k, angles, self.rotated_dims, self.interleaved, 1.0, self.key_scale, q, k, H, D)
         hidden = rt.buffer("ret_hidden", n, H * Dv, torch.float32)
-        ops.linear_scan(q, k, proj[:, self.col_v:self.col_v + H * Dv], cache.state, step.seq_q_start, step.seq_q_len,
-                        step.seq_slots, hidden, H, H, D, Dv, head_decay=self.decay_dev)
+        self.kernels.fixed(q, k, proj[:, self.col_v:self.col_v + H * Dv], self.decay_dev, cache.state, step, hidden, H, H, D, Dv)
         out = rt.buffer("ret_out", n, H * Dv)
         ops.headnorm_gate(hidden, None, proj if self.gate else None, self.col_g, out, H, self.eps, gate_kind=self.gate or "sigmoid")
         return Product(out, self.w_o)
@@ -299,7 +301,8 @@ class GatedLinearAttention(Mixer):
         return ("gated_linear_attention",)
 
     def step_signature(self, batch):
-        return ()
+        """Which requests go in chunks: all that this mixer decides from their lengths."""
+        return self.kernels.signature(batch)
 
     def tensors(self):
         W, H, D, Dv, R = self.hidden_size, self.n_heads, self.head_dim, self.value_dim, self.decay_rank
@@ -315,6 +318,7 @@ class GatedLinearAttention(Mixer):
         self.col_k, self.col_v = H * D, 2 * H * D
         self.col_g = self.col_v + H * Dv
         self.col_a = self.col_g + H * Dv
+        self.kernels = rt.kernels("linear_scan")
         self.w_a2 = (weights["a2.weight"].contiguous(), weights["a2.weight"].t().contiguous())
         self.b_a2 = weights["a2.bias"]
         self.norm = weights["norm.weight"].repeat(H).contiguous()          # one gain for every head, laid out heads x vdim
@@ -327,7 +331,7 @@ class GatedLinearAttention(Mixer):
         rt.gemm(x, self.w_in, proj)
         decay = ops.lowrank_gate(proj, self.col_a, *self.w_a2, self.b_a2, self.tau, rt.buffer("gla_decay", n, H * D, torch.float32))
         hidden = rt.buffer("gla_hidden", n, H * Dv, torch.float32)
-        ops.linear_scan_gated(proj[:, :H * D], proj[:, self.col_k:self.col_k + H * D], proj[:, self.col_v:self.col_v + H * Dv], decay,
+        self.kernels.gated(proj[:, :H * D], proj[:, self.col_k:self.col_k + H * D], proj[:, self.col_v:self.col_v + H * Dv], decay,
                               cache.state, step, hidden, H, H, D, Dv, out_scale=self.query_scale)
         out = rt.buffer("gla_out", n, H * Dv)
         ops.headnorm_gate(hidden, self.norm, proj, self.col_g, out, H, self.eps, gate_kind="silu")
@@ -365,7 +369,8 @@ class StateSpace(Mixer):
         return ("state_space",)
 
     def step_signature(self, batch):
-        return ()
+        """Which requests go in chunks: all that this mixer decides from their lengths."""
+        return self.kernels.signature(batch)
 
     def tensors(self):
         W, H, C = self.hidden_size, self.n_heads, self.channels
@@ -383,6 +388,7 @@ class StateSpace(Mixer):
         if not self.joined:
             self.w_in = rt.prepare_weight(weights["in.weight"])
             self.w_o = rt.prepare_weight(weights["o.weight"])
+        self.kernels = rt.kernels("linear_scan")
         self.conv_w = weights["conv.weight"].t().contiguous()              # [taps, channels]
         self.conv_b, self.dt_bias, self.a_log, self.skip = (weights[k] for k in ("conv.bias", "dt_bias", "A_log", "D"))
         self.norm, self._scaled = weights["norm.weight"], {}
@@ -411,6 +417,6 @@ class StateSpace(Mixer):
         ops.conv_steps(proj, col0 + inner, self.conv_w, self.conv_b, cache.state, self.conv_at, step, prep, col0 + inner + C, H, self.dt_bias,
                        self.a_log, gates)
         hidden = rt.buffer("ssd_hidden", n, inner, torch.float32)
-        ops.linear_scan_written(prep[:, inner + G * N:], prep[:, inner:inner + G * N], prep[:, :inner], gates, self.skip, cache.state, step,
-                                hidden, H, G, N, Dv)
+        self.kernels.written(prep[:, inner + G * N:], prep[:, inner:inner + G * N], prep[:, :inner], gates, self.skip, cache.state, step,
+                             hidden, H, G, N, Dv)
         ops.gated_group_norm(hidden, proj, col0, self._gain(factor), out, self.norm_parts, self.eps)

@@ -1302,6 +1302,117 @@ def test_linear_scan_in_whole_pieces_gives_the_same_bits(mode, D, Dv):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
+# ---------------------------------------------------------------- linear recurrences, a chunk of tokens at a time
+def _scan_case(mode, H, G, D, Dv, lens, pad=0):
+    """Inputs of a recurrence over ragged requests, and ``run(kernels)`` -> (outputs, states)."""
+    from types import SimpleNamespace
+    n, S = sum(lens), len(lens)
+    ints = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    step = SimpleNamespace(seq_q_start=ints([sum(lens[:i]) for i in range(S)]), seq_q_len=ints(lens), seq_slots=ints(list(range(S))[::-1]),
+                           host=SimpleNamespace(q_lens=lens))
+    c = SimpleNamespace(mode=mode, H=H, G=G, D=D, Dv=Dv, lens=lens, step=step)
+    rows = torch.empty(n, 2 * G * D + H * Dv + pad, dtype=torch.float32, device=DEV)           # q, k and v as columns of wider rows
+    rows.copy_(rnd(n, rows.shape[1], seed=60))
+    c.q, c.k, c.v = rows[:, :G * D], rows[:, G * D:2 * G * D], rows[:, 2 * G * D:2 * G * D + H * Dv]
+    c.k *= D ** -0.5
+    c.head_decay = 1 - 2.0 ** -(3 + torch.arange(H, dtype=torch.float32, device=DEV))
+    c.gates = torch.cat([torch.exp(-rnd(n, H, seed=61).abs() * 0.2), torch.sigmoid(rnd(n, H, seed=62))], dim=1).contiguous()
+    c.gates[n // 2, 0] = 0.0                                                                   # (a decay may be nothing at all)
+    c.key_decay = torch.sigmoid(rnd(n, H * D, seed=63)) ** (1 / 16)
+    c.skip, c.state0 = rnd(H, seed=64), rnd(S, H * D * Dv, seed=65)
+
+    def run(kernels):
+        state, out = c.state0.clone(), torch.full((n, H * Dv), float("nan"), dtype=torch.float32, device=DEV)
+        where = (state, step, out, H, G, D, Dv)
+        if mode == "fixed":
+            kernels.fixed(c.q, c.k, c.v, c.head_decay, *where)
+        elif mode == "gated":
+            kernels.gated(c.q, c.k, c.v, c.key_decay, *where, 0.5)
+        else:
+            kernels.written(c.q, c.k, c.v, c.gates, c.skip, *where)
+        return out, state
+    c.run = run
+    return c
+
+
+def _scan_in_64_bits(c):
+    H, G, D, Dv = c.H, c.G, c.D, c.Dv
+    q, k = (t.double().reshape(-1, G, D).repeat_interleave(H // G, dim=1) for t in (c.q, c.k))
+    v, out, states, at = c.v.double().reshape(-1, H, Dv), [], c.state0.double().reshape(-1, H, Dv, D).clone(), 0
+    for s, length in enumerate(c.lens):
+        S = states[int(c.step.seq_slots[s])]
+        for t in range(at, at + length):
+            decay = {"fixed": c.head_decay.double()[:, None, None], "gated": c.key_decay[t].double().reshape(H, 1, D),
+                     "written": c.gates[t, :H].double()[:, None, None]}[c.mode]
+            u = v[t] * c.gates[t, H:].double()[:, None] if c.mode == "written" else v[t]
+            S.mul_(decay).add_(u[:, :, None] * k[t][:, None, :])
+            o = (S * q[t][:, None, :]).sum(-1) * (0.5 if c.mode == "gated" else 1.0)
+            out.append(o + c.skip.double()[:, None] * v[t] if c.mode == "written" else o)
+        at += length
+    return torch.stack(out).reshape(at, H * Dv), states.reshape(len(c.lens), -1)
+
+
+def _scan_sets(max_tokens=4096):
+    from types import SimpleNamespace
+    from flambeau_amd.kernels import linear_scan as ls
+    rt = SimpleNamespace(max_batch_tokens=max_tokens, buffer=lambda name, rows, cols, dtype, max_rows=None: torch.full((rows, cols), float("nan"), dtype=dtype, device=DEV))
+    return ls.PlainLinearScan(rt), ls.TunedLinearScan(rt)
+
+
+@pytest.mark.parametrize("mode", ["fixed", "gated", "written"])
+@pytest.mark.parametrize("H,G,D,Dv,lens", [(2, 2, 64, 16, [192]), (3, 3, 128, 48, [193, 255, 256, 257]), (4, 2, 128, 64, [1, 320, 127, 191, 193, 7, 700]),
+                                           (2, 1, 256, 32, [207, 3, 192])])
+def test_scan_in_chunks_against_64_bits(mode, H, G, D, Dv, lens):
+    """Requests that end anywhere in a chunk and in 16 tokens, beside requests that walk: outputs and states are no further from 64
+    bits than the walk's, or than fewer than 40 roundings (a result is a sum of sums, in chains of at most 16 products and trees of
+    three, with a factor and a sum behind; a rounding to 24 bits is 2.4e-8 in the root mean square, 40 of them 1.5e-7)."""
+    if mode == "gated" and G != H:
+        G = H
+    c = _scan_case(mode, H, G, D, Dv, lens)
+    plain, chunked = _scan_sets()
+    want, walk, got = _scan_in_64_bits(c), c.run(plain), c.run(chunked)
+    assert not torch.equal(walk[0], got[0])                      # (the chunks did run)
+    for w, a, b in zip(want, walk, got):
+        err = lambda x: float((x.double() - w).norm() / w.norm())
+        assert err(b) < max(err(a), 1.5e-7), (err(a), err(b))
+    at = 0
+    for length in lens:                                          # (a request that walks: the walk's bits)
+        if length < (192 if mode == "gated" else 128):
+            assert torch.equal(walk[0][at:at + length], got[0][at:at + length])
+        at += length
+
+
+@pytest.mark.parametrize("mode", ["fixed", "gated", "written"])
+def test_scan_in_chunks_keeps_values_that_are_no_numbers_behind_their_token(mode):
+    """A NaN or an infinity in v reaches its own column from its token on, one in k or q nothing before its token."""
+    c = _scan_case(mode, 2, 2, 128, 32, [200])
+    _, chunked = _scan_sets()
+    before, _ = c.run(chunked)
+    for t in (0, 5, 15, 16, 70, 127, 199):
+        for bad in (float("nan"), float("inf")):
+            kept = c.v[t, 3].clone()
+            c.v[t, 3] = bad
+            out, _ = c.run(chunked)
+            c.v[t, 3] = kept
+            # (its column's tokens in the same 16 are then summed one by one: 80 sums of 3e-8)
+            assert not torch.isfinite(out[t, 3]) and bool(((out[:t, 3] - before[:t, 3]).abs() <= 2.5e-6 * before.abs().max()).all())
+            others = [j for j in range(out.shape[1]) if j != 3]
+            assert torch.equal(out[:, others], before[:, others])
+            for rows in (c.k, c.q):
+                kept = rows[t, 7].clone()
+                rows[t, 7] = bad
+                out, _ = c.run(chunked)
+                rows[t, 7] = kept
+                assert torch.equal(out[:t], before[:t])
+
+
+def test_scan_rows_that_the_chunks_do_not_take_walk():
+    """Rows that are no whole 16-byte pieces, and head sizes that the chunked kernels do not know: the walk's bits."""
+    plain, chunked = _scan_sets()
+    for c in (_scan_case("fixed", 2, 2, 128, 32, [200], pad=3), _scan_case("written", 2, 2, 96, 32, [200]), _scan_case("gated", 2, 2, 128, 24, [200])):
+        assert all(torch.equal(a, b) for a, b in zip(c.run(plain), c.run(chunked)))
+
+
 # ---------------------------------------------------------------- the 32-bit attention on the matrix cores
 @pytest.mark.parametrize("cap,sinks", [(0.0, False), (3.0, True)])
 @pytest.mark.parametrize("nh,nkv,hd,ps,window", [(8, 2, 128, 16, 0), (4, 4, 64, 8, 0), (40, 2, 64, 4, 37), (3, 1, 128, 32, 100), (6, 2, 64, 64, 64)])
