@@ -171,6 +171,7 @@ __global__ __launch_bounds__(128 * WT, OCC) void gemm_async_kernel(const bf16_t*
     // are issued here, ahead of all other loads, and wait in registers (where there is room: with 4 x 4
     // tiles per wave, not with 8 x 4).
     constexpr bool PREFETCH = EPI == TG_RESIDUAL && OCC == 1 && FT * TT <= 16;
+    constexpr int BATCH = FT * TT > 32 ? (FT + 1) / 2 : FT;           // tiles of a token that an epilogue looks values up for at a time: what registers leave room for
     const int j = lane & 15, g = lane >> 4;
     f32x4 pre[PREFETCH ? FT : 1][PREFETCH ? TT : 1];
     if (PREFETCH) {
@@ -299,9 +300,12 @@ __global__ __launch_bounds__(128 * WT, OCC) void gemm_async_kernel(const bf16_t*
         // resid += product; xg = bf16(resid * g); the block's sum of resid^2 per token: this wave's
         // features, then the four lanes of a token, then the two waves that share the tokens
         float* s_part = (float*)ring;                                 // [2][NTT * 16]
-        f32x4 gain[FT];                                               // the norm's weights of this lane's features
+        auto gain_of = [&](int ta) { return *(const f32x4*)(fu.g + min(n0 + (wf * FT + ta) * 16 + 4 * g, N - 4)); };
+        f32x4 gain[BATCH == FT ? FT : 1];                             // the norm's weights of this lane's features, where registers hold them
+        if constexpr (BATCH == FT) {
 #pragma unroll
-        for (int ta = 0; ta < FT; ++ta) gain[ta] = *(const f32x4*)(fu.g + min(n0 + (wf * FT + ta) * 16 + 4 * g, N - 4));
+            for (int ta = 0; ta < FT; ++ta) gain[ta] = gain_of(ta);
+        }
         const float dyt_a = fu.dyt_alpha ? fu.dyt_alpha[0] : 0.f;
         __syncthreads();                                              // the ring is no longer read
         // (which norm follows is chosen once, outside the loops: the usual form's code stays what it was)
@@ -310,30 +314,35 @@ __global__ __launch_bounds__(128 * WT, OCC) void gemm_async_kernel(const bf16_t*
             for (int tb = 0; tb < TT; ++tb) {
                 const int tok = m0 + (wt * TT + tb) * 16 + j;
                 float sq = 0.f;
-                f32x4 old[FT];                                        // the token's residual values, read together
 #pragma unroll
-                for (int ta = 0; ta < FT; ++ta) {
-                    const int f0 = min(n0 + (wf * FT + ta) * 16 + 4 * g, N - 4);
-                    old[ta] = PREFETCH ? pre[PREFETCH ? ta : 0][PREFETCH ? tb : 0]
-                                       : *(const f32x4*)(fu.resid + (size_t)min(tok, M - 1) * N + f0);
-                }
+                for (int t0 = 0; t0 < FT; t0 += BATCH) {
+                    f32x4 old[BATCH];                                 // the token's residual values, a batch read together
 #pragma unroll
-                for (int ta = 0; ta < FT; ++ta) {
-                    const int f0 = n0 + (wf * FT + ta) * 16 + 4 * g;
-                    if (tok < M && f0 < N) {
-                        const f32x4 nr = old[ta] + acc[ta][tb];
-                        const f32x4 gv = gain[ta];
-                        *(f32x4*)(fu.resid + (size_t)tok * N + f0) = nr;
-                        f32x4 xo = {nr[0] * gv[0], nr[1] * gv[1], nr[2] * gv[2], nr[3] * gv[3]};
-                        if (decltype(dyt)::value) {
-                            const f32x4 bv = fu.dyt_bias ? *(const f32x4*)(fu.dyt_bias + f0) : (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) xo[r] = tanhf(dyt_a * nr[r]) * gv[r] + bv[r];
-                        }
-                        const bf16x4 o = {(bf16_t)xo[0], (bf16_t)xo[1], (bf16_t)xo[2], (bf16_t)xo[3]};
-                        *(bf16x4*)(fu.xg + (size_t)tok * N + f0) = o;
-                        sq += (nr[0] * nr[0] + nr[1] * nr[1]) + (nr[2] * nr[2] + nr[3] * nr[3]);
+                    for (int u = 0; u < BATCH; ++u) {
+                        const int ta = min(t0 + u, FT - 1);
+                        const int f0 = min(n0 + (wf * FT + ta) * 16 + 4 * g, N - 4);
+                        old[u] = PREFETCH ? pre[PREFETCH ? ta : 0][PREFETCH ? tb : 0]
+                                          : *(const f32x4*)(fu.resid + (size_t)min(tok, M - 1) * N + f0);
                     }
+#pragma unroll
+                    for (int u = 0; u < BATCH && t0 + u < FT; ++u) {
+                        const int ta = t0 + u, f0 = n0 + (wf * FT + ta) * 16 + 4 * g;
+                        if (tok < M && f0 < N) {
+                            const f32x4 nr = old[u] + acc[ta][tb];
+                            const f32x4 gv = BATCH == FT ? gain[BATCH == FT ? ta : 0] : gain_of(ta);
+                            *(f32x4*)(fu.resid + (size_t)tok * N + f0) = nr;
+                            f32x4 xo = {nr[0] * gv[0], nr[1] * gv[1], nr[2] * gv[2], nr[3] * gv[3]};
+                            if (decltype(dyt)::value) {
+                                const f32x4 bv = fu.dyt_bias ? *(const f32x4*)(fu.dyt_bias + f0) : (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) xo[r] = tanhf(dyt_a * nr[r]) * gv[r] + bv[r];
+                            }
+                            const bf16x4 o = {(bf16_t)xo[0], (bf16_t)xo[1], (bf16_t)xo[2], (bf16_t)xo[3]};
+                            *(bf16x4*)(fu.xg + (size_t)tok * N + f0) = o;
+                            sq += (nr[0] * nr[0] + nr[1] * nr[1]) + (nr[2] * nr[2] + nr[3] * nr[3]);
+                        }
+                    }
+                    if constexpr (BATCH < FT) __builtin_amdgcn_sched_barrier(0);      // (the next batch's reads stay behind this one's use)
                 }
                 sq += __shfl_xor(sq, 16, 64);
                 sq += __shfl_xor(sq, 32, 64);
@@ -358,16 +367,20 @@ __global__ __launch_bounds__(128 * WT, OCC) void gemm_async_kernel(const bf16_t*
 #pragma unroll
         for (int tb = 0; tb < TT; ++tb) {
             const int tok = toks[tb];
-            RopeAngles an[FT];
-            if (rs.rot) {                                             // (no table without rotated dims)
 #pragma unroll
-                for (int ta = 0; ta < FT; ++ta)
-                    an[ta] = rope_angles(rs, min(tok, M - 1), n0 + (wf * FT + ta) * 16 + 4 * g, g);
-            }
+            for (int t0 = 0; t0 < FT; t0 += BATCH) {
+                RopeAngles an[BATCH];
+                if (rs.rot) {                                         // (no table without rotated dims)
 #pragma unroll
-            for (int ta = 0; ta < FT; ++ta) {
-                const int f0 = n0 + (wf * FT + ta) * 16 + 4 * g;
-                rope_store4<true>(rs, tok, places[tb], f0, g, acc[ta][tb], tok < M && f0 < N, an[ta]);
+                    for (int u = 0; u < BATCH; ++u)
+                        an[u] = rope_angles(rs, min(tok, M - 1), n0 + (wf * FT + min(t0 + u, FT - 1)) * 16 + 4 * g, g);
+                }
+#pragma unroll
+                for (int u = 0; u < BATCH && t0 + u < FT; ++u) {
+                    const int ta = t0 + u, f0 = n0 + (wf * FT + ta) * 16 + 4 * g;
+                    rope_store4<true>(rs, tok, places[tb], f0, g, acc[ta][tb], tok < M && f0 < N, an[u]);
+                }
+                if constexpr (BATCH < FT) __builtin_amdgcn_sched_barrier(0);
             }
         }
         return;
@@ -515,33 +528,38 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 // Shape of the block: 3 = 256 features x 128 tokens (4 waves, ring of 3, two blocks per compute unit),
 // 7 = 192 x 128 and 8 = 128 x 128 (the same with fewer features), 13 = 128 x 128 (4 waves, ring of 8, one block per
 // unit), 10 = 256 x 256 (8 waves, ring of 4, one block per compute unit), 11 = 224 x 256, 12 = 192 x 256 and
-// 6 = 128 x 256 (the same with fewer features; 6 on request only), 14 = 224 x 192 (8 waves, ring of 5); 0 = chosen
+// 6 = 128 x 256 (the same with fewer features; 6 on request only), 14 = 224 x 192 (8 waves, ring of 5), 15 = 256 x 320,
+// 16 = 224 x 320 and 17 = 224 x 384 (8 waves, ring of 4, more tokens per block); 0 = chosen
 // here, together with the number of K-splits.  The entry points whose names end in _ex take either from the caller,
 // for tests and measurements.
 //
-// What a shape costs, in us.  Four waves, two blocks per unit: bound by the copies into LDS, per k-step 0.115 a round of
-// resident blocks and 0.0193 per KB that a unit's blocks copy, 0.8 of it from the mean and 0.2 from the unit with the most
+// What a shape costs, in us.  Four waves, two blocks per unit: bound by the copies into LDS, per k-step 0.128 a round of
+// resident blocks and 0.0198 per KB that a unit's blocks copy, 0.8 of it from the mean and 0.2 from the unit with the most
 // blocks; a tile of w that few tiles of tokens share comes from HBM more often (a quarter more with one of them), and
-// blocks of 128 features copy 9 % faster.  Four waves alone on their unit have the whole LDS for stages on their way:
-// 0.377 per k-step, less where the tile's rows are few (28672 x 4096 at 65 rows 55.5 against 64 with three stages, at 97
-// 59.5 against 63).  Eight waves, one block after the other: bound by the matrix cores and by the wait for weights,
-// 0.69, 0.66, 0.60 per k-step with 256, 224, 192 features and 0.56 with 224 x 192, less where a tile's rows are few,
-// more where a unit gets a second block of another part of K, and 6 per block that nothing overlaps.  Splitting K adds the
-// parts' way to memory and back and the kernel that sums them: 2.38 us per million values and part.
-// What decides between 256, 224 and 192 features is how evenly the blocks fill the rounds: gate/up of 2,048 rows, 28672
-// features, is 3.5 rounds of 256 (422 us with its activation) and 4 of 224 (408; 512 with 4 waves before those
-// of a pair took turns), q/k/v of 2,048 rows, 6144 features, 0.75 rounds of 256 (108 us with its rotation) and 1
-// of 192 (102; 115 with 256 x 128).  192 tokens are mostly for rows that end soon behind a multiple of 256: 28672 x 4096
-// at 333 rows 90 us (96.6 with 256 tokens), 528 rows 157 (160), 1,040 rows 252 (257).  224 x 224 does not divide among
-// the waves, 192 x 192 and 256 x 192 gained nothing beside it (528 rows 161.8 and 168).
-// The constants are those that pick best among all that may be picked: 14 products (7B, 12B and 24B sizes and layers of
+// blocks of 128 features copy 12 % faster.  Four waves alone on their unit have the whole LDS for stages on their way:
+// 0.388 per k-step, less where the tile's rows are few (28672 x 4096 at 65 rows 55.5 against 64 with three stages, at 97
+// 59.5 against 63).  Eight waves, one block after the other: bound by the matrix cores, by LDS (a step of 256 x 256 takes as
+// many clocks of LDS as of the matrix cores, of 256 x 320 nine tenths) and by the wait for weights, 0.68, 0.68, 0.58 per k-step
+// with 256, 224, 192 features, 0.59 with 224 x 192 and 0.85, 0.75, 0.94 with 256 x 320, 224 x 320 and 224 x 384, less where a
+// tile's rows are few, more where a unit gets a second block of another part of K, and 7 per block that nothing overlaps.
+// Splitting K adds the parts' way to memory and back and the kernel that sums them: 1 us, and 2.35 per million values and part.
+// What decides among eight waves is how evenly the blocks fill the rounds, in features (gate/up of 2,048 rows, 28672 features, is
+// 3.5 rounds of 256 and 4 of 224, q/k/v of 2,048 rows, 6144 features, 0.75 rounds of 256 and 1 of 192) and in tokens: rows that
+// end soon behind a multiple of 256 are tiles of 192 (28672 x 4096 at 333 rows 90 us, 96.6 with 256) or of 320 and 384, which at
+// 528 rows are one round where 192 are two: 28672 x 4096 with its activation 163 us -> 121, at 768 rows 184 -> 150, at 1,100
+// rows 280 -> 243, at 3,072 rows 575 -> 535; 65536 x 5120 at 320 rows 258 -> 205, at 640 rows 421 -> 338; 5120 x 32768 at 3,328
+// rows 1,090 -> 850.  224 x 224 does not divide among the waves; 192 x 192, 256 x 192, 128 x 320 and 192 x 384 gained nothing
+// beside these (256 x 384 does not fit the registers).
+// The constants are those that pick best among all that may be picked: 15 products (7B, 12B and 24B sizes and layers of
 // width 2,048, each with the epilogue that it runs with: rotation and stores, sum into the stream, activation, none; where
 // K is split with the kernel that adds the parts) at 50 row counts from 65 to 4,001, weights from HBM, every shape with 1
-// to 6 and 8 parts, 26,000 timings.  Picks take 0.9 % more time than the best on average and 16 % at worst (4096 x 4096
-// at 768 rows, 53.7 against 46.2).  A formula fitted to plain products and fewer numbers of parts, with no sharing of w
-// and no rows per tile in it, was 1.9 % off and 44 % at worst (6144 x 5120 at 700 rows; 5120 x 32768 at 1,040 473 us against 358).
-struct TileShape { int variant, features, tokens, per_unit; };
-static const TileShape g_shapes[] = {{3, 256, 128, 2}, {7, 192, 128, 2}, {8, 128, 128, 2}, {10, 256, 256, 1}, {11, 224, 256, 1}, {12, 192, 256, 1}, {6, 128, 256, 1}, {13, 128, 128, 1}, {14, 224, 192, 1}};
+// to 6 and 8 parts, 52,000 timings.  Picks take 1.1 % more time than the best on average and 24 % at worst (2048 x 2048
+// at 3,584 rows, 53.6 against 43.1), 2.4 % less on average than those among the shapes of up to 256 tokens; five of 750 more than 3 %
+// longer (4096 x 14336 at 289 rows 65.9 against 62.3), 124 more than 3 % shorter.
+struct TileShape { int variant, features, tokens, per_unit; float step; };             // step: us per k-step of a block of eight waves
+static const TileShape g_shapes[] = {{3, 256, 128, 2, 0.f}, {7, 192, 128, 2, 0.f}, {8, 128, 128, 2, 0.f}, {10, 256, 256, 1, 0.6808f}, {11, 224, 256, 1, 0.6778f},
+                                     {12, 192, 256, 1, 0.5849f}, {6, 128, 256, 1, 0.58f}, {13, 128, 128, 1, 0.f}, {14, 224, 192, 1, 0.5855f},
+                                     {15, 256, 320, 1, 0.8539f}, {16, 224, 320, 1, 0.7514f}, {17, 224, 384, 1, 0.9405f}};
 static const TileShape& tile_shape(int variant) {
     for (const TileShape& t : g_shapes)
         if (t.variant == variant) return t;
@@ -559,17 +577,17 @@ static float tiled_cost(const TileShape& t, int splits, int M, int N, int K) {
     const int m_tiles = ceil_div(M, t.tokens);
     const float empty = 1.f - (float)M / ((long)m_tiles * t.tokens);   // share of the tiles' rows that are none
     float us;
-    if (t.variant == 14 && empty > 0.375f) return 1e9f;                // (tiles with so few rows: 28672 x 5120 at 207 rows 112.8 us, 106.4 with 256 x 128)
+    if (t.variant == 14 && empty > 0.4276f) return 1e9f;               // (tiles with so few rows: 28672 x 5120 at 207 rows 112.8 us, 106.4 with 256 x 128)
     if (t.variant == 13) {
-        us = most * steps * (0.377f - 0.104f * empty) + 1.72f;
+        us = most * steps * (0.3876f - 0.0892f * empty) + 1.73f;
     } else if (t.per_unit == 1) {
-        const float step = t.variant == 14 ? 0.563f : t.features == 256 ? 0.689f : t.features == 224 ? 0.662f : 0.601f;
-        us = most * (steps * (step * (1.f + 0.0864f / m_tiles + (splits > 1 && most > 1 ? 0.0543f : 0.f)) - 0.0736f * empty * t.tokens / 256.f) + 6.06f);
+        us = most * (steps * (t.step * (1.f + 0.1021f / m_tiles + (splits > 1 && most > 1 ? 0.0517f : 0.f)) - 0.0795f * empty * t.tokens / 256.f) +
+                     7.01f + 0.1918f * (t.tokens - 256) / 64.f);
     } else {
-        const float kb = (t.features * (1.f + 0.276f / m_tiles) + t.tokens) * 64 / 1024.f;      // copied per block and k-step
-        us = steps * (0.115f * rounds + (t.features == 128 ? 0.0175f : 0.0193f) * kb * (0.8f * mean + 0.2f * most));
+        const float kb = (t.features * (1.f + 0.2501f / m_tiles) + t.tokens) * 64 / 1024.f;     // copied per block and k-step
+        us = steps * (0.1277f * rounds + (t.features == 128 ? 0.0175f : 0.0198f) * kb * (0.8026f * mean + 0.1974f * most));
     }
-    if (splits > 1) us += 2.38e-6f * M * N * splits;
+    if (splits > 1) us += 1.06f + 2.351e-6f * M * N * splits;
     return us;
 }
 
@@ -622,6 +640,9 @@ static void launch_tiled(int variant, int splits, hipStream_t stream, const bf16
         case 12: launch_async<6, 4, 4, 4, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
         case 13: launch_async<4, 4, 2, 8, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
         case 14: launch_async<7, 3, 4, 5, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
+        case 15: launch_async<8, 5, 4, 4, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
+        case 16: launch_async<7, 5, 4, 4, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
+        case 17: launch_async<7, 6, 4, 4, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
         case 10: launch_async<8, 4, 4, 4, 1, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
         default: launch_async<8, 4, 2, 3, 2, TOut, EPI>(splits, stream, x, wp, out, M, N, K, n_steps, per, out_cols, rs, fu); break;
     }
@@ -655,7 +676,7 @@ static int tiled_entry(const void* x, const void* w_packed, void* out, float* wo
     FL_CHECK(!in_ssq || in_parts > 0, "gemm_tiled: a row scale over %d parts", in_parts);
     if (M == 0) return 0;
     const int n_steps = ceil_div(K, 32);
-    FL_CHECK(tiled_known(variant), "gemm_tiled: block shape %d (0, 3, 6, 7, 8 or 10 to 14)", variant);
+    FL_CHECK(tiled_known(variant), "gemm_tiled: block shape %d (0, 3, 6, 7, 8 or 10 to 17)", variant);
     const TilePlan plan = tiled_plan(M, N, K, !epilogue, variant, epilogue ? 1 : forced_splits);
     const int splits = plan.splits, v = plan.variant;
     FL_CHECK(splits == 1 || workspace, "gemm_tiled: this shape splits K %d ways and needs a workspace", splits);
@@ -725,7 +746,7 @@ FL_RECORDABLE(fl_gemm_tiled)
 extern "C" int fl_gemm_tiled_residual_ex(const void* x, const void* w_packed, float* workspace, int M, int N, int K,
                                          float* resid, const float* g, void* xg, float* out_ssq, int variant,
                                          hipStream_t stream) {
-    FL_CHECK(tiled_known(variant), "gemm_tiled_residual: block shape %d (0, 3, 6, 7, 8 or 10 to 14)", variant);
+    FL_CHECK(tiled_known(variant), "gemm_tiled_residual: block shape %d (0, 3, 6, 7, 8 or 10 to 17)", variant);
     FL_CHECK(M >= 0 && N > 0 && K > 0, "gemm_tiled_residual: bad sizes M=%d N=%d K=%d", M, N, K);
     FL_CHECK(K % 8 == 0, "gemm_tiled_residual: K=%d is no multiple of 8 (16-byte loads)", K);
     FL_CHECK(N % 4 == 0, "gemm_tiled_residual: N=%d is no multiple of 4 (16-byte accesses to the residual rows)", N);
@@ -816,7 +837,7 @@ extern "C" int fl_gemm_tiled_rope_ex(const void* x, const void* w_packed, int M,
                                      const int* block_table, int max_blocks, const float* cs, void* q_out,
                                      void* cache_base, int nh, int nkv, int hd, int page_size, int n_pages, int rot,
                                      int write_cache, int variant, hipStream_t stream) {
-    FL_CHECK(tiled_known(variant), "gemm_tiled_rope: block shape %d (0, 3, 6, 7, 8 or 10 to 14)", variant);
+    FL_CHECK(tiled_known(variant), "gemm_tiled_rope: block shape %d (0, 3, 6, 7, 8 or 10 to 17)", variant);
     FL_CHECK(M >= 0 && N > 0 && K > 0, "gemm_tiled_rope: bad sizes M=%d N=%d K=%d", M, N, K);
     FL_CHECK(K % 8 == 0, "gemm_tiled_rope: K=%d is no multiple of 8 (16-byte loads)", K);
     FL_CHECK(positions && tok_seq && block_table && cs && q_out && cache_base,

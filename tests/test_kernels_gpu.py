@@ -694,11 +694,11 @@ def test_gemm_tiled_against_plain(out_dtype, M, N, K):
     assert (got.double() - ref).abs().max() < tol * scale
 
 
-@pytest.mark.parametrize("variant", [3, 6, 7, 8, 10, 11, 12, 13, 14])
+@pytest.mark.parametrize("variant", [3, 6, 7, 8, 10, 11, 12, 13, 14, 15, 16, 17])
 @pytest.mark.parametrize("M,N,K", [(300, 520, 72), (129, 264, 96), (1100, 640, 256), (400, 452, 1032)])
 def test_gemm_tiled_block_shapes(variant, M, N, K):
     """Every block shape of the tiled product (features x tokens: 256, 192 or 128 x 128; 256, 224, 192 or 128 x 256;
-    128 x 128 alone on its unit; 224 x 192), whichever the sizes would choose, through the plain epilogue, SwiGLU, the row scale and
+    128 x 128 alone on its unit; 224 x 192; 256 or 224 x 320; 224 x 384), whichever the sizes would choose, through the plain epilogue, SwiGLU, the row scale and
     the add-to-the-stream epilogue."""
     from flambeau_amd.kernels.library import load
     from flambeau_amd.kernels.packing import pack_weight
@@ -743,10 +743,10 @@ def test_gemm_tiled_block_shapes(variant, M, N, K):
         assert (out2.double() - ref2).abs().max() < 1e-2 * ref2.abs().max()
 
 
-@pytest.mark.parametrize("M,N,K,gate,variant,splits", [(1040, 5120, 32768, False, 11, 2), (384, 16384, 2048, True, 8, 1)])
+@pytest.mark.parametrize("M,N,K,gate,variant,splits", [(1040, 5120, 32768, False, 11, 2), (384, 16384, 2048, True, 8, 1), (528, 28672, 4096, True, 16, 1)])
 def test_gemm_tiled_plan_knows_what_is_faster(M, N, K, gate, variant, splits):
     """Block shapes and parts that are a fifth faster than what the plan once picked for these sizes (473 and 50 us against
-    358 and 40): what it picks now is within a tenth of them.  Weights from memory: enough copies that none stays in a
+    358 and 40; 163 against 121): what it picks now is within a tenth of them.  Weights from memory: enough copies that none stays in a
     cache."""
     copies = max(2, -(-600_000_000 // (2 * N * K)))
     w = [rnd(N * K, dtype=torch.bfloat16, seed=22, scale=0.05) for _ in range(copies)]       # (N, K multiples of a tile: any values are a packed matrix)
@@ -1228,11 +1228,11 @@ def test_gemm_float_leaves_short_sums_to_the_plain_kernel(M, N, K):
 
 
 # ---------------------------------------------------------------- the tiled product's blocks
-@pytest.mark.parametrize("variant", [10, 11, 12, 13, 14])
-@pytest.mark.parametrize("M,N,K", [(1, 16, 8), (255, 223, 32), (257, 449, 40), (256, 192, 128), (193, 225, 160), (128, 129, 256), (300, 1000, 104),
+@pytest.mark.parametrize("variant", [10, 11, 12, 13, 14, 15, 16, 17])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 8), (255, 223, 32), (257, 449, 40), (256, 192, 128), (193, 225, 160), (385, 257, 96), (128, 129, 256), (300, 1000, 104),
                                    (512, 700, 4096)])
 def test_gemm_tiled_eight_waves_equal_four(variant, M, N, K):
-    """256, 224 and 192 features x 256 tokens, 224 x 192 and 128 x 128 in a deep ring against 256 x 128: every output is
+    """256, 224 and 192 features x 256 tokens, 224 x 192, 256 and 224 x 320, 224 x 384 and 128 x 128 in a deep ring against 256 x 128: every output is
     the same chain over K, so the same bits; one stage, fewer and more stages than the ring, K's and the tiles' remainders."""
     from flambeau_amd.kernels.packing import pack_weight
     x, w = rnd(M, K, dtype=torch.bfloat16, seed=41), rnd(N, K, dtype=torch.bfloat16, seed=42, scale=0.05)
@@ -1244,7 +1244,7 @@ def test_gemm_tiled_eight_waves_equal_four(variant, M, N, K):
     assert torch.equal(*got)
 
 
-@pytest.mark.parametrize("variant", [3, 7, 11, 12, 14])
+@pytest.mark.parametrize("variant", [3, 7, 11, 12, 14, 15, 17])
 @pytest.mark.parametrize("M,inter", [(1, 8), (130, 113), (257, 132), (300, 264), (193, 226)])
 def test_gemm_tiled_activation_for_rows_of_any_width(variant, M, inter):
     """Rows of results that are whole multiples of eight, of four and of neither, in tiles of features with four, six,
