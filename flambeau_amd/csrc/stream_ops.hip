@@ -65,23 +65,38 @@ extern "C" int fl_dyt(const float* x, const float* delta, float* resid_out, cons
 FL_RECORDABLE(fl_dyt)
 
 // ------------------------------------------------------------------ embedding with a factor
+// (a row over several blocks, four values a thread where rows are whole pieces of four: one trip to memory instead of one per 256
+// values; 8 rows of 4096 in bfloat16 10.1 -> 3.5 us, 2,048 rows 18.9 -> 14.1)
 template <typename T>
 __global__ __launch_bounds__(256) void embed_scaled_kernel(const T* __restrict__ table, const int* __restrict__ tokens,
-                                                           float* __restrict__ out, int H, int V, float scale) {
+                                                           float* __restrict__ out, int H, int V, float scale, int pieces) {
     int tok = tokens[blockIdx.x];
     if (tok < 0 || tok >= V) tok = 0;  // the host rejects such ids before the launch
     const T* src = table + (size_t)tok * H;
-    for (int i = threadIdx.x; i < H; i += 256) out[(size_t)blockIdx.x * H + i] = to_f32(src[i]) * scale;
+    float* dst = out + (size_t)blockIdx.x * H;
+    const int first = blockIdx.y * 256 + threadIdx.x, step = gridDim.y * 256;
+    if (pieces) {
+        for (int i = 4 * first; i < H; i += 4 * step) {
+            T v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = src[i + u];
+            *(f32x4*)(dst + i) = (f32x4){to_f32(v[0]) * scale, to_f32(v[1]) * scale, to_f32(v[2]) * scale, to_f32(v[3]) * scale};
+        }
+    } else {
+        for (int i = first; i < H; i += step) dst[i] = to_f32(src[i]) * scale;
+    }
 }
 
 extern "C" int fl_embed_scaled(const void* table, int dtype, const int* tokens, float* out, int n, int H, int V, float scale,
                                hipStream_t stream) {
     FL_CHECK(n >= 0 && H > 0 && V > 0, "embed_scaled: bad sizes");
     if (n == 0) return 0;
+    const int pieces = H % 4 == 0 && (uintptr_t)table % 16 == 0 && (uintptr_t)out % 16 == 0;
+    const dim3 grid(n, min(ceil_div(H, 1024), 64));
     if (dtype == FL_F32)
-        embed_scaled_kernel<float><<<n, 256, 0, stream>>>((const float*)table, tokens, out, H, V, scale);
+        embed_scaled_kernel<float><<<grid, 256, 0, stream>>>((const float*)table, tokens, out, H, V, scale, pieces);
     else if (dtype == FL_BF16)
-        embed_scaled_kernel<bf16_t><<<n, 256, 0, stream>>>((const bf16_t*)table, tokens, out, H, V, scale);
+        embed_scaled_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)table, tokens, out, H, V, scale, pieces);
     else
         FL_CHECK(false, "embed_scaled: unknown dtype %d", dtype);
     FL_LAUNCH_CHECK();
@@ -165,28 +180,70 @@ FL_RECORDABLE(fl_clamped_gate)
 
 // ------------------------------------------------------------------ weighted sum of two normed rows
 // out[t][i] = ca * a[t][i] / rms(a[t]) * wa[i] + cb * b[t][i] / rms(b[t]) * wb[i], rms with eps inside the root.
+// PIECES: the 16-byte pieces of each row that a thread holds in registers between the sums and the results (0: any sizes, rows read
+// twice a value at a time, a trip to memory per 256 values: 8 rows of 4096 10.5 us, 2,048 rows 27.7; with four pieces 4.6 and 18.9).
+template <int PIECES>
 __global__ __launch_bounds__(256) void norm_mix_kernel(const float* __restrict__ a, const float* __restrict__ wa, float ca,
                                                        const float* __restrict__ b, const float* __restrict__ wb, float cb,
                                                        float* __restrict__ out, int H, float eps) {
     __shared__ float lds[8];
     const float* ar = a + (size_t)blockIdx.x * H;
     const float* br = b + (size_t)blockIdx.x * H;
+    float* dst = out + (size_t)blockIdx.x * H;
     float sa = 0.f, sb = 0.f;
-    for (int i = threadIdx.x; i < H; i += 256) {
-        sa = fmaf(ar[i], ar[i], sa);
-        sb = fmaf(br[i], br[i], sb);
+    if constexpr (PIECES > 0) {
+        f32x4 va[PIECES], vb[PIECES];
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {
+            const int i = 4 * (threadIdx.x + 256 * p);
+            const bool in = i < H;
+            va[p] = *(const f32x4*)(ar + (in ? i : 0));
+            vb[p] = *(const f32x4*)(br + (in ? i : 0));
+        }
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (4 * (threadIdx.x + 256 * p) < H) {
+                    sa = fmaf(va[p][r], va[p][r], sa);
+                    sb = fmaf(vb[p][r], vb[p][r], sb);
+                }
+        sa = block_sum<4>(sa, lds);
+        sb = block_sum<4>(sb, lds + 4);
+        const float ia = ca / sqrtf(sa / (float)H + eps), ib = cb / sqrtf(sb / (float)H + eps);
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {
+            const int i = 4 * (threadIdx.x + 256 * p);
+            if (i < H) {
+                const f32x4 ga = *(const f32x4*)(wa + i), gb = *(const f32x4*)(wb + i);
+                f32x4 o;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[r] = va[p][r] * ia * ga[r] + vb[p][r] * ib * gb[r];
+                *(f32x4*)(dst + i) = o;
+            }
+        }
+    } else {
+        for (int i = threadIdx.x; i < H; i += 256) {
+            sa = fmaf(ar[i], ar[i], sa);
+            sb = fmaf(br[i], br[i], sb);
+        }
+        sa = block_sum<4>(sa, lds);
+        sb = block_sum<4>(sb, lds + 4);
+        const float ia = ca / sqrtf(sa / (float)H + eps), ib = cb / sqrtf(sb / (float)H + eps);
+        for (int i = threadIdx.x; i < H; i += 256) dst[i] = ar[i] * ia * wa[i] + br[i] * ib * wb[i];
     }
-    sa = block_sum<4>(sa, lds);
-    sb = block_sum<4>(sb, lds + 4);
-    const float ia = ca / sqrtf(sa / (float)H + eps), ib = cb / sqrtf(sb / (float)H + eps);
-    for (int i = threadIdx.x; i < H; i += 256) out[(size_t)blockIdx.x * H + i] = ar[i] * ia * wa[i] + br[i] * ib * wb[i];
 }
 
 extern "C" int fl_norm_mix(const float* a, const float* wa, float ca, const float* b, const float* wb, float cb, float* out,
                            int n, int H, float eps, hipStream_t stream) {
     FL_CHECK(n >= 0 && H > 0, "norm_mix: bad sizes");
     if (n == 0) return 0;
-    norm_mix_kernel<<<n, 256, 0, stream>>>(a, wa, ca, b, wb, cb, out, H, eps);
+    const bool whole = H % 4 == 0 && ((uintptr_t)a | (uintptr_t)wa | (uintptr_t)b | (uintptr_t)wb | (uintptr_t)out) % 16 == 0;
+    const int pieces = whole ? ceil_div(H, 1024) : 9;
+    if (pieces <= 2) norm_mix_kernel<2><<<n, 256, 0, stream>>>(a, wa, ca, b, wb, cb, out, H, eps);
+    else if (pieces <= 4) norm_mix_kernel<4><<<n, 256, 0, stream>>>(a, wa, ca, b, wb, cb, out, H, eps);
+    else if (pieces <= 8) norm_mix_kernel<8><<<n, 256, 0, stream>>>(a, wa, ca, b, wb, cb, out, H, eps);
+    else norm_mix_kernel<0><<<n, 256, 0, stream>>>(a, wa, ca, b, wb, cb, out, H, eps);
     FL_LAUNCH_CHECK();
     return 0;
 }
@@ -198,9 +255,30 @@ FL_RECORDABLE(fl_norm_mix)
 template <typename T>
 __global__ __launch_bounds__(256) void heads_gate_kernel(const T* __restrict__ x, int ldh, const float* __restrict__ gate, int ldg,
                                                          int gate_col0, int kind, int per_head, float scale, T* __restrict__ out,
-                                                         int ldo, int H, int Dv) {
+                                                         int ldo, int H, int Dv, int pieces) {
     const size_t t = blockIdx.x;
-    // (a token's values are spread over blocks, so that a step of few tokens still fills units)
+    // (a token's values are spread over blocks, so that a step of few tokens still fills units; pieces: four values a thread, 2,048
+    // tokens of 32 heads of 128 24.5 -> 17.3 us)
+    if (pieces) {
+        for (int e = 4 * (blockIdx.y * 256 + threadIdx.x); e < H * Dv; e += 1024 * gridDim.y) {
+            const int h = e / Dv, j = e - h * Dv;
+            T v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = x[(t * H + h) * ldh + j + r];
+            float z[4] = {0.f, 0.f, 0.f, 0.f};
+            if (kind) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) z[r] = gate[t * ldg + gate_col0 + (per_head ? h : e + r)];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float o = to_f32(v[r]) * scale;
+                if (kind) o *= kind == 1 ? 1.0f / (1.0f + expf(-z[r])) : z[r] / (1.0f + expf(-z[r]));
+                out[t * ldo + e + r] = from_f32<T>(o);
+            }
+        }
+        return;
+    }
     for (int e = blockIdx.y * 256 + threadIdx.x; e < H * Dv; e += 256 * gridDim.y) {
         const int h = e / Dv, j = e - h * Dv;
         float v = to_f32(x[(t * H + h) * ldh + j]) * scale;
@@ -218,11 +296,14 @@ extern "C" int fl_heads_gate(const void* x, int dtype, int ldh, const float* gat
     FL_CHECK(kind >= 0 && kind <= 2 && (kind == 0 || (gate && ldg >= gate_col0 + (per_head ? H : H * Dv))), "heads_gate: gate %d over rows %d wide", kind, ldg);
     FL_CHECK(ldo >= H * Dv, "heads_gate: output rows of %d values for %d heads of %d", ldo, H, Dv);
     if (n == 0) return 0;
-    const dim3 grid(n, min(ceil_div(H * Dv, 512), 64));
+    const dim3 grid(n, min(ceil_div(H * Dv, 1024), 64));
+    const size_t piece = dtype == FL_F32 ? 16 : 8;                     // four values of x and of out, and of the gate
+    const int pieces = Dv % 4 == 0 && ldh % 4 == 0 && ldo % 4 == 0 && (uintptr_t)x % piece == 0 && (uintptr_t)out % piece == 0 &&
+                       (!kind || per_head || (ldg % 4 == 0 && gate_col0 % 4 == 0 && (uintptr_t)gate % 16 == 0));
     if (dtype == FL_F32)
-        heads_gate_kernel<float><<<grid, 256, 0, stream>>>((const float*)x, ldh, gate, ldg, gate_col0, kind, per_head, scale, (float*)out, ldo, H, Dv);
+        heads_gate_kernel<float><<<grid, 256, 0, stream>>>((const float*)x, ldh, gate, ldg, gate_col0, kind, per_head, scale, (float*)out, ldo, H, Dv, pieces);
     else if (dtype == FL_BF16)
-        heads_gate_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldh, gate, ldg, gate_col0, kind, per_head, scale, (bf16_t*)out, ldo, H, Dv);
+        heads_gate_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldh, gate, ldg, gate_col0, kind, per_head, scale, (bf16_t*)out, ldo, H, Dv, pieces);
     else
         FL_CHECK(false, "heads_gate: unknown dtype %d", dtype);
     FL_LAUNCH_CHECK();

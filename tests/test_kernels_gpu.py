@@ -1585,3 +1585,89 @@ def test_attn_float_takes_no_longer_for_few_keys(context):
     """Eight requests of one token: measured 4 to 6 us, 11 to 13 with every row on the matrix cores (plain 3.7 to 12)."""
     fast, plain = attn_float_times(32, 8, 128, [(context, 1)] * 8)
     assert fast < 1.4 * plain + 1, (fast, plain)
+
+
+# ---------------------------------------------------------------- kernels that take whole pieces of four values, and any sizes
+def _near(got, want, roundings=8):
+    """A handful of 32-bit roundings (and, into the eight bits of bfloat16, one of 2^-8) of values of this size."""
+    step = 2.0 ** -8 if got.dtype == torch.bfloat16 else 0.0
+    assert bool(((got.double() - want).abs() <= roundings * 2.0 ** -23 * want.abs().max() + 1.01 * step * want.abs()).all())
+
+
+@pytest.mark.parametrize("n", [1, 9, 70])
+@pytest.mark.parametrize("H", [4, 1020, 1022, 1024, 2048, 4096, 4100, 8192, 8196])
+def test_rows_in_pieces_and_one_by_one(n, H):
+    """Scaled embedding rows and the sum of two normed rows: widths that are whole pieces of four or not, of one to eight pieces
+    a thread, and beyond."""
+    for dtype in (torch.float32, torch.bfloat16):
+        table, out = rnd(11, H, dtype=dtype, seed=70), torch.full((n, H), float("nan"), dtype=torch.float32, device=DEV)
+        tokens = torch.arange(n, dtype=torch.int32, device=DEV) % 11
+        ops().embed_scaled(table, tokens, out, 7.5)
+        assert torch.equal(out, table[tokens.long()].float() * 7.5)
+    a, b, wa, wb = rnd(n, H, seed=71), rnd(n, H, seed=72, scale=3.0), rnd(H, seed=73), rnd(H, seed=74)
+    out = torch.full((n, H), float("nan"), dtype=torch.float32, device=DEV)
+    ops().norm_mix(a, wa, 0.7, b, wb, 1.3, out, 1e-5)
+    normed = lambda t, w: t.double() * torch.rsqrt((t.double() ** 2).mean(1, keepdim=True) + 1e-5) * w.double()
+    _near(out, 0.7 * normed(a, wa) + 1.3 * normed(b, wb))
+
+
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("n,H,D,rot,col", [(3, 2, 128, 128, 0), (70, 3, 64, 24, 4), (5, 1, 128, 20, 0), (2, 2, 30, 30, 0), (9, 16, 128, 64, 3), (4, 2, 128, 0, 8)])
+def test_rotate_scale_in_pieces_and_one_by_one(interleaved, n, H, D, rot, col):
+    proj = rnd(n, col + 2 * H * D + 5, seed=75)
+    angle = rnd(n, max(rot // 2, 1), seed=76).double()
+    table = torch.stack([angle.cos(), angle.sin()], dim=-1).float().contiguous()
+    outs = [torch.full((n, H * D), float("nan"), dtype=torch.float32, device=DEV) for _ in range(2)]
+    ops().rotate_scale(proj, col, col + H * D, table if rot else None, rot, interleaved, 0.5, 2.0, *outs, H, D)
+    for out, c, scale in ((outs[0], col, 0.5), (outs[1], col + H * D, 2.0)):
+        x = proj[:, c:c + H * D].double().reshape(n, H, D)
+        want = x.clone()
+        if rot:
+            cos, sin = (t.double()[:, None, :] for t in (table[..., 0], table[..., 1]))
+            i, k = (slice(0, rot, 2), slice(1, rot, 2)) if interleaved else (slice(0, rot // 2), slice(rot // 2, rot))
+            want[..., i], want[..., k] = x[..., i] * cos - x[..., k] * sin, x[..., k] * cos + x[..., i] * sin
+        _near(out, (want * scale).reshape(n, H * D))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,H,Dv,ldh,col", [(3, 2, 128, 128, 4), (70, 4, 64, 96, 0), (2, 3, 30, 32, 1), (5, 33, 128, 128, 2), (4, 2, 256, 256, 0)])
+def test_gates_of_heads_in_pieces_and_one_by_one(dtype, n, H, Dv, ldh, col):
+    x, gate, act = rnd(n, H * ldh, dtype=dtype, seed=77), rnd(n, col + H * Dv + 4, seed=78), {"sigmoid": torch.sigmoid, "silu": torch.nn.functional.silu}
+    heads = x.double().reshape(n, H, ldh)[:, :, :Dv]
+    for kind in ("sigmoid", "silu"):
+        for per_head in (False, True):
+            out = torch.full((n, H * Dv), float("nan"), dtype=dtype, device=DEV)
+            ops().heads_gate(x, ldh, gate, col, kind, out, H, per_head, 1.25)
+            z = gate[:, col:col + (H if per_head else H * Dv)].double().reshape(n, H, -1)
+            _near(out, (heads * 1.25 * act[kind](z)).reshape(n, H * Dv))
+        y, w = x.float().reshape(n, H, ldh)[:, :, :Dv].contiguous(), rnd(H * Dv, seed=79)
+        out = torch.full((n, H * Dv), float("nan"), dtype=dtype, device=DEV)
+        ops().headnorm_gate(y.reshape(n, H * Dv), w, gate, col, out, H, 1e-5, gate_kind=kind)
+        z = gate[:, col:col + H * Dv].double().reshape(n, H, Dv)
+        normed = y.double() * torch.rsqrt((y.double() ** 2).mean(-1, keepdim=True) + 1e-5)
+        _near(out, (normed * w.double().reshape(H, Dv) * act[kind](z)).reshape(n, H * Dv))
+
+
+@pytest.mark.parametrize("lens", [[1024], [300, 1, 2, 5, 700, 8, 9], [3, 4, 1013], [20, 7]])
+@pytest.mark.parametrize("G,H,D,Dv", [(4, 12, 128, 128), (4, 16, 64, 32), (2, 16, 128, 48)])
+def test_convolution_of_runs_of_tokens(lens, G, H, D, Dv):
+    """Steps of many tokens take eight tokens a wave, others one: requests that end anywhere in such a run, one-token requests, kept
+    inputs of earlier steps."""
+    n, S, C = sum(lens), len(lens), 2 * G * D + H * Dv
+    ints = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    proj, w, old = rnd(n, C + 2 * H, seed=80), rnd(C, 4, seed=81), rnd(S, 3, C, seed=82)
+    a_log, dt_bias, state = rnd(H, seed=83), rnd(H, seed=84), old.reshape(S, 3 * C).clone()
+    prep, gates = (torch.full((n, k), float("nan"), dtype=torch.float32, device=DEV) for k in (C, 2 * H))
+    starts = [sum(lens[:i]) for i in range(S)]
+    seqs = [s for s, length in enumerate(lens) for _ in range(length)]
+    ops().conv_prepare(proj, 0, C, C + H, w, a_log, dt_bias, state, 0, ints(seqs), ints(starts), ints(lens), ints(list(range(S))), prep, gates,
+                       G, H, D, Dv, 4, 0.3, 1e-6)
+    for s, (at, length) in enumerate(zip(starts, lens)):
+        x = torch.cat([old[s], proj[at:at + length, :C]]).double()
+        y = torch.nn.functional.silu(sum(x[m:m + length] * w[:, m].double() for m in range(4)))
+        qk = y[:, :2 * G * D].reshape(length, 2, G, D)
+        qk = qk / (qk.square().sum(-1, keepdim=True) + 1e-6).sqrt() * torch.tensor([0.3, 1.0], device=DEV, dtype=torch.float64)[None, :, None, None]
+        _near(prep[at:at + length], torch.cat([qk.reshape(length, -1), y[:, 2 * G * D:]], dim=1), 16)
+        assert torch.equal(state[s].reshape(3, C), x[-3:].float())
+    _near(gates[:, H:], torch.sigmoid(proj[:, C:C + H].double()))
+    _near(gates[:, :H], torch.exp(-torch.exp(a_log.double()) * torch.nn.functional.softplus(proj[:, C + H:].double() + dt_bias.double())), 32)
