@@ -13,6 +13,10 @@
 // With a decay per key dim: the pairs, q times the decays up to its token [64][D], k times those behind its token [64][D], the
 // whole chunk's decays [D] and what their rounding left [D]
 #define SC_CHANNEL_Q (SC_CHUNK * SC_CHUNK)
+// The delta rule: as without it (no write strengths), then T diag(beta) [64][64] and T diag(beta p) k [64][D]
+#define SC_DELTA_T SC_RECORD
+#define SC_DELTA_W (SC_DELTA_T + SC_CHUNK * SC_CHUNK)
+#define SC_DELTA_RECORD(D) (SC_DELTA_W + SC_CHUNK * (D))
 #define SC_CHANNEL_RECORD(D) (SC_CHANNEL_Q + 2 * SC_CHUNK * (D) + 2 * (D))
 
 struct ScanChunks {
@@ -36,6 +40,7 @@ struct ScanChunks {
     const float* skip;
     const float* chan_decay;     // a decay per token, head and key dim (then neither of the other two, and no write strengths)
     int ldc;
+    int corrects;                // the delta rule: u = write (v - S^T k)
 };
 
 // Sizes that it takes, and the records (SC_RECORD floats per head each) that n tokens in n_seqs requests may need.

@@ -8,6 +8,14 @@
 //     of decays, one record per chunk and head in the workspace;
 //   scan_chunks: a block per request, head and 16 columns of S walks the chunks: per chunk and wave 16 tokens' outputs and
 //     D / 4 rows of S, the next chunk's operands on their way in registers meanwhile.
+// The delta rule writes u_i = beta_i (v_i - what the state before it holds at k_i), so that a chunk's u depend on each other:
+//     (I + L) U = diag(beta) V - diag(beta p) K S,      L_ij = beta_i d_ij (k_i . k_j) for j < i;
+// scan_pairs_delta forms T = (I + L)^-1 (unit lower triangular), T diag(beta) and T diag(beta p) K for every chunk at once, and the
+// walk makes U from v and S, exchanges it between the waves through LDS, and goes on with it in the place of v.
+// Measured, 2,048 tokens, the walk and the chunks (pairs + walk over chunks): a decay per head, 16 heads of 128 x 128, 304 us, 16 + 84;
+// with write strengths, 32 heads of 128 x 64, 309, 21 + 85; a decay per key dim, 32 heads of 128 x 128, 328, 45 + 108; the delta rule, 32
+// heads of 128 x 128, 371, 65 + 134.  A chunk of the second kernel is 2.6 to 4.2 us where its matrix instructions are 1.2 to 2.0.  Error
+// against 64 bits (2-norm) 7.6e-7 -> 1.4e-7, 3.7e-7 -> 1.0e-7, 1.4e-7 -> 1.2e-7, 3.7e-7 -> 1.7e-7.
 // Products of decays are formed by multiplying, never through logarithms or quotients: a decay of zero is one, and their rounding
 // is the walk's.  All values and sums are 32-bit; a chunk's sums are added to the state once, where the walk rounds the state at
 // every token, so results are nearer to 64 bits than the walk's.
@@ -262,6 +270,187 @@ __global__ __launch_bounds__(256) void scan_pairs_channel_kernel(ScanChunks a) {
     }
 }
 
+// The delta rule's pairs, T diag(beta) and T diag(beta p) K.  T by tiles of 16 tokens: the four on the diagonal by substitution, a
+// column per lane; the others from those before them, T_IJ = -T_II sum_{J <= M < I} L_IM T_MJ, by their distance from the diagonal.  A
+// chunk whose keys, decays or strengths are not all finite substitutes throughout, so that what is no number reaches no token before it.
+template <int D>
+__global__ __launch_bounds__(256) void scan_pairs_delta_kernel(ScanChunks a) {
+    constexpr int ROW = D + 4, LT = SC_CHUNK + 4;
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    float* ks = lds;                               // [64][ROW] keys
+    float* L = ks + SC_CHUNK * ROW;                // [64][LT]
+    float* T = L + SC_CHUNK * LT;                  // [64][LT]: the decays between tokens first, then T
+    float* X = T + SC_CHUNK * LT;                  // [4][16][20] a wave's tile on its way from one operand form to the other
+    float* decay = X + 4 * 16 * 20;                // [64] each
+    float* beta = decay + SC_CHUNK;
+    float* pre = beta + SC_CHUNK;
+    __shared__ int odd;
+    const int2 at = scan_find(a.seq_q_len, a.n_seqs, a.min_len, blockIdx.x);
+    const int s = at.x, c = at.y;
+    if (s < 0) return;
+    const int head = blockIdx.y, qk_head = head / (a.H / a.G);
+    const int t0 = a.seq_q_start[s] + c * SC_CHUNK, cnt = min(SC_CHUNK, a.seq_q_len[s] - c * SC_CHUNK);
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    float* rec = a.records + ((size_t)blockIdx.x * a.H + head) * SC_DELTA_RECORD(D);
+    const auto qrows = scan_rows(a.q + (size_t)t0 * a.ldq + qk_head * D, cnt, a.ldq, D), krows = scan_rows(a.k + (size_t)t0 * a.ldk + qk_head * D, cnt, a.ldk, D);
+    const int I = (wave + blockIdx.x) & 3;         // the wave's 16 tokens
+    f32x4 q[D / 16];
+#pragma unroll
+    for (int u = 0; u < D / 16; ++u) q[u] = scan_load<4>(qrows, 4 * ((16 * I + n) * a.ldq + 4 * g), 64 * u);
+    if (tid == 0) odd = 0;
+    float strange = 0.f;                           // NaN where something loaded is no finite number
+#pragma unroll
+    for (int u = 0; u < SC_CHUNK * D / 4 / 256; ++u) {
+        const int e = tid + 256 * u, t = e / (D / 4), d = 4 * (e % (D / 4));
+        const f32x4 k = scan_load<4>(krows, 4 * (t * a.ldk + d), 0);
+        strange += ((k[0] - k[0]) + (k[1] - k[1])) + ((k[2] - k[2]) + (k[3] - k[3]));
+        *(f32x4*)(ks + t * ROW + d) = k;
+    }
+    if (tid < SC_CHUNK) {
+        const size_t row = (size_t)(t0 + min(tid, cnt - 1)) * a.ldg + head;
+        const float own = a.tok_decay[row], strength = a.write[row];
+        decay[tid] = tid < cnt ? own : 1.f;
+        beta[tid] = tid < cnt ? strength : 0.f;
+        strange += (own - own) + (strength - strength);
+    }
+    __syncthreads();
+    if (strange != 0.f) odd = 1;
+    if (wave == 0) {                               // lane j: the decays behind token j, up to every later one
+        double p = 1.0;
+        for (int i = 0; i < SC_CHUNK; ++i) {
+            if (i > lane) p *= decay[i];
+            T[i * LT + lane] = (float)p;
+        }
+        rec[SC_SUF + lane] = (float)p;
+    } else if (wave == 1) {                        // lane i: the chunk's decays up to token i
+        double p = 1.0;
+        for (int m = 0; m < SC_CHUNK; ++m)
+            if (m <= lane) p *= decay[m];
+        pre[lane] = (float)p;
+        rec[SC_PRE + lane] = (float)p;
+        if (lane == SC_CHUNK - 1) rec[SC_REST] = p == p && p <= 1e30 ? (float)(p - (double)(float)p) : 0.f;
+    }
+    f32x4 pair[4], same[4];                        // q_i . k_j and k_i . k_j
+#pragma unroll
+    for (int J = 0; J < 4; ++J) {
+        if (J > I) break;
+        f32x4 sum[8] = {}, own[8] = {};
+#pragma unroll
+        for (int u = 0; u < D / 16; ++u) {
+            const f32x4 k = *(const f32x4*)(ks + (16 * J + n) * ROW + 16 * u + 4 * g), ki = *(const f32x4*)(ks + (16 * I + n) * ROW + 16 * u + 4 * g);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                sum[4 * (u & 1) + r] = mfma_f32(q[u][r], k[r], sum[4 * (u & 1) + r]);
+                own[4 * (u & 1) + r] = mfma_f32(ki[r], k[r], own[4 * (u & 1) + r]);
+            }
+        }
+        pair[J] = sum_of_8(sum);
+        same[J] = sum_of_8(own);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int J = 0; J < 4; ++J)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int i = 16 * I + 4 * g + r, j = 16 * J + n;
+            const float between = J <= I ? T[i * LT + j] : 0.f;
+            if (J <= I) rec[i * SC_CHUNK + j] = j <= i && j < cnt ? pair[J][r] * between : 0.f;
+            const float l = J <= I && j < i ? beta[i] * (same[J][r] * between) : 0.f;
+            L[i * LT + j] = l;
+            if (l - l != 0.f) odd = 1;             // (keys too large to multiply)
+        }
+    __syncthreads();                               // (the decays between tokens have been read: their room is T's)
+    if (odd) {
+        if (tid < SC_CHUNK) {                      // column tid, row by row; nothing above the diagonal is multiplied
+            for (int i = 0; i < SC_CHUNK; ++i) {
+                float t = i == tid ? 1.f : 0.f;
+                if (i > tid)
+                    for (int j = tid; j < i; ++j) t = fmaf(-L[i * LT + j], T[j * LT + tid], t);
+                T[i * LT + tid] = t;
+            }
+        }
+        __syncthreads();
+        for (int d = tid; d < D; d += 256)
+            for (int i = 0; i < SC_CHUNK; ++i) {
+                float w = 0.f;
+                for (int j = 0; j <= i; ++j) w = fmaf(T[i * LT + j] * (beta[j] * pre[j]), ks[j * ROW + d], w);
+                rec[SC_DELTA_W + i * D + d] = w;
+            }
+    } else {
+        {   // the tile on the diagonal: lane n has column n (all four lanes g the same)
+            float t[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                float row[16];
+#pragma unroll
+                for (int j = 0; j < 16; j += 4) *(f32x4*)(row + j) = *(const f32x4*)(L + (16 * wave + i) * LT + 16 * wave + j);
+                float sum = i == n ? 1.f : 0.f;
+#pragma unroll
+                for (int j = 0; j < i; ++j) sum = fmaf(-row[j], t[j], sum);
+                t[i] = sum;
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (g == i >> 2) T[(16 * wave + i) * LT + 16 * wave + n] = t[i];
+        }
+        __syncthreads();
+        float* x = X + wave * 16 * 20;
+#pragma unroll
+        for (int away = 1; away < 4; ++away) {
+            if (wave + away < 4) {
+                const int J = wave, R = wave + away;
+                f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+                for (int M = J; M < R; ++M) {
+                    const f32x4 l = *(const f32x4*)(L + (16 * R + n) * LT + 16 * M + 4 * g);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sum = mfma_f32(l[e], T[(16 * M + 4 * g + e) * LT + 16 * J + n], sum);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) x[(4 * g + r) * 20 + n] = sum[r];
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                f32x4 out = {0.f, 0.f, 0.f, 0.f};
+                const f32x4 t = *(const f32x4*)(T + (16 * R + n) * LT + 16 * R + 4 * g);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) out = mfma_f32(-t[e], x[(4 * g + e) * 20 + n], out);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) T[(16 * R + 4 * g + r) * LT + 16 * J + n] = out[r];
+            }
+            __syncthreads();
+        }
+        // T diag(beta p) K for the wave's 16 tokens
+        f32x4 t[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            t[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            if (b < I) t[b] = *(const f32x4*)(T + (16 * I + n) * LT + 16 * b + 4 * g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int j = 16 * b + 4 * g + e;
+                if (b == I) t[b][e] = 4 * g + e <= n ? T[(16 * I + n) * LT + j] : 0.f;
+                t[b][e] *= beta[j] * pre[j];
+            }
+        }
+#pragma unroll 2
+        for (int dt = 0; dt < D / 16; ++dt) {
+            f32x4 sum[4] = {};
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+                if (b <= I) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sum[e] = mfma_f32(t[b][e], ks[(16 * b + 4 * g + e) * ROW + 16 * dt + n], sum[e]);
+                }
+            const f32x4 w = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) rec[SC_DELTA_W + (16 * I + 4 * g + r) * D + 16 * dt + n] = w[r];
+        }
+    }
+    for (int e = tid; e < SC_CHUNK * SC_CHUNK; e += 256) {
+        const int i = e >> 6, j = e & 63;
+        rec[SC_DELTA_T + e] = j <= i ? T[i * LT + j] * beta[j] : 0.f;
+    }
+}
+
 // Block = (head, columns j0 .. j0 + 15, request), four waves (neighbouring blocks are neighbouring heads: the blocks of a head, which
 // read the same q and k, share a die's L2 where the number of heads is a multiple of eight).  Wave w has the outputs of the chunk's
 // tokens 16 w .. 16 w + 15 and the rows d = D / 4 w + NT n + i of S (n = lane % 16, i < NT) as S^T, whose operand form all waves
@@ -269,18 +458,18 @@ __global__ __launch_bounds__(256) void scan_pairs_channel_kernel(ScanChunks a) {
 // B) and the state (as A), and q, the pairs and S come in 16-byte pieces.  Every operand is asked for again, for the next chunk,
 // right behind its last use in this one, into the same registers: the trip hides behind the rest of the chunk (a second set of
 // registers did not fit: the compiler moved them through the accumulators, each move a wait).
-template <int D, bool CHAN>
+template <int D, bool CHAN, bool DELTA>
 __global__ __launch_bounds__(256, 1) void scan_chunks_kernel(ScanChunks a) {
     constexpr int NT = D / 64, ROW = D + 4;
     typedef __attribute__((ext_vector_type(NT))) float fNT;
-    __shared__ __attribute__((aligned(16))) float st_lds[2][SC_COLS * ROW];
+    __shared__ __attribute__((aligned(16))) float st_lds[2][SC_COLS * ROW], u_lds[DELTA ? SC_COLS * (SC_CHUNK + 4) : 1];
     const int s = blockIdx.z, len = a.seq_q_len[s];
     if (len < a.min_len || len == 0) return;
     const int head = blockIdx.x, qk_head = head / (a.H / a.G), j0 = blockIdx.y * SC_COLS;
     const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int start = a.seq_q_start[s], n_chunks = (len + SC_CHUNK - 1) / SC_CHUNK;
-    constexpr int RECORD = CHAN ? SC_CHANNEL_RECORD(D) : SC_RECORD;
+    constexpr int RECORD = CHAN ? SC_CHANNEL_RECORD(D) : DELTA ? SC_DELTA_RECORD(D) : SC_RECORD;
     const size_t rec_step = (size_t)a.H * RECORD;
     const float* rec0 = a.records + ((size_t)scan_first_record(a.seq_q_len, s, a.min_len) * a.H + head) * RECORD;
     float* st = a.state + (size_t)a.seq_slots[s] * a.slot_stride + (size_t)head * D * a.Dv;
@@ -295,6 +484,7 @@ __global__ __launch_bounds__(256, 1) void scan_chunks_kernel(ScanChunks a) {
     const float skip = a.skip ? a.skip[head] : 0.f;
 
     f32x4 q[D / 16], pairs[4], suf[4], pre;
+    f32x4 wk[DELTA ? D / 16 : 1], tb[DELTA ? 4 : 1];           // T diag(beta p) k of the wave's tokens, T diag(beta)
     float v[4][4];
     fNT k[4][4], last, rest;                       // last: the whole chunk's decay, rest: what its rounding left
     const int ldq = CHAN ? D : a.ldq, ldk = CHAN ? D : a.ldk;
@@ -312,13 +502,19 @@ __global__ __launch_bounds__(256, 1) void scan_chunks_kernel(ScanChunks a) {
                      scan_rows(a.v + (size_t)t0 * a.ldv + head * a.Dv + j0, cnt, a.ldv, SC_COLS), rec};
     };
     auto load_q = [&](const Chunk& c, int u) { q[u] = scan_load<4>(c.q, q_at, 64 * u); };
+    auto load_v = [&](const Chunk& c, int b, int e) { v[b][e] = scan_load<1>(c.v, v_at, 4 * (16 * b + e) * a.ldv)[0]; };
     auto load_rows = [&](const Chunk& c, int b, int e) {
-        v[b][e] = scan_load<1>(c.v, v_at, 4 * (16 * b + e) * a.ldv)[0];
+        if (!DELTA) load_v(c, b, e);
         k[b][e] = scan_load<NT>(c.k, k_at, 4 * (16 * b + e) * ldk);
     };
     auto load_pairs = [&](const Chunk& c) {
 #pragma unroll
         for (int b = 0; b < 4; ++b) pairs[b] = *(const f32x4*)(c.rec + (16 * w + n) * SC_CHUNK + 16 * min(b, w) + 4 * g);
+    };
+    auto load_wk = [&](const Chunk& c, int u) { wk[DELTA ? u : 0] = *(const f32x4*)(c.rec + SC_DELTA_W + (16 * w + n) * D + 16 * u + 4 * g); };
+    auto load_tb = [&](const Chunk& c) {
+#pragma unroll
+        for (int b = 0; b < (DELTA ? 4 : 1); ++b) tb[b] = *(const f32x4*)(c.rec + SC_DELTA_T + (16 * w + n) * SC_CHUNK + 16 * min(b, w) + 4 * g);
     };
     auto load_decays = [&](const Chunk& c) {
         if constexpr (CHAN) {
@@ -335,6 +531,18 @@ __global__ __launch_bounds__(256, 1) void scan_chunks_kernel(ScanChunks a) {
     };
     {
         const Chunk first = chunk(0);
+        if constexpr (DELTA) {
+#pragma unroll
+            for (int u = 0; u < D / 16; ++u) load_wk(first, u);
+            __builtin_amdgcn_sched_barrier(0);
+            load_tb(first);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) load_v(first, b, e);
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int u = 0; u < D / 16; ++u) load_q(first, u);
         __builtin_amdgcn_sched_barrier(0);         // (in the order of the loop: what a wait counts there holds for the first chunk too)
@@ -348,6 +556,45 @@ __global__ __launch_bounds__(256, 1) void scan_chunks_kernel(ScanChunks a) {
         load_decays(first);
         __builtin_amdgcn_sched_barrier(0);
     }
+    // A lower triangular matrix (this wave's 16 rows of it, the tiles' columns left of the diagonal in `rows`) times the chunk's `x`;
+    // own: x of this wave's tokens.  The tile on the diagonal is not to meet values above it that are no numbers.
+    auto lower = [&](const auto& rows, const float (&x)[4][4], f32x4& own) {
+        f32x4 sum[4] = {}, row = rows[0];
+        own = (f32x4){x[0][0], x[0][1], x[0][2], x[0][3]};
+#pragma unroll
+        for (int b = 0; b < 3; ++b)
+            if (b < w) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    sum[e] = mfma_f32(rows[b][e], x[b][e], sum[e]);
+                    own[e] = x[b + 1][e];
+                }
+                row = rows[b + 1];
+            }
+        const f32x4 none = own - own;              // zero for finite values, NaN for others
+        const unsigned long long odd = __ballot((none[0] + none[1]) + (none[2] + none[3]) != 0.f);
+        f32x4 apart = sum[0];                      // of a column with such a value: the tile's tokens one by one, none of them before its own
+        if (odd != 0) {
+#pragma unroll 1
+            for (int t = 0; t < 16; ++t) {
+                const float xt = __shfl((t & 2) ? ((t & 1) ? own[3] : own[2]) : ((t & 1) ? own[1] : own[0]), 16 * (t >> 2) + n, 64);
+                const float rt = (t & 2) ? ((t & 1) ? row[3] : row[2]) : ((t & 1) ? row[1] : row[0]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float p = __shfl(rt, 16 * (t >> 2) + 4 * g + r, 64);
+                    if (t <= 4 * g + r) apart[r] = fmaf(p, xt, apart[r]);
+                }
+            }
+        }
+        apart += (sum[1] + sum[2]) + sum[3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] = mfma_f32(row[e], own[e], sum[e]);
+        const bool is_odd = (odd >> n | odd >> (16 + n) | odd >> (32 + n) | odd >> (48 + n)) & 1;
+        f32x4 all = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) all[r] = is_odd ? apart[r] : all[r];
+        return all;
+    };
     for (int c = 0; c < n_chunks; ++c) {
         const Chunk next = chunk(min(c + 1, n_chunks - 1));    // (no branch: the compiler would wait for every load behind one)
         float* lds = st_lds[c & 1];
@@ -363,50 +610,52 @@ __global__ __launch_bounds__(256, 1) void scan_chunks_kernel(ScanChunks a) {
         f32x4 sb[D / 16];
 #pragma unroll
         for (int u = 0; u < D / 16; ++u) sb[u] = *(const f32x4*)(lds + n * ROW + 16 * u + 4 * g);
+        float u[4][4];                             // what the chunk's tokens write
+        if constexpr (DELTA) {
+            f32x4 held[8] = {};                    // T diag(beta p) K S
+#pragma unroll
+            for (int i = 0; i < D / 16; ++i) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) held[4 * (i & 1) + e] = mfma_f32(wk[DELTA ? i : 0][e], sb[i][e], held[4 * (i & 1) + e]);
+                __builtin_amdgcn_sched_barrier(0); // (loads go out where they are written)
+                load_wk(next, i);
+            }
+            f32x4 own;
+            f32x4 mine = lower(tb, v, own);
+            __builtin_amdgcn_sched_barrier(0);
+            load_tb(next);
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) load_v(next, b, e);
+            mine -= sum_of_8(held);
+            *(f32x4*)(u_lds + n * (SC_CHUNK + 4) + 16 * w + 4 * g) = mine;
+        }
         // the state's part of the outputs
         f32x4 seen[8] = {};
 #pragma unroll
-        for (int u = 0; u < D / 16; ++u) {
+        for (int i = 0; i < D / 16; ++i) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) seen[4 * (u & 1) + e] = mfma_f32(q[u][e], sb[u][e], seen[4 * (u & 1) + e]);
+            for (int e = 0; e < 4; ++e) seen[4 * (i & 1) + e] = mfma_f32(q[i][e], sb[i][e], seen[4 * (i & 1) + e]);
             __builtin_amdgcn_sched_barrier(0);     // (loads go out where they are written)
-            load_q(next, u);
+            load_q(next, i);
         }
-        // the tile on the diagonal: this wave's own tokens
-        f32x4 own = {v[0][0], v[0][1], v[0][2], v[0][3]}, pair = pairs[0];
-        f32x4 within[4] = {};
+        if constexpr (DELTA) {
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
-        for (int b = 0; b < 3; ++b)
-            if (b < w) {
+            for (int b = 0; b < 4; ++b) {
+                const f32x4 four = *(const f32x4*)(u_lds + n * (SC_CHUNK + 4) + 16 * b + 4 * g);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    within[e] = mfma_f32(pairs[b][e], v[b][e], within[e]);
-                    own[e] = v[b + 1][e];
-                }
-                pair = pairs[b + 1];
+                for (int e = 0; e < 4; ++e) u[b][e] = four[e];
             }
-        const f32x4 none = own - own;              // zero for finite values, NaN for others
-        const unsigned long long odd = __ballot((none[0] + none[1]) + (none[2] + none[3]) != 0.f);
-        f32x4 apart = within[0];                   // of a column with such a value: the tile's tokens one by one, none of them before its own
-        if (odd != 0) {
-#pragma unroll 1
-            for (int t = 0; t < 16; ++t) {
-                const float vt = __shfl((t & 2) ? ((t & 1) ? own[3] : own[2]) : ((t & 1) ? own[1] : own[0]), 16 * (t >> 2) + n, 64);
-                const float pt = (t & 2) ? ((t & 1) ? pair[3] : pair[2]) : ((t & 1) ? pair[1] : pair[0]);
+        } else {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float p = __shfl(pt, 16 * (t >> 2) + 4 * g + r, 64);
-                    if (t <= 4 * g + r) apart[r] = fmaf(p, vt, apart[r]);
-                }
-            }
+            for (int b = 0; b < 4; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) u[b][e] = v[b][e];
         }
-        apart += (within[1] + within[2]) + within[3];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) within[e] = mfma_f32(pair[e], own[e], within[e]);
-        const bool is_odd = (odd >> n | odd >> (16 + n) | odd >> (32 + n) | odd >> (48 + n)) & 1;
-        f32x4 mine = (within[0] + within[1]) + (within[2] + within[3]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) mine[r] = is_odd ? apart[r] : mine[r];
+        f32x4 own;
+        const f32x4 mine = lower(pairs, u, own);
         __builtin_amdgcn_sched_barrier(0);
         load_pairs(next);
         // the state: this chunk's sums apart, 16 tokens a chain, added once
@@ -415,7 +664,7 @@ __global__ __launch_bounds__(256, 1) void scan_chunks_kernel(ScanChunks a) {
         for (int b = 0; b < 4; ++b)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float behind = CHAN ? v[b][e] : v[b][e] * suf[b][e];
+                const float behind = CHAN ? u[b][e] : u[b][e] * suf[b][e];
 #pragma unroll
                 for (int i = 0; i < NT; ++i) sum[b][i] = mfma_f32(behind, k[b][e][i], sum[b][i]);
                 __builtin_amdgcn_sched_barrier(0);
@@ -453,10 +702,16 @@ static void scan_launch(const ScanChunks& a, int n, hipStream_t stream) {
         static const bool configured = hipFuncSetAttribute((const void*)scan_pairs_channel_kernel<D>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) == hipSuccess;
         (void)configured;
         scan_pairs_channel_kernel<D><<<pairs, 256, LDS, stream>>>(a);
-        scan_chunks_kernel<D, true><<<walk, 256, 0, stream>>>(a);
+        scan_chunks_kernel<D, true, false><<<walk, 256, 0, stream>>>(a);
+    } else if (a.corrects) {
+        constexpr int LDS = (SC_CHUNK * (D + 4) + 2 * SC_CHUNK * (SC_CHUNK + 4) + 4 * 16 * 20 + 3 * SC_CHUNK) * 4;
+        static const bool configured = hipFuncSetAttribute((const void*)scan_pairs_delta_kernel<D>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) == hipSuccess;
+        (void)configured;
+        scan_pairs_delta_kernel<D><<<pairs, 256, LDS, stream>>>(a);
+        scan_chunks_kernel<D, false, true><<<walk, 256, 0, stream>>>(a);
     } else {
         scan_pairs_kernel<D><<<pairs, 256, 0, stream>>>(a);
-        scan_chunks_kernel<D, false><<<walk, 256, 0, stream>>>(a);
+        scan_chunks_kernel<D, false, false><<<walk, 256, 0, stream>>>(a);
     }
 }
 void scan_chunks_launch(const ScanChunks& a, int D, int n, hipStream_t stream) {

@@ -85,7 +85,7 @@ _SIGNATURES = {
     "fl_softcap_inplace": [P, L, F, P],
     "fl_linear_scan_gated": [P, I, P, I, P, I, P, I, F, P, L, P, P, P, P, I, I, I, I, I, P],
     "fl_linear_scan_written": [P, I, P, I, P, I, P, P, I, P, P, L, P, P, P, P, I, I, I, I, I, P],
-    "fl_linear_scan_chunked": [P, I, P, I, P, I, P, P, P, I, P, I, F, P, P, L, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
+    "fl_linear_scan_chunked": [P, I, P, I, P, I, P, P, P, I, I, P, I, F, P, P, L, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
     "fl_lowrank_gate": [P, I, I, P, P, I, P, F, P, I, I, I, P],
     "fl_conv_steps": [P, I, I, P, P, P, L, P, P, P, P, P, P, I, I, I, I, I, P, P, P, P],
     "fl_gated_group_norm": [P, P, I, I, P, P, I, I, I, I, I, F, P],

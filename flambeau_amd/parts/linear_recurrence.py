@@ -150,7 +150,8 @@ class GatedDelta(Mixer):
         return ("gated_delta",)
 
     def step_signature(self, batch):
-        return ()
+        """Which requests go in chunks: all that this mixer decides from their lengths."""
+        return self.kernels.signature(batch)
 
     def tensors(self):
         W, H, G, D, Dv, K = self.hidden_size, self.n_heads, self.n_qk_heads, self.head_dim, self.value_dim, self.conv_taps
@@ -177,6 +178,7 @@ class GatedDelta(Mixer):
     def bind(self, weights, rt):
         self.rt = rt
         H, G, D, Dv = self.n_heads, self.n_qk_heads, self.head_dim, self.value_dim
+        self.kernels = rt.kernels("linear_scan")
         a_name, g_name = ("a1" if self.decay_rank is not None else "a"), ("g1" if self.gate_rank is not None else "g")
         self.w_in = rt.prepare_weight(torch.cat([weights[k + ".weight"] for k in ("q", "k", "v", "b", a_name, g_name)], dim=0).contiguous())
         self.col_b = self.channels
@@ -210,8 +212,12 @@ class GatedDelta(Mixer):
                 a, col = ops.lowrank_expand(proj, self.col_a, *self.w_a2, rt.buffer("gd_decay_in", n, H * D, torch.float32)), 0
             key_decay = ops.channel_decay(a, col, self.a_log, self.dt_bias, rt.buffer("gd_decay", n, H * D, torch.float32), H, D)
         hidden = rt.buffer("gd_hidden", n, H * Dv, torch.float32)
-        ops.linear_scan(prep[:, :G * D], prep[:, G * D:2 * G * D], prep[:, 2 * G * D:], cache.state, step.seq_q_start,
-                        step.seq_q_len, step.seq_slots, hidden, H, G, D, Dv, token_gates=gates, key_decay=key_decay)
+        q, k, v = prep[:, :G * D], prep[:, G * D:2 * G * D], prep[:, 2 * G * D:]
+        if key_decay is None:
+            self.kernels.delta(q, k, v, gates, cache.state, step, hidden, H, G, D, Dv)
+        else:
+            ops.linear_scan(q, k, v, cache.state, step.seq_q_start, step.seq_q_len, step.seq_slots, hidden, H, G, D, Dv,
+                            token_gates=gates, key_decay=key_decay)
         gate_rows, gate_col = proj, self.col_g
         if self.w_g2 is not None:
             gate_rows, gate_col = ops.lowrank_expand(proj, self.col_g, *self.w_g2, rt.buffer("gd_gate_in", n, H * Dv, torch.float32)), 0

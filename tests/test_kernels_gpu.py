@@ -1315,6 +1315,8 @@ def _scan_case(mode, H, G, D, Dv, lens, pad=0):
     rows.copy_(rnd(n, rows.shape[1], seed=60))
     c.q, c.k, c.v = rows[:, :G * D], rows[:, G * D:2 * G * D], rows[:, 2 * G * D:2 * G * D + H * Dv]
     c.k *= D ** -0.5
+    if mode == "delta":                                                                        # (unit keys, as this rule has them)
+        c.k.copy_(torch.nn.functional.normalize(c.k.reshape(n, G, D), dim=2).reshape(n, G * D))
     c.head_decay = 1 - 2.0 ** -(3 + torch.arange(H, dtype=torch.float32, device=DEV))
     c.gates = torch.cat([torch.exp(-rnd(n, H, seed=61).abs() * 0.2), torch.sigmoid(rnd(n, H, seed=62))], dim=1).contiguous()
     c.gates[n // 2, 0] = 0.0                                                                   # (a decay may be nothing at all)
@@ -1326,6 +1328,8 @@ def _scan_case(mode, H, G, D, Dv, lens, pad=0):
         where = (state, step, out, H, G, D, Dv)
         if mode == "fixed":
             kernels.fixed(c.q, c.k, c.v, c.head_decay, *where)
+        elif mode == "delta":
+            kernels.delta(c.q, c.k, c.v, c.gates, *where)
         elif mode == "gated":
             kernels.gated(c.q, c.k, c.v, c.key_decay, *where, 0.5)
         else:
@@ -1343,9 +1347,11 @@ def _scan_in_64_bits(c):
         S = states[int(c.step.seq_slots[s])]
         for t in range(at, at + length):
             decay = {"fixed": c.head_decay.double()[:, None, None], "gated": c.key_decay[t].double().reshape(H, 1, D),
-                     "written": c.gates[t, :H].double()[:, None, None]}[c.mode]
-            u = v[t] * c.gates[t, H:].double()[:, None] if c.mode == "written" else v[t]
-            S.mul_(decay).add_(u[:, :, None] * k[t][:, None, :])
+                     "written": c.gates[t, :H].double()[:, None, None], "delta": c.gates[t, :H].double()[:, None, None]}[c.mode]
+            S.mul_(decay)
+            u = v[t] - (S * k[t][:, None, :]).sum(-1) if c.mode == "delta" else v[t]
+            u = u * c.gates[t, H:].double()[:, None] if c.mode in ("written", "delta") else u
+            S.add_(u[:, :, None] * k[t][:, None, :])
             o = (S * q[t][:, None, :]).sum(-1) * (0.5 if c.mode == "gated" else 1.0)
             out.append(o + c.skip.double()[:, None] * v[t] if c.mode == "written" else o)
         at += length
@@ -1359,9 +1365,9 @@ def _scan_sets(max_tokens=4096):
     return ls.PlainLinearScan(rt), ls.TunedLinearScan(rt)
 
 
-@pytest.mark.parametrize("mode", ["fixed", "gated", "written"])
-@pytest.mark.parametrize("H,G,D,Dv,lens", [(2, 2, 64, 16, [192]), (3, 3, 128, 48, [193, 255, 256, 257]), (4, 2, 128, 64, [1, 320, 127, 191, 193, 7, 700]),
-                                           (2, 1, 256, 32, [207, 3, 192])])
+@pytest.mark.parametrize("mode", ["fixed", "gated", "written", "delta"])
+@pytest.mark.parametrize("H,G,D,Dv,lens", [(2, 2, 64, 16, [256]), (3, 3, 128, 48, [193, 255, 256, 257, 271]), (4, 2, 128, 64, [1, 320, 127, 191, 193, 7, 700]),
+                                           (2, 1, 256, 32, [207, 3, 272])])
 def test_scan_in_chunks_against_64_bits(mode, H, G, D, Dv, lens):
     """Requests that end anywhere in a chunk and in 16 tokens, beside requests that walk: outputs and states are no further from 64
     bits than the walk's, or than fewer than 40 roundings (a result is a sum of sums, in chains of at most 16 products and trees of
@@ -1377,15 +1383,15 @@ def test_scan_in_chunks_against_64_bits(mode, H, G, D, Dv, lens):
         assert err(b) < max(err(a), 1.5e-7), (err(a), err(b))
     at = 0
     for length in lens:                                          # (a request that walks: the walk's bits)
-        if length < (192 if mode == "gated" else 128):
+        if length < {"gated": 192, "delta": 256}.get(mode, 128):
             assert torch.equal(walk[0][at:at + length], got[0][at:at + length])
         at += length
 
 
-@pytest.mark.parametrize("mode", ["fixed", "gated", "written"])
+@pytest.mark.parametrize("mode", ["fixed", "gated", "written", "delta"])
 def test_scan_in_chunks_keeps_values_that_are_no_numbers_behind_their_token(mode):
     """A NaN or an infinity in v reaches its own column from its token on, one in k or q nothing before its token."""
-    c = _scan_case(mode, 2, 2, 128, 32, [200])
+    c = _scan_case(mode, 2, 2, 128, 32, [260])
     _, chunked = _scan_sets()
     before, _ = c.run(chunked)
     for t in (0, 5, 15, 16, 70, 127, 199):
@@ -1403,13 +1409,15 @@ def test_scan_in_chunks_keeps_values_that_are_no_numbers_behind_their_token(mode
                 rows[t, 7] = bad
                 out, _ = c.run(chunked)
                 rows[t, 7] = kept
-                assert torch.equal(out[:t], before[:t])
+                # (under the delta rule the whole chunk of such a key is substituted row by row: other sums, as above)
+                bound = 2.5e-6 * before.abs().max() if mode == "delta" and rows is c.k else 0.0
+                assert bool(((out[:t] - before[:t]).abs() <= bound).all())
 
 
 def test_scan_rows_that_the_chunks_do_not_take_walk():
     """Rows that are no whole 16-byte pieces, and head sizes that the chunked kernels do not know: the walk's bits."""
     plain, chunked = _scan_sets()
-    for c in (_scan_case("fixed", 2, 2, 128, 32, [200], pad=3), _scan_case("written", 2, 2, 96, 32, [200]), _scan_case("gated", 2, 2, 128, 24, [200])):
+    for c in (_scan_case("fixed", 2, 2, 128, 32, [200], pad=3), _scan_case("written", 2, 2, 96, 32, [200]), _scan_case("delta", 2, 2, 128, 32, [260], pad=1), _scan_case("gated", 2, 2, 128, 24, [200])):
         assert all(torch.equal(a, b) for a, b in zip(c.run(plain), c.run(chunked)))
 
 
