@@ -407,7 +407,7 @@ extern "C" int fl_linear_scan_chunked(const float* q, int ldq, const float* k, i
     FL_CHECK(pieces(q, ldq) && pieces(k, ldk) && (!chan_decay || pieces(chan_decay, ldc)) && (uintptr_t)state % 16 == 0 && slot_stride % 4 == 0 &&
              (uintptr_t)records % 16 == 0, "linear_scan_chunked: rows and states must be whole 16-byte pieces");
     FL_CHECK(slot_stride >= (long)H * D * Dv, "linear_scan_chunked: a slot of %ld floats does not hold %d heads", slot_stride, H);
-    FL_CHECK((long)SC_CHUNK * max(max(ldq, ldk), ldv) < (1l << 28), "linear_scan_chunked: rows of %d, %d and %d floats", ldq, ldk, ldv);
+    FL_CHECK((long)SC_CHUNK * max(max(ldq, ldk), max(ldv, ldc)) < (1l << 28), "linear_scan_chunked: rows %d, %d, %d and %d floats apart", ldq, ldk, ldv, ldc);
     if (n == 0 || n_seqs == 0) return 0;
     FL_CHECK(n_seqs <= 65535 && H <= 65535, "linear_scan_chunked: %d requests of %d heads are more than one grid takes", n_seqs, H);
     const ScanChunks a = {q, k, v, ldq, ldk, ldv, head_decay, tok_decay, write, ldg, state, (size_t)slot_stride, seq_q_start, seq_q_len,
