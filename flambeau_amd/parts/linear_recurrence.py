@@ -1,7 +1,8 @@
 """Mixers that keep a matrix per head instead of keys and values: retention and the gated delta rule.
 
-Both walk S [dim, vdim] per head through the tokens, S <- g S + k u^T, o = S^T q, in 32-bit, with the
-state in the request's slot (``StateSpec``), so that a prompt may be cut anywhere.
+Both take S [dim, vdim] per head through the tokens, S <- g S + k u^T, o = S^T q, in 32-bit, with the
+state in the request's slot (``StateSpec``), so that a prompt may be cut anywhere: token by token, or in
+bfloat16 runtimes 64 tokens at a time for requests of many (the kernel set ``linear_scan``).
 
 Retention: g is a constant per head, u = v; q and k are rotated by position, k is multiplied by
 dim^(-1/2) afterwards; there is no softmax and no denominator.  Every head's o is divided by its root
