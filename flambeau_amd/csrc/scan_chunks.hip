@@ -679,7 +679,10 @@ __global__ __launch_bounds__(256, 1) void scan_chunks_kernel(ScanChunks a) {
             const int t = 16 * w + 4 * g + r;
             if (t < cnt) a.out[((size_t)(t0 + t) * a.H + head) * a.Dv + j0 + n] = y;
 #pragma unroll
-            for (int i = 0; i < NT; ++i) S[i][r] = fmaf(S[i][r], last[i], fmaf(S[i][r], rest[i], (sum[0][i][r] + sum[1][i][r]) + (sum[2][i][r] + sum[3][i][r])));
+            for (int i = 0; i < NT; ++i) {
+                const float bounded = __builtin_isinf(S[i][r]) ? 0.f : S[i][r];            // (an infinity stays one, as in the walk: `rest` is zero or of either sign)
+                S[i][r] = fmaf(S[i][r], last[i], fmaf(bounded, rest[i], (sum[0][i][r] + sum[1][i][r]) + (sum[2][i][r] + sum[3][i][r])));
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
         load_decays(next);

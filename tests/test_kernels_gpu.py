@@ -1414,6 +1414,23 @@ def test_scan_in_chunks_keeps_values_that_are_no_numbers_behind_their_token(mode
                 assert bool(((out[:t] - before[:t]).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("mode", ["fixed", "gated", "written"])
+def test_scan_in_chunks_keeps_an_infinite_state(mode):
+    """A state that holds an infinity keeps it through whole chunks, as through the walk's tokens: the same outputs and states
+    are infinite, none becomes a NaN, and the other columns are those of a finite state."""
+    c = _scan_case(mode, 2, 2, 128, 32, [260])
+    plain, chunked = _scan_sets()
+    before = c.run(chunked)
+    for bad in (float("inf"), float("-inf")):
+        c.state0.reshape(2, 32, 128)[1, 3, 7] = bad                  # head 1 (head 0 forgets all at one token), column 3
+        for w, a, b in zip(c.run(plain), c.run(chunked), before):
+            w, a, b = (t.reshape(-1, 2, 32, t.numel() // (t.shape[0] * 64)) for t in (w, a, b))
+            assert torch.isinf(w[:, 1, 3]).any() and not torch.isnan(w).any()
+            assert torch.equal(torch.isinf(w), torch.isinf(a)) and torch.equal(w[torch.isinf(w)], a[torch.isinf(a)]) and not torch.isnan(a).any()
+            others = [j for j in range(32) if j != 3]
+            assert torch.equal(a[:, :, others], b[:, :, others])
+
+
 def test_scan_rows_that_the_chunks_do_not_take_walk():
     """Rows that are no whole 16-byte pieces, and head sizes that the chunked kernels do not know: the walk's bits."""
     plain, chunked = _scan_sets()
