@@ -171,7 +171,7 @@ __global__ __launch_bounds__(128 * WT, OCC) void gemm_async_kernel(const bf16_t*
     // are issued here, ahead of all other loads, and wait in registers (where there is room: with 4 x 4
     // tiles per wave, not with 8 x 4).
     constexpr bool PREFETCH = EPI == TG_RESIDUAL && OCC == 1 && FT * TT <= 16;
-    constexpr int BATCH = FT * TT > 32 ? (FT + 1) / 2 : FT;           // tiles of a token that an epilogue looks values up for at a time: what registers leave room for
+    constexpr int BATCH = FT * TT > 32 ? (FT + 1) / 2 : FT;           // tiles of a token that an epilogue looks values up for at a time: what registers leave room for beside 40 tiles of sums
     const int j = lane & 15, g = lane >> 4;
     f32x4 pre[PREFETCH ? FT : 1][PREFETCH ? TT : 1];
     if (PREFETCH) {
@@ -358,29 +358,35 @@ __global__ __launch_bounds__(128 * WT, OCC) void gemm_async_kernel(const bf16_t*
     }
     if (EPI == TG_ROPE) {
         // the joined q/k/v projection: rotate, store q and the cache rows (rope_store.h).  What the
-        // epilogue looks up (places, angles) is loaded in batches, each with one wait.
-        int toks[TT];
-        TokenPlace places[TT];
+        // epilogue looks up (places, angles) is loaded in batches, each with one wait: the places of all tokens of a
+        // lane together, in the larger blocks of each token by itself (all together the compiler kept what it forms from them
+        // for every token at once and spilled 134, 55 and 166 registers a lane with 8 x 5, 7 x 5 and 7 x 6 tiles per wave: 6144 x 4096 at 2,600 rows 131 us, 127 now, at 3,449 rows 163 -> 152, 7168 x 5120 at 3,072 199 -> 185).
+        constexpr int AT_ONCE = BATCH < FT ? 1 : TT;
 #pragma unroll
-        for (int tb = 0; tb < TT; ++tb) toks[tb] = m0 + (wt * TT + tb) * 16 + j;
-        rope_token_places<TT>(rs, toks, M, places);
+        for (int b0 = 0; b0 < TT; b0 += AT_ONCE) {
+            int toks[AT_ONCE];
+            TokenPlace places[AT_ONCE];
 #pragma unroll
-        for (int tb = 0; tb < TT; ++tb) {
-            const int tok = toks[tb];
+            for (int i = 0; i < AT_ONCE; ++i) toks[i] = m0 + (wt * TT + b0 + i) * 16 + j;
+            rope_token_places<AT_ONCE>(rs, toks, M, places);
 #pragma unroll
-            for (int t0 = 0; t0 < FT; t0 += BATCH) {
-                RopeAngles an[BATCH];
-                if (rs.rot) {                                         // (no table without rotated dims)
+            for (int i = 0; i < AT_ONCE; ++i) {
+                const int tok = toks[i];
 #pragma unroll
-                    for (int u = 0; u < BATCH; ++u)
-                        an[u] = rope_angles(rs, min(tok, M - 1), n0 + (wf * FT + min(t0 + u, FT - 1)) * 16 + 4 * g, g);
+                for (int t0 = 0; t0 < FT; t0 += BATCH) {
+                    RopeAngles an[BATCH];
+                    if (rs.rot) {                                     // (no table without rotated dims)
+#pragma unroll
+                        for (int u = 0; u < BATCH; ++u)
+                            an[u] = rope_angles(rs, min(tok, M - 1), n0 + (wf * FT + min(t0 + u, FT - 1)) * 16 + 4 * g, g);
+                    }
+#pragma unroll
+                    for (int u = 0; u < BATCH && t0 + u < FT; ++u) {
+                        const int ta = t0 + u, f0 = n0 + (wf * FT + ta) * 16 + 4 * g;
+                        rope_store4<true>(rs, tok, places[i], f0, g, acc[ta][b0 + i], tok < M && f0 < N, an[u]);
+                    }
+                    if constexpr (BATCH < FT) __builtin_amdgcn_sched_barrier(0);
                 }
-#pragma unroll
-                for (int u = 0; u < BATCH && t0 + u < FT; ++u) {
-                    const int ta = t0 + u, f0 = n0 + (wf * FT + ta) * 16 + 4 * g;
-                    rope_store4<true>(rs, tok, places[tb], f0, g, acc[ta][tb], tok < M && f0 < N, an[u]);
-                }
-                if constexpr (BATCH < FT) __builtin_amdgcn_sched_barrier(0);
             }
         }
         return;

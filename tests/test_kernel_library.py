@@ -2,8 +2,12 @@
 lists the Python side holds, and what the recorder of step programs knows."""
 import ctypes
 import re
+import struct
 from pathlib import Path
 
+import msgpack
+
+from flambeau_amd.csrc import build
 from flambeau_amd.kernels import library
 from flambeau_amd.kernels import tuned  # noqa: F401  (registers the tuned kernels' argument lists)
 from flambeau_amd.sampling import device  # noqa: F401
@@ -152,3 +156,36 @@ def test_which_products_of_9_to_16_rows_leave_the_skinny_kernel():
     assert [tuned.mid_preferred(m, 4096, 14336) for m in (9, 12, 13, 16)] == [False, False, True, True]
     assert not tuned.mid_preferred(16, 65536, 5120) and not tuned.mid_preferred(16, 4096, 4096)
     assert not tuned.mid_preferred(16, 5120, 32768 + 8)          # K must be whole steps of 32 for that kernel
+
+
+def _kernel_resources():
+    """``{mangled kernel name: its metadata}`` of every kernel in the built library: the notes of the device code objects
+    that the compiler bundled into it."""
+    data, found, at = build.library_path().read_bytes(), {}, 0
+    while (at := data.find(b"__CLANG_OFFLOAD_BUNDLE__", at)) >= 0:
+        p = at + 32
+        for _ in range(struct.unpack_from("<Q", data, at + 24)[0]):
+            offset, size, length = struct.unpack_from("<QQQ", data, p)
+            target, p = data[p + 24:p + 24 + length], p + 24 + length
+            if b"gfx950" not in target:
+                continue
+            elf = data[at + offset:at + offset + size]
+            sections, (entry, count) = struct.unpack_from("<Q", elf, 40)[0], struct.unpack_from("<HH", elf, 58)
+            for i in range(count):
+                kind, where = struct.unpack_from("<I", elf, sections + i * entry + 4)[0], struct.unpack_from("<Q", elf, sections + i * entry + 24)[0]
+                if kind == 7:                                            # a section of notes
+                    name, text, what = struct.unpack_from("<III", elf, where)
+                    if what == 32:                                       # the kernels' metadata
+                        notes = msgpack.unpackb(elf[where + 12 + (name + 3 & ~3):][:text])
+                        found.update({k[".name"]: k for k in notes["amdhsa.kernels"]})
+        at += 24
+    return found
+
+
+def test_the_rotating_product_keeps_its_values_in_registers():
+    """No block shape of the tiled product with rotation and stores in its kernel (the third kind of epilogue) spills registers,
+    the blocks of 320 and 384 tokens among them."""
+    kernels = {k: v for k, v in _kernel_resources().items() if re.match(r"_Z17gemm_async_kernelI(Li\d+E){5}DF16bLi2E", k)}
+    assert len(kernels) == 24, sorted(kernels)                            # (twelve shapes, K a multiple of 32 or not)
+    assert all(v[".vgpr_spill_count"] == 0 and v[".private_segment_fixed_size"] == 0 for v in kernels.values()), \
+        {k: v[".vgpr_spill_count"] for k, v in kernels.items()}
