@@ -388,15 +388,15 @@ int fl_linear_scan_written(const float* q, int ldq, const float* k, int ldk, con
                            long slot_stride, const int* seq_q_start, const int* seq_q_len, const int* seq_slots,
                            float* out, int n_seqs, int H, int G, int D, int Dv, hipStream_t stream);
 // The forms with a decay per head, with gates per token (corrects: the delta rule), or per key dim a chunk of 64 tokens at a time on the matrix cores (sizes: _takes): requests of at least min_len
-// tokens, and with walk_short the walk for the others (0: all requests go in chunks).  records: fl_linear_scan_records(n, n_seqs) x
-// fl_linear_scan_record_floats(H, D, kind) floats (kind 1: chan_decay, 2: corrects, else 0), n = the step's tokens.
+// tokens, and with walk_short the walk for the others (0: all requests go in chunks).  records: n_chunks x fl_linear_scan_record_floats(H, D, kind)
+// floats (kind 1: chan_decay, 2: corrects, else 0), n_chunks = the chunks of _chunk_tokens() tokens, begun ones too, of the requests that go in chunks.
 int fl_linear_scan_chunked_takes(int D, int Dv);
 int fl_linear_scan_record_floats(int H, int D, int kind);
-int fl_linear_scan_records(int n, int n_seqs);
+int fl_linear_scan_chunk_tokens(void);
 int fl_linear_scan_chunked(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* head_decay,
                            const float* tok_decay, const float* write, int ldg, int corrects, const float* chan_decay, int ldc,
                            float o_scale, const float* skip, float* state, long slot_stride, const int* seq_q_start, const int* seq_q_len,
-                           const int* seq_slots, float* out, float* records, int n, int n_seqs, int min_len, int walk_short, int H,
+                           const int* seq_slots, float* out, float* records, int n_chunks, int n_seqs, int min_len, int walk_short, int H,
                            int G, int D, int Dv, hipStream_t stream);
 int fl_rotate_scale(const float* proj, int ld, int col_a, int col_b, const float* cs, int rot, int interleaved,
                     float scale_a, float scale_b, float* out_a, float* out_b, int n, int H, int D,

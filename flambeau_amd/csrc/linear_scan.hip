@@ -388,17 +388,17 @@ FL_RECORDABLE(fl_linear_scan_written)
 // (walk_short), or for all requests (walk_short = 0).
 // a decay per head (head_decay), per token and head (tok_decay, with write strengths, rows ldg wide; corrects: the delta rule) or per token, head
 // and key dim (chan_decay, rows ldc wide); o = o_scale S^T q (with chan_decay; 1 otherwise) + skip v (skip: per head or null; with
-// write strengths).  records:
-// fl_linear_scan_records(n, n_seqs) x fl_linear_scan_record_floats(H, D, kind) floats (kind 1: chan_decay, 2: corrects), n = the step's tokens.
+// write strengths).  records: n_chunks x fl_linear_scan_record_floats(H, D, kind) floats (kind 1: chan_decay, 2: corrects), n_chunks = the chunks of
+// the requests that go in chunks, counted by the caller, who knows their lengths.
 extern "C" int fl_linear_scan_chunked_takes(int D, int Dv) { return scan_chunks_takes(D, Dv); }
 extern "C" int fl_linear_scan_record_floats(int H, int D, int kind) { return H * (kind == 1 ? SC_CHANNEL_RECORD(D) : kind == 2 ? SC_DELTA_RECORD(D) : SC_RECORD); }
-extern "C" int fl_linear_scan_records(int n, int n_seqs) { return scan_chunks_records(n, n_seqs); }
+extern "C" int fl_linear_scan_chunk_tokens(void) { return SC_CHUNK; }
 extern "C" int fl_linear_scan_chunked(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* head_decay,
                                       const float* tok_decay, const float* write, int ldg, int corrects, const float* chan_decay, int ldc,
                                       float o_scale, const float* skip, float* state, long slot_stride, const int* seq_q_start, const int* seq_q_len,
-                                      const int* seq_slots, float* out, float* records, int n, int n_seqs, int min_len, int walk_short, int H, int G,
+                                      const int* seq_slots, float* out, float* records, int n_chunks, int n_seqs, int min_len, int walk_short, int H, int G,
                                       int D, int Dv, hipStream_t stream) {
-    FL_CHECK(n >= 0 && n_seqs >= 0 && H > 0 && G > 0 && H % G == 0 && min_len >= 1, "linear_scan_chunked: bad sizes");
+    FL_CHECK(n_chunks >= 0 && n_seqs >= 0 && H > 0 && G > 0 && H % G == 0 && min_len >= 1, "linear_scan_chunked: bad sizes");
     FL_CHECK(scan_chunks_takes(D, Dv), "linear_scan_chunked: heads of %d x %d", D, Dv);
     FL_CHECK(!!head_decay + !!tok_decay + !!chan_decay == 1 && (!write == !tok_decay) && (!skip || (write && !corrects)) && (!corrects || write) && (chan_decay || o_scale == 1.f),
              "linear_scan_chunked: one decay per head, or one per token and head with write strengths, or one per token, head and key dim");
@@ -408,12 +408,14 @@ extern "C" int fl_linear_scan_chunked(const float* q, int ldq, const float* k, i
              (uintptr_t)records % 16 == 0, "linear_scan_chunked: rows and states must be whole 16-byte pieces");
     FL_CHECK(slot_stride >= (long)H * D * Dv, "linear_scan_chunked: a slot of %ld floats does not hold %d heads", slot_stride, H);
     FL_CHECK((long)SC_CHUNK * max(max(ldq, ldk), max(ldv, ldc)) < (1l << 28), "linear_scan_chunked: rows %d, %d, %d and %d floats apart", ldq, ldk, ldv, ldc);
-    if (n == 0 || n_seqs == 0) return 0;
+    if (n_seqs == 0) return 0;
     FL_CHECK(n_seqs <= 65535 && H <= 65535, "linear_scan_chunked: %d requests of %d heads are more than one grid takes", n_seqs, H);
     const ScanChunks a = {q, k, v, ldq, ldk, ldv, head_decay, tok_decay, write, ldg, state, (size_t)slot_stride, seq_q_start, seq_q_len,
                           seq_slots, out, records, n_seqs, walk_short ? min_len : 1, H, G, Dv, o_scale, skip, chan_decay, ldc, corrects};
-    scan_chunks_launch(a, D, n, stream);
-    FL_LAUNCH_CHECK();
+    if (n_chunks > 0) {
+        scan_chunks_launch(a, D, n_chunks, stream);
+        FL_LAUNCH_CHECK();
+    }
     if (!walk_short) return 0;
     return linear_scan_launch(q, ldq, k, ldk, v, ldv, head_decay, tok_decay, write, ldg, state, slot_stride, seq_q_start, seq_q_len,
                               seq_slots, out, n_seqs, H, G, D, Dv, false, stream, chan_decay, ldc, corrects != 0, o_scale, skip, min_len);

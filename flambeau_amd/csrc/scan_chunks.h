@@ -43,7 +43,7 @@ struct ScanChunks {
     int corrects;                // the delta rule: u = write (v - S^T k)
 };
 
-// Sizes that it takes, and the records (SC_RECORD floats per head each) that n tokens in n_seqs requests may need.
+// Sizes that it takes.
 inline bool scan_chunks_takes(int D, int Dv) { return (D == 64 || D == 128 || D == 256) && Dv % SC_COLS == 0; }
-inline int scan_chunks_records(int n, int n_seqs) { return n / SC_CHUNK + n_seqs; }
-void scan_chunks_launch(const ScanChunks& a, int D, int n, hipStream_t stream);
+// n_chunks: the chunks of all requests of at least min_len tokens, a record each.
+void scan_chunks_launch(const ScanChunks& a, int D, int n_chunks, hipStream_t stream);

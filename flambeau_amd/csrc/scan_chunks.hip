@@ -698,8 +698,8 @@ __global__ __launch_bounds__(256, 1) void scan_chunks_kernel(ScanChunks a) {
 }
 
 template <int D>
-static void scan_launch(const ScanChunks& a, int n, hipStream_t stream) {
-    const dim3 pairs(scan_chunks_records(n, a.n_seqs), a.H), walk(a.H, a.Dv / SC_COLS, a.n_seqs);
+static void scan_launch(const ScanChunks& a, int n_chunks, hipStream_t stream) {
+    const dim3 pairs(n_chunks, a.H), walk(a.H, a.Dv / SC_COLS, a.n_seqs);
     if (a.chan_decay) {
         constexpr int LDS = (2 * SC_CHUNK * (D + 4) + 12 * D) * 4;
         static const bool configured = hipFuncSetAttribute((const void*)scan_pairs_channel_kernel<D>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) == hipSuccess;
@@ -717,8 +717,8 @@ static void scan_launch(const ScanChunks& a, int n, hipStream_t stream) {
         scan_chunks_kernel<D, false, false><<<walk, 256, 0, stream>>>(a);
     }
 }
-void scan_chunks_launch(const ScanChunks& a, int D, int n, hipStream_t stream) {
-    if (D == 64) scan_launch<64>(a, n, stream);
-    else if (D == 128) scan_launch<128>(a, n, stream);
-    else scan_launch<256>(a, n, stream);
+void scan_chunks_launch(const ScanChunks& a, int D, int n_chunks, hipStream_t stream) {
+    if (D == 64) scan_launch<64>(a, n_chunks, stream);
+    else if (D == 128) scan_launch<128>(a, n_chunks, stream);
+    else scan_launch<256>(a, n_chunks, stream);
 }

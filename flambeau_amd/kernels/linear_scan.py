@@ -54,6 +54,16 @@ def lengths(batch, enough: int):
     return max(batch.q_lens) >= enough, min(batch.q_lens) < enough
 
 
+def chunks(q_lens, enough: int, size: int) -> int:
+    """How many chunks of ``size`` tokens the requests of at least ``enough`` go in: a record each."""
+    return sum(-(-q // size) for q in q_lens if q >= enough)
+
+
+def most_chunks(tokens: int, enough: int, size: int) -> int:
+    """The most that ``chunks`` can be for a step of ``tokens``: a chunk per ``size`` of them, and one that is not full per request."""
+    return tokens // size + tokens // enough
+
+
 class TunedLinearScan(PlainLinearScan):
     def signature(self, batch):
         return sum((lengths(batch, enough) for enough in (CHUNKED_TOKENS, CHUNKED_TOKENS_PER_DIM, CHUNKED_TOKENS_DELTA)), ())
@@ -72,10 +82,10 @@ class TunedLinearScan(PlainLinearScan):
         n, S = out.shape[0], step.seq_q_start.shape[0]
         f = lambda t, name, shape: ops._check(t, "linear_scan." + name, torch.float32, shape)
         i = lambda t, name: ops._check(t, "linear_scan." + name, torch.int32, (S,))
-        count = lib.fl_linear_scan_records(n, S)
-        most = lib.fl_linear_scan_records(self.rt.max_batch_tokens, max(self.rt.max_batch_tokens, 1))
+        size = lib.fl_linear_scan_chunk_tokens()
+        count = chunks(step.host.q_lens, enough, size)
         records = self.rt.buffer("scan_records", count, lib.fl_linear_scan_record_floats(int(H), int(D), 1 if key_decay is not None else 2 if corrects else 0),
-                                 torch.float32, max_rows=most)
+                                 torch.float32, max_rows=most_chunks(self.rt.max_batch_tokens, enough, size))
         pg = f(gates, "gates", (n, 2 * H)) if gates is not None else None
         call("fl_linear_scan_chunked", *ops._rows(q, "linear_scan.q", n, G * D), *ops._rows(k, "linear_scan.k", n, G * D),
              *ops._rows(v, "linear_scan.v", n, H * Dv), f(head_decay, "decay", (H,)) if head_decay is not None else None,
@@ -83,7 +93,7 @@ class TunedLinearScan(PlainLinearScan):
              *(ops._rows(key_decay, "linear_scan.key_decay", n, H * D) if key_decay is not None else (None, 0)), float(out_scale),
              f(skip, "skip", (H,)) if skip is not None else None, f(state, "state", (None, None)), state.shape[1],
              i(step.seq_q_start, "seq_q_start"), i(step.seq_q_len, "seq_q_len"), i(step.seq_slots, "seq_slots"), f(out, "out", (n, H * Dv)),
-             records.data_ptr(), n, S, enough, int(short), int(H), int(G), int(D), int(Dv), ops.stream_handle())
+             records.data_ptr(), count, S, enough, int(short), int(H), int(G), int(D), int(Dv), ops.stream_handle())
         return True
 
     def fixed(self, q, k, v, head_decay, state, step, out, n_heads, n_qk_heads, dim, vdim):

@@ -1,6 +1,8 @@
 """The lists that give every single row of a batch splits of its own for the decode attention
 (host side only): every row present with consecutive splits, the budget kept, no split shorter than
 the least, the list's length a function of the batch's shape alone."""
+import random
+
 import numpy as np
 
 from flambeau_amd.kernels import tuned
@@ -51,3 +53,22 @@ def test_long_contexts_get_the_splits_of_a_ragged_batch():
     assert tuned.balanced_items(rows[:0], 8)[0].shape == (0, 4)
     one, first = tuned.balanced_items(rows[:1], 8)
     assert (one[:, 0] >= 0).sum() == 63 and first[0].tolist() == [0, 0, 63, 0]
+
+
+# ---------------------------------------------------------------- chunks of the linear recurrences
+def test_chunks_are_counted_one_for_one():
+    """The records that a step asks for are the chunks of the requests that go in chunks, no more, and never beyond what the
+    buffer may grow to."""
+    from flambeau_amd.kernels.linear_scan import chunks, most_chunks
+    assert chunks([2048], 128, 64) == 32 and chunks([2049], 128, 64) == 33
+    assert chunks([1] * 64 + [512], 128, 64) == 8                # (requests that walk have none)
+    assert chunks([127, 128, 129], 128, 64) == 2 + 3 and chunks([1, 7], 128, 64) == 0
+    rng = random.Random(3)
+    for _ in range(2000):
+        enough, tokens = rng.choice([64, 128, 192, 256]), rng.randint(1, 4096)
+        left, lens = tokens, []
+        while left:
+            lens.append(min(left, rng.choice([1, rng.randint(1, 300), enough, enough + 1, rng.randint(1, 4096)])))
+            left -= lens[-1]
+        count = sum(1 for q in lens if q >= enough for _ in range(0, q, 64))
+        assert chunks(lens, enough, 64) == count <= most_chunks(tokens, enough, 64)
