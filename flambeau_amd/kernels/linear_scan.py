@@ -17,10 +17,6 @@ class PlainLinearScan:
     def __init__(self, rt):
         self.rt = rt
 
-    def signature(self, batch):
-        """What the kernels decide from the requests' lengths (part of a recorded step's key)."""
-        return ()
-
     def fixed(self, q, k, v, head_decay, state, step, out, n_heads, n_qk_heads, dim, vdim):
         """A decay per head, u = v (``ops.linear_scan``)."""
         return ops.linear_scan(q, k, v, state, step.seq_q_start, step.seq_q_len, step.seq_slots, out, n_heads, n_qk_heads, dim, vdim,
@@ -65,9 +61,6 @@ def most_chunks(tokens: int, enough: int, size: int) -> int:
 
 
 class TunedLinearScan(PlainLinearScan):
-    def signature(self, batch):
-        return sum((lengths(batch, enough) for enough in (CHUNKED_TOKENS, CHUNKED_TOKENS_PER_DIM, CHUNKED_TOKENS_DELTA)), ())
-
     def _chunked(self, q, k, v, state, step, out, H, G, D, Dv, head_decay=None, gates=None, skip=None, key_decay=None, out_scale=1.0,
                  corrects=False):
         """Whether the chunked kernels did it."""

@@ -71,8 +71,7 @@ class Retention(Mixer):
         return ("retention",)
 
     def step_signature(self, batch):
-        """Which requests go in chunks: all that this mixer decides from their lengths."""
-        return self.kernels.signature(batch)
+        return ()              # (which requests go in chunks follows from the rows per request, part of every recorded step's key)
 
     def tensors(self):
         W, H, D, Dv = self.hidden_size, self.n_heads, self.head_dim, self.value_dim
@@ -151,8 +150,7 @@ class GatedDelta(Mixer):
         return ("gated_delta",)
 
     def step_signature(self, batch):
-        """Which requests go in chunks: all that this mixer decides from their lengths."""
-        return self.kernels.signature(batch)
+        return ()              # (which requests go in chunks follows from the rows per request, part of every recorded step's key)
 
     def tensors(self):
         W, H, G, D, Dv, K = self.hidden_size, self.n_heads, self.n_qk_heads, self.head_dim, self.value_dim, self.conv_taps
@@ -308,8 +306,7 @@ class GatedLinearAttention(Mixer):
         return ("gated_linear_attention",)
 
     def step_signature(self, batch):
-        """Which requests go in chunks: all that this mixer decides from their lengths."""
-        return self.kernels.signature(batch)
+        return ()              # (which requests go in chunks follows from the rows per request, part of every recorded step's key)
 
     def tensors(self):
         W, H, D, Dv, R = self.hidden_size, self.n_heads, self.head_dim, self.value_dim, self.decay_rank
@@ -376,8 +373,7 @@ class StateSpace(Mixer):
         return ("state_space",)
 
     def step_signature(self, batch):
-        """Which requests go in chunks: all that this mixer decides from their lengths."""
-        return self.kernels.signature(batch)
+        return ()              # (which requests go in chunks follows from the rows per request, part of every recorded step's key)
 
     def tensors(self):
         W, H, C = self.hidden_size, self.n_heads, self.channels

@@ -72,3 +72,13 @@ def test_chunks_are_counted_one_for_one():
             left -= lens[-1]
         count = sum(1 for q in lens if q >= enough for _ in range(0, q, 64))
         assert chunks(lens, enough, 64) == count <= most_chunks(tokens, enough, 64)
+
+
+def test_recurrent_mixers_add_nothing_to_a_recorded_steps_key():
+    """What goes in chunks follows from the rows per request, which every recorded step's key holds: a step asks these
+    mixers for nothing else, whatever the lengths."""
+    from flambeau_amd.parts.base import HostBatch
+    from flambeau_amd.parts.linear_recurrence import GatedDelta, GatedLinearAttention, Retention, StateSpace
+    for cls in (GatedDelta, GatedLinearAttention, Retention, StateSpace):
+        for lens in ([1, 1], [300], [1, 300]):
+            assert object.__new__(cls).step_signature(HostBatch([0], lens, [5] * len(lens), [0], sum(lens), 1)) == ()
