@@ -539,7 +539,9 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 // here, together with the number of K-splits.  The entry points whose names end in _ex take either from the caller,
 // for tests and measurements.
 //
-// What a shape costs, in us.  Four waves, two blocks per unit: bound by the copies into LDS, per k-step 0.128 a round of
+// What a shape costs, in us.  Blocks go to the dies in turn, a die's share of the tiles times the parts of K: the unit with the most
+// blocks is one of that die (7168 x 5120 at 528 rows in three parts of 256 x 256 are 252 blocks, but 33 for a die's 32
+// units: 105 us, 73 in two parts of 224 x 192).  Four waves, two blocks per unit: bound by the copies into LDS, per k-step 0.128 a round of
 // resident blocks and 0.0198 per KB that a unit's blocks copy, 0.8 of it from the mean and 0.2 from the unit with the most
 // blocks; a tile of w that few tiles of tokens share comes from HBM more often (a quarter more with one of them), and
 // blocks of 128 features copy 12 % faster.  Four waves alone on their unit have the whole LDS for stages on their way:
@@ -549,6 +551,12 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 // with 256, 224, 192 features, 0.59 with 224 x 192 and 0.85, 0.75, 0.94 with 256 x 320, 224 x 320 and 224 x 384, less where a
 // tile's rows are few, more where a unit gets a second block of another part of K, and 7 per block that nothing overlaps.
 // Splitting K adds the parts' way to memory and back and the kernel that sums them: 1 us, and 2.35 per million values and part.
+// Parts that put a block of up to 256 tokens on nearly every unit at once are slower than their steps: launched back to back, the
+// chip lowers its clock under them, some cards more than others (4096 x 14336 at 289 rows in eight parts of 256 x 256, 256 blocks: 65 us
+// with weights of zeros, 85 with random ones, on one card of four 64; in six parts of 224 x 192, 228 blocks, 62 and 67; a prompt of 272
+// rows through four layers of the 7B model 1,139 -> 1,036 us).  A tenth where no unit is left idle, no more, picks best over
+// 20 products at 50 row counts, 11,000 timings in such a row, the mean of three cards: 30 of 1,000 picks more than 3 % faster
+// than without it, eight slower; blocks of 320 tokens do not show it (5120 x 32768 at 560 rows in six parts 204 to 212 us).
 // What decides among eight waves is how evenly the blocks fill the rounds, in features (gate/up of 2,048 rows, 28672 features, is
 // 3.5 rounds of 256 and 4 of 224, q/k/v of 2,048 rows, 6144 features, 0.75 rounds of 256 and 1 of 192) and in tokens: rows that
 // end soon behind a multiple of 256 are tiles of 192 (28672 x 4096 at 333 rows 90 us, 96.6 with 256) or of 320 and 384, which at
@@ -576,18 +584,21 @@ static bool tiled_known(int variant) { return variant == 0 || tile_shape(variant
 static float tiled_cost(const TileShape& t, int splits, int M, int N, int K) {
     const int units = fl_units();
     const int steps = ceil_div(ceil_div(K, 32), splits);
-    const long blocks = (long)ceil_div(N, t.features) * ceil_div(M, t.tokens) * splits;
-    const long most = (blocks + units - 1) / units;                    // blocks of the unit with the most
+    const int m_tiles = ceil_div(M, t.tokens);
+    const long tiles = (long)ceil_div(N, t.features) * m_tiles, blocks = tiles * splits;
+    const int die_units = max(units / 8, 1);
+    const long most = ((tiles + 7) / 8 * splits + die_units - 1) / die_units;              // blocks of the unit with the most
     const long rounds = (most + t.per_unit - 1) / t.per_unit;
     const float mean = blocks > units ? (float)blocks / units : 1.f;
-    const int m_tiles = ceil_div(M, t.tokens);
     const float empty = 1.f - (float)M / ((long)m_tiles * t.tokens);   // share of the tiles' rows that are none
+    // units at work at once beyond 0.88 of them
+    const float full = splits > 1 && most == 1 && t.tokens <= 256 ? fmaxf((float)blocks / units - 0.88f, 0.f) : 0.f;
     float us;
     if (t.variant == 14 && empty > 0.4276f) return 1e9f;               // (tiles with so few rows: 28672 x 5120 at 207 rows 112.8 us, 106.4 with 256 x 128)
     if (t.variant == 13) {
         us = most * steps * (0.3876f - 0.0892f * empty) + 1.73f;
     } else if (t.per_unit == 1) {
-        us = most * (steps * (t.step * (1.f + 0.1021f / m_tiles + (splits > 1 && most > 1 ? 0.0517f : 0.f)) - 0.0795f * empty * t.tokens / 256.f) +
+        us = most * (steps * (t.step * (1.f + 0.1021f / m_tiles + (splits > 1 && most > 1 ? 0.0517f : 0.f) + 0.8f * full) - 0.0795f * empty * t.tokens / 256.f) +
                      7.01f + 0.1918f * (t.tokens - 256) / 64.f);
     } else {
         const float kb = (t.features * (1.f + 0.2501f / m_tiles) + t.tokens) * 64 / 1024.f;     // copied per block and k-step

@@ -743,11 +743,13 @@ def test_gemm_tiled_block_shapes(variant, M, N, K):
         assert (out2.double() - ref2).abs().max() < 1e-2 * ref2.abs().max()
 
 
-@pytest.mark.parametrize("M,N,K,gate,variant,splits", [(1040, 5120, 32768, False, 11, 2), (384, 16384, 2048, True, 8, 1), (528, 28672, 4096, True, 16, 1)])
+@pytest.mark.parametrize("M,N,K,gate,variant,splits", [(1040, 5120, 32768, False, 11, 2), (384, 16384, 2048, True, 8, 1), (528, 28672, 4096, True, 16, 1),
+                                                       (528, 7168, 5120, False, 14, 2), (300, 4096, 14336, False, 14, 6)])
 def test_gemm_tiled_plan_knows_what_is_faster(M, N, K, gate, variant, splits):
     """Block shapes and parts that are a fifth faster than what the plan once picked for these sizes (473 and 50 us against
-    358 and 40; 163 against 121): what it picks now is within a tenth of them.  Weights from memory: enough copies that none stays in a
-    cache."""
+    358 and 40; 163 against 121; 105 against 73, where a die got one block more than it has units; 85 against 67, where a
+    block on every unit lowers the clock): what it picks now is within a tenth of them.  Weights from memory: enough copies
+    that none stays in a cache."""
     copies = max(2, -(-600_000_000 // (2 * N * K)))
     w = [rnd(N * K, dtype=torch.bfloat16, seed=22, scale=0.05) for _ in range(copies)]       # (N, K multiples of a tile: any values are a packed matrix)
     x, out = rnd(M, K, dtype=torch.bfloat16, seed=21), torch.empty(M, N // 2 if gate else N, dtype=torch.bfloat16, device=DEV)
