@@ -10,6 +10,7 @@
 // Two kernels: the gates and their running maximum for all tokens (only the maximum is a chain there), then the
 // memory's walk with the factors exp(f + m - m'), exp(i - m'), exp(-m') ready.
 // The walk is the recurrence itself, so a prompt cut anywhere leaves the same state and the same o.
+#include <type_traits>
 #include "common.h"
 #include "api.h"
 #include "recordable.h"
@@ -191,24 +192,29 @@ __global__ __launch_bounds__(256) void headnorm_gate_kernel(const float* __restr
     const float* xr = x + (size_t)unit * Dv;
     float ss = 0.f;
     if (Dv <= 128) {                               // everything a lane needs is asked for before the sum is formed (2,048 x 32 heads of 128 36.2 -> 22.5 us)
-        float v[2], z[2], g[2];
+        auto head = [&](auto values) {             // (a lane's values: one where a head has no more, 2,048 x 16 heads of 64 10.1 us with two, 9.4 with one)
+            constexpr int J = decltype(values)::value;
+            float v[J], z[J], g[J];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int i = lane + 64 * j, at = i < Dv ? i : 0;
-            v[j] = xr[at];
-            g[j] = w ? w[h * Dv + at] : 1.0f;
-            z[j] = gate ? gate[(size_t)t * ldg + gate_col0 + h * Dv + at] : 0.f;
-        }
+            for (int j = 0; j < J; ++j) {
+                const int i = lane + 64 * j, at = i < Dv ? i : 0;
+                v[j] = xr[at];
+                g[j] = w ? w[h * Dv + at] : 1.0f;
+                z[j] = gate ? gate[(size_t)t * ldg + gate_col0 + h * Dv + at] : 0.f;
+            }
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-            if (lane + 64 * j < Dv) ss += v[j] * v[j];
-        const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)Dv + eps);
+            for (int j = 0; j < J; ++j)
+                if (lane + 64 * j < Dv) ss += v[j] * v[j];
+            const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)Dv + eps);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            float o = v[j] * inv * g[j];
-            if (gate) o *= (gate_kind == 2 ? z[j] : 1.0f) / (1.0f + expf(-z[j]));
-            if (lane + 64 * j < Dv) out[(size_t)unit * Dv + lane + 64 * j] = from_f32<T>(o);
-        }
+            for (int j = 0; j < J; ++j) {
+                float o = v[j] * inv * g[j];
+                if (gate) o *= (gate_kind == 2 ? z[j] : 1.0f) / (1.0f + expf(-z[j]));
+                if (lane + 64 * j < Dv) out[(size_t)unit * Dv + lane + 64 * j] = from_f32<T>(o);
+            }
+        };
+        if (Dv <= 64) head(std::integral_constant<int, 1>{});
+        else head(std::integral_constant<int, 2>{});
         return;
     }
     for (int i = lane; i < Dv; i += 64) ss += xr[i] * xr[i];
