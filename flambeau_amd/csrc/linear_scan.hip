@@ -763,53 +763,73 @@ FL_RECORDABLE(fl_conv_prepare)
 // ------------------------------------------------------------------ rotation of float rows
 // out[t][h][d] of two row sets a (H heads) and b (H heads), both D wide per head: the first rot dims turned
 // by the step's table, pairs (i, i + rot/2) or (2i, 2i + 1); a times scale_a, b times scale_b afterwards.
-// PIECES: four neighbouring dims a thread (heads, rotated halves and rows are whole pieces of four), a token over several blocks: one
-// trip to memory instead of one per 256 values (8 tokens, 16 heads of 128 7.9 -> 4.8 us, 2,048 tokens 21.3 -> 14.7).
-template <bool PIECES>
 __global__ __launch_bounds__(256) void rotate_scale_kernel(const float* __restrict__ proj, int ld, int col_a, int col_b,
                                                            const float2* __restrict__ cs, int rot, int interleaved, float scale_a,
                                                            float scale_b, float* __restrict__ out_a, float* __restrict__ out_b,
                                                            int H, int D) {
-    constexpr int N = PIECES ? 4 : 1;
     const size_t token = blockIdx.x;
     const int half = rot >> 1;
-    for (int e = N * (blockIdx.y * 256 + threadIdx.x); e < 2 * H * D; e += N * 256 * gridDim.y) {
+    for (int e = threadIdx.x; e < 2 * H * D; e += 256) {
+        const bool is_b = e >= H * D;
+        const int f = is_b ? e - H * D : e;
+        const int h = f / D, d = f - h * D;
+        const float* src = proj + token * ld + (is_b ? col_b : col_a) + h * D;
+        float v = src[d];
+        if (d < rot) {
+            int i, partner;
+            bool first;
+            if (interleaved) { i = d >> 1; first = !(d & 1); partner = d ^ 1; }
+            else { first = d < half; i = first ? d : d - half; partner = first ? d + half : d - half; }
+            const float2 c = cs[token * half + i];
+            const float o = src[partner];
+            v = first ? v * c.x - o * c.y : v * c.x + o * c.y;
+        }
+        (is_b ? out_b : out_a)[token * H * D + f] = v * (is_b ? scale_b : scale_a);
+    }
+}
+
+// The same where heads, rotated halves and rows are whole pieces of four: four neighbouring dims a thread, a token over several
+// blocks, one trip to memory instead of one per 256 values (8 tokens, 16 heads of 128 7.9 -> 4.8 us, 2,048 tokens 21.3 -> 14.7; a
+// form for both that asks which it is took 5 % longer for 16 heads of 100).
+__global__ __launch_bounds__(256) void rotate_scale_pieces_kernel(const float* __restrict__ proj, int ld, int col_a, int col_b,
+                                                                  const float2* __restrict__ cs, int rot, int interleaved, float scale_a,
+                                                                  float scale_b, float* __restrict__ out_a, float* __restrict__ out_b,
+                                                                  int H, int D) {
+    const size_t token = blockIdx.x;
+    const int half = rot >> 1;
+    for (int e = 4 * (blockIdx.y * 256 + threadIdx.x); e < 2 * H * D; e += 4 * 256 * gridDim.y) {
         const bool is_b = e >= H * D;
         const int f = is_b ? e - H * D : e;
         const int h = f / D, d0 = f - h * D;
         const float* src = proj + token * ld + (is_b ? col_b : col_a) + h * D;
         float* dst = (is_b ? out_b : out_a) + token * H * D + f;
         const float scale = is_b ? scale_b : scale_a;
-        float v[N], o[N];
-        float2 c[N];
-        const bool turned = d0 < rot;                  // (of all N dims or none)
+        float v[4], o[4];
+        float2 c[4];
+        const bool turned = d0 < rot;                  // (of all four dims or none)
         const bool second = !interleaved && d0 >= half;
 #pragma unroll
-        for (int r = 0; r < N; ++r) v[r] = src[d0 + r];
+        for (int r = 0; r < 4; ++r) v[r] = src[d0 + r];
         if (turned) {
             if (interleaved) {
 #pragma unroll
-                for (int r = 0; r < N; ++r) { c[r] = cs[token * half + ((d0 + r) >> 1)]; o[r] = PIECES ? v[PIECES ? r ^ 1 : 0] : src[(d0 + r) ^ 1]; }
+                for (int r = 0; r < 4; ++r) { c[r] = cs[token * half + ((d0 + r) >> 1)]; o[r] = v[r ^ 1]; }
             } else {
                 const int i = second ? d0 - half : d0;
 #pragma unroll
-                for (int r = 0; r < N; ++r) { c[r] = cs[token * half + i + r]; o[r] = src[(second ? i : d0 + half) + r]; }
+                for (int r = 0; r < 4; ++r) { c[r] = cs[token * half + i + r]; o[r] = src[(second ? i : d0 + half) + r]; }
             }
         }
 #pragma unroll
-        for (int r = 0; r < N; ++r) {
+        for (int r = 0; r < 4; ++r) {
             float w = v[r];
             if (turned) {
-                const bool first = interleaved ? !((d0 + r) & 1) : !second;
+                const bool first = interleaved ? !(r & 1) : !second;
                 w = first ? v[r] * c[r].x - o[r] * c[r].y : v[r] * c[r].x + o[r] * c[r].y;
             }
             v[r] = w * scale;
         }
-        if constexpr (PIECES) {
-            *(f32x4*)dst = (f32x4){v[0], v[N - 3], v[N - 2], v[N - 1]};
-        } else {
-            dst[0] = v[0];
-        }
+        *(f32x4*)dst = (f32x4){v[0], v[1], v[2], v[3]};
     }
 }
 
@@ -823,10 +843,10 @@ extern "C" int fl_rotate_scale(const float* proj, int ld, int col_a, int col_b, 
     const bool pieces = D % 4 == 0 && rot % (interleaved ? 4 : 8) == 0 && ld % 4 == 0 && col_a % 4 == 0 && col_b % 4 == 0 &&
                         ((uintptr_t)proj | (uintptr_t)cs | (uintptr_t)out_a | (uintptr_t)out_b) % 16 == 0;
     if (pieces)
-        rotate_scale_kernel<true><<<dim3(n, min(ceil_div(2 * H * D, 1024), 64)), 256, 0, stream>>>(proj, ld, col_a, col_b, (const float2*)cs, rot, interleaved,
-                                                                                                 scale_a, scale_b, out_a, out_b, H, D);
+        rotate_scale_pieces_kernel<<<dim3(n, min(ceil_div(2 * H * D, 1024), 64)), 256, 0, stream>>>(proj, ld, col_a, col_b, (const float2*)cs, rot, interleaved,
+                                                                                                scale_a, scale_b, out_a, out_b, H, D);
     else
-        rotate_scale_kernel<false><<<n, 256, 0, stream>>>(proj, ld, col_a, col_b, (const float2*)cs, rot, interleaved, scale_a, scale_b, out_a, out_b, H, D);
+        rotate_scale_kernel<<<n, 256, 0, stream>>>(proj, ld, col_a, col_b, (const float2*)cs, rot, interleaved, scale_a, scale_b, out_a, out_b, H, D);
     FL_LAUNCH_CHECK();
     return 0;
 }
