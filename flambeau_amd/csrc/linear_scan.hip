@@ -660,6 +660,7 @@ __global__ __launch_bounds__(256) void conv_prepare_run_kernel(ConvPrepare a, in
     for (int i = 0; i < CP_RUN; ++i) ss[i] = 0.f;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {                                      // channels lane and lane + 64 (width <= 128, checked on the host)
+        if (64 * j >= width) break;                                    // (no lane has a second one)
         const int d = lane + 64 * j, c = c0 + (d < width ? d : 0);
         const f32x4 w = *(const f32x4*)(a.conv_w + (size_t)c * 4);
         float x[CP_RUN + 3];
@@ -744,8 +745,10 @@ extern "C" int fl_conv_prepare(const float* proj, int ld, int col0, int col_b, i
     FL_CHECK(D <= 64 * LS_QK_REGS, "conv_prepare: %d key dims per head, at most %d", D, 64 * LS_QK_REGS);
     dim3 pgrid(n, ceil_div(2 * G + H, 4));
     FL_CHECK(pgrid.y <= 65535, "conv_prepare: %d heads are more than one grid takes", 2 * G + H);
-    // (a run per wave needs enough tokens to give every compute unit several)
-    if (taps == 4 && D <= 128 && Dv <= 128 && (uintptr_t)conv_w % 16 == 0 && (long)ceil_div(n, CP_RUN) * pgrid.y >= 2 * fl_units())
+    // (a run per wave needs enough tokens to give every compute unit several blocks, of heads of up to 64 more than of wider ones: 512
+    // blocks of 48 heads of 128 17.6 -> 14.8 us, of 24 heads of 64 11.0 -> 11.8; 640 and 704 blocks of heads of 64 12.5 -> 11.9, 14.2 -> 12.0)
+    const int runs_for = max(D, Dv) > 64 ? 4 : 5;                      // halves of a block per unit
+    if (taps == 4 && D <= 128 && Dv <= 128 && (uintptr_t)conv_w % 16 == 0 && 2l * ceil_div(n, CP_RUN) * pgrid.y >= (long)runs_for * fl_units())
         conv_prepare_run_kernel<<<dim3(ceil_div(n, CP_RUN), pgrid.y), 256, 0, stream>>>(a, n);
     else
         conv_prepare_kernel<<<pgrid, 256, 0, stream>>>(a);
