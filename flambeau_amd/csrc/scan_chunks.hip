@@ -272,7 +272,8 @@ __global__ __launch_bounds__(256) void scan_pairs_channel_kernel(ScanChunks a) {
 
 // The delta rule's pairs, T diag(beta) and T diag(beta p) K.  T by tiles of 16 tokens: the four on the diagonal by substitution, a
 // column per lane; the others from those before them, T_IJ = -T_II sum_{J <= M < I} L_IM T_MJ, by their distance from the diagonal.  A
-// chunk whose keys, decays or strengths are not all finite substitutes throughout, so that what is no number reaches no token before it.
+// chunk whose keys, decays or strengths are not all finite, or whose products are not, substitutes throughout, so that what is no number
+// reaches no token before it.
 template <int D>
 __global__ __launch_bounds__(256) void scan_pairs_delta_kernel(ScanChunks a) {
     constexpr int ROW = D + 4, LT = SC_CHUNK + 4;
@@ -361,23 +362,7 @@ __global__ __launch_bounds__(256) void scan_pairs_delta_kernel(ScanChunks a) {
             if (l - l != 0.f) odd = 1;             // (keys too large to multiply)
         }
     __syncthreads();                               // (the decays between tokens have been read: their room is T's)
-    if (odd) {
-        if (tid < SC_CHUNK) {                      // column tid, row by row; nothing above the diagonal is multiplied
-            for (int i = 0; i < SC_CHUNK; ++i) {
-                float t = i == tid ? 1.f : 0.f;
-                if (i > tid)
-                    for (int j = tid; j < i; ++j) t = fmaf(-L[i * LT + j], T[j * LT + tid], t);
-                T[i * LT + tid] = t;
-            }
-        }
-        __syncthreads();
-        for (int d = tid; d < D; d += 256)
-            for (int i = 0; i < SC_CHUNK; ++i) {
-                float w = 0.f;
-                for (int j = 0; j <= i; ++j) w = fmaf(T[i * LT + j] * (beta[j] * pre[j]), ks[j * ROW + d], w);
-                rec[SC_DELTA_W + i * D + d] = w;
-            }
-    } else {
+    if (!odd) {
         {   // the tile on the diagonal: lane n has column n (all four lanes g the same)
             float t[16];
 #pragma unroll
@@ -408,6 +393,7 @@ __global__ __launch_bounds__(256) void scan_pairs_delta_kernel(ScanChunks a) {
                 }
 #pragma unroll
                 for (int r = 0; r < 4; ++r) x[(4 * g + r) * 20 + n] = sum[r];
+                if (((sum[0] - sum[0]) + (sum[1] - sum[1])) + ((sum[2] - sum[2]) + (sum[3] - sum[3])) != 0.f) odd = 1;      // (too large for 32 bits: its rows meet the others' zeros next)
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 f32x4 out = {0.f, 0.f, 0.f, 0.f};
                 const f32x4 t = *(const f32x4*)(T + (16 * R + n) * LT + 16 * R + 4 * g);
@@ -418,6 +404,24 @@ __global__ __launch_bounds__(256) void scan_pairs_delta_kernel(ScanChunks a) {
             }
             __syncthreads();
         }
+    }
+    if (odd) {
+        if (tid < SC_CHUNK) {                      // column tid, row by row; nothing above the diagonal is multiplied
+            for (int i = 0; i < SC_CHUNK; ++i) {
+                float t = i == tid ? 1.f : 0.f;
+                if (i > tid)
+                    for (int j = tid; j < i; ++j) t = fmaf(-L[i * LT + j], T[j * LT + tid], t);
+                T[i * LT + tid] = t;
+            }
+        }
+        __syncthreads();
+        for (int d = tid; d < D; d += 256)
+            for (int i = 0; i < SC_CHUNK; ++i) {
+                float w = 0.f;
+                for (int j = 0; j <= i; ++j) w = fmaf(T[i * LT + j] * (beta[j] * pre[j]), ks[j * ROW + d], w);
+                rec[SC_DELTA_W + i * D + d] = w;
+            }
+    } else {
         // T diag(beta p) K for the wave's 16 tokens
         f32x4 t[4];
 #pragma unroll

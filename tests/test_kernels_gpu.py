@@ -1437,6 +1437,26 @@ def test_scan_in_chunks_keeps_an_infinite_state(mode):
             assert torch.equal(a[:, :, others], b[:, :, others])
 
 
+def test_scan_in_chunks_overflows_at_its_token_and_not_before():
+    """The delta rule with three keys so large that what the third corrects is beyond 32 bits, though no product of two keys is:
+    tokens before it, in its 16 too, are what the walk makes of them."""
+    c = _scan_case("delta", 2, 2, 64, 16, [320])
+    plain, chunked = _scan_sets()
+    k = c.k.reshape(320, 2, 64)
+    k[:, :, 0] = 0
+    k /= k.norm(dim=2, keepdim=True)                             # (the others do not see them)
+    for t in (3, 9, 21):
+        k[t] = 0
+        k[t, :, 0] = 1e10
+    c.gates[:, :2], c.gates[:, 2:] = 1.0, 1.0
+    c.state0.zero_()
+    (want, _), (got, _) = c.run(plain), c.run(chunked)
+    assert not torch.isfinite(want[21:]).all() and not torch.isfinite(got[21:]).all()
+    for t in range(21):                                          # (80 sums of 3e-8, of values as large as the token's largest per head)
+        w, a = want[t].reshape(2, 16), got[t].reshape(2, 16)
+        assert bool(((w - a).abs() <= 2.5e-6 * w.abs().max(dim=1, keepdim=True).values).all()), t
+
+
 def test_scan_rows_that_the_chunks_do_not_take_walk():
     """Rows that are no whole 16-byte pieces, and head sizes that the chunked kernels do not know: the walk's bits."""
     plain, chunked = _scan_sets()
