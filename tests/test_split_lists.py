@@ -82,3 +82,20 @@ def test_recurrent_mixers_add_nothing_to_a_recorded_steps_key():
     for cls in (GatedDelta, GatedLinearAttention, Retention, StateSpace):
         for lens in ([1, 1], [300], [1, 300]):
             assert object.__new__(cls).step_signature(HostBatch([0], lens, [5] * len(lens), [0], sum(lens), 1)) == ()
+
+
+def test_what_goes_in_chunks_is_what_takes_less_time_so():
+    """Sizes of both sides that were measured (us walked, us in chunks), few requests and a full chip, whole chunks and begun ones."""
+    from flambeau_amd.kernels.linear_scan import FORMS, chunked_from
+    for kind, heads, dim, vdim, lens, walked, in_chunks in [
+            ("fixed", 16, 128, 128, [2048], 304, 103), ("written", 32, 128, 64, [2048], 310, 106), ("gated", 32, 128, 128, [2048], 311, 150),
+            ("delta", 32, 128, 128, [2048], 355, 189), ("delta", 16, 128, 128, [384], 72, 54), ("gated", 32, 128, 128, [129], 29.1, 30.4),
+            ("gated", 4, 128, 64, [193] * 4, 31, 34), ("delta", 64, 64, 64, [257], 38, 46), ("delta", 64, 64, 64, [257] * 16, 272, 493),
+            ("delta", 64, 64, 64, [1024] * 16, 991, 1475), ("delta", 64, 64, 128, [256], 48.7, 58.1), ("delta", 16, 128, 128, [256], 50, 46),
+            ("fixed", 64, 128, 64, [129] * 64, 684, 904), ("fixed", 64, 128, 128, [512] * 16, 1207, 949),
+            ("gated", 64, 128, 64, [193] * 64, 1134, 1606), ("written", 64, 64, 64, [129] * 64, 455, 526)]:
+        expected = FORMS[kind].tokens if in_chunks < walked else 0
+        assert chunked_from(kind, lens, heads, dim, vdim, 64) == expected, (kind, heads, dim, vdim, lens[0], len(lens))
+        assert chunked_from(kind, lens + [1], heads, dim, vdim, 64) == expected       # (a token beside them changes nothing)
+    for kind in FORMS:
+        assert chunked_from(kind, [1] * 8, 32, 128, 128, 64) == 0
