@@ -160,7 +160,7 @@ def test_a_product_that_norms_in_its_epilogue(n, K, H):
     kernel, many: the tiled one) against product, addition and norm apart."""
     from flambeau_amd.kernels import ops, tuned
     from flambeau_amd.parts import NORMS, PartSpec, Product, ResidualStream
-    rt = make_rt("bfloat16", max_tokens=1024)
+    rt = make_rt("bfloat16", max_tokens=512)
     norm, plain = bound_part(NORMS, PartSpec("dynamic_tanh", dict(hidden_size=H)), "bfloat16", rt, seed=n, prefix="n.")
     gen = torch.Generator().manual_seed(K)
     x = (torch.randn(n, K, generator=gen) * 0.5).to(torch.bfloat16).to(DEV)
@@ -290,7 +290,7 @@ def test_attention_with_a_window(dtype, D, Dv, window):
             want[i, a] = (p / p.sum()) @ v[lo:i + 1, a // (H // G)]
     want = (want.reshape(n, H * Dv) * pb.silu(h @ plain["m.g"].T)) @ plain["m.o"].T
     for cuts in ([150], [60, 4, 1, 1, 70, 2, 12], [1] * 30 + [120]):
-        got = run_mixer(mixer, rt, x, cuts, n_pages=60)
+        got = run_mixer(mixer, rt, x, cuts, n_pages=90)
         assert np.abs(got - want).max() < TOL[dtype] * np.abs(want).max(), cuts
 
 
@@ -347,6 +347,71 @@ def test_gated_delta_rule_alone(dtype, H, G, D, Dv, taps):
         assert np.abs(got - want).max() < (5e-5 if dtype == "float32" else 5e-2) * np.abs(want).max()
     if dtype == "float32":
         assert np.array_equal(results[0], results[1]) and np.array_equal(results[0], results[2])
+
+
+# requests long enough for chunks of 64 tokens: whole, in two portions that both go in chunks, and in chunks, single
+# tokens and short portions by turns (what walks picks the state up where a chunk left it, and the other way round)
+LONG_CUTS = ([640], [320, 320], [1, 300, 1, 1, 337], [560, 80], [2] * 20 + [600])
+
+
+def run_mixer_in_chunks(mixer, rt, x, want, tol):
+    """Every cutting against the plain numbers, and that chunks did run."""
+    for cuts in LONG_CUTS:
+        got = run_mixer(mixer, rt, x, cuts, n_pages=90)
+        assert np.abs(got - want).max() < tol * np.abs(want).max(), cuts
+    assert any(name == "scan_records" for _, name, _, _ in rt._buffers)
+
+
+@pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 64, 16), (2, 2, 128, 32)])
+def test_gated_delta_rule_in_chunks(H, G, D, Dv):
+    from flambeau_amd.parts import MIXERS, PartSpec
+    rt = make_rt("bfloat16", max_tokens=1024)
+    fix = {"A_log": lambda v: v * 3 - 1.0, "dt_bias": lambda v: v * 3}
+    mixer, plain = bound_part(MIXERS, PartSpec("gated_delta", dict(hidden_size=40, n_heads=H, n_qk_heads=G, head_dim=D, value_dim=Dv, conv_taps=4,
+                                                                    eps=1e-5)), "bfloat16", rt, seed=D, fix=fix)
+    x = _x(640, 40, "bfloat16", 8)
+    want = pb.gated_delta(x.double().numpy(), plain, "m.", dict(heads=H, kv_heads=G, dim=D, vdim=Dv, conv=4), 1e-5)
+    run_mixer_in_chunks(mixer, rt, x, want, 5e-2)
+
+
+def replayed_in_chunks(runner, reqs, ref, what):
+    """Long prompts, one of them beside another request's single token, and single tokens after them, again and again: steps are
+    recorded, replayed and turned into graphs, a longer prompt makes the chunks' workspace grow in between, and every
+    round gives the first one's bits, which are the plain model's numbers."""
+    a, b, c = (reqs[f"r{i}"] for i in range(3))
+
+    def a_round():
+        n, m = len(a) - 4, len(b) - 3
+        steps = [dict(entries=[dict(id="r0", tokens=a[:n], want=[0, n // 2, n - 1])], end=[]),
+                 dict(entries=[dict(id="r1", tokens=b[:m], want=[0, m // 3, m - 1]), dict(id="r0", tokens=a[n:n + 1], want=[0])], end=[])]
+        steps += [dict(entries=[dict(id="r0", tokens=a[n + 1 + i:n + 2 + i], want=[0]), dict(id="r1", tokens=b[m + i:m + 1 + i], want=[0])], end=[])
+                  for i in range(3)]
+        steps[-1]["end"] = ["r0", "r1"]
+        return rh.run_in_process(runner, steps)
+
+    first = a_round()
+    for turn in range(10):
+        if turn == 5:
+            grown = rh.run_in_process(runner, [dict(entries=[dict(id="r2", tokens=c, want=list(range(0, len(c), 50)))], end=["r2"])])
+        again = a_round()
+        assert all(np.array_equal(first[k], again[k]) for k in first), (what, turn)
+    assert runner.n_replayed > 0 and any(hit.graphs for hit in runner._programs.values())
+    rows = {buf.shape[0] for (_, name, _, _), buf in runner.rt._buffers.items() if name == "scan_records"}
+    assert rows and all(-(-len(c) // 64) <= n < len(c) // 16 for n in rows), rows
+    close({**first, **grown}, ref, "bfloat16", what)
+
+
+def test_chunks_recorded_and_replayed(tmp_path):
+    from bugidra_configs import att, delta, dense, model, par, ret
+    from flambeau_amd.weights import write_random_model
+    config = model(90, 64, 1e-5, 4.0, [
+        (delta(4, 2, 64, 16, 4), dense(64)),
+        (par(att(4, 2, 16, 16, 0.25, rot(10000.0, 16)), ret(2, 64, 16, [0.99, 0.999], rot(1e4, 32))), dense(48)),
+        (delta(2, 2, 64, 32, 3), None)])
+    d = write_random_model(config, tmp_path / "long", seed=31, std=0.12, gain_std=0.1, store_dtype=torch.bfloat16)
+    (d / "config.json").write_text(json.dumps(config, indent=1))
+    reqs = rh.make_requests(90, [300, 340, 700], seed=9)
+    replayed_in_chunks(runner_for(d, "bfloat16", n_pages=100, page_size=16, max_tokens=1024), reqs, reference(d, reqs), "Bugidra")
 
 
 @pytest.mark.parametrize("dtype", DTYPES)

@@ -10,7 +10,7 @@ import torch
 import plain_fipitar as pf
 import replay_helpers as rh
 from fipitar_configs import CONFIGS, left, long_memory, read_model, right, rot, write_model
-from test_bugidra_gpu import CUTS, TOL, _x, run_mixer, runner_for
+from test_bugidra_gpu import CUTS, TOL, _x, replayed_in_chunks, run_mixer, run_mixer_in_chunks, runner_for
 from test_bugidra_gpu import bound_part as _bound_part
 from test_kuvidra_gpu import close, make_rt, make_step
 
@@ -206,6 +206,40 @@ def test_the_state_space_mixer_alone(dtype, m, slow):
         assert np.abs(got - want).max() < TOL[dtype] * np.abs(want).max(), cuts
 
 
+@pytest.mark.parametrize("H,D,Dv", [(4, 64, 16), (2, 128, 32)])
+def test_gated_linear_attention_in_chunks(H, D, Dv):
+    from flambeau_amd.parts import MIXERS
+    rt = make_rt("bfloat16", max_tokens=1024)
+    mixer, plain = bound_part(MIXERS, gla_spec(40, H, D, Dv, 8, 8.0, 2e-5), "bfloat16", rt, seed=H + D, fix={"a2.bias": lambda v: v + 2.0})
+    x = _x(640, 40, "bfloat16", 5)
+    want = pf.gated_linear_attention(x.double().numpy(), dict(heads=H, dim=D, vdim=Dv, tau=8.0), plain, "m.", 2e-5)
+    run_mixer_in_chunks(mixer, rt, x, want, TOL["bfloat16"])
+
+
+@pytest.mark.parametrize("m", [right(8, 16, 64, 2, 4, 1), right(4, 32, 128, 4, 4, 2)])
+def test_the_state_space_mixer_in_chunks(m):
+    from flambeau_amd.parts import MIXERS
+    rt = make_rt("bfloat16", max_tokens=1024)
+    mixer, plain = bound_part(MIXERS, ssd_spec(40, m, 2e-5), "bfloat16", rt, seed=m["heads"] + m["state"], fix={"A_log": lambda v: v - 2.0})
+    x = _x(640, 40, "bfloat16", 6)
+    want = pf.state_space(x.double().numpy(), m, plain, "m.", 2e-5)
+    run_mixer_in_chunks(mixer, rt, x, want, TOL["bfloat16"])
+
+
+def test_chunks_recorded_and_replayed(tmp_path):
+    from fipitar_configs import dense, gla, model, pair
+    from flambeau_amd.weights import write_random_model
+    config = model(90, 64, 1e-5, [(gla(4, 64, 16, 8.0, 8), dense(64, 1.5)),
+                                  (pair(left(4, 2, 16, 16, 0.25, 10.0, rot(16)), right(8, 16, 64, 2, 4, 2), 0.8, 1.1), dense(48, 2.0)),
+                                  (gla(2, 128, 16, 4.0, 4), None)])
+    d = write_random_model(config, tmp_path / "long", seed=31, std=0.12, gain_std=0.1, store_dtype=torch.bfloat16)
+    for layer in config["layers"]:                                           # (a file's ranks are its tensors')
+        layer["mixer"].pop("decay_rank", None)
+    (d / "config.json").write_text(json.dumps(config, indent=1))
+    reqs = rh.make_requests(90, [300, 340, 700], seed=9)
+    replayed_in_chunks(runner_for(d, "bfloat16", n_pages=100, page_size=16, max_tokens=1024), reqs, reference(d, reqs), "Fipitar")
+
+
 # ---------------------------------------------------------------- latent attention with neighbours turned and a sink
 def latent_spec(W, H, D, Dr, Dv, Rq, R, scale, eps, r):
     from flambeau_amd.models.fipitar import _position
@@ -383,7 +417,7 @@ def test_the_tuned_attention_kernels_with_a_sink(H, G, D, ps, cap):
     from flambeau_amd.cache.storage import CacheStorage
     from flambeau_amd.kernels import ops, tuned
     from flambeau_amd.parts import PagedKVSpec
-    rt = make_rt("bfloat16", max_tokens=1024)
+    rt = make_rt("bfloat16", max_tokens=512)
     n_pages = -(-9000 // ps)
     store = CacheStorage([PagedKVSpec(G, D)], [None], torch.device(DEV), torch.bfloat16, n_pages=n_pages, page_size=ps, max_slots=6)
     kv = store.entries[0].kv
