@@ -551,12 +551,14 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 // with 256, 224, 192 features, 0.59 with 224 x 192 and 0.85, 0.75, 0.94 with 256 x 320, 224 x 320 and 224 x 384, less where a
 // tile's rows are few, more where a unit gets a second block of another part of K, and 7 per block that nothing overlaps.
 // Splitting K adds the parts' way to memory and back and the kernel that sums them: 1 us, and 2.35 per million values and part.
-// Parts that put a block of up to 256 tokens on nearly every unit at once are slower than their steps: launched back to back, the
-// chip lowers its clock under them, some cards more than others (4096 x 14336 at 289 rows in eight parts of 256 x 256, 256 blocks: 65 us
-// with weights of zeros, 85 with random ones, on one card of four 64; in six parts of 224 x 192, 228 blocks, 62 and 67; a prompt of 272
-// rows through four layers of the 7B model 1,139 -> 1,036 us).  A tenth where no unit is left idle, no more, picks best over
-// 20 products at 50 row counts, 11,000 timings in such a row, the mean of three cards: 30 of 1,000 picks more than 3 % faster
-// than without it, eight slower; blocks of 320 tokens do not show it (5120 x 32768 at 560 rows in six parts 204 to 212 us).
+// Parts that put a block of up to 256 tokens on nearly every unit at once are slower than their steps where a good share of the tiles' rows
+// are none: launched back to back, the chip lowers its clock under them, some cards more than others (4096 x 14336 at 289 rows in eight
+// parts of 256 x 256, 256 blocks: 65 us with weights of zeros, 85 with random ones, on one card of four 64; in six parts of 224 x 192, 228
+// blocks, 62 and 67; a prompt of 272 rows through four layers of the 7B model 1,139 -> 1,036 us).  A tenth where no unit is left
+// idle, no more, picks best over 20 products at 50 row counts, 11,000 timings in such a row, the mean of three cards: 20 of 1,000
+// picks more than 3 % faster than without it, three slower.  Tiles whose rows are there do not show it in a model (4096 x 14336 at 512
+// rows in those eight parts 71 us in a prompt's steps, in five parts of 192 x 256 82; prompts of 480 and 500 rows 1,272 and 1,291 us,
+// 1,289 and 1,318), and blocks of 320 tokens do not (5120 x 32768 at 560 rows in six parts 204 to 212 us).
 // What decides among eight waves is how evenly the blocks fill the rounds, in features (gate/up of 2,048 rows, 28672 features, is
 // 3.5 rounds of 256 and 4 of 224, q/k/v of 2,048 rows, 6144 features, 0.75 rounds of 256 and 1 of 192) and in tokens: rows that
 // end soon behind a multiple of 256 are tiles of 192 (28672 x 4096 at 333 rows 90 us, 96.6 with 256) or of 320 and 384, which at
@@ -591,8 +593,8 @@ static float tiled_cost(const TileShape& t, int splits, int M, int N, int K) {
     const long rounds = (most + t.per_unit - 1) / t.per_unit;
     const float mean = blocks > units ? (float)blocks / units : 1.f;
     const float empty = 1.f - (float)M / ((long)m_tiles * t.tokens);   // share of the tiles' rows that are none
-    // units at work at once beyond 0.88 of them
-    const float full = splits > 1 && most == 1 && t.tokens <= 256 ? fmaxf((float)blocks / units - 0.88f, 0.f) : 0.f;
+    // units at work at once beyond 0.88 of them, where more than a tenth of the tiles' rows are none
+    const float full = splits > 1 && most == 1 && t.tokens <= 256 ? fmaxf((float)blocks / units - 0.88f, 0.f) * fminf(fmaxf(10.f * empty - 1.f, 0.f), 1.f) : 0.f;
     float us;
     if (t.variant == 14 && empty > 0.4276f) return 1e9f;               // (tiles with so few rows: 28672 x 5120 at 207 rows 112.8 us, 106.4 with 256 x 128)
     if (t.variant == 13) {
