@@ -160,7 +160,7 @@ def test_a_product_that_norms_in_its_epilogue(n, K, H):
     kernel, many: the tiled one) against product, addition and norm apart."""
     from flambeau_amd.kernels import ops, tuned
     from flambeau_amd.parts import NORMS, PartSpec, Product, ResidualStream
-    rt = make_rt("bfloat16", max_tokens=512)
+    rt = make_rt("bfloat16", max_tokens=1024)
     norm, plain = bound_part(NORMS, PartSpec("dynamic_tanh", dict(hidden_size=H)), "bfloat16", rt, seed=n, prefix="n.")
     gen = torch.Generator().manual_seed(K)
     x = (torch.randn(n, K, generator=gen) * 0.5).to(torch.bfloat16).to(DEV)
@@ -290,7 +290,7 @@ def test_attention_with_a_window(dtype, D, Dv, window):
             want[i, a] = (p / p.sum()) @ v[lo:i + 1, a // (H // G)]
     want = (want.reshape(n, H * Dv) * pb.silu(h @ plain["m.g"].T)) @ plain["m.o"].T
     for cuts in ([150], [60, 4, 1, 1, 70, 2, 12], [1] * 30 + [120]):
-        got = run_mixer(mixer, rt, x, cuts, n_pages=90)
+        got = run_mixer(mixer, rt, x, cuts, n_pages=60)
         assert np.abs(got - want).max() < TOL[dtype] * np.abs(want).max(), cuts
 
 

@@ -417,7 +417,7 @@ def test_the_tuned_attention_kernels_with_a_sink(H, G, D, ps, cap):
     from flambeau_amd.cache.storage import CacheStorage
     from flambeau_amd.kernels import ops, tuned
     from flambeau_amd.parts import PagedKVSpec
-    rt = make_rt("bfloat16", max_tokens=512)
+    rt = make_rt("bfloat16", max_tokens=1024)
     n_pages = -(-9000 // ps)
     store = CacheStorage([PagedKVSpec(G, D)], [None], torch.device(DEV), torch.bfloat16, n_pages=n_pages, page_size=ps, max_slots=6)
     kv = store.entries[0].kv
