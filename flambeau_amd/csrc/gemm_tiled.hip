@@ -12,8 +12,8 @@
 //    lane with four consecutive features of one token, one 16-byte store;
 //  * blocks of four waves (256, 192 or 128 features x 128 tokens, a wave computes 8 x 4 tiles: 12 operand
 //    reads feed 32 products; ring of 3; two blocks per compute unit; with 128 features also a ring of 8 and one
-//    block per unit) and of eight (256, 224 or 192 features x 256 tokens, 224 x 192; ring of 4 or 5, one block per
-//    unit, the two waves of a SIMD taking turns at the matrix cores);
+//    block per unit) and of eight (256, 224 or 192 features x 256 tokens, 224 x 192, 256 or 224 x 320, 224 x 384; ring of
+//    4 or 5, one block per unit, the two waves of a SIMD taking turns at the matrix cores);
 //    blocks are handed to the eight dies in turn, each die working on a compact patch of tiles;
 //  * with few rows and a narrow matrix even that grid is small: K is then split over
 //    blockIdx.z, the parts are written as float partial sums and a second kernel adds them in
@@ -569,9 +569,11 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 // The constants are those that pick best among all that may be picked: 15 products (7B, 12B and 24B sizes and layers of
 // width 2,048, each with the epilogue that it runs with: rotation and stores, sum into the stream, activation, none; where
 // K is split with the kernel that adds the parts) at 50 row counts from 65 to 4,001, weights from HBM, every shape with 1
-// to 6 and 8 parts, 52,000 timings.  Picks take 1.1 % more time than the best on average and 24 % at worst (2048 x 2048
-// at 3,584 rows, 53.6 against 43.1), 2.4 % less on average than those among the shapes of up to 256 tokens; five of 750 more than 3 %
-// longer (4096 x 14336 at 289 rows 65.9 against 62.3), 124 more than 3 % shorter.
+// to 6 and 8 parts, 52,000 timings with a pause behind every five launches, which keeps the clock up.  Launched back to back, 20 products
+// at those row counts, the mean of three cards, picks take 1.6 % more time than the best on average and 18 % at worst (2048 x 2048 at
+// 3,328 rows 49.3 against 41.9, as before there were blocks of 320 tokens), 2 % less on average than the picks among blocks of up
+// to 256 tokens by the formula before; 18 of 1,000 more than 3 % longer, the worst 10 % (28672 x 4096 with its activation at 2,816 rows
+// 579 against 524; a prompt of 2,816 rows 4,910 us all the same, 5,150 before).
 struct TileShape { int variant, features, tokens, per_unit; float step; };             // step: us per k-step of a block of eight waves
 static const TileShape g_shapes[] = {{3, 256, 128, 2, 0.f}, {7, 192, 128, 2, 0.f}, {8, 128, 128, 2, 0.f}, {10, 256, 256, 1, 0.6808f}, {11, 224, 256, 1, 0.6778f},
                                      {12, 192, 256, 1, 0.5849f}, {6, 128, 256, 1, 0.58f}, {13, 128, 128, 1, 0.f}, {14, 224, 192, 1, 0.5855f},

@@ -12,9 +12,10 @@
 //     (I + L) U = diag(beta) V - diag(beta p) K S,      L_ij = beta_i d_ij (k_i . k_j) for j < i;
 // scan_pairs_delta forms T = (I + L)^-1 (unit lower triangular), T diag(beta) and T diag(beta p) K for every chunk at once, and the
 // walk makes U from v and S, exchanges it between the waves through LDS, and goes on with it in the place of v.
-// Measured, 2,048 tokens, the walk and the chunks (pairs + walk over chunks): a decay per head, 16 heads of 128 x 128, 304 us, 16 + 84;
-// with write strengths, 32 heads of 128 x 64, 309, 21 + 85; a decay per key dim, 32 heads of 128 x 128, 328, 45 + 108; the delta rule, 32
-// heads of 128 x 128, 371, 65 + 134.  A chunk of the second kernel is 2.6 to 4.2 us where its matrix instructions are 1.2 to 2.0.  Error
+// Measured, 2,048 tokens of one request alone on the device, the walk and the chunks: a decay per head, 16 heads of 128 x 128, 304 and 103
+// us; with write strengths, 32 heads of 128 x 64, 310 and 106; a decay per key dim, 32 heads of 128 x 128, 311 and 150; the delta rule, 32
+// heads of 128 x 128, 355 and 189; traced in a model's prompt the pairs and the walk over chunks take 16 + 99, 24 + 98, 57 + 113 and 73 +
+// 150.  A chunk of the second kernel is 2.6 to 4.7 us where its matrix instructions are 1.2 to 2.0.  Error
 // against 64 bits (2-norm) 7.6e-7 -> 1.4e-7, 3.7e-7 -> 1.0e-7, 1.4e-7 -> 1.2e-7, 3.7e-7 -> 1.7e-7.
 // Products of decays are formed by multiplying, never through logarithms or quotients: a decay of zero is one, and their rounding
 // is the walk's.  All values and sums are 32-bit; a chunk's sums are added to the state once, where the walk rounds the state at

@@ -2,8 +2,8 @@
 
 ``PlainLinearScan`` walks token by token (``fl_linear_scan*``), which gives a prompt cut anywhere the same bits.
 ``TunedLinearScan`` takes requests of many tokens 64 at a time on the 32-bit matrix cores (``fl_linear_scan_chunked``): the same
-sums in another order, in 32 bits, nearer to 64 bits than the walk's.  Requests of few tokens, and sizes, strides or addresses that
-the chunked kernels do not take, walk."""
+sums in another order, in 32 bits, nearer to 64 bits than the walk's.  Requests of few tokens, steps whose walk is the faster way
+(``chunked_from``), and sizes, strides or addresses that the chunked kernels do not take, walk."""
 from __future__ import annotations
 
 from typing import NamedTuple
