@@ -1311,33 +1311,48 @@ def test_gemm_tiled_activation_of_weights_read_once(variant, tokens):
     assert (both.float() - ref).abs().max() < 2.0 ** -8 * ref.abs().max()          # (a rounding to bf16, sums good to 1e-5)
 
 
-@pytest.mark.parametrize("gate", ["silu", "gelu_tanh", "gelu"])
+@pytest.mark.parametrize("gate", ["silu", "gelu_tanh", "gelu", "clamped"])
 def test_gemm_tiled_gates_over_the_whole_range(gate):
-    """The tiled product's own gates against 64 bits, ups of one.  silu is a quotient of values good to a unit or two of the last place; the two
-    gelus are z times a share (of the logistic function, whose argument is rounded, and of the normal distribution) good to 2e-7.  Zeros where e^-z overflows, NaN where the formula has them."""
-    z = torch.cat([torch.linspace(-95, 95, 3000), torch.linspace(-6, 6, 3000), torch.tensor([0.0, -0.0, 1e-30, -1e-30, 300.0, -300.0, 3e38, -3e38, float("inf"), float("nan")])]).to(DEV)
-    z = z.bfloat16()
+    """The tiled product's own gates against 64 bits, ups of one.  silu and the clamped gate are quotients of values good to a unit or two of the last place; the two
+    gelus are z times a share (of the logistic function, whose argument is rounded, and of the normal distribution) good to 2e-7.  Zeros where e^-z overflows.
+    Gates that are infinite or none, as sums that leave 32 bits make them: what the formula gives, as in the kernels for few rows."""
+    inf = float("inf")
+    z = torch.cat([torch.linspace(-95, 95, 3000), torch.linspace(-6, 6, 3000), torch.linspace(-88.6, -86, 300),
+                   torch.tensor([0.0, -0.0, 1e-30, -1e-30, 300.0, -300.0, 3e38, -3e38, inf, -inf, float("nan")])]).to(DEV).bfloat16()
     M = z.numel()
     finite = torch.isfinite(z)
-    x = torch.zeros(M, 16, dtype=torch.bfloat16, device=DEV)
-    x[:, 0], x[:, 1] = z, finite.to(torch.bfloat16)
-    gate_w, up_w = torch.zeros(8, 16, dtype=torch.bfloat16, device=DEV), torch.zeros(8, 16, dtype=torch.bfloat16, device=DEV)
-    gate_w[:, 0], up_w[:, 1] = 1.0, 1.0
+    x = torch.zeros(M, 64, dtype=torch.bfloat16, device=DEV)
+    x[:, 0], x[:, 1] = torch.where(finite, z, 0), 1.0
+    x[-3:, 2] = torch.tensor([3e38, -3e38, 3e38])                       # (times 128: an infinite sum beside an up of one)
+    x[-1, 40] = -3e38
+    gate_w, up_w = torch.zeros(8, 64, dtype=torch.bfloat16, device=DEV), torch.zeros(8, 64, dtype=torch.bfloat16, device=DEV)
+    gate_w[:, 0], gate_w[:, 2], gate_w[:, 40], up_w[:, 1] = 1.0, 128.0, 128.0, 1.0
     W = tuned().prepare_gate_up(gate_w, up_w)
-    got = torch.empty(M, 8, dtype=torch.float32, device=DEV)
-    tuned().gemm_tiled(x, W.packed, got, swiglu_rows=W.packed_rows, gate=gate)
+    def product(x):
+        out = torch.empty(x.shape[0], 8, dtype=torch.float32, device=DEV)
+        if gate == "clamped":
+            assert tuned().gemm_clamped(x, W, out, None, 1.25, inf, 0.5) is not None
+        elif x.shape[0] > 64:
+            tuned().gemm_tiled(x, W.packed, out, swiglu_rows=W.packed_rows, gate=gate)
+        else:
+            tuned().gemm_skinny(x, W.packed, out, swiglu_rows=W.packed_rows, gate=gate)
+        return out
+    got = product(x)
     d = z.double()[:, None].expand(M, 8)
     want = {"silu": lambda v: v / (1 + torch.exp(-v)), "gelu_tanh": lambda v: v / (1 + torch.exp(-2 * 0.7978845608028654 * (v + 0.044715 * v ** 3))),
-            "gelu": lambda v: 0.5 * v * torch.special.erfc(-v / 2 ** 0.5)}[gate](d)
+            "gelu": lambda v: 0.5 * v * torch.special.erfc(-v / 2 ** 0.5), "clamped": lambda v: v / (1 + torch.exp(-1.25 * v)) * 1.5}[gate](d)
     off = (got.double() - want).abs()
-    if gate == "silu":
-        ok = finite & (z > -87)                                         # (below, e^-z is about to leave 32 bits)
-        assert (off[ok] <= 4 * 2.0 ** -23 * want[ok].abs() + 1e-44).all()
+    if gate in ("silu", "clamped"):
+        # (as far as e^-z stays in 32 bits: silu to -88.7, and the clamped gate, whose exponent is rounded by up to half a unit of 64, to -70)
+        ok = finite & (z > (-88.7 if gate == "silu" else -70)) & (z < 2e38)
+        assert (off[ok] <= (4 if gate == "silu" else 40) * 2.0 ** -23 * want[ok].abs() + 1e-44).all(), (off[ok] / want[ok].abs()).max()
     else:
         ok = finite & (z > -30)
         assert (off[ok] <= 2e-7 * d[ok].abs() + 1e-44).all(), (off[ok] / d[ok].abs()).max()
-    assert (got[finite & (z <= -87)].abs() < 2e-36).all()
-    assert torch.isnan(got[~finite]).all()                              # (an infinity times the ups' zeros)
+    assert (got[finite & (z <= -88)].abs() < 2e-36).all()
+    few = product(x[-11:].contiguous())
+    assert torch.equal(torch.isnan(got[-11:]), torch.isnan(few)) and torch.equal(torch.isinf(got[-11:]), torch.isinf(few))
+    assert (got[-3] == inf).all() and torch.isnan(got[-2]).all() and (gate == "clamped" or torch.isnan(got[-1]).all())         # (min(NaN, limit) is the limit)
 
 
 @pytest.mark.parametrize("variant", [3, 7, 11, 12, 14, 15, 17])
