@@ -1355,6 +1355,36 @@ def test_gemm_tiled_gates_over_the_whole_range(gate):
     assert (got[-3] == inf).all() and torch.isnan(got[-2]).all() and (gate == "clamped" or torch.isnan(got[-1]).all())         # (min(NaN, limit) is the limit)
 
 
+@pytest.mark.parametrize("gate", ["silu", "gelu_tanh", "gelu"])
+def test_gemm_tiled_gates_are_as_near_to_64_bits_as_the_formulas(gate):
+    """The tiled product's own gates in 32 bits against the kernels for few rows, which call the library's functions: over every range the largest
+    relative error from 64 bits is no larger.  Any 32-bit gate is a sum of three bfloat16 values; ups of one."""
+    G, M, few = 128, 1024, 64
+    gate_w, up_w = torch.zeros(G, 3 * G + 32, dtype=torch.bfloat16, device=DEV), torch.zeros(G, 3 * G + 32, dtype=torch.bfloat16, device=DEV)
+    i = torch.arange(G, device=DEV)
+    gate_w[i, i] = gate_w[i, G + i] = gate_w[i, 2 * G + i] = 1.0
+    up_w[:, 3 * G] = 1.0
+    W = tuned().prepare_gate_up(gate_w, up_w)
+    formula = {"silu": lambda v: v / (1 + torch.exp(-v)), "gelu_tanh": lambda v: v / (1 + torch.exp(-2 * 0.7978845608028654 * (v + 0.044715 * v ** 3))),
+               "gelu": lambda v: 0.5 * v * torch.special.erfc(-v / 2 ** 0.5)}[gate]
+    for low, high in [(1e-3, 1.4), (1.4, 5.0), (5.0, 80.0), (-0.5, -1e-3), (-1.4, -0.5), (-3.0, -1.4), (-5.0, -3.0)] + ([(-87.0, -5.0), (-88.7, -87.0)] if gate == "silu" else []):
+        z = torch.linspace(low, high, M * G, dtype=torch.float64).float().to(DEV).view(M, G)
+        x = torch.zeros(M, 3 * G + 32, dtype=torch.bfloat16, device=DEV)
+        x[:, :G] = z
+        rest = z - x[:, :G].float()
+        x[:, G:2 * G] = rest
+        x[:, 2 * G:3 * G] = rest - x[:, G:2 * G].float()
+        x[:, 3 * G] = 1.0
+        assert torch.equal(x[:, :G].double() + x[:, G:2 * G].double() + x[:, 2 * G:3 * G].double(), z.double())
+        got, plain = torch.empty(M, G, dtype=torch.float32, device=DEV), torch.empty(M, G, dtype=torch.float32, device=DEV)
+        tuned().gemm_tiled(x, W.packed, got, swiglu_rows=W.packed_rows, gate=gate)
+        for at in range(0, M, few):
+            tuned().gemm_mid(x[at:at + few], W.packed, plain[at:at + few], swiglu_rows=W.packed_rows, gate=gate)
+        want = formula(z.double())
+        far = [((v.double() - want).abs() / want.abs()).max().item() for v in (got, plain)]
+        assert far[0] <= far[1], (low, high, far)
+
+
 @pytest.mark.parametrize("variant", [3, 7, 11, 12, 14, 15, 17])
 @pytest.mark.parametrize("M,inter", [(1, 8), (130, 113), (257, 132), (300, 264), (193, 226)])
 def test_gemm_tiled_activation_for_rows_of_any_width(variant, M, inter):
