@@ -28,14 +28,6 @@ __device__ __forceinline__ void gf_add(float part, float& acc, float& lost) {
     acc = t;
 }
 
-// LDS written by some lanes of a wave and read by others of the same wave: its operations run in order, this keeps
-// the compiler from moving them.
-__device__ __forceinline__ void gf_wave_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // ------------------------------------------------------------------ few rows of x
 // Block = 16 rows of w x 16 MT rows of x, four waves.  A step is 64 CH k: wave v forms CH chunks of it, the ones
 // from v CH on, of rows of w and x that it fetches itself (AHEAD steps ahead, in registers; a row's piece by
@@ -89,7 +81,7 @@ __global__ __launch_bounds__(256, 2) void gemm_float_few_kernel(const float* __r
 #pragma unroll
             for (int u = 0; u < XF; ++u) *(f32x4*)&xs[wave][u / F][((ROWS * u + fr) & 15) * LD + fk] = in ? px[a][u] : zero;
             fetch(step + AHEAD, pw[a], px[a]);
-            gf_wave_fence();
+            wave_fence();
             f32x4 part[MT][CH];
 #pragma unroll
             for (int s = 0; s < 4; ++s)
@@ -103,7 +95,7 @@ __global__ __launch_bounds__(256, 2) void gemm_float_few_kernel(const float* __r
                         part[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, xv, from, 0, 0, 0);
                     }
                 }
-            gf_wave_fence();
+            wave_fence();
             float(*to)[4 * CH * 256] = sums[step & 1];
 #pragma unroll
             for (int t = 0; t < MT; ++t)
