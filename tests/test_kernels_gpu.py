@@ -1269,6 +1269,27 @@ def test_gemm_tiled_where_a_pair_of_steps_is_not_full(variant, M, N, K, splits):
     assert (out[:M][~bad].double() - ref[~bad]).abs().max() < 1e-5 * ref[~bad].abs().max()
 
 
+@pytest.mark.parametrize("variant", [3, 6, 7, 8, 10, 11, 12, 13, 14, 15, 16, 17])
+@pytest.mark.parametrize("K,splits", [(96, 1), (24, 1), (352, 1), (1056, 3)])
+def test_gemm_tiled_fetches_no_weights_behind_the_last_step(variant, K, splits):
+    """Odd numbers of steps: the pair's second half multiplies zeros.  What lies there in memory is the next 16 features' first step, made infinite here (and,
+    behind the matrix, what is no number): had it been fetched, even x of zero would make NaN of the features before."""
+    from flambeau_amd.kernels.packing import pack_weight
+    M, N = 70, 400
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=55), rnd(N, K, dtype=torch.bfloat16, seed=56, scale=0.05)
+    odd = torch.arange(N, device=DEV) // 16 % 2 == 1
+    w[odd, :32] = float("inf")
+    packed = pack_weight(w)
+    room = torch.full((packed.numel() + (1 << 16),), float("nan"), dtype=torch.bfloat16, device=DEV)
+    room[:packed.numel()] = packed.flatten()
+    out = torch.empty(M, N, dtype=torch.float32, device=DEV)
+    ws = torch.empty(splits * M * N, dtype=torch.float32, device=DEV)
+    tuned().gemm_tiled(x, room[:packed.numel()].view(packed.shape), out, ws, variant=variant, splits=splits)
+    ref = x.double() @ w[~odd].double().T
+    assert not torch.isfinite(out[:, odd]).any()
+    assert (out[:, ~odd].double() - ref).abs().max() < 1e-5 * ref.abs().max()              # (sums of at most 1,056 products in 32 bits)
+
+
 @pytest.mark.parametrize("M,N,K,cols", [(1286, 16384, 512, 8192), (1175, 16400, 1000, 8195), (2063, 16384, 512, 8180), (842, 28672, 4096, 14336)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_gemm_tiled_activation_in_two_launches(dtype, M, N, K, cols):
