@@ -68,8 +68,6 @@ static const TileShape& tile_shape(int variant) {
 }
 static bool tiled_known(int variant) { return variant == 0 || tile_shape(variant).variant == variant; }
 
-#define TG_MOST_K (1 << 22)
-
 // k-steps of a part of K: an even number, so that only K's last pair of steps is half empty
 static int tiled_steps(int K, int splits) { return 2 * ceil_div(ceil_div(K, 32), 2 * splits); }
 
@@ -106,6 +104,7 @@ static TilePlan tiled_plan(int M, int N, int K, bool may_split, int forced_varia
             }
         }
     }
+    if (K > TG_MOST_K) return {8, splits};                 // (whichever is asked for: the block whose kernel has 64-bit addresses)
     if (forced_variant) return {forced_variant, splits};
     TilePlan best = {3, splits};
     float best_us = 0.f;
@@ -162,7 +161,6 @@ static int tiled_entry(const void* x, const void* w_packed, void* out, float* wo
                        int forced_splits, const GateConstants& gate, hipStream_t stream) {
     FL_CHECK(M >= 0 && N > 0 && K > 0, "gemm_tiled: bad sizes M=%d N=%d K=%d", M, N, K);
     FL_CHECK(K % 8 == 0, "gemm_tiled: K=%d is no multiple of 8 (16-byte loads)", K);
-    FL_CHECK(K <= TG_MOST_K, "gemm_tiled: K=%d is beyond %d (32-bit offsets within a block's rows)", K, TG_MOST_K);
     FL_CHECK(out_dtype == FL_F32 || out_dtype == FL_BF16, "gemm_tiled: unknown output dtype %d", out_dtype);
     const int gate_kind = epilogue >> 4;          // the bits above the low four: the activation of the gate (epilogue 1)
     epilogue &= 15;
@@ -262,7 +260,6 @@ extern "C" int fl_gemm_tiled_residual_ex(const void* x, const void* w_packed, fl
     FL_CHECK(tiled_known(variant), "gemm_tiled_residual: block shape %d (0, 3, 6, 7, 8 or 10 to 17)", variant);
     FL_CHECK(M >= 0 && N > 0 && K > 0, "gemm_tiled_residual: bad sizes M=%d N=%d K=%d", M, N, K);
     FL_CHECK(K % 8 == 0, "gemm_tiled_residual: K=%d is no multiple of 8 (16-byte loads)", K);
-    FL_CHECK(K <= TG_MOST_K, "gemm_tiled_residual: K=%d is beyond %d (32-bit offsets within a block's rows)", K, TG_MOST_K);
     FL_CHECK(N % 4 == 0, "gemm_tiled_residual: N=%d is no multiple of 4 (16-byte accesses to the residual rows)", N);
     FL_CHECK(resid && g && xg && out_ssq, "gemm_tiled_residual: needs resid, g, xg and out_ssq");
     FL_CHECK(((uintptr_t)x % 16 == 0) && ((uintptr_t)w_packed % 16 == 0) && ((uintptr_t)resid % 16 == 0) &&
@@ -292,7 +289,6 @@ extern "C" int fl_gemm_tiled_dyt(const void* x, const void* w_packed, int M, int
                                  const float* alpha, const float* g, const float* bias, void* xn, hipStream_t stream) {
     FL_CHECK(M >= 0 && N > 0 && K > 0, "gemm_tiled_dyt: bad sizes M=%d N=%d K=%d", M, N, K);
     FL_CHECK(K % 8 == 0, "gemm_tiled_dyt: K=%d is no multiple of 8 (16-byte loads)", K);
-    FL_CHECK(K <= TG_MOST_K, "gemm_tiled_dyt: K=%d is beyond %d (32-bit offsets within a block's rows)", K, TG_MOST_K);
     FL_CHECK(N % 4 == 0, "gemm_tiled_dyt: N=%d is no multiple of 4 (16-byte accesses to the residual rows)", N);
     FL_CHECK(resid && alpha && g && xn, "gemm_tiled_dyt: needs resid, alpha, g and xn");
     FL_CHECK(((uintptr_t)x % 16 == 0) && ((uintptr_t)w_packed % 16 == 0) && ((uintptr_t)resid % 16 == 0) &&
@@ -328,7 +324,6 @@ extern "C" int fl_gemm_tiled_partials(const void* x, const void* w_packed, float
                                       const float* in_ssq, int in_parts, float eps, hipStream_t stream) {
     FL_CHECK(M >= 0 && N > 0 && K > 0, "gemm_tiled_partials: bad sizes M=%d N=%d K=%d", M, N, K);
     FL_CHECK(K % 8 == 0, "gemm_tiled_partials: K=%d is no multiple of 8 (16-byte loads)", K);
-    FL_CHECK(K <= TG_MOST_K, "gemm_tiled_partials: K=%d is beyond %d (32-bit offsets within a block's rows)", K, TG_MOST_K);
     FL_CHECK(workspace && ((uintptr_t)x % 16 == 0) && ((uintptr_t)w_packed % 16 == 0) && ((uintptr_t)workspace % 16 == 0),
              "gemm_tiled_partials: operands must be 16-byte aligned");
     FL_CHECK(!in_ssq || in_parts > 0, "gemm_tiled_partials: a row scale over %d parts", in_parts);
@@ -356,7 +351,6 @@ extern "C" int fl_gemm_tiled_rope_ex(const void* x, const void* w_packed, int M,
     FL_CHECK(tiled_known(variant), "gemm_tiled_rope: block shape %d (0, 3, 6, 7, 8 or 10 to 17)", variant);
     FL_CHECK(M >= 0 && N > 0 && K > 0, "gemm_tiled_rope: bad sizes M=%d N=%d K=%d", M, N, K);
     FL_CHECK(K % 8 == 0, "gemm_tiled_rope: K=%d is no multiple of 8 (16-byte loads)", K);
-    FL_CHECK(K <= TG_MOST_K, "gemm_tiled_rope: K=%d is beyond %d (32-bit offsets within a block's rows)", K, TG_MOST_K);
     FL_CHECK(positions && tok_seq && block_table && cs && q_out && cache_base,
              "gemm_tiled_rope: needs positions, requests, block table, angles, q and the cache");
     FL_CHECK(hd % 16 == 0 && rot % 16 == 0 && rot <= hd && N == (nh + 2 * nkv) * hd,

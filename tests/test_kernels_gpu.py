@@ -1290,6 +1290,41 @@ def test_gemm_tiled_fetches_no_weights_behind_the_last_step(variant, K, splits):
     assert (out[:, ~odd].double() - ref).abs().max() < 1e-5 * ref.abs().max()              # (sums of at most 1,056 products in 32 bits)
 
 
+@pytest.mark.parametrize("K", [(1 << 22) - 8, 1 << 22, (1 << 22) + 8, (1 << 23) + 72])
+def test_gemm_tiled_takes_rows_of_any_length(K):
+    """Rows longer than a block's 32-bit offsets reach, and the longest that they do, through the plain, the stream's and the activation's epilogue.
+    Values of -1, 0 and 1: every sum is a whole number below 2^24, so exact in any order.  Rows and features end within a tile; behind both lies what is no number."""
+    M, N, steps = 131, 80, -(-K // 32)
+    g = torch.Generator(device=DEV).manual_seed(7)
+    x = torch.full((M * K + 4096,), float("nan"), dtype=torch.bfloat16, device=DEV)[:M * K].view(M, K)
+    for r in range(M):
+        x[r] = torch.randint(-1, 2, (K,), generator=g, device=DEV, dtype=torch.int8).bfloat16()
+    w = torch.full((N * steps * 32 + 4096,), float("nan"), dtype=torch.bfloat16, device=DEV)[:N * steps * 32]
+    tiles = w.view(N // 16, steps, 4, 16, 8)                             # (a tile of 16 features x 32 values of k: lane 16 g + i holds feature i's piece g)
+    rows = torch.zeros(N, steps * 32, dtype=torch.bfloat16, device=DEV)
+    for r in range(N):
+        rows[r, :K] = torch.randint(-1, 2, (K,), generator=g, device=DEV, dtype=torch.int8).bfloat16()
+    tiles.copy_(rows.view(N // 16, 16, steps, 4, 8).permute(0, 2, 3, 1, 4))
+    ref = torch.zeros(M, N, dtype=torch.float64, device=DEV)
+    for at in range(0, K, 1 << 20):
+        ref += (x[:, at:at + (1 << 20)].float() @ rows[:, at:min(at + (1 << 20), K)].float().T).double()
+    splits = tuned().gemm_tiled_splits(M, N, K)
+    ws = torch.empty(max(splits, 3) * M * N, dtype=torch.float32, device=DEV)
+    for variant, parts in ((0, 0), (8, 1), (10, 3)):
+        out = torch.full((M + 1, N), 7.0, dtype=torch.float32, device=DEV)
+        tuned().gemm_tiled(x, w, out[:M], ws, variant=variant, splits=parts)
+        assert torch.equal(out[:M].double(), ref) and (out[M] == 7.0).all()
+    resid, gain = torch.zeros(M, N, dtype=torch.float32, device=DEV), torch.ones(N, dtype=torch.float32, device=DEV)
+    xg, ssq = torch.empty(M, N, dtype=torch.bfloat16, device=DEV), torch.empty(M, tuned().tiled_parts(M, N, K), dtype=torch.float32, device=DEV)
+    tuned().gemm_tiled_residual(x, w, resid, gain, xg, ssq, 1e-5, ws)
+    assert torch.equal(resid.double(), ref) and torch.equal(xg, ref.bfloat16())
+    act = torch.empty(M, N // 2, dtype=torch.float32, device=DEV)
+    tuned().gemm_tiled(x, w, act, swiglu_rows=N)
+    gate, up = ref.view(M, N // 8, 2, 4).unbind(2)
+    want = (gate / (1 + torch.exp(-gate)) * up).reshape(M, N // 2)
+    assert ((act.double() - want).abs() <= 4 * 2.0 ** -23 * want.abs() + 1e-30).all()
+
+
 @pytest.mark.parametrize("M,N,K,cols", [(1286, 16384, 512, 8192), (1175, 16400, 1000, 8195), (2063, 16384, 512, 8180), (842, 28672, 4096, 14336)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_gemm_tiled_activation_in_two_launches(dtype, M, N, K, cols):
