@@ -1461,6 +1461,32 @@ def test_gemm_tiled_activation_for_rows_of_any_width(variant, M, inter):
         assert torch.equal(got[0].bfloat16(), got[1])
 
 
+@pytest.mark.parametrize("variant", [3, 7, 11, 12, 16, 17])
+@pytest.mark.parametrize("M,N", [(130, 100), (257, 132), (65, 4), (300, 1028), (193, 226)])
+def test_gemm_tiled_stores_rows_of_any_width(variant, M, N):
+    """The plain epilogue's bfloat16 rows of a multiple of four values and of neither: the float results' rounding to the bit, nothing behind a row or the last."""
+    from flambeau_amd.kernels.packing import pack_weight
+    x, w, got = rnd(M, 72, dtype=torch.bfloat16, seed=43), pack_weight(rnd(N, 72, dtype=torch.bfloat16, seed=44, scale=0.3)), []
+    for dtype in (torch.float32, torch.bfloat16):
+        out = torch.full((M + 1, N), float("nan"), dtype=dtype, device=DEV)
+        tuned().gemm_tiled(x, w, out[:M], variant=variant, splits=1)
+        assert torch.isnan(out[M]).all()
+        got.append(out[:M])
+    assert torch.equal(got[0].bfloat16(), got[1])
+
+
+@pytest.mark.parametrize("gate", [False, True])
+def test_gemm_tiled_stores_rows_of_fours_in_fours(gate):
+    """bfloat16 rows of 4,100 values beside rows of 4,104, which are stored eight at a time: a third slower at most (value by value they took 1.6 times as long)."""
+    M, K, times = 2000, 1024, []
+    x = rnd(M, K, dtype=torch.bfloat16, seed=21)
+    for N in (4100, 4104):
+        rows = -(-(2 * N if gate else N) // 16) * 16
+        w, out = rnd(rows * K, dtype=torch.bfloat16, seed=22, scale=0.05), torch.empty(M, N, dtype=torch.bfloat16, device=DEV)       # (any values are a packed matrix)
+        times.append(time_of(lambda: tuned().gemm_tiled(x, w, out, swiglu_rows=rows if gate else 0, splits=0 if gate else 1)))
+    assert times[0] < 4 / 3 * times[1], times
+
+
 # ---------------------------------------------------------------- the walk of the linear recurrences
 @pytest.mark.parametrize("mode", ["fixed", "delta", "forget", "delta_per_dim", "gated", "written"])
 @pytest.mark.parametrize("D,Dv", [(64, 16), (128, 48), (256, 32)])
