@@ -139,6 +139,9 @@ __device__ __forceinline__ RopeColumns rope_columns(const RopeStore& rs, int f0)
     return {head, within, within + 8, -1};
 }
 
+// (q and the cache begin at 8 bytes, as rope_store4 has them: one 16-byte store all the same)
+typedef bf16x8 bf16x8_at8 __attribute__((aligned(8)));
+
 // v: the group's values of token tok, a valid one.  The same products and sums as rope_store4.
 __device__ __forceinline__ void rope_store16(const RopeStore& rs, int tok, const TokenPlace& tp, const RopeColumns& col, const f32x4 (&v)[4]) {
     const int hd = rs.cache.head_dim, nkv = rs.cache.n_kv_heads;
@@ -171,12 +174,12 @@ __device__ __forceinline__ void rope_store16(const RopeStore& rs, int tok, const
     }
     if (col.head < rs.nh) {
         bf16_t* row = rs.q_out + ((size_t)tok * rs.nh + col.head) * hd;
-        *(bf16x8*)(row + col.dim) = lo;
-        *(bf16x8*)(row + col.other) = hi;
+        *(bf16x8_at8*)(row + col.dim) = lo;
+        *(bf16x8_at8*)(row + col.other) = hi;
     } else if (col.head < rs.nh + nkv) {
         bf16_t* base = (bf16_t*)rs.cache.base + cache_k_offset(rs.cache, tp.page, col.head - rs.nh, tp.row, 0);
-        *(bf16x8*)(base + col.dim) = lo;
-        *(bf16x8*)(base + col.other) = hi;
+        *(bf16x8_at8*)(base + col.dim) = lo;
+        *(bf16x8_at8*)(base + col.other) = hi;
     } else {
         bf16_t* p = (bf16_t*)rs.cache.base + cache_v_offset(rs.cache, tp.page, col.head - rs.nh - nkv, tp.row, col.dim);
 #pragma unroll

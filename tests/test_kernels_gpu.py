@@ -938,6 +938,28 @@ def test_gemm_with_rotation_and_stores_in_its_kernel(M, nh, nkv, hd, rot, ps, H)
     assert tuned().gemm_rope_store(x, W, store_c) and not cache_c.pool.any() and torch.equal(store_c.q_out, q_b)
 
 
+@pytest.mark.parametrize("variant", [3, 7, 16, 17])
+def test_gemm_tiled_rotates_into_queries_that_begin_at_8_bytes(variant):
+    """Queries and cache pages that begin 8 bytes behind a 16-byte boundary: the bits of those that begin at one, and nothing beside them."""
+    from flambeau_amd.kernels.ops import PagedLayerCache
+    from flambeau_amd.kernels.packing import pack_weight
+    M, nh, nkv, hd, rot, ps, K = 130, 3, 2, 48, 32, 16, 72
+    N, pages = (nh + 2 * nkv) * hd, 9
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=62), pack_weight(rnd(N, K, dtype=torch.bfloat16, seed=61, scale=0.1))
+    pos, table = torch.arange(M, dtype=torch.int32, device=DEV), torch.arange(pages, dtype=torch.int32, device=DEV)[None].contiguous()
+    angles, got = rnd(M, rot // 2, 2, seed=63), []
+    for offset in (0, 4):
+        room = [torch.full((n + 16,), 7.0, dtype=torch.bfloat16, device=DEV) for n in (M * nh * hd, pages * 2 * nkv * ps * hd)]
+        q, pool = (r[offset:r.numel() - 16 + offset] for r in room)
+        cache = PagedLayerCache(pool.view(pages, 2, nkv, ps, hd))
+        store = tuned().RopeStore(pos, torch.zeros_like(pos), table, angles, q.view(M, nh * hd), cache, nh, rot, True)
+        tuned().gemm_tiled_rope(x, w, N, store, variant=variant)
+        for r, v in zip(room, (q, pool)):
+            assert (r[:offset] == 7.0).all() and (r[v.numel() + offset:] == 7.0).all()
+        got.append((q.clone(), pool.clone()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and (got[0][0] != 7.0).all()
+
+
 def test_gemm_dispatch_rows_agree_across_kernels():
     """The same rows through the skinny, the middle and the tiled kernel: equal up to float rounding of sums."""
     w = rnd(512, 1024, dtype=torch.bfloat16, seed=23, scale=0.05)
