@@ -18,6 +18,7 @@
 #include "recordable.h"
 
 #define QKV_FEW_TOKENS 64     // up to this many tokens a block forms the projection's sums of squares for itself
+#define QKV_MANY_VALUES (1L << 20)      // values of q, k and v from which the kernel for many tokens is the faster one (fl_qkv_prepare)
 
 struct QkvPrepare {
     const float* proj; int ld; int col_q, col_k, col_v;
@@ -329,9 +330,13 @@ extern "C" int fl_qkv_prepare(const float* proj, int ld, int col_q, int col_k, i
         FL_LAUNCH_CHECK();
     }
     // Many tokens of heads as wide as they are stored, whose columns, tables and pages 16-byte accesses meet; pages hold whole eights of tokens.
+    // Its chain of lookups and LDS takes 4.4 us at least, 5 where every token is another request's (v stored value by value), the kernel above 3.7: wave per
+    // head and here, a prompt's tokens and as many requests': 8 + 1 + 1 heads of 128, 256 tokens 4.1 us and 4.6, 4.0 and 5.3, 512 tokens 5.0 and 4.8, 4.7 and 5.6,
+    // 2,048 tokens 10.8 and 6.0, 10.4 and 6.8; 2 + 1 + 1 heads, 2,048 tokens (the line) 6.6 and 5.0, 6.1 and 6.0; 32 + 8 + 8 heads, 96 tokens 4.5 and
+    // 4.9, 4.3 and 5.4, 192 tokens (just above it) 6.1 and 5.1, 5.8 and 5.7.
     const bool by16 = ((uintptr_t)proj | (uintptr_t)bias | (uintptr_t)qnorm_w | (uintptr_t)knorm_w | (uintptr_t)q_head_gain | (uintptr_t)k_head_gain |
                        (uintptr_t)v_first | (uintptr_t)q_out | (uintptr_t)cache_base) % 16 == 0 && (ld | col_q) % 4 == 0 && (col_k < 0 || (col_k | col_v) % 4 == 0);
-    if (n > QKV_FEW_TOKENS && by16 && hdp == D && Dv == D && (D == 64 || D == 128 || D == 256) && rot % 8 == 0 && page_size % 8 == 0 && (!qnorm_w || row_scales) &&
+    if (n > QKV_FEW_TOKENS && (long)n * (nh + (col_k >= 0 ? 2 * nkv : 0)) * D >= QKV_MANY_VALUES && by16 && hdp == D && Dv == D && (D == 64 || D == 128 || D == 256) && rot % 8 == 0 && page_size % 8 == 0 && (!qnorm_w || row_scales) &&
         dtype == FL_BF16) {
         const long units = (long)n * (nh + (col_k >= 0 ? nkv : 0)), qk = (units + 2048 / D - 1) / (2048 / D), v = col_k >= 0 ? (long)ceil_div(n, 64) * (nkv * D / 64) : 0;
         if (units + 256 < (1L << 31) && qk + v < (1L << 31)) {

@@ -2002,11 +2002,12 @@ def test_convolution_takes_no_leap_where_runs_begin():
 
 # ---------------------------------------------------------------- between a projection and attention, many tokens
 @pytest.mark.parametrize("D,nh,nkv,ps,n,rot,interleaved,head_norm,mix,whole_norm,bias", [
-    (128, 32, 8, 16, 200, 128, False, 0, 0, False, False), (128, 5, 3, 16, 65, 64, False, 1, 1, False, True), (64, 6, 2, 8, 130, 64, True, 2, 2, False, False),
-    (256, 3, 1, 32, 100, 128, True, 1, 2, False, True), (64, 7, 5, 64, 333, 16, False, 0, 1, True, False), (128, 4, 0, 16, 129, 128, False, 2, 0, False, False),
-    (256, 2, 2, 24, 71, 0, False, 2, 2, False, False), (128, 8, 2, 8, 96, 8, True, 0, 0, True, True)])
+    (128, 32, 8, 16, 200, 128, False, 0, 0, False, False), (128, 5, 3, 16, 745, 64, False, 1, 1, False, True), (64, 6, 2, 8, 1650, 64, True, 2, 2, False, False),
+    (256, 3, 1, 32, 820, 128, True, 1, 2, False, True), (64, 7, 5, 64, 965, 16, False, 0, 1, True, False), (128, 4, 0, 16, 2049, 128, False, 2, 0, False, False),
+    (256, 2, 2, 24, 691, 0, False, 2, 2, False, False), (128, 8, 2, 8, 700, 8, True, 0, 0, True, True), (128, 5, 3, 16, 744, 64, False, 1, 1, False, True),
+    (64, 6, 2, 8, 130, 64, True, 2, 2, False, False)])
 def test_qkv_prepare_of_many_tokens(D, nh, nkv, ps, n, rot, interleaved, head_norm, mix, whole_norm, bias):
-    """Steps of more than 64 tokens against the same tokens at most 64 at a time (a wave per head): queries, cache pages and kept values. Requests that begin
+    """Steps of 2^20 values and more (the last two: just fewer, and far fewer) against the same tokens at most 64 at a time (a wave per head): queries, cache pages and kept values. Requests that begin
     anywhere in a page, some rows without a page; columns behind others. The sums of squares are in another order and the rotations' products may be fused
     otherwise: one rounding to bfloat16 at most, and one unit of 32 bits of what cancels."""
     ops_ = ops()
@@ -2049,3 +2050,16 @@ def test_qkv_prepare_of_many_tokens(D, nh, nkv, ps, n, rot, interleaved, head_no
         assert ((a - w).abs() <= 2.0 ** -7 * w.abs() + 2.0 ** -20 * w.abs().max()).all()          # (neighbours of 8 significant bits lie at most 2^-7 apart)
     if has_kv:                                            # (values are neither normed nor turned: the same bits)
         assert torch.equal(c1[:, 1], c2[:, 1]) and (c1 != 0).any()
+
+
+@pytest.mark.parametrize("nh,nkv,D", [(2, 1, 128), (8, 2, 64), (8, 1, 128)])
+def test_qkv_prepare_takes_no_leap_behind_64_tokens(nh, nkv, D):
+    """A decode step of 65 requests beside one of 64, which a wave per head does: no leap (where the kernel for many tokens began there it took a third longer)."""
+    times = []
+    for n in (64, 65):
+        proj, angles = rnd(n, (nh + 2 * nkv) * D, seed=5), rnd(n, D // 2, 2, seed=6)
+        seq, pos = torch.arange(n, dtype=torch.int32, device=DEV), torch.full((n,), 5, dtype=torch.int32, device=DEV)
+        cache, q = make_cache(n, nkv, 16, D, torch.bfloat16), torch.empty(n, nh * D, dtype=torch.bfloat16, device=DEV)
+        table = seq[:, None].contiguous()
+        times.append(time_of(lambda: ops().qkv_prepare(proj, (0, nh * D, (nh + nkv) * D), pos, seq, table, q, cache, nh, D, D, D, False, angles, None, None, 0, 1e-5)))
+    assert times[1] < 1.12 * times[0] + 0.1, times
