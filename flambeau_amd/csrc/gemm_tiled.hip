@@ -54,9 +54,10 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 // whose best is nearest to the best of all: 20 products (7B, 12B and 24B sizes and layers of width 2,048 and 3,072, each with the epilogue
 // that it runs with: rotation and stores, sum into the stream, activation, none; where K is split with the kernel that adds the parts) at 51 row
 // counts from 65 to 4,001, weights from HBM, shapes and 1 to 6 and 8 parts, 19,600 timings launched back to back.  Picks take 0.9 %
-// more time than the best on average and 18 % at worst (7168 x 5120 at 400 rows 52 us, 43 with 128 x 128 whole).  Splits count a little less
-// than they cost, which keeps products of few tiles in parts where whole they would be up to 7 % faster (6144 x 4096 at 512 rows 46.7 us
-// in two parts of 192 x 128 with the rotation's kernel, 43.6 whole in 128 x 128).
+// more time than the best on average; over another 384 products (twelve matrices, 32 row counts) 2.4 % and 19 % at worst.  Where they are known to be wrong: 97 to 128 rows
+// of a narrow matrix, which 128 x 96 takes in two tiles of tokens (4096 x 4096 at 97 rows 18.9 us in four parts, 16.5 in six of 128 x 128), narrow matrices in more
+// parts than pay, and splits count less than they cost with what stands behind them (7168 x 5120 at 400 rows with the rotation 49 us in two parts, 42 whole in
+// 128 x 128; 6144 x 4096 at 512 rows 46 and 42).
 struct TileShape { int variant, features, tokens, tiles; float step; };       // tiles: of a wave; step: us per k-step
 #define TG_SHAPE(variant, FT, TT, WT, NSW, XP, step) {variant, 64 / WT * FT, 16 * WT * TT, FT * TT, step},
 static const TileShape g_shapes[] = {TG_SHAPES(TG_SHAPE)};
@@ -340,8 +341,8 @@ FL_RECORDABLE(fl_gemm_tiled_partials)
 
 // The joined q/k/v projection of many rows with its rows in paired order: q is rotated and written to
 // q_out[M, nh * hd], k rotated and v as it is into the cache pages at the tokens' positions; cs[M,
-// rot / 2, 2] are the step's cosines and sines.  K is never split here (for shapes whose K the plain
-// product would split, that product followed by the rotation kernel is the faster way).  in_ssq as in
+// rot / 2, 2] are the step's cosines and sines.  K is never split here (shapes whose K the plain
+// product would split go to that product and the rotation kernel).  in_ssq as in
 // fl_gemm_tiled_scaled.
 extern "C" int fl_gemm_tiled_rope_ex(const void* x, const void* w_packed, int M, int N, int K, const float* in_ssq,
                                      int in_parts, float eps, const int* positions, const int* tok_seq,

@@ -222,8 +222,9 @@ def gemm_rope_store(x, w: Weight, store: RopeStore, rt=None) -> bool:
         gemm_skinny_rope(x, w.packed, w.rows, store, row_scale=scale)
         return True
     # many rows: the tiled product rotates and stores itself where its K is not split; where it is, it
-    # leaves the splits apart and the rotation kernel adds them (at 7B sizes and 512 rows the product
-    # with K split in two takes 45 us and the rotation kernel 13, the whole product in one kernel 82)
+    # leaves the splits apart and the rotation kernel adds them (6144 x 4096 at 65 rows in five parts 20 us, 34 in one kernel, at
+    # 160 rows in two parts 29 and 33).  The plan weighs the product alone, which is known to be up to a fifth too slow for some
+    # sizes of more rows: 207 rows in four parts 33 us and 31, 512 rows in two parts 46 and 42, 7168 x 5120 at 400 rows in two parts 49 and 42
     if M > SKINNY_MAX_ROWS and K % 8 == 0:
         x, scale = _rows_for(x, w, rt)
         N = w.rows
