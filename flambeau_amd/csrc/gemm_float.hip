@@ -1,55 +1,56 @@
 // The 32-bit matrix product on the matrix cores: out[m][n] = sum_k x[m][k] w[n][k], floats in, floats out,
 // the same bits as gemm_plain_kernel (plain.hip) gives.
 //
-// What an output element is: its k in rising chunks of 16, every chunk a chain of 16 fused multiply-adds
-// from zero, the chunks' sums added in rising order with a compensated (Kahan) addition.  A
-// v_mfma_f32_16x16x4_f32 is such a chain of four (rising k, one rounding each: 1 M random results and
-// products below the smallest normal number are bit for bit those of fmaf), so four of them on one
-// accumulator are a chunk.  Nothing else about the sum is free: K cannot be split, but the chunks' chains
-// are independent of one another; only the compensated addition, four operations per chunk, is serial.
+// What an output element is: its k in rising groups of 64, a group two halves of 32, a half three chains of 12, 12 and 8 fused
+// multiply-adds from zero, (12 + 12) + 8, the halves and the chains added in 32 bits, the groups in rising order in 64; k behind K
+// are zeros.  Its distance from the exact sum, root mean square over normal values, is 8.06e-8 at K 4096 and 8.03e-8 at 14336 (chains of
+// 16 with a compensated addition in 32 bits: 8.10e-8 and 8.17e-8).  A v_mfma_f32_16x16x4_f32 is such a chain of four (rising k, one rounding
+// each: 1 M random results and products below the smallest normal number are bit for bit those of fmaf).  Nothing else
+// about the sum is free: K cannot be split, but groups are independent of one another up to their addition.
+// Additions and 32-bit matrix instructions share the vector unit, at 2.7 clocks an addition in 32 bits, 5.4 one in 64 or a
+// conversion to it, and 32.3 a matrix instruction (measured, any number of waves): 258 clocks of products and 48 of
+// additions per 16 x 16 x 32, where chains of 16 took 86 of additions in either way (four compensated in 32 bits, or two in 64).
 //
-// Operand of the instruction for the chunk's k = 4 s .. 4 s + 3 (s = 0 .. 3): lane l gives row l % 16 at
+// Operand of the instruction for the k = 4 s .. 4 s + 3 of a half (s = 0 .. 7): lane l gives row l % 16 at
 // k = 4 s + l / 16.  Rows lie in LDS as in memory, an odd multiple of 4 floats apart (68 or 36): 16 such rows
 // begin at 16 different multiples of 4 of the 64 banks, so that the 16 rows x 4 neighbours of a read meet no bank twice.
 //
-// Two kernels: `few` streams w for a few rows of x (bound by HBM), `many` tiles both (bound by the matrix and the
-// vector unit, which 32-bit matrix instructions share: 128 clocks of products and 64 of compensated additions per
-// 16 x 16 x 16, so 105 of 157 TFLOP/s at most).  The bits do not depend on which one runs.
+// Two kernels: `few` streams w for a few rows of x (bound by HBM), `many` tiles both (bound by the vector unit, which 32-bit matrix
+// instructions share: 132 of 157 TFLOP/s at most).  The bits do not depend on which one runs.
 #include "common.h"
 #include "gemm_float.h"
 
-#define GF_CHUNK 16
-
-// One compensated addition of a chunk's sum to (acc, lost).
-__device__ __forceinline__ void gf_add(float part, float& acc, float& lost) {
-    const float y = part - lost;
-    const float t = acc + y;
-    lost = (t - acc) - y;
-    acc = t;
+// Instruction s of a half's eight: the next four k of its chain (of 12, 12 and 8).
+__device__ __forceinline__ void gf_chain(float w, float x, int s, f32x4* part) {
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4& p = part[s / 3];
+    p = __builtin_amdgcn_mfma_f32_16x16x4f32(w, x, s % 3 == 0 ? zero : p, 0, 0, 0);
 }
+__device__ __forceinline__ f32x4 gf_half(const f32x4* part) { return (part[0] + part[1]) + part[2]; }
 
 // ------------------------------------------------------------------ few rows of x
-// Block = 16 rows of w x 16 MT rows of x, four waves.  A step is 64 CH k: wave v forms CH chunks of it, the ones
-// from v CH on, of rows of w and x that it fetches itself (AHEAD steps ahead, in registers; a row's piece by
-// neighbouring lanes, every line asked for once) and turns into operands through LDS of its own; the chunks' sums
-// go to LDS, one barrier, and every thread adds the sums of its own output elements in their order, while other
-// waves are already in the next step.  Bound by the stream of w up to 16 rows, by the sums' way through LDS beyond.
-// Measured with weights from HBM, one row of x (gemm_plain_kernel in brackets): 28672 x 4096 98.7 us = 4.8 TB/s (832),
-// 4096 x 14336 53.4 us (2,650), 6144 x 4096 29.4 us (747), 4096 x 4096 21.2 us (739); 16 rows: 111, 72, 33.5, 24 us.
-template <int MT, int CH, int XF, int AHEAD>
+// Block = 16 rows of w x 16 MT rows of x, four waves.  A step is 128 HALVES k: wave v forms HALVES halves of groups of it, the ones
+// from v HALVES on, of rows of w and x that it fetches itself (AHEAD steps ahead, in registers; a row's piece by
+// neighbouring lanes, every line asked for once) and turns into operands through LDS of its own; their sums
+// go to LDS, one barrier, and every thread adds those of its own output elements in their order, while other
+// waves are already in the next step.  Bound by the stream of w and, at 4096 rows of w, by a block's chain of steps (one block to a
+// unit).  Measured with weights from HBM, one row of x (chains of 16, whose sums all went through LDS, in brackets):
+// 28672 x 4096 91 us = 5.2 TB/s (99), 4096 x 14336 46 (53), 6144 x 4096 25.6 (29.4), 4096 x 4096 20.6 (21.2); 16 rows: 100 (111),
+// 59 (72), 30 (33.5), 22 (24).  Three and four steps ahead are up to 10 % slower but at 4096 x 14336 (up to 6 % faster).
+template <int MT, int HALVES, int XF, int AHEAD>
 __global__ __launch_bounds__(256, 2) void gemm_float_few_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                 float* __restrict__ out, int M, int N, int K) {
-    constexpr int STEP = 64 * CH, WK = 16 * CH;      // k per step, and of a wave
+    constexpr int STEP = 128 * HALVES, WK = 32 * HALVES;   // k per step, and of a wave
     constexpr int LD = WK + 4;                       // floats between rows in LDS
     constexpr int LANES = WK / 4, ROWS = 64 / LANES; // a fetch: ROWS rows by LANES lanes each
     constexpr int F = 16 / ROWS;                     // fetches per 16 rows
     __shared__ __attribute__((aligned(16))) float ws[4][16 * LD];
     __shared__ __attribute__((aligned(16))) float xs[4][MT][16 * LD];
-    __shared__ __attribute__((aligned(16))) float sums[2][MT][4 * CH * 256];
+    __shared__ __attribute__((aligned(16))) float sums[2][MT][4 * 256];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int n0 = blockIdx.x * 16, i = lane & 15, g = lane >> 4;
     const int fr = lane / LANES, fk = 4 * (lane % LANES);
-    const int steps = (K + STEP - 1) / STEP, chunks = (K + GF_CHUNK - 1) / GF_CHUNK;
+    const int steps = (K + STEP - 1) / STEP;
     const float* xrow[XF];
     const float* wrow[F];
 #pragma unroll
@@ -65,16 +66,16 @@ __global__ __launch_bounds__(256, 2) void gemm_float_few_kernel(const float* __r
 #pragma unroll
         for (int u = 0; u < XF; ++u) fx[u] = *(const f32x4*)(xrow[u] + k);
     };
-    float acc[MT], lost[MT];
+    double acc[MT];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) acc[t] = lost[t] = 0.f;
+    for (int t = 0; t < MT; ++t) acc[t] = 0.0;
 #pragma unroll
     for (int a = 0; a < AHEAD; ++a) fetch(a, pw[a], px[a]);
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = 0; s0 < steps; s0 += AHEAD) {
 #pragma unroll
         for (int a = 0; a < AHEAD; ++a) {
-            const int step = s0 + a;                 // (one behind the last adds nothing: cnt is 0 or less)
+            const int step = s0 + a;                 // (what lies behind K, a step behind the last too, is zeros: they add nothing)
             const bool in = step * STEP + WK * wave + fk < K;
 #pragma unroll
             for (int u = 0; u < F; ++u) *(f32x4*)&ws[wave][(ROWS * u + fr) * LD + fk] = in ? pw[a][u] : zero;
@@ -82,39 +83,35 @@ __global__ __launch_bounds__(256, 2) void gemm_float_few_kernel(const float* __r
             for (int u = 0; u < XF; ++u) *(f32x4*)&xs[wave][u / F][((ROWS * u + fr) & 15) * LD + fk] = in ? px[a][u] : zero;
             fetch(step + AHEAD, pw[a], px[a]);
             wave_fence();
-            f32x4 part[MT][CH];
+            f32x4 part[HALVES][MT][3];
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
+            for (int s = 0; s < 8; ++s)
 #pragma unroll
-                for (int c = 0; c < CH; ++c) {
-                    const float wv = ws[wave][i * LD + 16 * c + 4 * s + g];
+                for (int h = 0; h < HALVES; ++h) {
+                    const float wv = ws[wave][i * LD + 32 * h + 4 * s + g];
 #pragma unroll
-                    for (int t = 0; t < MT; ++t) {
-                        const float xv = xs[wave][t][i * LD + 16 * c + 4 * s + g];
-                        const f32x4 from = s ? part[t][c] : (f32x4){0.f, 0.f, 0.f, 0.f};
-                        part[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, xv, from, 0, 0, 0);
-                    }
+                    for (int t = 0; t < MT; ++t) gf_chain(wv, xs[wave][t][i * LD + 32 * h + 4 * s + g], s, part[h][t]);
                 }
             wave_fence();
-            float(*to)[4 * CH * 256] = sums[step & 1];
-#pragma unroll
-            for (int t = 0; t < MT; ++t)
-#pragma unroll
-                for (int c = 0; c < CH; ++c) *(f32x4*)&to[t][(CH * wave + c) * 256 + 4 * lane] = part[t][c];
-            __syncthreads();                         // (who writes these sums again has passed the next barrier, behind these reads)
-            const int cnt = min(4 * CH, chunks - step * 4 * CH);
+            float(*to)[4 * 256] = sums[step & 1];
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
-                float v[4 * CH];
+                f32x4 sum = gf_half(part[0][t]);
+                if (HALVES == 2) sum += gf_half(part[HALVES - 1][t]);
+                *(f32x4*)&to[t][wave * 256 + 4 * lane] = sum;
+            }
+            __syncthreads();                         // (who writes these sums again has passed the next barrier, behind these reads)
 #pragma unroll
-                for (int c = 0; c < 4 * CH; ++c) v[c] = to[t][c * 256 + threadIdx.x];
-                if (cnt == 4 * CH) {
+            for (int t = 0; t < MT; ++t) {
+                float v[4];
 #pragma unroll
-                    for (int c = 0; c < 4 * CH; ++c) gf_add(v[c], acc[t], lost[t]);
+                for (int c = 0; c < 4; ++c) v[c] = to[t][c * 256 + threadIdx.x];
+                if (HALVES == 2) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) acc[t] += v[c];
                 } else {
-#pragma unroll
-                    for (int c = 0; c < 4 * CH; ++c)
-                        if (c < cnt) gf_add(v[c], acc[t], lost[t]);
+                    acc[t] += v[0] + v[1];
+                    acc[t] += v[2] + v[3];
                 }
             }
         }
@@ -124,16 +121,16 @@ __global__ __launch_bounds__(256, 2) void gemm_float_few_kernel(const float* __r
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
         const int m = 16 * t + ((threadIdx.x >> 2) & 15);
-        if (m < M && n < N) out[(size_t)m * N + n] = acc[t];
+        if (m < M && n < N) out[(size_t)m * N + n] = (float)acc[t];
     }
 }
 
 // ------------------------------------------------------------------ many rows of x
 // Block = 64 rows of w x 16 TM rows of x, wave v the 16 rows of w from 16 v on against all of x's.  Stages of 32 k in
-// two LDS slots, AHEAD stages asked for (into registers) before the products of this one.  2 TM chains are in flight
-// per wave.  Counters at 28672 x 4096 x 333: matrix unit busy 67 % of the time, vector unit 41 %.  Measured at 333 rows
-// (gemm_plain_kernel in brackets): 28672 x 4096 837 us = 93 TFLOP/s (1,948), 4096 x 14336 538 us (2,624), 6144 x 4096
-// 222 us (736), 4096 x 4096 163 us (691); at 1,000 rows 81 to 100 TFLOP/s.
+// two LDS slots, two stages asked for (into registers) before the products of this one.  3 TM chains are in flight
+// per wave.  Measured at 333 rows (chains of 16 in brackets): 28672 x 4096 745 us = 105 TFLOP/s (837), 4096 x 14336 429 us (538),
+// 6144 x 4096 180 (222), 4096 x 4096 131 (163).  No faster: four stages ahead, the next stage's first operands read and this
+// one's sums added behind the barrier, 32 rows of w to a wave, waves side by side along x.
 #define GF_K 32
 #define GF_LDM 36
 
@@ -141,7 +138,7 @@ template <int TM>
 __global__ __launch_bounds__(256, 2) void gemm_float_many_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                  float* __restrict__ out, int M, int N, int K, int m_tiles, int tiles,
                                                                  int per_die) {
-    constexpr int AHEAD = 2;
+    constexpr int AHEAD = 2;                         // (two stages are a group)
     constexpr int XR = 16 * TM, XF = (XR * 8 + 255) / 256;           // float4 of x per thread and stage
     __shared__ __attribute__((aligned(16))) float ws[2][64 * GF_LDM];
     __shared__ __attribute__((aligned(16))) float xs[2][XR * GF_LDM];
@@ -186,11 +183,13 @@ __global__ __launch_bounds__(256, 2) void gemm_float_many_kernel(const float* __
         for (int u = 0; u < XF; ++u)
             if (XR % 32 == 0 || row + 32 * u < XR) *(f32x4*)&xs[slot][(row + 32 * u) * GF_LDM + kq] = fx[u];
     };
-    f32x4 acc[TM], lost[TM];
+    double acc[TM][4];
+    f32x4 first[TM];                                 // the first half of a group
 #pragma unroll
-    for (int t = 0; t < TM; ++t) acc[t] = lost[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < TM; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[t][r] = 0.0;
     const int stages = (K + GF_K - 1) / GF_K;
-    const int chunks = (K + GF_CHUNK - 1) / GF_CHUNK;
     fetch(0, pw[0], px[0]);
     put(0, 0, pw[0], px[0]);
 #pragma unroll
@@ -199,35 +198,27 @@ __global__ __launch_bounds__(256, 2) void gemm_float_many_kernel(const float* __
     for (int s0 = 0; s0 < stages; s0 += AHEAD) {
 #pragma unroll
         for (int a = 0; a < AHEAD; ++a) {
-            const int st = s0 + a;                   // (one behind the last adds nothing)
-            const int slot = a & 1;
-            f32x4 part[2][TM];
+            const int st = s0 + a;                   // (one behind the last is zeros and adds nothing)
+            const int slot = a;
+            f32x4 part[TM][3];
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
+            for (int s = 0; s < 8; ++s) {
+                const int at = i * GF_LDM + 4 * s + g;
+                const float wv = ws[slot][16 * wave * GF_LDM + at];
 #pragma unroll
-                for (int c = 0; c < 2; ++c) {
-                    const int at = i * GF_LDM + 16 * c + 4 * s + g;
-                    const float wv = ws[slot][16 * wave * GF_LDM + at];
-#pragma unroll
-                    for (int t = 0; t < TM; ++t) {
-                        const f32x4 from = s ? part[c][t] : (f32x4){0.f, 0.f, 0.f, 0.f};
-                        part[c][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, xs[slot][16 * t * GF_LDM + at], from, 0, 0, 0);
-                    }
-                }
+                for (int t = 0; t < TM; ++t) gf_chain(wv, xs[slot][16 * t * GF_LDM + at], s, part[t]);
+            }
             put(slot ^ 1, (st + 1) * GF_K, pw[a], px[a]);
             fetch((st + 1 + AHEAD) * GF_K, pw[a], px[a]);
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                if (2 * st + c >= chunks) break;
+            for (int t = 0; t < TM; ++t) {
+                const f32x4 half = gf_half(part[t]);
+                if (a == 0) {
+                    first[t] = half;
+                } else {
 #pragma unroll
-                for (int t = 0; t < TM; ++t)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        float sum = acc[t][r], l = lost[t][r];
-                        gf_add(part[c][t][r], sum, l);
-                        acc[t][r] = sum;
-                        lost[t][r] = l;
-                    }
+                    for (int r = 0; r < 4; ++r) acc[t][r] += first[t][r] + half[r];
+                }
             }
             __syncthreads();
         }
@@ -238,17 +229,39 @@ __global__ __launch_bounds__(256, 2) void gemm_float_many_kernel(const float* __
         const int m = m0 + 16 * t + i;
         if (m >= M) continue;
         if (n + 3 < N && N % 4 == 0) {
-            *(f32x4*)(out + (size_t)m * N + n) = acc[t];
+            *(f32x4*)(out + (size_t)m * N + n) = (f32x4){(float)acc[t][0], (float)acc[t][1], (float)acc[t][2], (float)acc[t][3]};
         } else {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                if (n + r < N) out[(size_t)m * N + n + r] = acc[t][r];
+                if (n + r < N) out[(size_t)m * N + n + r] = (float)acc[t][r];
         }
     }
 }
 
-// Which of the two kernels takes a product (gemm_float_launch says why).
-static bool gf_few(int M, int N) { return M <= 32 || (M <= 64 && N <= 8192); }
+// Which of the two kernels takes a product: to 16 rows `few`, to 48 where `many` would have too few blocks.  Microseconds, few against
+// many: 32 rows 28672 x 4096 125 / 100, 4096 x 14336 94 / 152, 6144 x 4096 43 / 48, 4096 x 4096 30 / 46; 48 rows 185 / 136, 131 / 154,
+// 57 / 62, 41 / 47; 64 rows 242 / 168, 178 / 156, 75 / 63, 53 / 48.
+static bool gf_few(int M, int N) { return M <= 16 || (M <= 48 && N <= 8192); }
+
+// Tiles of 16 rows of x to a block of `many`: what a stage takes by the blocks that a unit gets, r (fitted to 43 products of 17 to
+// 1,000 rows with 4096 to 32768 rows of w; its picks take 0.03 % more than the best on average, 0.9 % at most; four tiles, measured too, are nowhere more than 2 % faster).  `full` blocks share a
+// unit; to two rounds of those the unit with the most blocks decides.
+static int gf_tiles(int M, int N) {
+    static const struct { float stage, tile; int full; } cost[3] = {{0.193f, 0.153f, 6}, {0.241f, 0.259f, 4}, {0.281f, 0.381f, 3}};
+    int best = 1;
+    float least = 0.f;
+    for (int tm = 1; tm <= 3; ++tm) {
+        const auto& c = cost[tm - 1];
+        const long blocks = (long)ceil_div(M, 16 * tm) * ceil_div(N, 64), units = fl_units();
+        const float r = (float)blocks / units, most = r <= 2 * c.full ? (float)((blocks + units - 1) / units) : r;
+        const float t = c.stage * (r > c.full ? r / c.full : 1.f) + c.tile * most;
+        if (tm == 1 || t < least) {
+            best = tm;
+            least = t;
+        }
+    }
+    return best;
+}
 
 bool gemm_float_takes(const void* x, const void* w, const void* out, int M, int N, int K) {
     // 16-byte pieces of rows; a grid of fewer than 2^31 blocks, and 64 rows within a 32-bit offset
@@ -259,32 +272,25 @@ bool gemm_float_takes(const void* x, const void* w, const void* out, int M, int 
     // gemm_plain_kernel, the same bits.  Microseconds here / there, one row: 32768 x 4 15.0 / 4.3, x 32 14.8 / 6.5, x 64 14.9 / 10.9, x 128
     // 15 / 20; 16384 x 32 1.27 times as long, x 64 0.73; 131072 x 128 1.5 times; 64 rows: 8192 x 32 1.5 times, x 64 0.93, 4096 x 20
     // 0.89; 1,000 rows: 4096 x 16 1.13 times, 1024 x 16 0.95, 4096 x 20 0.96.
-    if (K <= 16) return !gf_few(M, N) && (long)M * N <= (1l << 20);
-    if (!gf_few(M, N)) return true;
+    const bool few = M <= 32 || (M <= 64 && N <= 8192);
+    if (K <= 16) return !few && (long)M * N <= (1l << 20);
+    if (!few) return true;
     return M <= 32 ? 256l * K >= N : N <= 4096 || K >= 64;
 }
 
 void gemm_float_launch(const float* x, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
     const int blocks = ceil_div(N, 16);
-    // rows of x per block: 32, 48 or 64, whichever leaves the fewest empty (the larger of two that leave as many: w is
-    // read by fewer blocks)
-    int best = 4;
-    for (int tm = 3; tm >= 2; --tm)
-        if (ceil_div(M, 16 * tm) * tm < ceil_div(M, 16 * best) * best) best = tm;
-    const int m_tiles = ceil_div(M, 16 * best), tiles = m_tiles * ceil_div(N, 64), per_die = ceil_div(tiles, 8);
-    // 33 to 64 rows of x: a narrow matrix gives `many` too few blocks (N / 64) and goes to `few` (N / 16).  Microseconds at
-    // 33 / 64 rows, few against many: 4096 x 4096 52 / 64 against 131 / 146, 4096 x 14336 172 / 218 against 461 / 507, 6144 x
-    // 4096 97 / 122 against 133 / 148, 28672 x 4096 339 / 424 against 170 / 224.  17 to 32 rows: 28672 x 4096 few 172, many 170.
-#define GF_FEW(MT, CH, XF) gemm_float_few_kernel<MT, CH, XF, 2><<<blocks, 256, 0, stream>>>(x, w, out, M, N, K)
+    const int tm = gf_tiles(M, N);
+    const int m_tiles = ceil_div(M, 16 * tm), tiles = m_tiles * ceil_div(N, 64), per_die = ceil_div(tiles, 8);
+#define GF_FEW(MT, HALVES, XF) gemm_float_few_kernel<MT, HALVES, XF, 2><<<blocks, 256, 0, stream>>>(x, w, out, M, N, K)
 #define GF_MANY(TM) gemm_float_many_kernel<TM><<<8 * per_die, 256, 0, stream>>>(x, w, out, M, N, K, m_tiles, tiles, per_die)
-    if (M <= 4) GF_FEW(1, 4, 1);
-    else if (M <= 16) GF_FEW(1, 4, 4);
-    else if (M <= 32) GF_FEW(2, 2, 4);
-    else if (gf_few(M, N) && M <= 48) GF_FEW(3, 2, 6);
-    else if (gf_few(M, N)) GF_FEW(4, 2, 8);
-    else if (best == 4) GF_MANY(4);
-    else if (best == 3) GF_MANY(3);
-    else GF_MANY(2);
+    if (M <= 4) GF_FEW(1, 2, 1);
+    else if (M <= 16) GF_FEW(1, 2, 4);
+    else if (gf_few(M, N) && M <= 32) GF_FEW(2, 1, 4);
+    else if (gf_few(M, N)) GF_FEW(3, 1, 6);
+    else if (tm == 3) GF_MANY(3);
+    else if (tm == 2) GF_MANY(2);
+    else GF_MANY(1);
 #undef GF_FEW
 #undef GF_MANY
 }

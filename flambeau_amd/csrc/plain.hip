@@ -186,10 +186,10 @@ extern "C" int fl_add_inplace(float* x, const float* delta, long n, hipStream_t 
 FL_RECORDABLE(fl_add_inplace)
 
 // ------------------------------------------------------------------ plain GEMM
-// out[m, n] = sum_k x[m,k] * w[n,k]; 64x64 tile per block, 4x4 per thread, k in steps of 16.
+// out[m, n] = sum_k x[m,k] * w[n,k]; 64x64 tile per block, 4x4 per thread, k in steps of 32.
 // Each output element is summed in a fixed order (rising k): the result of a row does not depend on
-// how many rows the call has.  The 16 products of a step are added in a chain of their own and the
-// steps' sums with a compensated (Kahan) addition, still all in float: over K = 14336 a single
+// how many rows the call has.  A step's products are added in chains of 12, 12 and 8, the chains and the steps of a
+// pair in float and the pairs in double: over K = 14336 a single
 // chain loses about sqrt(K) roundings, which is what showed in the 32-bit path's logits (6.6e-5 at
 // 7B layer sizes against a float64 reference, against a bound of 1e-4).  Floats whose rows are whole 16-byte
 // pieces go to gemm_float.hip, which forms the same sums on the matrix cores; this kernel takes the rest.
@@ -198,31 +198,31 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const TIn* __restrict__
                                                          const TIn* __restrict__ w,
                                                          TOut* __restrict__ out, int M, int N, int K,
                                                          int ldo) {
-    __shared__ float xs[16][68];
-    __shared__ float ws[16][68];
+    __shared__ float xs[32][68];
+    __shared__ float ws[32][68];
     const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
     const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    float acc[4][4], lost[4][4];              // the running sums and what their roundings have lost so far
+    double acc[4][4];
+    float first[4][4];                        // the first half of a group
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) { acc[i][j] = 0.f; lost[i][j] = 0.f; }
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        for (int e = threadIdx.x; e < 1024; e += 256) {
-            const int row = e >> 4, kk = e & 15;
+        for (int j = 0; j < 4; ++j) {
+            acc[i][j] = 0.0;
+            first[i][j] = 0.f;
+        }
+    for (int k0 = 0; k0 < K; k0 += 32) {
+        for (int e = threadIdx.x; e < 2048; e += 256) {
+            const int row = e >> 5, kk = e & 31;
             const int gk = k0 + kk;
             const int gm = m0 + row, gn = n0 + row;
             xs[kk][row] = (gm < M && gk < K) ? to_f32(x[(size_t)gm * K + gk]) : 0.f;
             ws[kk][row] = (gn < N && gk < K) ? to_f32(w[(size_t)gn * K + gk]) : 0.f;
         }
         __syncthreads();
-        float part[4][4];
+        float half[4][4], part[4][4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) part[i][j] = 0.f;
-#pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
+        for (int kk = 0; kk < 32; ++kk) {
             float a[4], b[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) a[i] = xs[kk][ty * 4 + i];
@@ -231,16 +231,20 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const TIn* __restrict__
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) part[i][j] = fmaf(a[i], b[j], part[i][j]);
+                for (int j = 0; j < 4; ++j) {
+                    part[i][j] = fmaf(a[i], b[j], kk % 12 == 0 ? 0.f : part[i][j]);
+                    if (kk == 11) half[i][j] = part[i][j];
+                    if (kk == 23 || kk == 31) half[i][j] += part[i][j];
+                }
         }
+        const bool second = (k0 & 32) != 0, last = k0 + 32 >= K;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const float y = part[i][j] - lost[i][j];
-                const float t = acc[i][j] + y;
-                lost[i][j] = (t - acc[i][j]) - y;
-                acc[i][j] = t;
+                const float sum = first[i][j] + half[i][j];
+                if (second || last) acc[i][j] += sum;
+                first[i][j] = second ? 0.f : half[i][j];
             }
         __syncthreads();
     }
@@ -251,7 +255,7 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const TIn* __restrict__
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int gn = n0 + tx * 4 + j;
-            if (gn < N) out[(size_t)gm * ldo + gn] = from_f32<TOut>(acc[i][j]);
+            if (gn < N) out[(size_t)gm * ldo + gn] = from_f32<TOut>((float)acc[i][j]);
         }
     }
 }

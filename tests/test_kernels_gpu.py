@@ -1242,6 +1242,12 @@ def test_gemm_float_gives_the_plain_kernel_s_bits(M, N, K):
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("M,N,K", [(100, 4100, 68), (130, 6148, 100), (47, 28676, 36), (333, 6148, 132), (500, 4100, 20), (16, 28676, 196), (17, 28676, 60)])
+def test_gemm_float_blocks_of_one_to_three_tiles_give_the_plain_kernel_s_bits(M, N, K):
+    """Sizes at which each number of tiles of x to a block is the cheapest, and where the kernel for few rows ends; K that ends in every kind of chain."""
+    test_gemm_float_gives_the_plain_kernel_s_bits(M, N, K)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 32768, 32), (8, 16384, 20), (16, 131072, 64), (40, 8192, 16), (64, 6144, 32), (1000, 4096, 16)])
 def test_gemm_float_leaves_short_sums_to_the_plain_kernel(M, N, K):
     """Where the blocks' beginnings would take longer than their sums (measured 1.12 to 2.9 times the plain kernel's time):
