@@ -392,198 +392,232 @@ __global__ __launch_bounds__(64 * LT_WAVES) void latent_attention_shared_kernel(
         if (t < 2 * ns) *(f32x4*)(zr + 16 * t + 4 * g) = o[t] * inv;
 }
 
-// The same tiles for latents of 128, 256 or 512 values, eight waves to a block.  No wave holds a whole head: for the
-// scores of a chunk of 64 keys the waves deal out the keys (four runs of 16) and the steps of 32 values (two halves),
-// for the weighted sum the latent's dims, so that every row and every value of a chunk is read from memory by exactly
-// one wave of the block, straight into the registers it multiplies from (the values of a chunk are asked for before its
-// scores are formed, the rows of the next chunk before this one's are weighted).  What the waves share lies in LDS: the
-// folded queries of the tile's 64 (token, head) rows for the whole walk, the halves' scores, and the weights.
+// The same tiles for latents of 128, 256 or 512 values, up to eight units (token, group of 16 heads) to a tile and eight waves to a
+// block: a wave is a unit, with its folded queries and its weighted sums in registers and its weights formed and used in
+// place (a wave behind the tile's units only copies).  Chunks of 32 keys lie in LDS twice, the next one on its way (memory straight to
+// LDS, one barrier per chunk) while this one is read: rows as they are, the pages' transposed copies run by run of 16 keys, 16-byte
+// pieces exchanged so that the reads of an operand meet no bank twice.
 //
-// Softmax: eight neighbouring threads take a row, eight keys each; a row's maximum and sum live in their registers.
-// The base of the exponents follows the maximum lazily, as in the kernel above; where it moved, all waves rescale.
-#define LS_S 68               // floats per row of scores (64 and four, so that rows start in different banks)
-#define LS_P 72               // values per row of weights
-// a barrier that waits for this wave's LDS accesses and not for its loads in flight
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-template <int NKH, int NDT>
-__global__ __launch_bounds__(512, 2) void latent_attention_spread_kernel(
+// Bound by LDS: an operand of a kilobyte serves one matrix instruction, 4,352 clocks per chunk of eight units of 576 and 512 values where
+// the matrix cores take 2,176; a chunk takes about 6,700 (5,450 without its copies, 3,400 the copies alone).  Why not eight waves that
+// deal out the keys, the steps and the dims of 64 rows, as it was: their chunks' 137 KB for half the rows came in 5.6 us.  Microseconds,
+// before and now: 32 heads of 576 and 512 values, 2,048 tokens 320 / 171, 1,024 94 / 73, 512 47 / 37, 512 behind 2,048 183 / 135, 4,096
+// 1,202 / 627; 16 heads of 320 and 256, 2,048 119 / 83, 300 22 / 17.  The asks ahead of an operand's use, three to five, make no
+// difference; the compiler's own order, one at a time, takes 242 where this takes 183.
+template <int KB, int NS>                                           // steps of 64 values of a row as a key, of 32 as a value
+__global__ __launch_bounds__(512, 2) void latent_attention_units_kernel(
     const bf16_t* __restrict__ qa, float* __restrict__ z, const bf16_t* __restrict__ pool,
     const int* __restrict__ positions, const int* __restrict__ tok_seq, const int* __restrict__ block_table,
-    int max_blocks, int H, int K, int R, int page_size, int n_pages, float scale, int window, const int* __restrict__ tiles,
+    int max_blocks, int H, int K, int page_size, int n_pages, float scale, int window, const int* __restrict__ tiles,
     const float* __restrict__ sink) {
-    constexpr int QS = NKH * 64 + 8;
+    constexpr int R = 32 * NS, NK = 2 * KB, CHUNK = 32, AHEAD = 4;
+    constexpr int KEYS = CHUNK * KB * 64, VALUES = R * CHUNK;       // values of a chunk in LDS
+    constexpr int K_COPIES = 4 * KB, V_COPIES = 2 * NS;             // copies of a kilobyte by one wave
+    constexpr int KU = (K_COPIES + 7) / 8, VU = (V_COPIES + 7) / 8;
     extern __shared__ __attribute__((aligned(16))) unsigned char lt_smem[];
-    bf16_t* qs = (bf16_t*)lt_smem;                                  // [64 rows][QS]
-    float* ss = (float*)(qs + 64 * QS);                             // [2 halves][64 rows][LS_S]
-    bf16_t* ps = (bf16_t*)(ss + 2 * 64 * LS_S);                     // [64 rows][LS_P]
-    float* rs = (float*)(ps + 64 * LS_P);                           // [64 rows]: factor of a chunk, at the end 1 / sum
-    int* moved_at = (int*)(rs + 64);                                // the chunk in which some row's base moved last
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int col = lane & 15, g = lane >> 4;
-    const int half = wave >> 2, kt = wave & 3;
     const int tile = gridDim.x - 1 - blockIdx.x;                    // (a prompt's last tokens see the most keys: first)
     const int t_first = tiles[4 * tile], n_tok = tiles[4 * tile + 1], g_first = tiles[4 * tile + 2], n_grp = tiles[4 * tile + 3];
-    const int nk = K >> 5;
+    const int tw = wave / n_grp, gw = wave - tw * n_grp;
+    const bool active = tw < n_tok;
+    const int token = t_first + (active ? tw : 0), h0 = (g_first + gw) * 16;
+    const int p = active ? positions[token] : -1;
     const int p_max = positions[t_first + n_tok - 1];
     const int* table = block_table + (size_t)tok_seq[t_first] * max_blocks;
+    const int lo = window > 0 ? max(0, p - window + 1) : 0;
     const int lo_min = window > 0 ? max(0, positions[t_first] - window + 1) : 0;
     const size_t page_stride = (size_t)page_size * (K + R);
+    const bool head_live = active && h0 + col < H;
 
-    // this thread's row in the softmax (and in filling the queries): unit row / 16 = (token, group of 16 heads)
-    const int row = tid >> 3, kk = tid & 7;
-    const int unit = row >> 4, tw = unit / n_grp, head = (g_first + unit - tw * n_grp) * 16 + (row & 15);
-    const bool live = tw < n_tok && head < H;
-    const int p = live ? positions[t_first + tw] : -1;
-    const int lo = window > 0 ? max(0, p - window + 1) : 0;
+    bf16x8 qreg[NK];
     {
-        const bf16_t* qr = qa + ((size_t)(t_first + (live ? tw : 0)) * H + (live ? head : 0)) * K;
+        const bf16_t* qr = qa + ((size_t)token * H + (head_live ? h0 + col : 0)) * K;
         const bf16x8 zero = {(bf16_t)0.f, (bf16_t)0.f, (bf16_t)0.f, (bf16_t)0.f, (bf16_t)0.f, (bf16_t)0.f, (bf16_t)0.f, (bf16_t)0.f};
-        for (int c = kk; c < NKH * 8; c += 8) {
-            const bool inside = live && 8 * c < K;
-            const bf16x8 v = *(const bf16x8*)(qr + (inside ? 8 * c : 0));
-            *(bf16x8*)(qs + row * QS + 8 * c) = inside ? v : zero;
+#pragma unroll
+        for (int st = 0; st < NK; ++st) {
+            const bool inside = head_live && 32 * st < K;
+            const bf16x8 v = *(const bf16x8*)(qr + (32 * st < K ? 32 * st : 0) + 8 * g);
+            qreg[st] = inside ? v : zero;
         }
-        if (tid == 0) *moved_at = -1;
     }
-    auto page_of = [&](int key) {                                   // (a run beyond the newest token: that token's page, masked below)
-        const int page = table[min(key, p_max & ~15) / page_size];
-        return pool + (size_t)min(max(page, 0), n_pages - 1) * page_stride;
-    };
-    bf16x8 kreg[NKH], vreg[NDT][2];
-    auto load_keys = [&](int t0) {
-        const int key = t0 + 16 * kt;
-        const bf16_t* src = page_of(key) + (size_t)(min(key, p_max & ~15) % page_size + col) * K + 8 * g;
+    // the runs of 16 keys whose copies are sent next, two at a time (behind the newest token's run: that one again, masked below)
+    const int t_begin = lo_min & ~(CHUNK - 1), runs_of_page = page_size / 16, last_run = p_max / 16;
+    int run = min(t_begin / 16, last_run), page_at = run / runs_of_page, in_run = run - page_at * runs_of_page;
+    int page[2], in_page[2];
+    auto next_runs = [&]() {
 #pragma unroll
-        for (int i = 0; i < NKH; ++i) {
-            const int st = half * NKH + i;
-            kreg[i] = *(const bf16x8*)(src + (st < nk ? 32 * st : 0));
-        }
-    };
-    auto load_values = [&](int t0) {
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int run = t0 + 32 * q + 16 * (g >> 1);
-            const bf16_t* src = page_of(run) + (size_t)page_size * K + min(run, p_max & ~15) % page_size + 8 * (g & 1);
-#pragma unroll
-            for (int d = 0; d < NDT; ++d) vreg[d][q] = *(const bf16x8*)(src + (size_t)(16 * (NDT * wave + d) + col) * page_size);
-        }
-    };
-    f32x4 o[NDT][4];                                                // dims 16 (NDT wave + d) + 4 g + r of row 16 u + col
-#pragma unroll
-    for (int d = 0; d < NDT; ++d)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) o[d][u] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;
-    const int t_begin = lo_min & ~(LT_CHUNK - 1);
-    load_keys(t_begin);
-    __syncthreads();                                                // the queries are in place
-    for (int t0 = t_begin; t0 <= p_max; t0 += LT_CHUNK) {
-        load_values(t0);
-        f32x4 sacc[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) sacc[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < NKH; ++i)
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                sacc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kreg[i], *(const bf16x8*)(qs + (16 * u + col) * QS + (half * NKH + i) * 32 + 8 * g), sacc[u], 0, 0, 0);
-        // lane (row col, g): keys 16 kt + 4 g .. + 3
-#pragma unroll
-        for (int u = 0; u < 4; ++u) *(f32x4*)(ss + (half * 64 + 16 * u + col) * LS_S + 16 * kt + 4 * g) = sacc[u];
-        if (t0 + LT_CHUNK <= p_max) load_keys(t0 + LT_CHUNK);
-        lds_barrier();
-        {
-            float sv[8], cmax = -INFINITY;
-#pragma unroll
-            for (int h4 = 0; h4 < 2; ++h4) {
-                const f32x4 a = *(const f32x4*)(ss + row * LS_S + 8 * kk + 4 * h4), b = *(const f32x4*)(ss + (64 + row) * LS_S + 8 * kk + 4 * h4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int key = t0 + 8 * kk + 4 * h4 + e;
-                    sv[4 * h4 + e] = key > p || key < lo ? -INFINITY : (a[e] + b[e]) * scale;
-                    cmax = fmaxf(cmax, sv[4 * h4 + e]);
+        for (int r = 0; r < 2; ++r) {
+            page[r] = min(max(__builtin_amdgcn_readfirstlane(table[page_at]), 0), n_pages - 1);
+            in_page[r] = 16 * in_run;
+            if (run < last_run) {
+                ++run;
+                if (++in_run == runs_of_page) {
+                    in_run = 0;
+                    ++page_at;
                 }
             }
-            cmax = fmaxf(cmax, __shfl_xor(cmax, 1, FL_WAVE));
-            cmax = fmaxf(cmax, __shfl_xor(cmax, 2, FL_WAVE));
-            cmax = fmaxf(cmax, __shfl_xor(cmax, 4, FL_WAVE));
-            const float m_new = cmax > m + 8.0f ? cmax : m;         // minus infinity while the row has seen no key
+        }
+    };
+    auto send = [&](int at) {
+        const auto first = __builtin_amdgcn_make_buffer_rsrc((void*)(pool + (size_t)page[0] * page_stride), 0, (int)(page_stride * 2), 0x00020000);
+        const auto second = __builtin_amdgcn_make_buffer_rsrc((void*)(pool + (size_t)page[1] * page_stride), 0, (int)(page_stride * 2), 0x00020000);
+        unsigned char* ks = lt_smem + at * (KEYS + VALUES) * 2;
+        unsigned char* vs = ks + KEYS * 2;
+        int l = lane;                                               // (where a lane's 16 bytes come from is formed anew each time: no register is left to keep it)
+        asm volatile("" : "+v"(l));
+#pragma unroll
+        for (int u = 0; u < KU; ++u) {
+            const int c = wave + 8 * u;
+            if (K_COPIES % 8 != 0 && c >= K_COPIES) break;
+            const int slot = c % (2 * KB) * 64 + l, row = slot / (8 * KB), piece = slot % (8 * KB) ^ ((row & 3) | (row >> 1 & 4));
+            const unsigned from = 8 * piece < K ? (unsigned)(row * K + 8 * piece) * 2 : 0x80000000u;      // (beyond the range: zeros)
+            if (c < 2 * KB) __builtin_amdgcn_raw_ptr_buffer_load_lds(first, (__attribute__((address_space(3))) void*)(ks + c * 1024), 16, from, in_page[0] * K * 2, 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(second, (__attribute__((address_space(3))) void*)(ks + c * 1024), 16, from, in_page[1] * K * 2, 0, 0);
+        }
+        const unsigned v_from = (unsigned)((l >> 1) * page_size + 8 * ((l & 1) ^ (l >> 3 & 1))) * 2;      // of 32 dims
+#pragma unroll
+        for (int u = 0; u < VU; ++u) {
+            const int c = wave + 8 * u;
+            if (V_COPIES % 8 != 0 && c >= V_COPIES) break;
+            const int from = (page_size * (K + c % NS * 32) + in_page[c / NS]) * 2;
+            if (c < NS) __builtin_amdgcn_raw_ptr_buffer_load_lds(first, (__attribute__((address_space(3))) void*)(vs + c * 1024), 16, v_from, from, 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(second, (__attribute__((address_space(3))) void*)(vs + c * 1024), 16, v_from, from, 0, 0);
+        }
+    };
+    f32x4 o[2 * NS];
+#pragma unroll
+    for (int t = 0; t < 2 * NS; ++t) o[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;                                   // (l: of the keys that this lane weighs)
+    next_runs();
+    send(0);
+    next_runs();
+    int at = 0;
+    const float scale2 = scale * 1.4426950408889634f;               // (scores in powers of two)
+    // a chunk; EDGE: some token of the tile does not see all of it
+    auto chunk = [&](int t0, auto EDGE) {
+        constexpr bool edge = decltype(EDGE)::value;
+        __builtin_amdgcn_s_waitcnt(0x0F70);                         // this wave's copies of the chunk are there ...
+        asm volatile("s_barrier" ::: "memory");                     // ... everyone's, and the other half is read
+        if (t0 + CHUNK <= p_max) {
+            send(at ^ 1);
+            next_runs();
+        }
+        if (active && (!edge || (t0 <= p && t0 + CHUNK - 1 >= lo))) {
+            const bf16_t* ks = (const bf16_t*)(lt_smem + at * (KEYS + VALUES) * 2);
+            const bf16_t* vs = ks + KEYS;
+            // row i of tile a is key 8 (i / 4) + 4 a + i % 4, so that lane (g, head col) gets keys 8 g + 4 a + e in sacc[a][e]
+            int lc = lane;                                          // (as above)
+            asm volatile("" : "+v"(lc));
+            const int c = lc & 15, q = lc >> 4;
+            const bf16_t* row = ks + (8 * (c >> 2) + (c & 3)) * KB * 64;
+            const bf16_t* even = row + (q ^ (c & 7)) * 8;           // its 16 bytes of steps 0, 2, ..., and of 1, 3, ...
+            const bf16_t* odd = row + ((4 + q) ^ (c & 7)) * 8;
+            const bf16_t* dims = vs + ((q >> 1) * R + c) * 16 + ((q & 1) ^ (c >> 2 & 1)) * 8;
+            // the operands of the scores and, behind them, of the sums, in the order of their use, AHEAD of them on their way (left to
+            // itself the compiler, short of registers, asks for one and waits for it)
+            auto operand = [&](auto J) {
+                constexpr int j = decltype(J)::value, t = j - 2 * NK;
+                if constexpr (t < 0) return *(const bf16x8*)((j & 2 ? odd : even) + (j >> 2) * 64 + (j & 1) * 4 * KB * 64);
+                else return *(const bf16x8*)(dims + t * 256);
+            };
+            bf16x8 ring[AHEAD];
+            static_for<AHEAD>([&](auto J) { ring[J] = operand(J); });
+            f32x4 sacc[2];
+#pragma unroll
+            for (int a = 0; a < 2; ++a) sacc[a] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            static_for<2 * NK>([&](auto J) {
+                constexpr int j = decltype(J)::value;
+                sacc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring[j % AHEAD], qreg[j >> 1], sacc[j & 1], 0, 0, 0);
+                ring[j % AHEAD] = operand(std::integral_constant<int, j + AHEAD>{});
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            float cmax = -INFINITY;
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int key = t0 + 8 * q + 4 * a + e;
+                    sacc[a][e] = edge && (key > p || key < lo) ? -INFINITY : sacc[a][e] * scale2;
+                    cmax = fmaxf(cmax, sacc[a][e]);
+                }
+            cmax = fmaxf(cmax, __shfl_xor(cmax, 16, FL_WAVE));
+            cmax = fmaxf(cmax, __shfl_xor(cmax, 32, FL_WAVE));
+            // (the base of the exponents follows the maximum lazily: weights stay below 2^11.5)
+            const float m_new = cmax > m + 11.5f ? cmax : m;
             const float base = m_new == -INFINITY ? 0.f : m_new;
-            const float corr = expf(m - base);
-            bf16x8 w;
-            float lsum = 0.f;
+            if (__any(m_new != m)) {
+                const float corr = __builtin_amdgcn_exp2f(m - base);
+                l *= corr;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                w[e] = (bf16_t)expf(sv[e] - base);
-                lsum += (float)w[e];                                // the sum of the weights as they are multiplied
+                for (int t = 0; t < 2 * NS; ++t) o[t] *= corr;
+                m = m_new;
             }
-            lsum += __shfl_xor(lsum, 1, FL_WAVE);
-            lsum += __shfl_xor(lsum, 2, FL_WAVE);
-            lsum += __shfl_xor(lsum, 4, FL_WAVE);
-            l = l * corr + lsum;
-            *(bf16x8*)(ps + row * LS_P + 8 * kk) = w;
-            if (kk == 0) rs[row] = corr;
-            if (m_new != m) *moved_at = t0;
-            m = m_new;
-        }
-        lds_barrier();
-        if (*moved_at == t0) {
+            bf16x8 pb;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const float corr = rs[16 * u + col];
+            for (int a = 0; a < 2; ++a)
 #pragma unroll
-                for (int d = 0; d < NDT; ++d) o[d][u] *= corr;
+                for (int e = 0; e < 4; ++e) {
+                    pb[4 * a + e] = (bf16_t)__builtin_amdgcn_exp2f(sacc[a][e] - base);
+                    l += (float)pb[4 * a + e];                      // the sum of the weights as they are multiplied
+                }
+            // values of keys that the token does not see are zero, whatever the page holds
+            u32x4 keep = {};
+            if constexpr (edge) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int key = t0 + 8 * q + 2 * e;
+                    keep[e] = (key > p || key < lo ? 0u : 0xffffu) | (key + 1 > p || key + 1 < lo ? 0u : 0xffff0000u);
+                }
             }
+            static_for<2 * NS>([&](auto T) {
+                constexpr int t = decltype(T)::value, j = 2 * NK + t;
+                bf16x8 v = ring[j % AHEAD];
+                if constexpr (edge) v = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, v) & keep);
+                o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pb, o[t], 0, 0, 0);
+                if constexpr (t + AHEAD < 2 * NS) ring[j % AHEAD] = operand(std::integral_constant<int, j + AHEAD>{});
+                __builtin_amdgcn_sched_barrier(0);
+            });
         }
-        const bool edge = t0 + LT_CHUNK - 1 > p_max || t0 < lo_min;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");          // (the reads are done before the barrier lets anyone copy into their place)
+        at ^= 1;
+    };
+    const int p_least = positions[t_first], lo_most = window > 0 ? max(0, p_max - window + 1) : 0;
+    int t0 = t_begin;
+    for (; t0 <= p_max && t0 < lo_most; t0 += CHUNK) chunk(t0, std::true_type{});
+    for (; t0 + CHUNK - 1 <= p_least; t0 += CHUNK) chunk(t0, std::false_type{});
+    for (; t0 <= p_max; t0 += CHUNK) chunk(t0, std::true_type{});
+    if (!head_live) return;
+    l += __shfl_xor(l, 16, FL_WAVE);
+    l += __shfl_xor(l, 32, FL_WAVE);
+    const float inv = sink ? softmax_factor_with_sink(m * 0.6931471805599453f, l, sink[h0 + col]) : l > 0.f ? 1.0f / l : 0.f;
+    float* zr = z + ((size_t)token * H + h0 + col) * R;
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            bf16x8 pb[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) pb[u] = *(const bf16x8*)(ps + (16 * u + col) * LS_P + 32 * q + 8 * g);
-#pragma unroll
-            for (int d = 0; d < NDT; ++d) {
-                bf16x8 v = vreg[d][q];
-                if (edge) v = keep_keys(v, t0 + 32 * q + 8 * g, lo_min, p_max);          // (what no row of the tile sees is zero, whatever the page holds)
-#pragma unroll
-                for (int u = 0; u < 4; ++u) o[d][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pb[u], o[d][u], 0, 0, 0);
-            }
-        }
-    }
-    __syncthreads();
-    if (kk == 0) rs[row] = sink && live ? softmax_factor_with_sink(m, l, sink[head]) : l > 0.f ? 1.0f / l : 0.f;
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int tu = u / n_grp, hu = (g_first + u - tu * n_grp) * 16 + col;
-        if (tu >= n_tok || hu >= H) continue;
-        const float inv = rs[16 * u + col];
-        float* zr = z + ((size_t)(t_first + tu) * H + hu) * R;
-#pragma unroll
-        for (int d = 0; d < NDT; ++d) *(f32x4*)(zr + 16 * (NDT * wave + d) + 4 * g) = o[d][u] * inv;
-    }
+    for (int t = 0; t < 2 * NS; ++t) *(f32x4*)(zr + 16 * t + 4 * g) = o[t] * inv;
 }
 
-template <int NKH, int NDT>
-static int launch_spread(const void* qa, float* z, const void* pool, const int* positions, const int* tok_seq, const int* block_table,
-                         int max_blocks, int H, int K, int R, int page_size, int n_pages, float scale, int window, const int* tiles,
-                         int n_tiles, const float* sink, hipStream_t stream) {
-    constexpr int LDS = 64 * (NKH * 64 + 8) * 2 + 2 * 64 * LS_S * 4 + 64 * LS_P * 2 + 64 * 4 + 16;
+template <int KB, int NS>
+static int launch_units(const void* qa, float* z, const void* pool, const int* positions, const int* tok_seq, const int* block_table,
+                        int max_blocks, int H, int K, int page_size, int n_pages, float scale, int window, const int* tiles, int n_tiles,
+                        const float* sink, hipStream_t stream) {
+    constexpr int LDS = 2 * 32 * (KB * 64 + NS * 32) * 2;
     static bool sized = false;
     if (!sized) {
-        hipError_t e_ = hipFuncSetAttribute((const void*)latent_attention_spread_kernel<NKH, NDT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
-        FL_CHECK(e_ == hipSuccess, "latent_attention_spread: %s", hipGetErrorString(e_));
+        hipError_t e_ = hipFuncSetAttribute((const void*)latent_attention_units_kernel<KB, NS>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        FL_CHECK(e_ == hipSuccess, "latent_attention_units: %s", hipGetErrorString(e_));
         sized = true;
     }
-    latent_attention_spread_kernel<NKH, NDT><<<n_tiles, 512, LDS, stream>>>((const bf16_t*)qa, z, (const bf16_t*)pool, positions, tok_seq, block_table,
-                                                                            max_blocks, H, K, R, page_size, n_pages, scale, window, tiles, sink);
+    latent_attention_units_kernel<KB, NS><<<n_tiles, 512, LDS, stream>>>((const bf16_t*)qa, z, (const bf16_t*)pool, positions, tok_seq, block_table,
+                                                                         max_blocks, H, K, page_size, n_pages, scale, window, tiles, sink);
     return 0;
 }
 
 extern "C" long fl_latent_attention_shared_lds(int K, int R) { return (long)LT_CHUNK * (K + 8) * 2 + (long)R * (LT_CHUNK + 8) * 2; }
 
-// tiles [n_tiles][4] = (first token, tokens, first group of 16 heads, groups): tokens x groups <= 4, the tokens of one request
+// how many units (token, group of 16 heads) a tile of the kernel below may hold (eight: in pages that lie within a 31-bit offset)
+extern "C" int fl_latent_attention_units(int R) { return R == 128 || R == 256 || R == 512 ? 8 : 4; }
+
+// tiles [n_tiles][4] = (first token, tokens, first group of 16 heads, groups): tokens x groups <= fl_latent_attention_units, the tokens of one request
 extern "C" int fl_latent_attention_shared(const void* qa, float* z, const void* pool, const int* positions,
                                           const int* tok_seq, const int* block_table, int max_blocks, int H, int K, int R,
                                           int page_size, int n_pages, float scale, int window, const int* tiles, int n_tiles,
@@ -593,10 +627,10 @@ extern "C" int fl_latent_attention_shared(const void* qa, float* z, const void* 
     FL_CHECK((uintptr_t)qa % 16 == 0 && (uintptr_t)pool % 16 == 0 && (uintptr_t)z % 16 == 0, "latent_attention_shared: operands must be 16-byte aligned");
     FL_CHECK(window >= 0, "latent_attention_shared: negative window");
     if (n_tiles == 0) return 0;
-    if (R == 128 || R == 256 || R == 512) {
-#define FL_LSP(NKH, NDT) launch_spread<NKH, NDT>(qa, z, pool, positions, tok_seq, block_table, max_blocks, H, K, R, page_size, n_pages, scale, window, tiles, n_tiles, sink, stream)
-        const int rc = R == 128 ? (K == R ? FL_LSP(2, 1) : FL_LSP(3, 1)) : R == 256 ? (K == R ? FL_LSP(4, 2) : FL_LSP(5, 2)) : K == R ? FL_LSP(8, 4) : FL_LSP(9, 4);
-#undef FL_LSP
+    if (fl_latent_attention_units(R) == 8 && (long)page_size * (K + R) < (1l << 30)) {
+#define FL_LUN(KB, NS) launch_units<KB, NS>(qa, z, pool, positions, tok_seq, block_table, max_blocks, H, K, page_size, n_pages, scale, window, tiles, n_tiles, sink, stream)
+        const int rc = R == 128 ? (K == R ? FL_LUN(2, 4) : FL_LUN(3, 4)) : R == 256 ? (K == R ? FL_LUN(4, 8) : FL_LUN(5, 8)) : K == R ? FL_LUN(8, 16) : FL_LUN(9, 16);
+#undef FL_LUN
         if (rc != 0) return rc;
         FL_LAUNCH_CHECK();
         return 0;

@@ -198,6 +198,35 @@ SHAPES = [
 ]
 
 
+@pytest.mark.parametrize("H,R,rot,ps", [(20, 128, 32, 16), (5, 128, 64, 32), (32, 256, 64, 16), (64, 256, 0, 32), (70, 512, 64, 16), (16, 512, 32, 64), (130, 512, 0, 16)])
+@pytest.mark.parametrize("window", [0, 40, 131])
+def test_latent_attention_in_tiles_of_eight_units_gives_the_same_bits(H, R, rot, ps, window):
+    """A unit is a wave's own work: neither who shares its keys nor how many do shows, whatever keys behind its token (in the
+    tile's chunks, NaN for the last request's newest token) the others see."""
+    from types import SimpleNamespace
+    from flambeau_amd.kernels import latent_attention as la
+    K, groups, blocks = R + rot, -(-H // 16), -(-400 // ps)
+    seqs = [(0, 150), (300, 7), (63, 1), (122, 70)]
+    g = torch.Generator().manual_seed(H + R)
+    pool = (torch.randn(4 * blocks, ps * (K + R), generator=g) * 0.7).to(torch.bfloat16).to(DEV)
+    table = torch.arange(4 * blocks, dtype=torch.int32, device=DEV).view(4, blocks)
+    last = seqs[3][0] + seqs[3][1] - 1
+    page = pool[int(table[3, last // ps])]
+    page[last % ps * K:(last % ps + 1) * K] = float("nan")
+    page[ps * K:].view(R, ps)[:, last % ps] = float("nan")
+    cache = SimpleNamespace(pool=pool, width=K, value_width=R, page_size=ps, n_pages=4 * blocks)
+    starts = [sum(q for _, q in seqs[:i]) for i in range(4)]
+    batch, n = SimpleNamespace(q_starts=starts, q_lens=[q for _, q in seqs]), sum(q for _, q in seqs)
+    positions = torch.cat([torch.arange(st, st + q) for st, q in seqs]).int().to(DEV)
+    tok_seq = torch.repeat_interleave(torch.arange(4), torch.tensor([q for _, q in seqs])).int().to(DEV)
+    qa = (torch.randn(n, H * K, generator=g) * 0.4).to(torch.bfloat16).to(DEV)
+    got = []
+    for units in (4, 8):
+        tiles = torch.tensor(la.shared_tiles(batch, groups, units), dtype=torch.int32, device=DEV)
+        got.append(la.latent_attention_shared(qa, torch.full((n, H * R), 7.0, device=DEV), cache, positions, tok_seq, table, H, 0.25, window, tiles))
+    assert torch.isfinite(got[0][:-1]).all() and torch.equal(got[0][:-1], got[1][:-1])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,D,Dr,Dv,Rq,R,window,base,dims", SHAPES)
 def test_latent_attention_with_a_rotated_part_alone(dtype, H, D, Dr, Dv, Rq, R, window, base, dims):
