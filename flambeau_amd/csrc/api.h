@@ -423,6 +423,8 @@ int fl_layernorm(const float* x, const float* delta, float* resid_out, const int
 // resid += layernorm(delta); cast (or null) receives the new resid in cast_dtype
 int fl_layernorm_add(const float* delta, const float* w, const float* b, float* resid, void* cast, int cast_dtype,
                      int n, int H, float eps, hipStream_t stream);
+int fl_layernorm_add_parts(const float* part, int splits, const float* w, const float* b, float* resid, void* cast, int cast_dtype,
+                           int n, int H, float eps, hipStream_t stream);
 // out[t] = table[tokens[t]] + pos_table[positions[t]] (both tables in dtype, the sum float)
 int fl_embed_positions(const void* table, const void* pos_table, int dtype, const int* tokens, const int* positions,
                        float* out, int n, int H, int V, int P, hipStream_t stream);

@@ -153,8 +153,9 @@ FL_RECORDABLE(fl_layernorm)
 
 // A row's VPT groups of four values per thread stay in registers; the number of threads follows from the row's length
 // alone, so a row's bits do not depend on what else the step holds.
+// `parts` > 1: delta is the sum of that many matrices, `stride` values apart, added in their order.
 template <int NT, int VPT, typename TC>
-__global__ __launch_bounds__(NT) void layernorm_add_kernel(const float* __restrict__ delta, const float* __restrict__ w,
+__global__ __launch_bounds__(NT) void layernorm_add_kernel(const float* __restrict__ delta, int parts, size_t stride, const float* __restrict__ w,
                                                            const float* __restrict__ b, float* __restrict__ resid,
                                                            TC* __restrict__ cast, int H, float eps) {
     __shared__ float red[2 * (NT / 64)];
@@ -168,6 +169,7 @@ __global__ __launch_bounds__(NT) void layernorm_add_kernel(const float* __restri
         if (i >= H) continue;
         v[k] = *(const f32x4*)(delta + at + i);
         r[k] = *(const f32x4*)(resid + at + i);
+        for (int z = 1; z < parts; ++z) v[k] += *(const f32x4*)(delta + z * stride + at + i);
         s += (v[k][0] + v[k][1]) + (v[k][2] + v[k][3]);
     }
     const float mean = block_sum<NT / 64>(s, red) / (float)H;
@@ -211,21 +213,26 @@ __global__ __launch_bounds__(256) void layernorm_add_any_kernel(const float* __r
     }
 }
 
-extern "C" int fl_layernorm_add(const float* delta, const float* w, const float* b, float* resid, void* cast, int cast_dtype,
+static bool layernorm_add_whole(const float* delta, const float* w, const float* b, const float* resid, const void* cast, int H) {
+    auto aligned = [](const void* p) { return (uintptr_t)p % 16 == 0; };
+    return (H & 3) == 0 && H <= 4 * 1024 * 4 && aligned(delta) && aligned(w) && aligned(b) && aligned(resid) && aligned(cast);
+}
+
+static int layernorm_add_launch(const float* delta, int parts, const float* w, const float* b, float* resid, void* cast, int cast_dtype,
                                 int n, int H, float eps, hipStream_t stream) {
     FL_CHECK(n >= 0 && H > 0 && delta && w && resid, "layernorm_add: bad sizes or a missing tensor");
     if (n == 0) return 0;
-    auto aligned = [](const void* p) { return (uintptr_t)p % 16 == 0; };
-    const bool whole = (H & 3) == 0 && H <= 4 * 1024 * 4 && aligned(delta) && aligned(w) && aligned(b) && aligned(resid) && aligned(cast);
+    const bool whole = layernorm_add_whole(delta, w, b, resid, cast, H);
+    const size_t stride = (size_t)n * H;
     auto run = [&](auto* c) {
         typedef typename std::remove_pointer<decltype(c)>::type T;
         if (!whole) layernorm_add_any_kernel<T><<<n, 256, 0, stream>>>(delta, w, b, resid, c, H, eps);
-        else if (H <= 4 * 64) layernorm_add_kernel<64, 1, T><<<n, 64, 0, stream>>>(delta, w, b, resid, c, H, eps);
-        else if (H <= 4 * 256) layernorm_add_kernel<256, 1, T><<<n, 256, 0, stream>>>(delta, w, b, resid, c, H, eps);
-        else if (H <= 4 * 512) layernorm_add_kernel<512, 1, T><<<n, 512, 0, stream>>>(delta, w, b, resid, c, H, eps);
-        else if (H <= 4 * 1024) layernorm_add_kernel<1024, 1, T><<<n, 1024, 0, stream>>>(delta, w, b, resid, c, H, eps);
-        else if (H <= 8 * 1024) layernorm_add_kernel<1024, 2, T><<<n, 1024, 0, stream>>>(delta, w, b, resid, c, H, eps);
-        else layernorm_add_kernel<1024, 4, T><<<n, 1024, 0, stream>>>(delta, w, b, resid, c, H, eps);
+        else if (H <= 4 * 64) layernorm_add_kernel<64, 1, T><<<n, 64, 0, stream>>>(delta, parts, stride, w, b, resid, c, H, eps);
+        else if (H <= 4 * 256) layernorm_add_kernel<256, 1, T><<<n, 256, 0, stream>>>(delta, parts, stride, w, b, resid, c, H, eps);
+        else if (H <= 4 * 512) layernorm_add_kernel<512, 1, T><<<n, 512, 0, stream>>>(delta, parts, stride, w, b, resid, c, H, eps);
+        else if (H <= 4 * 1024) layernorm_add_kernel<1024, 1, T><<<n, 1024, 0, stream>>>(delta, parts, stride, w, b, resid, c, H, eps);
+        else if (H <= 8 * 1024) layernorm_add_kernel<1024, 2, T><<<n, 1024, 0, stream>>>(delta, parts, stride, w, b, resid, c, H, eps);
+        else layernorm_add_kernel<1024, 4, T><<<n, 1024, 0, stream>>>(delta, parts, stride, w, b, resid, c, H, eps);
     };
     if (!cast || cast_dtype == FL_F32) run((float*)cast);
     else if (cast_dtype == FL_BF16) run((bf16_t*)cast);
@@ -233,7 +240,23 @@ extern "C" int fl_layernorm_add(const float* delta, const float* w, const float*
     FL_LAUNCH_CHECK();
     return 0;
 }
+
+extern "C" int fl_layernorm_add(const float* delta, const float* w, const float* b, float* resid, void* cast, int cast_dtype,
+                                int n, int H, float eps, hipStream_t stream) {
+    return layernorm_add_launch(delta, 1, w, b, resid, cast, cast_dtype, n, H, eps, stream);
+}
 FL_RECORDABLE(fl_layernorm_add)
+
+// the same from a product's K-splits left apart (part[splits][n][H]): 2,048 rows of 4,096, in a model's prompt, half
+// of them in two parts 26 us on average where the kernel above took 23 and one that adds the parts, reading and writing the sum once
+// more, 19
+extern "C" int fl_layernorm_add_parts(const float* part, int splits, const float* w, const float* b, float* resid, void* cast, int cast_dtype,
+                                      int n, int H, float eps, hipStream_t stream) {
+    FL_CHECK(splits >= 1, "layernorm_add_parts: %d parts", splits);
+    FL_CHECK(splits == 1 || layernorm_add_whole(part, w, b, resid, cast, H), "layernorm_add_parts: rows of %d values, or operands that do not begin at 16 bytes", H);
+    return layernorm_add_launch(part, splits, w, b, resid, cast, cast_dtype, n, H, eps, stream);
+}
+FL_RECORDABLE(fl_layernorm_add_parts)
 
 template <typename T>
 __global__ __launch_bounds__(256) void embed_positions_kernel(const T* __restrict__ table, const T* __restrict__ pos_table,

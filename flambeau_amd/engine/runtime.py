@@ -122,6 +122,13 @@ class Runtime:
             return tuned.gemm(x, w, out, rt=self)
         return ops.gemm_plain(x, w.rowmajor, out)
 
+    def gemm_parts(self, x, w):
+        """``x @ w.T`` in parts that a kernel which reads the product once adds itself (``kernels.tuned.gemm_parts``), or ``None``."""
+        if not self.tuned:
+            return None
+        from ..kernels import tuned
+        return tuned.gemm_parts(x, w, self)
+
     def gemm_add_norm(self, x, w, resid, norm_weight, eps: float):
         """``resid += x @ w.T`` with the norm that follows left in factors, where a kernel does both
         (``kernels.tuned.gemm_add_norm``); ``None`` if none does: the caller adds and norms itself."""

@@ -66,6 +66,7 @@ _SIGNATURES = {
     "fl_rotate_scale": [P, I, I, I, P, I, I, F, F, P, P, I, I, I, P],
     "fl_layernorm": [P, P, P, P, P, P, P, I, I, I, F, P],
     "fl_layernorm_add": [P, P, P, P, P, I, I, I, F, P],
+    "fl_layernorm_add_parts": [P, I, P, P, P, P, I, I, I, F, P],
     "fl_embed_positions": [P, P, I, P, P, P, I, I, I, I, P],
     "fl_cast_rows": [P, P, I, L, P],
     "fl_scale_inplace": [P, L, F, P],

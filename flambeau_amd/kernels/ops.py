@@ -805,10 +805,13 @@ def layernorm(x, weight, bias, out, eps, delta=None, store_sum=False, rows=None)
 
 
 def layernorm_add(delta, weight, bias, resid, eps, cast=None):
-    """``resid += layernorm(delta) * weight + bias``; ``cast`` (optional) receives the new ``resid`` in its dtype."""
+    """``resid += layernorm(delta) * weight + bias``; ``cast`` (optional) receives the new ``resid`` in its dtype.  A ``delta``
+    of three dims is a product's K-splits left apart, ``[splits, n, H]``, whose sum is meant."""
     n, H = resid.shape
-    call("fl_layernorm_add", _check(delta, "layernorm_add.delta", torch.float32, (n, H)),
-         _check(weight, "layernorm_add.weight", torch.float32, (H,)),
+    apart = delta.dim() == 3
+    shape = (None, n, H) if apart else (n, H)
+    call("fl_layernorm_add_parts" if apart else "fl_layernorm_add", _check(delta, "layernorm_add.delta", torch.float32, shape),
+         *((delta.shape[0],) if apart else ()), _check(weight, "layernorm_add.weight", torch.float32, (H,)),
          _check(bias, "layernorm_add.bias", torch.float32, (H,)) if bias is not None else None,
          _check(resid, "layernorm_add.resid", torch.float32),
          _check(cast, "layernorm_add.cast", None, (n, H)) if cast is not None else None,

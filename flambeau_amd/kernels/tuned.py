@@ -526,6 +526,22 @@ def gemm(x, w: Weight, out, rt=None):
     return ops.gemm_plain(x, w.rowmajor, out)
 
 
+def gemm_parts(x, w: Weight, rt):
+    """``x @ w.T`` as K-splits left apart, ``[splits, n, H]`` float32, for a kernel that adds them itself, or ``None`` where the
+    product is computed in one part (or by a kernel that leaves none)."""
+    if w.packed is None or w.swiglu_cols or isinstance(x, NormedRows) or x.dtype != torch.bfloat16 or x.shape[1] % 8:
+        return None
+    M, K = x.shape
+    N = w.rows
+    if SKINNY_BEST_ROWS < M <= SKINNY_MAX_ROWS and K % 32 == 0:
+        splits, partials = gemm_mid_splits(M, N, K), gemm_mid_partials
+    elif M > SKINNY_MAX_ROWS:
+        splits, partials = gemm_tiled_splits(M, N, K), gemm_tiled_partials
+    else:
+        return None
+    return partials(x, w.packed, _split_workspace(rt, splits * M * N, x.device), N) if splits > 1 else None
+
+
 def gemm_swiglu(x, w: Weight, out, rt, gate: str = "silu"):
     """``out = act(x Wg^T) * (x Wu^T)``, act = ``gate`` (silu, gelu_tanh or gelu); ``w`` comes from
     ``prepare_gate_up``; ``x`` may be ``NormedRows``."""

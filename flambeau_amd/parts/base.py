@@ -382,6 +382,10 @@ class Norm(Part):
         tensor); ``cast`` (or None) receives the new stream in its own dtype."""
         raise NotImplementedError(f"{type(self).__name__} cannot norm a sublayer's output into the stream")
 
+    def takes_parts(self, resid) -> bool:
+        """Whether ``add_to`` takes a ``delta`` in parts, ``[parts, n, H]`` float32 whose sum is meant."""
+        return False
+
     def after_product(self, rt, resid, product: Product):
         """Optional fusion: add ``product`` to ``resid`` and return the normed sum as an object
         that ``rt.gemm`` and ``rt.gemm_swiglu`` take in place of a tensor, or ``None`` if this

@@ -102,6 +102,9 @@ class LayerNorm(Norm):
     def forward(self, x, out, delta=None, store_sum=False, rows=None):
         return ops.layernorm(x, self.weight, self.bias, out, self.eps, delta=delta, store_sum=store_sum, rows=rows)
 
+    def takes_parts(self, resid):
+        return self.hidden_size % 4 == 0 and self.hidden_size <= 16384        # (rows that its kernel holds, 16 bytes at a time)
+
     def add_to(self, resid, delta, cast=None):
         """``resid += norm(delta)``; ``cast`` (a tensor of the compute dtype, or None) receives the new stream."""
         return ops.layernorm_add(delta, self.weight, self.bias, resid, self.eps, cast=cast)

@@ -139,6 +139,26 @@ def test_a_norm_on_its_way_into_the_stream_alone(W):
         assert torch.equal(outs[0][:3], outs[1])
 
 
+@pytest.mark.parametrize("W,parts", [(40, 2), (516, 1), (4096, 3), (16384, 5)])
+def test_a_norm_of_a_product_in_parts_on_its_way_into_the_stream(W, parts):
+    """The parts' sum in their order, the same bits as the sum first and the norm then; rows that the kernel does not hold are refused."""
+    from flambeau_amd.kernels import ops
+    from flambeau_amd.kernels.library import KernelError
+    g = torch.Generator().manual_seed(W)
+    part, x = dev(torch.randn(parts, 70, W, generator=g)), dev(torch.randn(70, W, generator=g))
+    w, b = dev(1 + 0.3 * torch.randn(W, generator=g)), dev(torch.randn(W, generator=g))
+    total = part[0].clone()
+    for p in part[1:]:
+        total += p
+    whole, apart = x.clone(), x.clone()
+    casts = [torch.empty(70, W, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    ops.layernorm_add(total, w, b, whole, 3e-4, cast=casts[0])
+    ops.layernorm_add(part, w, b, apart, 3e-4, cast=casts[1])
+    assert torch.equal(whole, apart) and torch.equal(*casts)
+    with pytest.raises(KernelError):
+        ops.layernorm_add(dev(torch.randn(2, 3, 37)), dev(torch.ones(37)), None, dev(torch.ones(3, 37)), 3e-4)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n,N,R,tau", [(1, 30, 5, 4.0), (16, 700, 1, 1.0), (17, 513, 64, 16.0), (50, 33, 200, 0.5)])
 def test_a_forget_gate_of_low_rank_alone(dtype, n, N, R, tau):
