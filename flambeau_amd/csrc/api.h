@@ -298,6 +298,8 @@ int fl_attn_prefill_max_pages(int hd);
 int fl_attn_prefill_takes(int hd, int page_size, int max_blocks, int window);
 int fl_attn_prefill_splits(int n_tiles, int nh, int nkv, int hd, int max_keys);
 int fl_attn_prefill_heads(int n_tiles, int nh, int nkv, int hd, int max_keys);      // query heads per wave: the qt_hint to pass
+int fl_attn_prefill_splits_beside(int n_tiles, int nh, int nkv, int hd, int max_keys, int beside);      // the same with that many blocks of single rows in the same launch (fl_attn_both)
+int fl_attn_prefill_heads_beside(int n_tiles, int nh, int nkv, int hd, int max_keys, int beside);
 int fl_attn_prefill_workspace(int n_rows, int nh, int hd, int n_split, long* o_floats, long* ml_floats);
 int fl_attn_decode_workspace(int n_items, int nh, int hd, int n_split, long* o_floats, long* ml_floats);
 
@@ -326,6 +328,11 @@ int fl_attn_prefill_capped(const void* q, void* out, const void* cache_base, con
                            int max_blocks, int nh, int nkv, int hd, int page_size, int n_pages,
                            float scale, int window, float softcap, const float* sink, int qt_hint, float* part_o, float* part_ml,
                            int n_split, hipStream_t stream);
+// Tiles and items of one step in one launch: fl_attn_prefill(_capped) and fl_attn_decode_items(_capped) at once, the same bits.
+int fl_attn_both(const void* q, void* out, const void* cache_base, const int* block_table, int max_blocks, int nh, int nkv, int hd, int page_size,
+                 int n_pages, float scale, int window, float softcap, const float* sink, const int* tiles, int n_tiles, const int* positions, int qt_hint,
+                 float* tile_part_o, float* tile_part_ml, int tile_splits, const int* items, int n_items, float* row_part_o, float* row_part_ml,
+                 const int* firsts, int n_rows, hipStream_t stream);
 
 // ---- rows of the residual stream and of mixers' outputs (stream_ops.hip) ----
 // out = tanh(alpha * (x + delta)) * w + b (Dynamic Tanh); resid_out, rows as for fl_rmsnorm

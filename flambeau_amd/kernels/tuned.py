@@ -41,6 +41,8 @@ register_signatures({
     "fl_attn_prefill": [P, P, P, P, I, P, P, I, I, I, I, I, I, F, I, I, P, P, I, P],
     "fl_attn_prefill_splits": [I, I, I, I, I],
     "fl_attn_prefill_heads": [I, I, I, I, I],
+    "fl_attn_prefill_splits_beside": [I, I, I, I, I, I],
+    "fl_attn_prefill_heads_beside": [I, I, I, I, I, I],
     "fl_attn_prefill_max_pages": [I],
     "fl_attn_prefill_takes": [I, I, I, I],
     "fl_attn_decode": [P, P, P, P, P, P, I, P, I, I, I, I, I, I, F, I, I, P],
@@ -50,6 +52,7 @@ register_signatures({
     "fl_reduce_dyt": [P, P, P, P, P, P, I, I, I, P],
     "fl_attn_decode_items_capped": [P, P, P, P, P, P, I, P, I, I, I, I, I, I, F, I, F, P, P, I, P],
     "fl_attn_prefill_capped": [P, P, P, P, I, P, P, I, I, I, I, I, I, F, I, F, P, I, P, P, I, P],
+    "fl_attn_both": [P, P, P, P, I, I, I, I, I, I, F, I, F, P, P, I, P, I, P, P, I, P, I, P, P, P, I, P],
     "fl_gemm_skinny_clamped": [P, P, P, I, I, I, I, I, F, F, F, P],
     "fl_gemm_mid_clamped": [P, P, P, I, I, I, I, I, F, F, F, P],
     "fl_gemm_tiled_clamped": [P, P, P, I, I, I, I, I, F, F, F, P],
@@ -646,6 +649,8 @@ def attention_metadata(batch, shapes=()) -> dict:
         items, firsts = balanced_items(rows, per_row, window)
         out[f"attn_items/{per_row}/{window}"], out[f"attn_item_rows/{per_row}/{window}"] = items, firsts
         # whether any row is split at all decides if the kernel that merges runs: a part of the step's signature
+        # (blocks of the tiles' launch that are theirs, as far as they count)
+        batch.notes[("attn_row_blocks", per_row, window)] = min(DECODE_UNITS, int(firsts[:, 2].sum()) * per_row)
         batch.notes[("attn_rows_split", per_row, window)] = bool(firsts.shape[0] and int(firsts[:, 2].max()) > 1)
     return out
 
@@ -802,18 +807,18 @@ def attn_decode(q, out, cache, rows, table, n_heads, scale, window, n_split, par
     return out
 
 
-def attn_prefill_splits(n_tiles: int, n_heads: int, n_kv_heads: int, head_dim: int, max_keys: int) -> int:
+def attn_prefill_splits(n_tiles: int, n_heads: int, n_kv_heads: int, head_dim: int, max_keys: int, beside: int = 0) -> int:
     """Into how many parts the tiled kernel wants the keys split for a batch of this shape (1: not
-    at all; more when few tiles face a long context)."""
+    at all; more when few tiles face a long context; fewer with ``beside`` blocks of single rows in the same launch)."""
     from .library import load
-    return load().fl_attn_prefill_splits(n_tiles, n_heads, n_kv_heads, head_dim, max_keys)
+    return load().fl_attn_prefill_splits_beside(n_tiles, n_heads, n_kv_heads, head_dim, max_keys, beside)
 
 
-def attn_prefill_heads(n_tiles: int, n_heads: int, n_kv_heads: int, head_dim: int, max_keys: int) -> int:
+def attn_prefill_heads(n_tiles: int, n_heads: int, n_kv_heads: int, head_dim: int, max_keys: int, beside: int = 0) -> int:
     """Query heads per wave that the tiled kernel wants for a batch of this shape (``heads_per_wave`` of
     ``attn_prefill``; the splits of ``attn_prefill_splits`` go with it)."""
     from .library import load
-    return load().fl_attn_prefill_heads(n_tiles, n_heads, n_kv_heads, head_dim, max_keys)
+    return load().fl_attn_prefill_heads_beside(n_tiles, n_heads, n_kv_heads, head_dim, max_keys, beside)
 
 
 def attn_prefill(q, out, cache, tiles, positions, table, n_heads, scale, window, heads_per_wave: int = 0,
@@ -842,6 +847,31 @@ def attn_prefill(q, out, cache, tiles, positions, table, n_heads, scale, window,
          *((float(softcap), _check(sink, "attn.sink", torch.float32, (n_heads,)) if sink is not None else None) if extras else ()), int(heads_per_wave),
          _check(part_o, "attn.part_o", torch.float32) if part_o is not None else None,
          _check(part_ml, "attn.part_ml", torch.float32) if part_ml is not None else None, int(n_split), stream_handle())
+    return out
+
+
+def attn_both(q, out, cache, tiles, positions, items, table, n_heads, scale, window, heads_per_wave: int = 0, n_split: int = 1, tile_part_o=None,
+              tile_part_ml=None, row_part_o=None, row_part_ml=None, firsts=None, softcap: float = 0.0, sink=None):
+    """``attn_prefill`` of ``tiles`` and ``attn_decode`` of ``items`` (rows with splits of their own) in one launch, their merges in another."""
+    n = q.shape[0]
+    hd = cache.head_dim
+    n_tiles, n_items = tiles.shape[0], items.shape[0]
+    hdp = -(-hd // 32) * 32
+    if n_split > 1 and (tile_part_o is None or tile_part_ml is None):
+        raise KernelError("attn_both: splits of the tiles' keys need a workspace")
+    if firsts is not None:
+        slots = n_items * n_heads
+        if row_part_o is None or row_part_o.numel() < slots * hdp or row_part_ml is None or row_part_ml.numel() < slots * 2:
+            raise KernelError("attn_both: workspace too small for the rows' splits")
+    part = lambda t, name: _check(t, name, torch.float32) if t is not None else None
+    call("fl_attn_both", _check(q, "attn.q", torch.bfloat16, (n, n_heads * hd)), _check(out, "attn.out", torch.bfloat16, (n, n_heads * hd)),
+         _check(cache.pool, "attn.cache", torch.bfloat16), _check(table, "attn.block_table", torch.int32, (None, None)), table.shape[1], n_heads,
+         cache.n_kv_heads, hd, cache.page_size, cache.n_pages, float(scale), int(window), float(softcap),
+         _check(sink, "attn.sink", torch.float32, (n_heads,)) if sink is not None else None,
+         _check(tiles, "attn.tiles", torch.int32, (n_tiles, 4)), n_tiles, _check(positions, "attn.positions", torch.int32, (n,)), int(heads_per_wave),
+         part(tile_part_o, "attn.tile_part_o"), part(tile_part_ml, "attn.tile_part_ml"), int(n_split),
+         _check(items, "attn.rows", torch.int32, (n_items, 4)), n_items, part(row_part_o, "attn.part_o"), part(row_part_ml, "attn.part_ml"),
+         _check(firsts, "attn.firsts", torch.int32, (None, 4)) if firsts is not None else None, firsts.shape[0] if firsts is not None else 0, stream_handle())
     return out
 
 
@@ -877,8 +907,9 @@ def attention_splits(batch, n_heads: int, n_kv_heads: int, head_dim: int, window
     if n_tiles:
         # few tiles before a long context: the keys are split too, so that the chip has blocks enough
         longest = batch.max_ctx_len if not window else min(batch.max_ctx_len, window + PREFILL_TILE)
-        p_split = attn_prefill_splits(n_tiles, n_heads, n_kv_heads, head_dim, longest) \
-            + 64 * attn_prefill_heads(n_tiles, n_heads, n_kv_heads, head_dim, longest)
+        beside = batch.notes.get(("attn_row_blocks", decode_blocks_per_row(n_heads, n_kv_heads), window or 0), 0) if with_items and head_dim <= 128 else 0
+        p_split = attn_prefill_splits(n_tiles, n_heads, n_kv_heads, head_dim, longest, beside) \
+            + 64 * attn_prefill_heads(n_tiles, n_heads, n_kv_heads, head_dim, longest, beside)
     if n_items and not with_items:
         max_ctx = batch.ctx_bound or batch.max_ctx_len
         if window:
@@ -907,13 +938,14 @@ def attention(rt, q, out, cache, step, table, n_heads, scale, window, softcap: f
                                                        with_items=items is not None)
     p_split, n_split = splits
     p_heads, p_split = p_split >> 6, p_split & 63
-    if tiles.shape[0]:
-        p_o = p_ml = None
-        if p_split > 1:
-            n_rows = sum(ql for ql in batch.q_lens if ql > SHORT_PORTION)
-            hdp = -(-cache.head_dim // 32) * 32
-            p_o = rt.buffer("attn_tile_part_o", n_rows * n_heads * p_split, hdp, torch.float32, max_rows=1 << 24)
-            p_ml = rt.buffer("attn_tile_part_ml", n_rows * n_heads * p_split, 2, torch.float32, max_rows=1 << 24)
+    p_o = p_ml = None
+    if tiles.shape[0] and p_split > 1:
+        n_rows = sum(ql for ql in batch.q_lens if ql > SHORT_PORTION)
+        hdp = -(-cache.head_dim // 32) * 32
+        p_o = rt.buffer("attn_tile_part_o", n_rows * n_heads * p_split, hdp, torch.float32, max_rows=1 << 24)
+        p_ml = rt.buffer("attn_tile_part_ml", n_rows * n_heads * p_split, 2, torch.float32, max_rows=1 << 24)
+    both = tiles.shape[0] and rows.shape[0] and items is not None
+    if tiles.shape[0] and not both:
         attn_prefill(q, out, cache, tiles, step.positions, table, n_heads, scale, window, heads_per_wave=p_heads,
                      n_split=p_split, part_o=p_o, part_ml=p_ml, softcap=softcap, sink=sink)
     if rows.shape[0] and items is not None:
@@ -928,7 +960,11 @@ def attention(rt, q, out, cache, step, table, n_heads, scale, window, softcap: f
             slots = items.shape[0] * n_heads
             part_o = rt.buffer("attn_part_o", slots, hdp, torch.float32, max_rows=1 << 24)
             part_ml = rt.buffer("attn_part_ml", slots, 2, torch.float32, max_rows=1 << 24)
-        attn_decode(q, out, cache, items, table, n_heads, scale, window, 0, part_o, part_ml, firsts=firsts, softcap=softcap, sink=sink)
+        if both:
+            attn_both(q, out, cache, tiles, step.positions, items, table, n_heads, scale, window, heads_per_wave=p_heads, n_split=p_split, tile_part_o=p_o,
+                      tile_part_ml=p_ml, row_part_o=part_o, row_part_ml=part_ml, firsts=firsts, softcap=softcap, sink=sink)
+        else:
+            attn_decode(q, out, cache, items, table, n_heads, scale, window, 0, part_o, part_ml, firsts=firsts, softcap=softcap, sink=sink)
     elif rows.shape[0]:
         part_o = part_ml = None
         if n_split > 1:

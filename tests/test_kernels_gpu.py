@@ -1017,6 +1017,51 @@ def test_attn_prefill_against_plain_and_reference(nh, nkv, hd, ps, window, heads
     assert (out.double() - plain.double()).abs().max() < 1.5e-2 * top
 
 
+@pytest.mark.parametrize("nh,nkv,hd,ps,window,heads,n_split,softcap,sinks", [
+    (32, 8, 128, 16, 0, 0, 1, 0.0, False), (32, 8, 128, 16, 300, 2, 3, 0.0, False), (32, 8, 128, 64, 0, 1, 4, 20.0, True), (6, 1, 24, 16, 0, 1, 2, 0.0, True),
+    (8, 2, 64, 8, 0, 4, 1, 0.0, False), (20, 1, 64, 8, 90, 2, 2, 0.0, False), (8, 2, 96, 16, 70, 0, 1, 0.0, False), (5, 5, 32, 16, 24, 1, 5, 0.0, False),
+    (4, 2, 256, 32, 100, 2, 2, 9.0, True)])
+@pytest.mark.parametrize("rows_of", ["many", "one"])
+def test_attn_both_gives_the_bits_of_the_two(nh, nkv, hd, ps, window, heads, n_split, softcap, sinks, rows_of):
+    """Tiles and single rows in one launch (numbers of blocks that are no multiples of eight, rows that are split, rows that are not, unused places):
+    exactly what the two launches give; heads beyond 128 take those."""
+    singles = [(1500, 1), (33, 1), (257, 3), (31, 1)] if rows_of == "many" else [(700, 1)]
+    seqs = [(300, 70)] + singles + [(200, 200), (131, 130)]
+    case = build_attention_case(torch.bfloat16, nh, nkv, hd, ps, seqs, seed=11)
+    n = case["n"]
+    q2 = case["q"].reshape(n, nh * hd)
+    tiles, single, at = [], [], 0
+    for s, (_, ql) in enumerate(seqs):
+        if ql > 8:
+            tiles += [(s, at + off, min(64, ql - off), at + off) for off in range(0, ql, 64)]
+        else:
+            single += range(at, at + ql)
+        at += ql
+    tiles = torch.tensor(tiles, dtype=torch.int32, device=DEV)
+    items, firsts = (torch.tensor(a, device=DEV) for a in tuned().balanced_items(decode_rows(case, single).cpu().numpy(), tuned().decode_blocks_per_row(nh, nkv), window))
+    sink = torch.linspace(-3, 3, nh, device=DEV) if sinks else None
+    args = (nh, 1 / math.sqrt(hd), window)
+    extras = dict(softcap=softcap, sink=sink)
+
+    def run(both, merge):
+        out = torch.full((n, nh * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+        tile_o, tile_ml = split_workspace(n, nh, hd, n_split) if n_split > 1 else (None, None)
+        row_o, row_ml = split_workspace(items.shape[0], nh, hd, 1)
+        its, f = (items, firsts) if merge else (torch.cat([decode_rows(case, single)[:, :3], torch.full((len(single), 1), 256, dtype=torch.int32, device=DEV)], 1), None)
+        if both:
+            tuned().attn_both(q2, out, case["cache"], tiles, case["pos_d"], its, case["table"], *args, heads_per_wave=heads, n_split=n_split, tile_part_o=tile_o,
+                              tile_part_ml=tile_ml, row_part_o=row_o, row_part_ml=row_ml, firsts=f, **extras)
+        else:
+            tuned().attn_prefill(q2, out, case["cache"], tiles, case["pos_d"], case["table"], *args, heads, n_split=n_split, part_o=tile_o, part_ml=tile_ml, **extras)
+            tuned().attn_decode(q2, out, case["cache"], its, case["table"], *args, 0, row_o, row_ml, firsts=f, **extras)
+        return out
+
+    for merge in (True, False):
+        want = run(False, merge)
+        assert not torch.isnan(want).any()
+        assert torch.equal(run(True, merge), want)
+
+
 def test_attn_prefill_refuses_page_sizes_it_cannot_take():
     from flambeau_amd.kernels import KernelError
     for ps in (4, 12):
