@@ -177,6 +177,24 @@ def test_a_forget_gate_of_low_rank_alone(dtype, n, N, R, tau):
     assert np.abs(plain - pf.sigmoid(z - b.double().numpy()) ** (1 / tau)).max() < 1e-5
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n,N,R", [(17, 257, 13), (24, 256, 8), (31, 1, 7), (40, 600, 65)])
+def test_a_forget_gate_of_low_rank_of_many_tokens(dtype, n, N, R):
+    """Numbers of tokens, features and ranks that are no multiples of what the kernel takes at a time.  32-bit sums of R products of values below 6 and 1: off by
+    R 2^-24 of their sizes' sum at most, a tenth of 1e-5 here; without the gate's bias, and with gates at infinity, that are none, and at zero."""
+    from flambeau_amd.kernels import ops
+    g = torch.Generator().manual_seed(n * R)
+    x, w = torch.randn(n, R, generator=g), (torch.randn(N, R, generator=g) / R ** 0.5).to(TORCH[dtype])
+    x[3], x[5, 0], x[6, 0], w[0] = 0.0, float("inf"), float("nan"), 1.0
+    got = ops.lowrank_gate(dev(x), 0, dev(w), dev(w.t()), None, 16.0, torch.empty(n, N, device=DEV)).cpu()
+    few = torch.cat([ops.lowrank_gate(dev(x[a:a + 16]), 0, dev(w), dev(w.t()), None, 16.0, torch.empty(min(16, n - a), N, device=DEV)).cpu() for a in range(0, n, 16)])
+    assert torch.equal(torch.nan_to_num(got, nan=-1.0), torch.nan_to_num(few, nan=-1.0))         # (the kernel of few tokens: the same sums in the same order)
+    z = x.double() @ w.double().t()
+    want = torch.exp(-(torch.clamp(-z, min=0) + torch.log1p(torch.exp(-z.abs()))) / 16.0)
+    there = torch.isfinite(z)
+    assert (got.double() - want)[there].abs().max() < 1e-5 and got[5, 0] == 1.0 and torch.isnan(got[6]).all()
+
+
 # ---------------------------------------------------------------- the recurrent mixers
 def gla_spec(W, H, D, Dv, R, tau, eps):
     from flambeau_amd.parts import PartSpec
