@@ -1,52 +1,54 @@
 // The 32-bit matrix product on the matrix cores: out[m][n] = sum_k x[m][k] w[n][k], floats in, floats out,
 // the same bits as gemm_plain_kernel (plain.hip) gives.
 //
-// What an output element is: its k in rising groups of 64, a group two halves of 32, a half three chains of 12, 12 and 8 fused
-// multiply-adds from zero, (12 + 12) + 8, the halves and the chains added in 32 bits, the groups in rising order in 64; k behind K
-// are zeros.  Its distance from the exact sum, root mean square over normal values, is 8.06e-8 at K 4096 and 8.03e-8 at 14336 (chains of
-// 16 with a compensated addition in 32 bits: 8.10e-8 and 8.17e-8).  A v_mfma_f32_16x16x4_f32 is such a chain of four (rising k, one rounding
-// each: 1 M random results and products below the smallest normal number are bit for bit those of fmaf).  Nothing else
-// about the sum is free: K cannot be split, but groups are independent of one another up to their addition.
+// What an output element is: its k in rising groups of 32, a group three chains of 12, 8 and 12 fused multiply-adds from zero,
+// (12 + 8) + 12 added in 32 bits, the groups in rising order in 64; k behind K are zeros.  A v_mfma_f32_16x16x4_f32 is such a chain
+// of four (rising k, one rounding each: 1 M random results and products below the smallest normal number are bit for bit those of
+// fmaf).  Nothing else about the sum is free: K cannot be split, but groups are independent of one another up to their addition.
+// How far the sums are from the exact ones (2-norm of the difference over 2-norm of the exact sums, x normal, w normal times 0.02), and
+// in brackets chains of 16 with a compensated addition in 32 bits: K 14336 7.55e-8 (8.14e-8), 4096 7.55e-8 (8.14e-8), 100 7.47e-8 (7.98e-8);
+// of absolute values, whose sums grow, K 4096 2.153e-8 (2.154e-8), 1000 2.323e-8 (2.326e-8), 100 3.74e-8 (3.75e-8).  Groups of 64 whose
+// halves were joined in 32 bits were further off than the latter: 2.18e-8, 2.43e-8, 4.44e-8.
 // Additions and 32-bit matrix instructions share the vector unit, at 2.7 clocks an addition in 32 bits, 5.4 one in 64 or a
-// conversion to it, and 32.3 a matrix instruction (measured, any number of waves): 258 clocks of products and 48 of
+// conversion to it, and 32.3 a matrix instruction (measured, any number of waves): 258 clocks of products and 65 of
 // additions per 16 x 16 x 32, where chains of 16 took 86 of additions in either way (four compensated in 32 bits, or two in 64).
 //
-// Operand of the instruction for the k = 4 s .. 4 s + 3 of a half (s = 0 .. 7): lane l gives row l % 16 at
+// Operand of the instruction for the k = 4 s .. 4 s + 3 of a group (s = 0 .. 7): lane l gives row l % 16 at
 // k = 4 s + l / 16.  Rows lie in LDS as in memory, an odd multiple of 4 floats apart (68 or 36): 16 such rows
 // begin at 16 different multiples of 4 of the 64 banks, so that the 16 rows x 4 neighbours of a read meet no bank twice.
 //
 // Two kernels: `few` streams w for a few rows of x (bound by HBM), `many` tiles both (bound by the vector unit, which 32-bit matrix
-// instructions share: 132 of 157 TFLOP/s at most).  The bits do not depend on which one runs.
+// instructions share: 125 of 157 TFLOP/s at most).  The bits do not depend on which one runs.
 #include "common.h"
 #include "gemm_float.h"
 
-// Instruction s of a half's eight: the next four k of its chain (of 12, 12 and 8).
+// Instruction s of a group's eight: the next four k of its chain (of 12, 8 and 12).
 __device__ __forceinline__ void gf_chain(float w, float x, int s, f32x4* part) {
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4& p = part[s / 3];
-    p = __builtin_amdgcn_mfma_f32_16x16x4f32(w, x, s % 3 == 0 ? zero : p, 0, 0, 0);
+    f32x4& p = part[(s >= 3) + (s >= 5)];
+    p = __builtin_amdgcn_mfma_f32_16x16x4f32(w, x, s == 0 || s == 3 || s == 5 ? zero : p, 0, 0, 0);
 }
-__device__ __forceinline__ f32x4 gf_half(const f32x4* part) { return (part[0] + part[1]) + part[2]; }
+__device__ __forceinline__ f32x4 gf_group(const f32x4* part) { return (part[0] + part[1]) + part[2]; }
 
 // ------------------------------------------------------------------ few rows of x
-// Block = 16 rows of w x 16 MT rows of x, four waves.  A step is 128 HALVES k: wave v forms HALVES halves of groups of it, the ones
-// from v HALVES on, of rows of w and x that it fetches itself (AHEAD steps ahead, in registers; a row's piece by
+// Block = 16 rows of w x 16 MT rows of x, four waves.  A step is 128 GROUPS k: wave v forms GROUPS groups of it, the ones
+// from v GROUPS on, of rows of w and x that it fetches itself (AHEAD steps ahead, in registers; a row's piece by
 // neighbouring lanes, every line asked for once) and turns into operands through LDS of its own; their sums
 // go to LDS, one barrier, and every thread adds those of its own output elements in their order, while other
 // waves are already in the next step.  Bound by the stream of w and, at 4096 rows of w, by a block's chain of steps (one block to a
 // unit).  Measured with weights from HBM, one row of x (chains of 16, whose sums all went through LDS, in brackets):
 // 28672 x 4096 91 us = 5.2 TB/s (99), 4096 x 14336 46 (53), 6144 x 4096 25.6 (29.4), 4096 x 4096 20.6 (21.2); 16 rows: 100 (111),
 // 59 (72), 30 (33.5), 22 (24).  Three and four steps ahead are up to 10 % slower but at 4096 x 14336 (up to 6 % faster).
-template <int MT, int HALVES, int XF, int AHEAD>
+template <int MT, int GROUPS, int XF, int AHEAD>
 __global__ __launch_bounds__(256, 2) void gemm_float_few_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                 float* __restrict__ out, int M, int N, int K) {
-    constexpr int STEP = 128 * HALVES, WK = 32 * HALVES;   // k per step, and of a wave
+    constexpr int STEP = 128 * GROUPS, WK = 32 * GROUPS;   // k per step, and of a wave
     constexpr int LD = WK + 4;                       // floats between rows in LDS
     constexpr int LANES = WK / 4, ROWS = 64 / LANES; // a fetch: ROWS rows by LANES lanes each
     constexpr int F = 16 / ROWS;                     // fetches per 16 rows
     __shared__ __attribute__((aligned(16))) float ws[4][16 * LD];
     __shared__ __attribute__((aligned(16))) float xs[4][MT][16 * LD];
-    __shared__ __attribute__((aligned(16))) float sums[2][MT][4 * 256];
+    __shared__ __attribute__((aligned(16))) float sums[2][MT][4 * GROUPS * 256];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int n0 = blockIdx.x * 16, i = lane & 15, g = lane >> 4;
     const int fr = lane / LANES, fk = 4 * (lane % LANES);
@@ -83,36 +85,29 @@ __global__ __launch_bounds__(256, 2) void gemm_float_few_kernel(const float* __r
             for (int u = 0; u < XF; ++u) *(f32x4*)&xs[wave][u / F][((ROWS * u + fr) & 15) * LD + fk] = in ? px[a][u] : zero;
             fetch(step + AHEAD, pw[a], px[a]);
             wave_fence();
-            f32x4 part[HALVES][MT][3];
+            f32x4 part[GROUPS][MT][3];
 #pragma unroll
             for (int s = 0; s < 8; ++s)
 #pragma unroll
-                for (int h = 0; h < HALVES; ++h) {
+                for (int h = 0; h < GROUPS; ++h) {
                     const float wv = ws[wave][i * LD + 32 * h + 4 * s + g];
 #pragma unroll
                     for (int t = 0; t < MT; ++t) gf_chain(wv, xs[wave][t][i * LD + 32 * h + 4 * s + g], s, part[h][t]);
                 }
             wave_fence();
-            float(*to)[4 * 256] = sums[step & 1];
+            float(*to)[4 * GROUPS * 256] = sums[step & 1];
 #pragma unroll
-            for (int t = 0; t < MT; ++t) {
-                f32x4 sum = gf_half(part[0][t]);
-                if (HALVES == 2) sum += gf_half(part[HALVES - 1][t]);
-                *(f32x4*)&to[t][wave * 256 + 4 * lane] = sum;
-            }
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int h = 0; h < GROUPS; ++h) *(f32x4*)&to[t][(GROUPS * wave + h) * 256 + 4 * lane] = gf_group(part[h][t]);
             __syncthreads();                         // (who writes these sums again has passed the next barrier, behind these reads)
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
-                float v[4];
+                float v[4 * GROUPS];
 #pragma unroll
-                for (int c = 0; c < 4; ++c) v[c] = to[t][c * 256 + threadIdx.x];
-                if (HALVES == 2) {
+                for (int c = 0; c < 4 * GROUPS; ++c) v[c] = to[t][c * 256 + threadIdx.x];
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) acc[t] += v[c];
-                } else {
-                    acc[t] += v[0] + v[1];
-                    acc[t] += v[2] + v[3];
-                }
+                for (int c = 0; c < 4 * GROUPS; ++c) acc[t] += v[c];
             }
         }
     }
@@ -128,8 +123,8 @@ __global__ __launch_bounds__(256, 2) void gemm_float_few_kernel(const float* __r
 // ------------------------------------------------------------------ many rows of x
 // Block = 64 rows of w x 16 TM rows of x, wave v the 16 rows of w from 16 v on against all of x's.  Stages of 32 k in
 // two LDS slots, two stages asked for (into registers) before the products of this one.  3 TM chains are in flight
-// per wave.  Measured at 333 rows (chains of 16 in brackets): 28672 x 4096 745 us = 105 TFLOP/s (837), 4096 x 14336 429 us (538),
-// 6144 x 4096 180 (222), 4096 x 4096 131 (163).  No faster: four stages ahead, the next stage's first operands read and this
+// per wave.  Measured at 333 rows (chains of 16 in brackets, and the groups of 64): 28672 x 4096 766 us = 102 TFLOP/s (828, 750),
+// 4096 x 14336 443 us (520, 435), 6144 x 4096 184 (207, 181), 4096 x 4096 136 (153, 131).  No faster: four stages ahead, the next stage's first operands read and this
 // one's sums added behind the barrier, 32 rows of w to a wave, waves side by side along x.
 #define GF_K 32
 #define GF_LDM 36
@@ -138,7 +133,7 @@ template <int TM>
 __global__ __launch_bounds__(256, 2) void gemm_float_many_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                  float* __restrict__ out, int M, int N, int K, int m_tiles, int tiles,
                                                                  int per_die) {
-    constexpr int AHEAD = 2;                         // (two stages are a group)
+    constexpr int AHEAD = 2;
     constexpr int XR = 16 * TM, XF = (XR * 8 + 255) / 256;           // float4 of x per thread and stage
     __shared__ __attribute__((aligned(16))) float ws[2][64 * GF_LDM];
     __shared__ __attribute__((aligned(16))) float xs[2][XR * GF_LDM];
@@ -184,7 +179,6 @@ __global__ __launch_bounds__(256, 2) void gemm_float_many_kernel(const float* __
             if (XR % 32 == 0 || row + 32 * u < XR) *(f32x4*)&xs[slot][(row + 32 * u) * GF_LDM + kq] = fx[u];
     };
     double acc[TM][4];
-    f32x4 first[TM];                                 // the first half of a group
 #pragma unroll
     for (int t = 0; t < TM; ++t)
 #pragma unroll
@@ -212,13 +206,9 @@ __global__ __launch_bounds__(256, 2) void gemm_float_many_kernel(const float* __
             fetch((st + 1 + AHEAD) * GF_K, pw[a], px[a]);
 #pragma unroll
             for (int t = 0; t < TM; ++t) {
-                const f32x4 half = gf_half(part[t]);
-                if (a == 0) {
-                    first[t] = half;
-                } else {
+                const f32x4 sum = gf_group(part[t]);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[t][r] += first[t][r] + half[r];
-                }
+                for (int r = 0; r < 4; ++r) acc[t][r] += sum[r];
             }
             __syncthreads();
         }
@@ -282,7 +272,7 @@ void gemm_float_launch(const float* x, const float* w, float* out, int M, int N,
     const int blocks = ceil_div(N, 16);
     const int tm = gf_tiles(M, N);
     const int m_tiles = ceil_div(M, 16 * tm), tiles = m_tiles * ceil_div(N, 64), per_die = ceil_div(tiles, 8);
-#define GF_FEW(MT, HALVES, XF) gemm_float_few_kernel<MT, HALVES, XF, 2><<<blocks, 256, 0, stream>>>(x, w, out, M, N, K)
+#define GF_FEW(MT, GROUPS, XF) gemm_float_few_kernel<MT, GROUPS, XF, 2><<<blocks, 256, 0, stream>>>(x, w, out, M, N, K)
 #define GF_MANY(TM) gemm_float_many_kernel<TM><<<8 * per_die, 256, 0, stream>>>(x, w, out, M, N, K, m_tiles, tiles, per_die)
     if (M <= 4) GF_FEW(1, 2, 1);
     else if (M <= 16) GF_FEW(1, 2, 4);

@@ -188,11 +188,12 @@ FL_RECORDABLE(fl_add_inplace)
 // ------------------------------------------------------------------ plain GEMM
 // out[m, n] = sum_k x[m,k] * w[n,k]; 64x64 tile per block, 4x4 per thread, k in steps of 32.
 // Each output element is summed in a fixed order (rising k): the result of a row does not depend on
-// how many rows the call has.  A step's products are added in chains of 12, 12 and 8, the chains and the steps of a
-// pair in float and the pairs in double: over K = 14336 a single
+// how many rows the call has.  A step's products are added in chains of 12, 8 and 12, the chains in float and the
+// steps in double (gemm_float.hip says why): over K = 14336 a single
 // chain loses about sqrt(K) roundings, which is what showed in the 32-bit path's logits (6.6e-5 at
 // 7B layer sizes against a float64 reference, against a bound of 1e-4).  Floats whose rows are whole 16-byte
-// pieces go to gemm_float.hip, which forms the same sums on the matrix cores; this kernel takes the rest.
+// pieces go to gemm_float.hip, which forms the same sums on the matrix cores; this kernel takes the rest: 4096 x 4100 in
+// bfloat16 at 1 and 333 rows 543 and 619 us (steps of 16, compensated in 32 bits: 809 and 830), 4096 x 4101 in 32 bits 518 and 617 (764, 757).
 template <typename TIn, typename TOut>
 __global__ __launch_bounds__(256) void gemm_plain_kernel(const TIn* __restrict__ x,
                                                          const TIn* __restrict__ w,
@@ -203,14 +204,10 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const TIn* __restrict__
     const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
     const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
     double acc[4][4];
-    float first[4][4];                        // the first half of a group
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            acc[i][j] = 0.0;
-            first[i][j] = 0.f;
-        }
+        for (int j = 0; j < 4; ++j) acc[i][j] = 0.0;
     for (int k0 = 0; k0 < K; k0 += 32) {
         for (int e = threadIdx.x; e < 2048; e += 256) {
             const int row = e >> 5, kk = e & 31;
@@ -220,7 +217,7 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const TIn* __restrict__
             ws[kk][row] = (gn < N && gk < K) ? to_f32(w[(size_t)gn * K + gk]) : 0.f;
         }
         __syncthreads();
-        float half[4][4], part[4][4];
+        float sum[4][4], part[4][4];
 #pragma unroll
         for (int kk = 0; kk < 32; ++kk) {
             float a[4], b[4];
@@ -232,20 +229,15 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const TIn* __restrict__
             for (int i = 0; i < 4; ++i)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    part[i][j] = fmaf(a[i], b[j], kk % 12 == 0 ? 0.f : part[i][j]);
-                    if (kk == 11) half[i][j] = part[i][j];
-                    if (kk == 23 || kk == 31) half[i][j] += part[i][j];
+                    part[i][j] = fmaf(a[i], b[j], kk == 0 || kk == 12 || kk == 20 ? 0.f : part[i][j]);
+                    if (kk == 11) sum[i][j] = part[i][j];
+                    if (kk == 19 || kk == 31) sum[i][j] += part[i][j];
                 }
         }
-        const bool second = (k0 & 32) != 0, last = k0 + 32 >= K;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float sum = first[i][j] + half[i][j];
-                if (second || last) acc[i][j] += sum;
-                first[i][j] = second ? 0.f : half[i][j];
-            }
+            for (int j = 0; j < 4; ++j) acc[i][j] += sum[i][j];
         __syncthreads();
     }
 #pragma unroll

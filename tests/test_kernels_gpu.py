@@ -1307,6 +1307,29 @@ def test_gemm_float_gives_the_plain_kernel_s_bits(M, N, K):
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("M,N,K", [(4, 4096, 14336), (16, 4096, 4096), (40, 4096, 1000), (333, 4096, 4096), (100, 4096, 14336), (200, 4096, 100)])
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("one_sign", [False, True])
+def test_32_bit_products_are_as_close_to_64_bits_as_chains_of_16_with_a_compensated_addition(M, N, K, offset, one_sign):
+    """Both kernels on the matrix cores and (rows that do not begin at 16 bytes) the plain one.  The bounds are those chains' own distances,
+    2-norm of the difference over 2-norm of the sums: 8.0e-8 at K 100 and 8.1e-8 beyond for normal values; 3.75e-8 at 100, 2.33e-8 at 1000, 2.16e-8 at 4096 and
+    2.42e-8 at 14336 where all products have one sign.  The kernels' are 7.5e-8, and the same within 0.3 % with one sign, which half a percent over the bound leaves room for; groups
+    of 64 joined in 32 bits are 2 to 18 % beyond the latter at K up to 4096, 32-bit accumulators 2 to 4 times beyond the former.  Single values: seven of these deviations, and the last rounding
+    of the largest sums (at most 6 deviations of them, 2^-24 each)."""
+    g = torch.Generator(device=DEV).manual_seed(K + M)
+    def at(rows, scale):
+        view = torch.empty(rows * K + 4, dtype=torch.float32, device=DEV)[offset:offset + rows * K].view(rows, K)
+        view.copy_(torch.randn(rows, K, generator=g, device=DEV) * scale)
+        return view.abs_() if one_sign else view
+    x, w, out = at(M, 1.0), at(N, 0.02), torch.empty(M, N, dtype=torch.float32, device=DEV)
+    ops().gemm_plain(x, w, out)
+    want = x.double() @ w.double().t()
+    off, size = out.double() - want, want.square().mean().sqrt()
+    bound = {100: 3.75e-8, 1000: 2.33e-8, 4096: 2.16e-8, 14336: 2.42e-8}[K] * 1.005 if one_sign else 8.0e-8
+    assert off.square().mean().sqrt() < bound * size
+    assert off.abs().max() < 7 * bound * size + (0.0 if one_sign else 6 * 2 ** -24 * size)
+
+
 @pytest.mark.parametrize("M,N,K", [(100, 4100, 68), (130, 6148, 100), (47, 28676, 36), (333, 6148, 132), (500, 4100, 20), (16, 28676, 196), (17, 28676, 60)])
 def test_gemm_float_blocks_of_one_to_three_tiles_give_the_plain_kernel_s_bits(M, N, K):
     """Sizes at which each number of tiles of x to a block is the cheapest, and where the kernel for few rows ends; K that ends in every kind of chain."""
