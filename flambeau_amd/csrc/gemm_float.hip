@@ -258,14 +258,15 @@ bool gemm_float_takes(const void* x, const void* w, const void* out, int M, int 
     const bool fits = K % 4 == 0 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 == 0 && K < (1 << 24) &&
                       (long)(N / 64 + 1) * (M / 32 + 1) < (1l << 30);
     if (!fits) return false;
-    // A block's beginning and end take as long as some hundred k, so a K that is short beside the number of blocks is left to
-    // gemm_plain_kernel, the same bits.  Microseconds here / there, one row: 32768 x 4 15.0 / 4.3, x 32 14.8 / 6.5, x 64 14.9 / 10.9, x 128
-    // 15 / 20; 16384 x 32 1.27 times as long, x 64 0.73; 131072 x 128 1.5 times; 64 rows: 8192 x 32 1.5 times, x 64 0.93, 4096 x 20
-    // 0.89; 1,000 rows: 4096 x 16 1.13 times, 1024 x 16 0.95, 4096 x 20 0.96.
-    const bool few = M <= 32 || (M <= 64 && N <= 8192);
+    // A block's beginning and end take as long as some ten k, so a K that is short beside the number of blocks is left to
+    // gemm_plain_kernel, the same bits.  Microseconds here / there, for few rows: one row 32768 x 16 12.0 / 3.7, x 64 12.0 / 9.1, x 128 12.4 / 19.8,
+    // 8192 x 32 4.8 / 4.9, 16384 x 32 7.3 / 5.0, x 64 7.4 / 7.8; 40 rows 6144 x 32 6.3 / 5.7, x 48 6.4 / 8.4, 4096 x 20 4.6 / 5.7.  For many: K up to 16 0.7 to 0.95
+    // of the time there to 2^20 results (64 rows 6144 x 16 3.9 / 4.7, 17 of 32768 4.5 / 4.5), 1.03 to 1.25 of it beyond (65 of 16384 5.8 / 5.1, 1,000 of 4096 12.0 /
+    // 10.6); from 20 on 0.5 to 1.0.
+    const bool few = gf_few(M, N);
     if (K <= 16) return !few && (long)M * N <= (1l << 20);
     if (!few) return true;
-    return M <= 32 ? 256l * K >= N : N <= 4096 || K >= 64;
+    return M <= 32 ? 256l * K >= N : N <= 4096 || K > 32;
 }
 
 void gemm_float_launch(const float* x, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
