@@ -382,7 +382,7 @@ class Norm(Part):
         tensor); ``cast`` (or None) receives the new stream in its own dtype."""
         raise NotImplementedError(f"{type(self).__name__} cannot norm a sublayer's output into the stream")
 
-    def takes_parts(self, resid) -> bool:
+    def takes_parts(self) -> bool:
         """Whether ``add_to`` takes a ``delta`` in parts, ``[parts, n, H]`` float32 whose sum is meant."""
         return False
 

@@ -81,7 +81,7 @@ class ResidualStream:
         tensor or a ``Product``.  The kernel leaves the new stream in the compute dtype too, for the sublayer
         that reads it next."""
         resid = self.flush()
-        if type(delta) is Product and norm.takes_parts(resid):
+        if type(delta) is Product and norm.takes_parts():
             parts = self.rt.gemm_parts(delta.x, delta.weight)
             delta = parts if parts is not None else delta
         if isinstance(delta, Product):

@@ -102,8 +102,10 @@ class LayerNorm(Norm):
     def forward(self, x, out, delta=None, store_sum=False, rows=None):
         return ops.layernorm(x, self.weight, self.bias, out, self.eps, delta=delta, store_sum=store_sum, rows=rows)
 
-    def takes_parts(self, resid):
-        return self.hidden_size % 4 == 0 and self.hidden_size <= 16384        # (rows that its kernel holds, 16 bytes at a time)
+    def takes_parts(self):
+        # (rows that its kernel holds, 16 bytes at a time; an ``add_to`` of a subclass's own is handed the sum)
+        return type(self).add_to is LayerNorm.add_to and self.hidden_size % 4 == 0 and self.hidden_size <= 16384 \
+            and all(t is None or t.data_ptr() % 16 == 0 for t in (self.weight, self.bias))
 
     def add_to(self, resid, delta, cast=None):
         """``resid += norm(delta)``; ``cast`` (a tensor of the compute dtype, or None) receives the new stream."""

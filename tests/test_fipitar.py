@@ -204,3 +204,29 @@ def test_the_framework_s_ladder_is_the_plain_one():
         f, m = blended_frequencies(dims, base, *sc)
         want, mag = pf.frequencies(rot(dims, base, sc))
         assert np.allclose(f, want, rtol=1e-14) and np.isclose(m, mag)
+
+
+def test_who_is_handed_a_product_in_parts():
+    """``LayerNorm``'s own kernel adds the parts of a product itself.  A subclass with an ``add_to`` of its own, rows that the kernel does not hold and
+    vectors that do not begin at 16 bytes get the sum, as ever."""
+    from types import SimpleNamespace
+    from flambeau_amd.parts.base import Product
+    from flambeau_amd.parts.block import ResidualStream
+    from flambeau_amd.parts.norm import LayerNorm
+    handed = []
+
+    class Own(LayerNorm):
+        def add_to(self, resid, delta, cast=None):
+            handed.append(tuple(delta.shape))
+
+    rt = SimpleNamespace(dtype=torch.bfloat16, buffer=lambda name, rows, cols, dtype=torch.bfloat16, **_: torch.empty(rows, cols, dtype=dtype),
+                         gemm=lambda x, w, out: out.zero_(), gemm_parts=lambda x, w: torch.zeros(2, x.shape[0], w.rows))
+    norm = Own(64, 1e-5)
+    norm.bind({"weight": torch.ones(64), "bias": torch.zeros(64)}, rt)
+    ResidualStream(torch.zeros(3, 64), rt).add_normed(norm, Product(torch.zeros(3, 8), SimpleNamespace(rows=64)))
+    assert handed == [(3, 64)]
+    off = torch.zeros(72)
+    for width, weight, takes in ((64, torch.ones(64), True), (66, torch.ones(66), False), (16388, torch.ones(16388), False), (64, off[1:65], False)):
+        norm = LayerNorm(width, 1e-5, bias=False)
+        norm.bind({"weight": weight}, rt)
+        assert norm.takes_parts() is takes
