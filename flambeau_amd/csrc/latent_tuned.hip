@@ -398,12 +398,18 @@ __global__ __launch_bounds__(64 * LT_WAVES) void latent_attention_shared_kernel(
 // LDS, one barrier per chunk) while this one is read: rows as they are, the pages' transposed copies run by run of 16 keys, 16-byte
 // pieces exchanged so that the reads of an operand meet no bank twice.
 //
+// A key whose score is the base has a weight of exactly one, and where a few keys have most of the weight, that is most of what rounding the weights to 16
+// bits costs: the base follows the maximum for the first LT_FOLLOW keys.  Distance from 64 bits (2-norms, 32 heads of 576 and 512, 600 tokens, scores of deviation 0.18, 0.7
+// and 2.1): 1.290e-3, 1.220e-3 and 0.89e-3; following it for the first 32 keys alone 1.282e-3, 1.263e-3 and 1.06e-3, for 64 (the kernel before) 1.294e-3, 1.248e-3 and
+// 1.00e-3, for all of them 1.292e-3, 1.206e-3 and 0.71e-3 but 3 to 8 % slower.
+//
 // Bound by LDS: an operand of a kilobyte serves one matrix instruction, 4,352 clocks per chunk of eight units of 576 and 512 values where
 // the matrix cores take 2,176; a chunk takes about 6,700 (5,450 without its copies, 3,400 the copies alone).  Why not eight waves that
 // deal out the keys, the steps and the dims of 64 rows, as it was: their chunks' 137 KB for half the rows came in 5.6 us.  Microseconds,
-// before and now: 32 heads of 576 and 512 values, 2,048 tokens 320 / 171, 1,024 94 / 73, 512 47 / 37, 512 behind 2,048 183 / 135, 4,096
-// 1,202 / 627; 16 heads of 320 and 256, 2,048 119 / 83, 300 22 / 17.  The asks ahead of an operand's use, three to five, make no
+// before and now: 32 heads of 576 and 512 values, 2,048 tokens 329 / 191, 1,024 95 / 78, 512 47 / 38, 512 behind 2,048 183 / 134, 4,096
+// 1,200 / 635; 16 heads of 320 and 256, 2,048 123 / 86, 300 22 / 18.  The asks ahead of an operand's use, three to five, make no
 // difference; the compiler's own order, one at a time, takes 242 where this takes 183.
+#define LT_FOLLOW 128
 template <int KB, int NS>                                           // steps of 64 values of a row as a key, of 32 as a value
 __global__ __launch_bounds__(512, 2) void latent_attention_units_kernel(
     const bf16_t* __restrict__ qa, float* __restrict__ z, const bf16_t* __restrict__ pool,
@@ -543,8 +549,8 @@ __global__ __launch_bounds__(512, 2) void latent_attention_units_kernel(
                 }
             cmax = fmaxf(cmax, __shfl_xor(cmax, 16, FL_WAVE));
             cmax = fmaxf(cmax, __shfl_xor(cmax, 32, FL_WAVE));
-            // (the base of the exponents follows the maximum lazily: weights stay below 2^11.5)
-            const float m_new = cmax > m + 11.5f ? cmax : m;
+            // (the base of the exponents follows the maximum, behind the first LT_FOLLOW keys lazily: weights stay below 2^11.5)
+            const float m_new = cmax > (t0 < t_begin + LT_FOLLOW ? m : m + 11.5f) ? cmax : m;
             const float base = m_new == -INFINITY ? 0.f : m_new;
             if (__any(m_new != m)) {
                 const float corr = __builtin_amdgcn_exp2f(m - base);

@@ -227,6 +227,33 @@ def test_latent_attention_in_tiles_of_eight_units_gives_the_same_bits(H, R, rot,
     assert torch.isfinite(got[0][:-1]).all() and torch.equal(got[0][:-1], got[1][:-1])
 
 
+@pytest.mark.parametrize("H,R,rot,ps,n,window", [(32, 512, 64, 16, 600, 0), (16, 256, 64, 32, 700, 0), (20, 128, 0, 16, 500, 131)])
+@pytest.mark.parametrize("spread,bound", [(1.0, 1.30e-3), (3.0, 1.0e-3)])
+def test_latent_attention_of_prompts_is_as_close_to_64_bits_where_few_keys_have_the_weight(H, R, rot, ps, n, window, spread, bound):
+    """Weights are rounded to 16 bits relative to the base of the exponents, and a key at the base has a weight of exactly one.  The bounds are the distances
+    (2-norms) of a kernel whose base is the maximum of the first 64 keys, 1.25e-3 to 1.32e-3 and 0.97e-3 to 1.03e-3; with the first 128 they are 1.22e-3 to 1.26e-3 and 0.75e-3
+    to 0.93e-3, with the first 32 1.26e-3 to 1.33e-3 and 1.03e-3 to 1.08e-3."""
+    from types import SimpleNamespace
+    from flambeau_amd.kernels import latent_attention as la
+    K, blocks, g = R + rot, -(-n // ps), torch.Generator().manual_seed(H + R)
+    pool = (torch.randn(blocks, ps * (K + R), generator=g) * 0.7).to(torch.bfloat16).to(DEV)
+    table = torch.arange(blocks, dtype=torch.int32, device=DEV).view(1, blocks)
+    cache = SimpleNamespace(pool=pool, width=K, value_width=R, page_size=ps, n_pages=blocks)
+    qa = (torch.randn(n, H * K, generator=g) * spread).to(torch.bfloat16).to(DEV)
+    tiles = torch.tensor(la.shared_tiles(SimpleNamespace(q_starts=[0], q_lens=[n]), -(-H // 16), 8), dtype=torch.int32, device=DEV)
+    z = la.latent_attention_shared(qa, torch.empty(n, H * R, device=DEV), cache, torch.arange(n, dtype=torch.int32, device=DEV),
+                                   torch.zeros(n, dtype=torch.int32, device=DEV), table, H, K ** -0.5, window, tiles)
+    keys = pool[:, :ps * K].reshape(-1, K)[:n].double()
+    values = pool[:, ps * K:].view(blocks, R, ps).transpose(1, 2).reshape(-1, R)[:n].double()
+    i, j = torch.arange(n, device=DEV)[:, None], torch.arange(n, device=DEV)[None, :]
+    off, size = 0.0, 0.0
+    for h in range(0, H, 4):
+        s = (qa.view(n, H, K)[:, h].double() @ keys.t() * K ** -0.5).masked_fill_((j > i) | ((j <= i - window) if window else (j < 0)), -torch.inf)
+        want = torch.softmax(s, -1) @ values
+        off, size = off + (z.view(n, H, R)[:, h] - want).square().sum(), size + want.square().sum()
+    assert (off / size).sqrt() < bound
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,D,Dr,Dv,Rq,R,window,base,dims", SHAPES)
 def test_latent_attention_with_a_rotated_part_alone(dtype, H, D, Dr, Dv, Rq, R, window, base, dims):
