@@ -95,7 +95,7 @@ int fl_latent_attention_shared(const void* qa, float* z, const void* pool, const
                                const int* tok_seq, const int* block_table, int max_blocks, int H, int K, int R,
                                int page_size, int n_pages, float scale, int window, const int* tiles, int n_tiles,
                                const float* sink, hipStream_t stream);
-int fl_latent_attention_units(int R);
+int fl_latent_attention_units(int K, int R, int page_size);
 long fl_latent_attention_shared_lds(int K, int R);
 // and for steps of few rows: a block of four waves per (token, 16 heads, part of the keys) that deal the latent's dims out among them
 int fl_latent_attention_dealt(const void* qa, float* z, const void* pool, const int* positions,

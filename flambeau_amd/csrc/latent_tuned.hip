@@ -621,7 +621,9 @@ static int launch_units(const void* qa, float* z, const void* pool, const int* p
 extern "C" long fl_latent_attention_shared_lds(int K, int R) { return (long)LT_CHUNK * (K + 8) * 2 + (long)R * (LT_CHUNK + 8) * 2; }
 
 // how many units (token, group of 16 heads) a tile of the kernel below may hold (eight: in pages that lie within a 31-bit offset)
-extern "C" int fl_latent_attention_units(int R) { return R == 128 || R == 256 || R == 512 ? 8 : 4; }
+extern "C" int fl_latent_attention_units(int K, int R, int page_size) {
+    return (R == 128 || R == 256 || R == 512) && (long)page_size * (K + R) < (1l << 30) ? 8 : 4;
+}
 
 // tiles [n_tiles][4] = (first token, tokens, first group of 16 heads, groups): tokens x groups <= fl_latent_attention_units, the tokens of one request
 extern "C" int fl_latent_attention_shared(const void* qa, float* z, const void* pool, const int* positions,
@@ -633,7 +635,7 @@ extern "C" int fl_latent_attention_shared(const void* qa, float* z, const void* 
     FL_CHECK((uintptr_t)qa % 16 == 0 && (uintptr_t)pool % 16 == 0 && (uintptr_t)z % 16 == 0, "latent_attention_shared: operands must be 16-byte aligned");
     FL_CHECK(window >= 0, "latent_attention_shared: negative window");
     if (n_tiles == 0) return 0;
-    if (fl_latent_attention_units(R) == 8 && (long)page_size * (K + R) < (1l << 30)) {
+    if (fl_latent_attention_units(K, R, page_size) == 8) {
 #define FL_LUN(KB, NS) launch_units<KB, NS>(qa, z, pool, positions, tok_seq, block_table, max_blocks, H, K, page_size, n_pages, scale, window, tiles, n_tiles, sink, stream)
         const int rc = R == 128 ? (K == R ? FL_LUN(2, 4) : FL_LUN(3, 4)) : R == 256 ? (K == R ? FL_LUN(4, 8) : FL_LUN(5, 8)) : K == R ? FL_LUN(8, 16) : FL_LUN(9, 16);
 #undef FL_LUN

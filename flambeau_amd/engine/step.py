@@ -180,7 +180,7 @@ class ModelRunner:
             rows = list(range(pad_to))          # a fixed-shape step computes every row's logits
         batch = HostBatch(q_starts, q_lens, starts, slots, n + n_pad, len(rows),
                           ctx_bound=self.max_seq_len if pad_to is not None else None,
-                          every_row=rows == list(range(n + n_pad)))
+                          every_row=rows == list(range(n + n_pad)), page_size=mgr.page_size)
         if pad_to is not None:
             width = mgr.max_blocks
         else:

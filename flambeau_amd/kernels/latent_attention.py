@@ -101,7 +101,7 @@ class TunedLatentAttention(PlainLatentAttention):
         lib, units = load(), {}
         for m in mixers:
             g = -(-m.n_heads // 16)
-            units[g] = min(units.get(g, 8), lib.fl_latent_attention_units(m.value_width))
+            units[g] = min(units.get(g, 8), lib.fl_latent_attention_units(m.row_width, m.value_width, batch.page_size))
         return {f"latent_tiles_{g}": prompt_tiles(batch, g, units[g], lib.fl_compute_units()) for g in sorted(units)}
 
     def prepare(self, uk, uv, n_heads):
@@ -125,7 +125,7 @@ class TunedLatentAttention(PlainLatentAttention):
         tiles = step.extra.get(f"latent_tiles_{-(-H // 16)}") if on_cores else None
         n_split = key_splits(step.host, H, window)
         few = bool(window) and n * -(-H // 16) <= DEALT_UNITS
-        if on_cores and tiles is not None and n_split == 1 and not few and cache.page_size * (cache.width + R) < 1 << 30:
+        if on_cores and tiles is not None and n_split == 1 and not few:
             # a step of many rows (prompt portions): the waves of a block share every chunk of keys through LDS
             latent_attention_shared(qa, z, cache, step.positions, step.tok_seq, table, H, scale, window, tiles, sink=sink)
         elif on_cores:

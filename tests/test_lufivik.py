@@ -194,3 +194,21 @@ def test_key_parts_follow_the_window():
     from flambeau_amd.parts import HostBatch
     one = HostBatch([0], [1], [4000], [0], 1, 0)
     assert key_splits(one, 32) == 32 and key_splits(one, 32, 1024) == 16 and key_splits(one, 32, 40) == 1 and key_splits(one, 32, 1 << 20) == 32
+
+
+def test_a_tile_holds_the_units_that_its_kernel_has():
+    """Eight units share their keys where latent and page are such that the kernel of eight takes them; the kernel of four would leave the others out."""
+    from types import SimpleNamespace
+    from flambeau_amd.kernels.latent_attention import TunedLatentAttention
+    from flambeau_amd.kernels.library import load
+    from flambeau_amd.parts import HostBatch
+    units = load().fl_latent_attention_units
+    assert [units(K, R, 16) for K, R in ((576, 512), (512, 512), (320, 256), (128, 128), (96, 96), (448, 384))] == [8, 8, 8, 8, 4, 4]
+    assert units(576, 512, 1 << 19) == 8 and units(576, 512, 1 << 20) == 4 and units(128, 128, 1 << 21) == 8 and units(128, 128, 1 << 22) == 4
+    for page_size, most in ((16, 8), (1 << 20, 4)):
+        batch = HostBatch([0], [4096], [0], [0], 4096, 1, page_size=page_size)
+        mixers = [SimpleNamespace(n_heads=32, row_width=576, value_width=512), SimpleNamespace(n_heads=70, row_width=576, value_width=512)]
+        lists = TunedLatentAttention(None).metadata(batch, mixers)
+        assert sorted(lists) == ["latent_tiles_2", "latent_tiles_5"]
+        for groups, tiles in ((2, lists["latent_tiles_2"]), (5, lists["latent_tiles_5"])):
+            assert (tiles[:, 1] * tiles[:, 3]).max() == min(most, most // groups * groups or most) and (tiles[:, 1] * tiles[:, 3]).sum() == 4096 * groups

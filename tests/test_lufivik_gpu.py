@@ -227,6 +227,24 @@ def test_latent_attention_in_tiles_of_eight_units_gives_the_same_bits(H, R, rot,
     assert torch.isfinite(got[0][:-1]).all() and torch.equal(got[0][:-1], got[1][:-1])
 
 
+def test_latent_attention_of_prompts_in_pages_beyond_a_31_bit_offset():
+    """A page of 2^20 rows of 576 and 512 values: tiles of four units, whose kernel has 64-bit offsets, against the kernel that shares nothing."""
+    from types import SimpleNamespace
+    from flambeau_amd.kernels import latent_attention as la
+    from flambeau_amd.kernels.library import load
+    H, R, K, ps, n = 40, 512, 576, 1 << 20, 37
+    assert load().fl_latent_attention_units(K, R, ps) == 4
+    pool = torch.empty(1, ps * (K + R), dtype=torch.bfloat16, device=DEV).normal_()
+    cache = SimpleNamespace(pool=pool, width=K, value_width=R, page_size=ps, n_pages=1)
+    table, seq = torch.zeros(1, 1, dtype=torch.int32, device=DEV), torch.zeros(n, dtype=torch.int32, device=DEV)
+    positions = torch.arange(ps - n, ps, dtype=torch.int32, device=DEV)
+    qa = (torch.randn(n, H * K, generator=torch.Generator().manual_seed(1)) * 0.5).to(torch.bfloat16).to(DEV)
+    tiles = torch.tensor(la.shared_tiles(SimpleNamespace(q_starts=[0], q_lens=[n]), 3, 4), dtype=torch.int32, device=DEV)
+    got = la.latent_attention_shared(qa, torch.full((n, H * R), float("nan"), device=DEV), cache, positions, seq, table, H, K ** -0.5, 200, tiles)
+    want = la.latent_attention_mfma(qa, torch.empty(n, H * R, device=DEV), cache, positions, seq, table, H, K ** -0.5, 200, dealt=True)
+    assert (got - want).abs().max() < 2e-2 * want.abs().max()            # (weights in 16 bits, from bases that differ)
+
+
 @pytest.mark.parametrize("H,R,rot,ps,n,window", [(32, 512, 64, 16, 600, 0), (16, 256, 64, 32, 700, 0), (20, 128, 0, 16, 500, 131)])
 @pytest.mark.parametrize("spread,bound", [(1.0, 1.30e-3), (3.0, 1.0e-3)])
 def test_latent_attention_of_prompts_is_as_close_to_64_bits_where_few_keys_have_the_weight(H, R, rot, ps, n, window, spread, bound):
