@@ -6,8 +6,9 @@
 // blocks as there are units, in proportion to their numbers (a unit's first and second block are that far apart; changed every 8 blocks, units got two of
 // one kind: 47 us, every 256 blocks 45, every 512 49).  The tiles' keys are then split over fewer blocks (pf_plan), which leaves less to merge.
 // What bounds it: the lines in flight, which the tiles' keys and values share: of 512 tokens behind up to 1,536 beside 16 rows of 500 to 4,096 keys the
-// kernels of their own take 24 + 27 us and 9 + 6 of merges, these 42 + 10.  Steps of 7B layers, apart and in one: 2 rows of 500 and 512 tokens 2 % less,
-// 4 rows beside 128 6 %, 32 rows of 1,000 to 8,000 beside 256 3 %, 32 of 2,000 to 8,000 beside 1,024 4 %.
+// kernels of their own take 24 + 27 us and 9 + 6 of merges, these 42 + 10.  A layer's attention apart and in one: 64 tokens behind 2,000 beside one row of 1,500
+// 42 / 34 us, 128 behind 4,000 beside 16 of 1,000 53 / 40, 512 behind 1,536 beside 16 of 2,000 67 / 49, 1,024 behind 2,000 beside 32 of 4,000 158 / 113, a prompt of
+// 2,048 beside one row of 300 72 / 66 (whose tiles run longest first here: in the order of attn_prefill.hip, mirrored, 69, beside more rows up to 30 % slower), of 1,280 59 / 45.
 //
 // Both are the code of the kernels of their own, so results are the same bits.
 #include "common.h"
@@ -88,7 +89,9 @@ static void launch_both(const PrefillLaunch& l, hipStream_t stream, const bf16_t
 }
 
 // fl_attn_prefill(_capped) of the tiles and fl_attn_decode_items(_capped) of the items (splits of their own) at once; tile_* are the workspaces, parts and heads of the
-// former, row_* and firsts those of the latter.  Heads beyond 128 run one behind the other: there a unit has one block of either.
+// former, row_* and firsts those of the latter.  Heads beyond 128 run one behind the other: there a unit has one block of either.  So do tables that
+// leave a unit one block, where the tiles fill the chip by themselves (6,000 pages, a prompt of 2,048 tokens beside one row of 1,500 keys 81 us joined, 79 apart, beside 16
+// of 2,000 94 and 97; with fewer blocks or parts of the keys joined is the faster one there too: 512 tokens 31 and 35).
 extern "C" int fl_attn_both(const void* q, void* out, const void* cache_base, const int* block_table, int max_blocks, int nh, int nkv, int hd, int page_size,
                             int n_pages, float scale, int window, float softcap, const float* sink, const int* tiles, int n_tiles, const int* positions, int qt_hint,
                             float* tile_part_o, float* tile_part_ml, int tile_splits, const int* items, int n_items, float* row_part_o, float* row_part_ml,
@@ -102,8 +105,10 @@ extern "C" int fl_attn_both(const void* q, void* out, const void* cache_base, co
     const int q_tiles = ceil_div(nh / nkv, 16), per_item = nkv * q_tiles;
     const int row_rows = firsts ? n_rows : 0;
     const long long merges = (tile_splits > 1 ? (long long)n_tiles * l.merge_blocks_per_tile : 0) + (long long)row_rows * nh;
-    const bool in_range = (long long)l.grid.x * l.grid.y * l.grid.z + (long long)n_items * per_item < (1ll << 23) && merges < (1ll << 23);        // (a grid has 2^32 threads)
-    if (l.hdp > 128 || n_tiles == 0 || n_items == 0 || !in_range) {
+    const long long tile_blocks_all = (long long)l.grid.x * l.grid.y * l.grid.z;
+    const bool in_range = tile_blocks_all + (long long)n_items * per_item < (1ll << 23) && merges < (1ll << 23);        // (a grid has 2^32 threads)
+    const bool one_place = 2 * (2 * 256 * l.hdp + l.lds_pages * (long long)sizeof(int)) > PF_LDS_BYTES;        // (a table of more than 4,096 pages with heads of 128)
+    if (l.hdp > 128 || n_tiles == 0 || n_items == 0 || !in_range || (one_place && tile_splits == 1 && tile_blocks_all > fl_units())) {
         const int rc = fl_attn_prefill_capped(q, out, cache_base, tiles, n_tiles, positions, block_table, max_blocks, nh, nkv, hd, page_size, n_pages, scale, window,
                                               softcap, sink, qt_hint, tile_part_o, tile_part_ml, tile_splits, stream);
         if (rc) return rc;

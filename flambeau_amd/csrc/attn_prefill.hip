@@ -86,8 +86,9 @@ static void launch_prefill(int qt, dim3 grid, hipStream_t stream, const bf16_t* 
 //    with one head and 2; behind 32,256: 314 against 422; 64 tokens behind 32,704: 83 against 115).
 //  * Where the keys are too few for that (a whole prompt of 1,024 tokens: 16 stages at most), fewer heads
 //    per wave give the blocks (29 us with one head, 35 with two).
-//  * Blocks of single rows that run beside (fl_attn_both) take up to one of a unit's two places: the grid then is as many blocks fewer (512
-//    tokens behind up to 1,536 beside 16 rows of 500 to 4,096 keys: 57 us with 4 parts of the keys, 51 with 2, merges and all; 1: 55).
+//  * Blocks of single rows that run beside (fl_attn_both) may have one of a unit's two places (beside = units): the grid then is as many
+//    blocks fewer (512 tokens behind up to 1,536 beside 16 rows of 500 to 4,096 keys: 57 us with 4 parts of the keys, 51 with 2, merges
+//    and all; 1: 55).  When they have is the caller's rule: beside few rows' keys half a grid is the slower one.
 struct PrefillPlan { int qt, splits; };
 static PrefillPlan pf_plan(int n_tiles, int nh, int nkv, int hd, int max_keys, int beside) {
     const int G = nh / nkv;

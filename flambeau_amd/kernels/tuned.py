@@ -649,8 +649,6 @@ def attention_metadata(batch, shapes=()) -> dict:
         items, firsts = balanced_items(rows, per_row, window)
         out[f"attn_items/{per_row}/{window}"], out[f"attn_item_rows/{per_row}/{window}"] = items, firsts
         # whether any row is split at all decides if the kernel that merges runs: a part of the step's signature
-        # (blocks of the tiles' launch that are theirs, as far as they count)
-        batch.notes[("attn_row_blocks", per_row, window)] = min(DECODE_UNITS, int(firsts[:, 2].sum()) * per_row)
         batch.notes[("attn_rows_split", per_row, window)] = bool(firsts.shape[0] and int(firsts[:, 2].max()) > 1)
     return out
 
@@ -894,22 +892,50 @@ def prefill_supported(cache, table, window: int = 0) -> bool:
         load().fl_attn_prefill_takes(cache.head_dim, cache.page_size, table.shape[1], int(window or 0)))
 
 
+# When the tiles of a step's prompt portions and its single rows share a launch (``attn_both``), and whether the tiles are then laid out for both of a unit's two
+# places or for one.  A row counts its keys and ROW_KEYS more, once per kv head; a tile its own keys once per query head (measured with four of these to one of
+# those).  32 query and 8 kv heads, 843 steps of 1 to 64 rows of 100 to 8,000 keys beside 9 to 2,048 tokens behind up to 8,000; us by the rows' part of the tiles' work, tiles for one
+# place / for both / the two launches apart:
+#   0.6   512 tokens behind 5,000 beside 16 rows of 1,000   93 / 82 / 87       0.5   1,024 behind 2,000 beside 8 of 2,000   93 / 82 / 90
+#   1.2   the same beside 24 of 2,000                       98 / 112 / 109     1.1   the same beside 24 of 2,000            96 / 112 / 111
+#   3 to 50   one place the faster by up to 30 %            110   256 beside 64 of 1,500   86 / 86 / 82        113   128 beside 17 of 200 to 5,400   6 less than apart
+# Between 0.7 and 1.1 either is within 6 us.  For fewer rows than tiles one place was up to 27 % slower than both and up to 20 % slower than apart.  Rows that
+# keep every unit at its keys for 80 us (3,400 of a head) beside a twentieth of that work lose 2 to 6 % by the tiles' blocks among theirs.  With these lines the steps took
+# 0.66 to 1.03 of the time apart, 0.87 on average.
+ROW_KEYS = 256
+ROWS_TAKE_A_PLACE = 7 / 8
+ROWS_APART, ROWS_APART_KEYS = 20.0, 3400
+
+
+def tiles_beside_rows(rows: int, tiles: int, n_heads: int, n_kv_heads: int):
+    """Whether a step's single rows go into the launch of its tiles, and the blocks of theirs that the tiles leave room for (``rows``, ``tiles``: what they count)."""
+    part = 4.0 * rows * n_kv_heads / (tiles * n_heads)
+    joined = part > 0.0 and not (part > ROWS_APART and rows * n_kv_heads >= ROWS_APART_KEYS * DECODE_UNITS)
+    return joined, DECODE_UNITS if joined and part >= ROWS_TAKE_A_PLACE else 0
+
+
 def attention_splits(batch, n_heads: int, n_kv_heads: int, head_dim: int, window: int, with_items: bool = True):
-    """``(parts of the keys for the tiled kernel + 64 x its query heads per wave, parts for the single-row
-    kernel)`` for a batch: everything that ``attention`` decides from the contexts' lengths (the rest
+    """``(parts of the keys for the tiled kernel + 64 x its query heads per wave + 512 where the single rows are in its launch, parts for the
+    single-row kernel)`` for a batch: everything that ``attention`` decides from the contexts' lengths (the rest
     follows from the batch's shape).
     ``with_items``: the single rows come with splits of their own (``balanced_items``), which are
     data of the step; all they decide here is whether any row is split at all (0 if so: the kernel
     that merges runs; -1 if not: it is left out)."""
-    n_tiles = sum(-(-ql // PREFILL_TILE) for ql in batch.q_lens if ql > SHORT_PORTION)
-    n_items = sum(ql for ql in batch.q_lens if ql <= SHORT_PORTION)
+    long = [(ql, p0 + ql) for ql, p0 in zip(batch.q_lens, batch.start_pos) if ql > SHORT_PORTION]
+    n_tiles = sum([-(-ql // PREFILL_TILE) for ql, _ in long])
+    n_items = sum(batch.q_lens) - sum([ql for ql, _ in long])
     p_split = n_split = 1
     if n_tiles:
         # few tiles before a long context: the keys are split too, so that the chip has blocks enough
         longest = batch.max_ctx_len if not window else min(batch.max_ctx_len, window + PREFILL_TILE)
-        beside = batch.notes.get(("attn_row_blocks", decode_blocks_per_row(n_heads, n_kv_heads), window or 0), 0) if with_items and head_dim <= 128 else 0
+        joined, beside = False, 0
+        if n_items and with_items and head_dim <= 128:
+            most = window or longest
+            rows = sum([ql * (p0 + ql if p0 + ql < most else most) for ql, p0 in zip(batch.q_lens, batch.start_pos) if ql <= SHORT_PORTION]) + ROW_KEYS * n_items
+            tiles = sum([-(-ql // PREFILL_TILE) * min(end, most + PREFILL_TILE) for ql, end in long])
+            joined, beside = tiles_beside_rows(rows, tiles, n_heads, n_kv_heads)
         p_split = attn_prefill_splits(n_tiles, n_heads, n_kv_heads, head_dim, longest, beside) \
-            + 64 * attn_prefill_heads(n_tiles, n_heads, n_kv_heads, head_dim, longest, beside)
+            + 64 * attn_prefill_heads(n_tiles, n_heads, n_kv_heads, head_dim, longest, beside) + 512 * joined
     if n_items and not with_items:
         max_ctx = batch.ctx_bound or batch.max_ctx_len
         if window:
@@ -937,15 +963,14 @@ def attention(rt, q, out, cache, step, table, n_heads, scale, window, softcap: f
         splits = step.scratch[key] = attention_splits(batch, n_heads, cache.n_kv_heads, cache.head_dim, window,
                                                        with_items=items is not None)
     p_split, n_split = splits
-    p_heads, p_split = p_split >> 6, p_split & 63
+    joined, p_heads, p_split = p_split >> 9, p_split >> 6 & 7, p_split & 63
     p_o = p_ml = None
     if tiles.shape[0] and p_split > 1:
         n_rows = sum(ql for ql in batch.q_lens if ql > SHORT_PORTION)
         hdp = -(-cache.head_dim // 32) * 32
         p_o = rt.buffer("attn_tile_part_o", n_rows * n_heads * p_split, hdp, torch.float32, max_rows=1 << 24)
         p_ml = rt.buffer("attn_tile_part_ml", n_rows * n_heads * p_split, 2, torch.float32, max_rows=1 << 24)
-    both = tiles.shape[0] and rows.shape[0] and items is not None
-    if tiles.shape[0] and not both:
+    if tiles.shape[0] and not joined:
         attn_prefill(q, out, cache, tiles, step.positions, table, n_heads, scale, window, heads_per_wave=p_heads,
                      n_split=p_split, part_o=p_o, part_ml=p_ml, softcap=softcap, sink=sink)
     if rows.shape[0] and items is not None:
@@ -960,7 +985,7 @@ def attention(rt, q, out, cache, step, table, n_heads, scale, window, softcap: f
             slots = items.shape[0] * n_heads
             part_o = rt.buffer("attn_part_o", slots, hdp, torch.float32, max_rows=1 << 24)
             part_ml = rt.buffer("attn_part_ml", slots, 2, torch.float32, max_rows=1 << 24)
-        if both:
+        if joined:
             attn_both(q, out, cache, tiles, step.positions, items, table, n_heads, scale, window, heads_per_wave=p_heads, n_split=p_split, tile_part_o=p_o,
                       tile_part_ml=p_ml, row_part_o=part_o, row_part_ml=part_ml, firsts=firsts, softcap=softcap, sink=sink)
         else:

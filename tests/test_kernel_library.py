@@ -189,3 +189,29 @@ def test_the_rotating_product_keeps_its_values_in_registers():
     assert len(kernels) == 24, sorted(kernels)                            # (twelve shapes, K a multiple of 64 or not)
     assert all(v[".vgpr_spill_count"] == 0 and v[".private_segment_fixed_size"] == 0 for v in kernels.values()), \
         {k: v[".vgpr_spill_count"] for k, v in kernels.items()}
+
+
+def test_tiles_beside_single_rows_are_laid_out_for_half_the_chip_where_the_rows_have_as_much_work():
+    """Few rows' keys leave the plan of the tiles as it is without them; rows with as many keys as the tiles take one of a unit's two places; rows that
+    keep all units busy for long beside a twentieth of their work run apart.  The rows' contexts decide nothing else: while they grow, the plan changes once."""
+    from flambeau_amd.parts import HostBatch
+
+    def splits(portion, behind, rows, keys, window=0, heads=(32, 8, 128)):
+        lens, starts = [1] * rows + [portion], [keys - 1] * rows + [behind]
+        batch = HostBatch([sum(lens[:i]) for i in range(len(lens))], lens, starts, [0] * len(lens), sum(lens), 0)
+        tuned.attention_metadata(batch, [(tuned.decode_blocks_per_row(*heads[:2]), window)])
+        code = tuned.attention_splits(batch, *heads, window)[0]
+        return code & 63, code >> 6 & 7, code >> 9                 # parts, heads, joined
+    alone = lambda tokens, keys: (tuned.attn_prefill_splits(-(-tokens // 64), 32, 8, 128, keys), tuned.attn_prefill_heads(-(-tokens // 64), 32, 8, 128, keys))
+    for rows, keys in ((1, 300), (1, 4000), (4, 600), (4, 4000), (8, 300), (16, 200), (16, 2000)):
+        assert splits(512, 7680, rows, keys) == (*alone(512, 8192), 1) == (4, 2, 1)
+        assert splits(1024, 3000, rows, keys)[:2] == alone(1024, 4024)
+    assert splits(512, 1536, 16, 2000) == (2, 2, 1) and alone(512, 2048) == (2, 1)
+    assert splits(1024, 2000, 32, 4000) == (1, 2, 1) and splits(512, 5000, 24, 2000) == (2, 2, 1)
+    assert splits(256, 0, 64, 1500) == (*alone(256, 1500), 0) and splits(256, 0, 16, 4000)[2] == splits(128, 0, 17, 1500)[2] == splits(512, 1536, 64, 1500)[2] == 1
+    assert splits(512, 0, 0, 1) == (*alone(512, 512), 0) and splits(512, 0, 4, 600, heads=(4, 2, 256))[2] == 0
+    # a window bounds what both see
+    assert splits(512, 30000, 16, 30000, window=1000) == splits(512, 1000, 16, 1000, window=1000)
+    for rows in (1, 2, 3, 16):
+        seen = [splits(512, 1536, rows, keys) for keys in range(2, 2049)]
+        assert sum(a != b for a, b in zip(seen, seen[1:])) <= 1

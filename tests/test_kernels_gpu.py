@@ -1082,6 +1082,33 @@ def test_attn_both_gives_the_bits_of_the_two(nh, nkv, hd, ps, window, heads, n_s
         assert torch.equal(run(True, merge), want)
 
 
+@pytest.mark.parametrize("heads,n_split", [(2, 1), (2, 2), (1, 1)])
+def test_attn_both_with_tables_that_leave_a_unit_one_block(heads, n_split):
+    """6,000 pages: tiles that fill the chip by themselves, whole (the two launches) or in parts (one)."""
+    nh, nkv, hd, ps, window = 32, 8, 128, 16, 0
+    seqs = [(1100, 1100), (900, 1), (40, 1)]
+    case = build_attention_case(torch.bfloat16, nh, nkv, hd, ps, seqs, seed=12)
+    n, q2 = case["n"], case["q"].reshape(case["n"], nh * hd)
+    table = torch.full((3, 6000), -1, dtype=torch.int32, device=DEV)
+    table[:, :case["table"].shape[1]] = case["table"]
+    tiles = torch.tensor([(0, off, min(64, 1100 - off), off) for off in range(0, 1100, 64)], dtype=torch.int32, device=DEV)
+    items, firsts = (torch.tensor(a, device=DEV) for a in tuned().balanced_items(decode_rows(case, [1100, 1101]).cpu().numpy(), tuned().decode_blocks_per_row(nh, nkv), window))
+    outs = []
+    for both, t in ((True, table), (False, table), (True, case["table"])):
+        out = torch.full((n, nh * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+        tile_o, tile_ml = split_workspace(n, nh, hd, n_split) if n_split > 1 else (None, None)
+        row_o, row_ml = split_workspace(items.shape[0], nh, hd, 1)
+        rest = (nh, 1 / math.sqrt(hd), window)
+        if both:
+            tuned().attn_both(q2, out, case["cache"], tiles, case["pos_d"], items, t, *rest, heads_per_wave=heads, n_split=n_split, tile_part_o=tile_o, tile_part_ml=tile_ml,
+                              row_part_o=row_o, row_part_ml=row_ml, firsts=firsts)
+        else:
+            tuned().attn_prefill(q2, out, case["cache"], tiles, case["pos_d"], t, *rest, heads, n_split=n_split, part_o=tile_o, part_ml=tile_ml)
+            tuned().attn_decode(q2, out, case["cache"], items, t, *rest, 0, row_o, row_ml, firsts=firsts)
+        outs.append(out)
+    assert not torch.isnan(outs[0]).any() and torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 def test_attn_prefill_refuses_page_sizes_it_cannot_take():
     from flambeau_amd.kernels import KernelError
     for ps in (4, 12):
