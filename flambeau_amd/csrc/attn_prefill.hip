@@ -125,16 +125,14 @@ static int pf_heads_per_wave(int n_tiles, int nh, int nkv, int hd, int qt_hint, 
 
 // Query heads per wave for a batch of this shape (what fl_attn_prefill takes as its hint), and into how
 // many parts its keys are split (1: not at all); `beside`: blocks of single rows in the same launch (fl_attn_both).
-extern "C" int fl_attn_prefill_heads_beside(int n_tiles, int nh, int nkv, int hd, int max_keys, int beside) {
+extern "C" int fl_attn_prefill_heads(int n_tiles, int nh, int nkv, int hd, int max_keys, int beside) {
     if (n_tiles <= 0 || nh <= 0 || nkv <= 0 || nh % nkv) return 1;
     return pf_plan(n_tiles, nh, nkv, hd, max_keys, beside).qt;
 }
-extern "C" int fl_attn_prefill_splits_beside(int n_tiles, int nh, int nkv, int hd, int max_keys, int beside) {
+extern "C" int fl_attn_prefill_splits(int n_tiles, int nh, int nkv, int hd, int max_keys, int beside) {
     if (n_tiles <= 0 || nh <= 0 || nkv <= 0 || nh % nkv) return 1;
     return pf_plan(n_tiles, nh, nkv, hd, max_keys, beside).splits;
 }
-extern "C" int fl_attn_prefill_heads(int n_tiles, int nh, int nkv, int hd, int max_keys) { return fl_attn_prefill_heads_beside(n_tiles, nh, nkv, hd, max_keys, 0); }
-extern "C" int fl_attn_prefill_splits(int n_tiles, int nh, int nkv, int hd, int max_keys) { return fl_attn_prefill_splits_beside(n_tiles, nh, nkv, hd, max_keys, 0); }
 
 // Block-table entries per request that the kernel takes at a head size: the table of a request sits in
 // LDS beside the ring of two stages of 64 keys and values (256 bytes per padded head dim and stage).

@@ -39,10 +39,8 @@ register_signatures({
     "fl_gemm_tiled_splits": [I, I, I],
     "fl_gemm_tiled_shape": [I, I, I, I],
     "fl_attn_prefill": [P, P, P, P, I, P, P, I, I, I, I, I, I, F, I, I, P, P, I, P],
-    "fl_attn_prefill_splits": [I, I, I, I, I],
-    "fl_attn_prefill_heads": [I, I, I, I, I],
-    "fl_attn_prefill_splits_beside": [I, I, I, I, I, I],
-    "fl_attn_prefill_heads_beside": [I, I, I, I, I, I],
+    "fl_attn_prefill_splits": [I, I, I, I, I, I],
+    "fl_attn_prefill_heads": [I, I, I, I, I, I],
     "fl_attn_prefill_max_pages": [I],
     "fl_attn_prefill_takes": [I, I, I, I],
     "fl_attn_decode": [P, P, P, P, P, P, I, P, I, I, I, I, I, I, F, I, I, P],
@@ -809,14 +807,14 @@ def attn_prefill_splits(n_tiles: int, n_heads: int, n_kv_heads: int, head_dim: i
     """Into how many parts the tiled kernel wants the keys split for a batch of this shape (1: not
     at all; more when few tiles face a long context; fewer with ``beside`` blocks of single rows in the same launch)."""
     from .library import load
-    return load().fl_attn_prefill_splits_beside(n_tiles, n_heads, n_kv_heads, head_dim, max_keys, beside)
+    return load().fl_attn_prefill_splits(n_tiles, n_heads, n_kv_heads, head_dim, max_keys, beside)
 
 
 def attn_prefill_heads(n_tiles: int, n_heads: int, n_kv_heads: int, head_dim: int, max_keys: int, beside: int = 0) -> int:
     """Query heads per wave that the tiled kernel wants for a batch of this shape (``heads_per_wave`` of
     ``attn_prefill``; the splits of ``attn_prefill_splits`` go with it)."""
     from .library import load
-    return load().fl_attn_prefill_heads_beside(n_tiles, n_heads, n_kv_heads, head_dim, max_keys, beside)
+    return load().fl_attn_prefill_heads(n_tiles, n_heads, n_kv_heads, head_dim, max_keys, beside)
 
 
 def attn_prefill(q, out, cache, tiles, positions, table, n_heads, scale, window, heads_per_wave: int = 0,
