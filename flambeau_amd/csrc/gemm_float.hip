@@ -229,12 +229,13 @@ __global__ __launch_bounds__(256, 2) void gemm_float_many_kernel(const float* __
 }
 
 // Which of the two kernels takes a product: to 16 rows `few`, to 48 where `many` would have too few blocks.  Microseconds, few against
-// many: 32 rows 28672 x 4096 125 / 100, 4096 x 14336 94 / 152, 6144 x 4096 43 / 48, 4096 x 4096 30 / 46; 48 rows 185 / 136, 131 / 154,
-// 57 / 62, 41 / 47; 64 rows 242 / 168, 178 / 156, 75 / 63, 53 / 48.
+// many: 17 rows 28672 x 4096 125 / 109, 32 rows 28672 x 4096 128 / 102, 4096 x 14336 92 / 153, 6144 x 4096 43 / 46, 4096 x 4096 30 / 46; 48 rows 190 / 138,
+// 127 / 153, 59 / 61, 40 / 46.
 static bool gf_few(int M, int N) { return M <= 16 || (M <= 48 && N <= 8192); }
 
-// Tiles of 16 rows of x to a block of `many`: what a stage takes by the blocks that a unit gets, r (fitted to 43 products of 17 to
-// 1,000 rows with 4096 to 32768 rows of w; its picks take 0.03 % more than the best on average, 0.9 % at most; four tiles, measured too, are nowhere more than 2 % faster).  `full` blocks share a
+// Tiles of 16 rows of x to a block of `many`: what a stage takes by the blocks that a unit gets, r.  Fitted to 43 products of 17 to
+// 1,000 rows with 4096 to 32768 rows of w; of 108 with 2048 to 32768 none takes more than 2 % longer than with the best number (100 and 128 rows of
+// 4096 x 4096, 63 us with one tile and 62 with two).  Four tiles were nowhere more than 2 % faster.  `full` blocks share a
 // unit; to two rounds of those the unit with the most blocks decides.
 static int gf_tiles(int M, int N) {
     static const struct { float stage, tile; int full; } cost[3] = {{0.193f, 0.153f, 6}, {0.241f, 0.259f, 4}, {0.281f, 0.381f, 3}};

@@ -353,8 +353,8 @@ extern "C" int fl_moe_identity(const void* x, int dtype, const int* src_row, con
 }
 FL_RECORDABLE(fl_moe_identity)
 
-// The plain product (64 x 64 tile, 4 x 4 per thread, k in steps of 16, the steps' sums added with a
-// compensated addition) over the rows of one tile of one expert.  src_row / src_scale may be null (the
+// A product (64 x 64 tile, 4 x 4 per thread, k in steps of 16, each a chain, the steps' sums added with a compensated
+// addition in 32 bits: not the sums of dense layers, see gemm_float.hip) over the rows of one tile of one expert.  src_row / src_scale may be null (the
 // rows are then the sorted places themselves, unscaled).  A scaled row is rounded to the storage type
 // before it is multiplied, as a stored activation would be.
 template <typename TIn>
