@@ -338,7 +338,10 @@ FL_RECORDABLE(fl_rope_table)
 // table of cosines and sines, or null (then they are computed here).  paired: the rotated dims of
 // a q or k head arrive in the order of fl_rotary_paired_rows (8 dims, their 8 partners, the next
 // 8 dims, ...), as the projection's fused kernels want them.
-template <typename TIn, typename T>
+// PARTS: n_parts where it is 2 or 3, all asked for at once, or 0 (four at a time).  One by one, as it was, and now, 2, 4 and 8 parts: 207 rows of 48 heads
+// of 128 10.0 / 10.1, 11.0 / 10.5 and 16.1 / 11.7 us, 528 rows 20.6 / 21.0, 24.0 / 21.1 and 35 / 24; 2,048 rows of 12 heads of 256, 64 dims rotated, 25.0 / 24.7 and 37.5 / 28.3 (two parts
+// asked for by fours 27.5).
+template <int PARTS, typename TIn, typename T>
 __global__ __launch_bounds__(64) void rope_kv_write_kernel(
     const TIn* __restrict__ qkv, int ld, const int* __restrict__ positions,
     const int* __restrict__ tok_seq, const int* __restrict__ block_table, int max_blocks,
@@ -349,22 +352,23 @@ __global__ __launch_bounds__(64) void rope_kv_write_kernel(
     const int nkv = cache.n_kv_heads;
     const int pos = positions[token];
     const TIn* src = qkv + (size_t)token * ld + (size_t)head * hd;
-    // the projection may arrive as n_parts partial sums (a product that split K): added here, in rising order.  Those of a pair's two values come four parts at a time: waiting for every
-    // one before the next was asked for, 207 rows of 48 heads of 128 in four parts took 9.8 us, now 8.2.
+    // The projection may arrive as n_parts partial sums (a product that split K): added here, in rising order
     auto pair_of = [&](int i, int k, float& a, float& b) {
+        constexpr int AT = PARTS > 0 ? PARTS - 1 : 4;
         a = to_f32(src[i]), b = to_f32(src[k]);
-        for (int part = 1; part < n_parts; part += 4) {
-            float u[4], v[4];
+        if constexpr (AT > 0)
+            for (int part = 1; part < (PARTS > 0 ? 2 : n_parts); part += AT) {
+                float u[AT], v[AT];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const TIn* from = src + (size_t)min(part + q, n_parts - 1) * part_stride;
-                u[q] = to_f32(from[i]);
-                v[q] = to_f32(from[k]);
+                for (int q = 0; q < AT; ++q) {
+                    const TIn* from = src + (size_t)(PARTS > 0 ? part + q : min(part + q, n_parts - 1)) * part_stride;
+                    u[q] = to_f32(from[i]);
+                    v[q] = to_f32(from[k]);
+                }
+#pragma unroll
+                for (int q = 0; q < AT; ++q)
+                    if (PARTS > 0 || part + q < n_parts) { a += u[q]; b += v[q]; }
             }
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (part + q < n_parts) { a += u[q]; b += v[q]; }
-        }
     };
     T* dst;
     size_t stride = 1;      // distance between consecutive head dims at the destination
@@ -430,15 +434,22 @@ extern "C" int fl_rope_kv_write(const void* qkv, int in_dtype, int ld, const int
     if (n == 0) return 0;
     PagedCache c{cache_base, nkv, page_size, hd, n_pages};
     dim3 grid(n, nh + 2 * nkv);
+#define FL_ROPE_PARTS(PARTS, TIN, TT)                                                          \
+    rope_kv_write_kernel<PARTS, TIN, TT><<<grid, 64, 0, stream>>>((const TIN*)qkv, ld, positions, tok_seq, \
+                                                                  block_table, max_blocks, (TT*)q_out, c, \
+                                                                  nh, hd, rot, theta, write_cache, (const float2*)cs, paired, n_parts, (size_t)part_stride)
 #define FL_ROPE(TIN, TT)                                                                       \
-    rope_kv_write_kernel<TIN, TT><<<grid, 64, 0, stream>>>((const TIN*)qkv, ld, positions, tok_seq, \
-                                                           block_table, max_blocks, (TT*)q_out, c, \
-                                                           nh, hd, rot, theta, write_cache, (const float2*)cs, paired, n_parts, (size_t)part_stride)
+    do {                                                                                       \
+        if (n_parts == 2) FL_ROPE_PARTS(2, TIN, TT);                                      \
+        else if (n_parts == 3) FL_ROPE_PARTS(3, TIN, TT);                                      \
+        else FL_ROPE_PARTS(0, TIN, TT);                                                        \
+    } while (0)
     if (in_dtype == FL_F32 && dtype == FL_F32) FL_ROPE(float, float);
     else if (in_dtype == FL_F32 && dtype == FL_BF16) FL_ROPE(float, bf16_t);
     else if (in_dtype == FL_BF16 && dtype == FL_BF16) FL_ROPE(bf16_t, bf16_t);
     else FL_CHECK(false, "rope_kv_write: unsupported dtypes in=%d store=%d", in_dtype, dtype);
 #undef FL_ROPE
+#undef FL_ROPE_PARTS
     FL_LAUNCH_CHECK();
     return 0;
 }

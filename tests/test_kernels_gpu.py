@@ -265,7 +265,7 @@ def rope_ref(x, pos, theta, rot):
     return out
 
 
-@pytest.mark.parametrize("parts", [2, 4, 5, 6, 8])
+@pytest.mark.parametrize("parts", [2, 3, 4, 5, 6, 7, 8])
 @pytest.mark.parametrize("nh,nkv,hd,rot,paired", [(4, 2, 128, 128, True), (3, 1, 200, 64, False), (2, 2, 24, 0, False), (5, 1, 16, 16, True)])
 def test_rope_kv_write_adds_parts_in_order(nh, nkv, hd, rot, paired, parts):
     """Partial sums, whatever their number and the heads' size: the bits of their sum in rising order."""
@@ -283,6 +283,19 @@ def test_rope_kv_write_adds_parts_in_order(nh, nkv, hd, rot, paired, parts):
     ops().rope_kv_write(whole, pos, seq, table, outs[1], again, nh, rot, 1e4, paired=paired)
     live = [5, 2]
     assert torch.equal(outs[0], outs[1]) and torch.equal(cache.pool[live].nan_to_num(), again.pool[live].nan_to_num())
+
+
+@pytest.mark.parametrize("nh,nkv,hd,rot", [(8, 2, 256, 64), (32, 8, 128, 64)])
+def test_rope_kv_write_reads_the_parts_there_are_and_no_more(nh, nkv, hd, rot):
+    """Two parts are one read more per value: measured 1.03 to 1.06 of one part's time, and 1.15 to 1.21 where four reads are asked for whatever there is."""
+    n, ps = 2048, 16
+    cache = make_cache(n // ps, nkv, ps, hd, torch.bfloat16)
+    pos, seq = torch.arange(n, dtype=torch.int32, device=DEV), torch.zeros(n, dtype=torch.int32, device=DEV)
+    table = torch.arange(n // ps, dtype=torch.int32, device=DEV).view(1, -1)
+    qkv, out, times = rnd(2, n, (nh + 2 * nkv) * hd, seed=3), torch.zeros(n, nh * hd, dtype=torch.bfloat16, device=DEV), []
+    for parts in (1, 2):
+        times.append(time_of(lambda: ops().rope_kv_write(qkv if parts == 2 else qkv[0], pos, seq, table, out, cache, nh, rot, 1e4, parts=parts)))
+    assert times[1] < 1.12 * times[0], times
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
