@@ -151,19 +151,28 @@ extern "C" int fl_layernorm(const float* x, const float* delta, float* resid_out
 }
 FL_RECORDABLE(fl_layernorm)
 
-// v += the parts behind the first, in their order, AT of them asked for at a time.  Waited for one by one, the norm of eight parts of 65 rows of 512 values took
-// 3.43 us where one part takes 2.74 (now 3.04), and product and norm of 80 rows and 2048 x 2048 12.6 us where a kernel of its own that adds the parts made
-// it 11.9 (now 11.7; of 96 rows 13.2 and 12.0, now 12.2: nowhere else of 264 products of 512 to 5120 features was the sum apart the faster one).
-template <int AT>
-__device__ __forceinline__ void add_parts(f32x4& v, const float* first, int parts, size_t stride) {
-    for (int z = 1; z < parts; z += AT) {
-        f32x4 part[AT];
+// v += the parts behind the first, in their order, all of up to five asked for at once, seven at a time of more.  Waited for one by one, the norm of eight
+// parts of 65 rows of 512 values took 3.43 us where one part takes 2.74 (now 3.04), and product and norm of 80 rows and 2048 x 2048 12.6 us where a kernel of its
+// own that adds the parts made it 11.9 (now 11.7; of 96 rows 13.2 and 12.0, now 12.2: nowhere else of 264 products of 512 to 5120 features was the sum apart the
+// faster one).  Four asked for whatever there is: three parts up to 8 % slower than one by one.
+template <int N>
+__device__ __forceinline__ void add_parts(f32x4& v, const float* part, size_t stride) {
+    f32x4 p[N];
 #pragma unroll
-        for (int q = 0; q < AT; ++q) part[q] = *(const f32x4*)(first + min(z + q, parts - 1) * stride);
+    for (int q = 0; q < N; ++q) p[q] = *(const f32x4*)(part + q * stride);
 #pragma unroll
-        for (int q = 0; q < AT; ++q)
-            if (z + q < parts) v += part[q];
-    }
+    for (int q = 0; q < N; ++q) v += p[q];
+}
+__device__ __forceinline__ void add_parts_behind(f32x4& v, const float* first, int parts, size_t stride) {
+    const float* part = first + stride;
+    for (; parts > 8; parts -= 7, part += 7 * stride) add_parts<7>(v, part, stride);
+    if (parts == 2) add_parts<1>(v, part, stride);
+    else if (parts == 3) add_parts<2>(v, part, stride);
+    else if (parts == 4) add_parts<3>(v, part, stride);
+    else if (parts == 5) add_parts<4>(v, part, stride);
+    else if (parts == 6) add_parts<5>(v, part, stride);
+    else if (parts == 7) add_parts<6>(v, part, stride);
+    else if (parts == 8) add_parts<7>(v, part, stride);
 }
 
 // A row's VPT groups of four values per thread stay in registers; the number of threads follows from the row's length
@@ -184,8 +193,11 @@ __global__ __launch_bounds__(NT) void layernorm_add_kernel(const float* __restri
         if (i >= H) continue;
         v[k] = *(const f32x4*)(delta + at + i);
         r[k] = *(const f32x4*)(resid + at + i);
-        if (parts <= 5) add_parts<4>(v[k], delta + at + i, parts, stride);
-        else add_parts<7>(v[k], delta + at + i, parts, stride);
+        if constexpr (VPT == 1) {
+            if (parts > 1) add_parts_behind(v[k], delta + at + i, parts, stride);
+        } else {
+            for (int z = 1; z < parts; ++z) v[k] += *(const f32x4*)(delta + z * stride + at + i);      // (the other groups' reads are in flight beside it)
+        }
         s += (v[k][0] + v[k][1]) + (v[k][2] + v[k][3]);
     }
     const float mean = block_sum<NT / 64>(s, red) / (float)H;
