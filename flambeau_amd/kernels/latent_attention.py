@@ -101,7 +101,8 @@ class TunedLatentAttention(PlainLatentAttention):
         lib, units = load(), {}
         for m in mixers:
             g = -(-m.n_heads // 16)
-            units[g] = min(units.get(g, 8), lib.fl_latent_attention_units(m.row_width, m.value_width, batch.page_size))
+            # (a batch that does not say its pages: tiles that the kernels for pages of any size take)
+            units[g] = min(units.get(g, 8), lib.fl_latent_attention_units(m.row_width, m.value_width, batch.page_size or 1 << 30))
         return {f"latent_tiles_{g}": prompt_tiles(batch, g, units[g], lib.fl_compute_units()) for g in sorted(units)}
 
     def prepare(self, uk, uv, n_heads):

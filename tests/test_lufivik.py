@@ -205,7 +205,7 @@ def test_a_tile_holds_the_units_that_its_kernel_has():
     units = load().fl_latent_attention_units
     assert [units(K, R, 16) for K, R in ((576, 512), (512, 512), (320, 256), (128, 128), (96, 96), (448, 384))] == [8, 8, 8, 8, 4, 4]
     assert units(576, 512, 1 << 19) == 8 and units(576, 512, 1 << 20) == 4 and units(128, 128, 1 << 21) == 8 and units(128, 128, 1 << 22) == 4
-    for page_size, most in ((16, 8), (1 << 20, 4)):
+    for page_size, most in ((16, 8), (1 << 20, 4), (0, 4)):                   # (0: a batch that does not say it)
         batch = HostBatch([0], [4096], [0], [0], 4096, 1, page_size=page_size)
         mixers = [SimpleNamespace(n_heads=32, row_width=576, value_width=512), SimpleNamespace(n_heads=70, row_width=576, value_width=512)]
         lists = TunedLatentAttention(None).metadata(batch, mixers)
