@@ -162,12 +162,12 @@ def test_a_norm_of_a_product_in_parts_on_its_way_into_the_stream(W, parts):
 @pytest.mark.parametrize("W", [512, 1024])
 def test_a_norm_asks_for_the_parts_of_a_product_side_by_side(W):
     """Eight parts of few rows are a few reads in flight: 1.11 to 1.14 of one part's time (measured); waited for one by one 1.24 and more."""
-    from test_kernels_gpu import time_of
+    from test_kernels_gpu import times_in_turn
     from flambeau_amd.kernels import ops
     g = torch.Generator().manual_seed(W)
     part, x, cast = dev(torch.randn(8, 65, W, generator=g)), dev(torch.randn(65, W, generator=g)), torch.empty(65, W, dtype=torch.bfloat16, device=DEV)
     w, b = dev(torch.ones(W)), dev(torch.zeros(W))
-    times = [min(time_of(lambda: ops.layernorm_add(d, w, b, x, 3e-4, cast=cast), times=50) for _ in range(3)) for d in (part[0].clone(), part)]
+    times = times_in_turn(*(lambda d=d: ops.layernorm_add(d, w, b, x, 3e-4, cast=cast) for d in (part[0].clone(), part)), times=50)
     assert times[1] < 1.19 * times[0], times
 
 

@@ -292,9 +292,8 @@ def test_rope_kv_write_reads_the_parts_there_are_and_no_more(nh, nkv, hd, rot):
     cache = make_cache(n // ps, nkv, ps, hd, torch.bfloat16)
     pos, seq = torch.arange(n, dtype=torch.int32, device=DEV), torch.zeros(n, dtype=torch.int32, device=DEV)
     table = torch.arange(n // ps, dtype=torch.int32, device=DEV).view(1, -1)
-    qkv, out, times = rnd(2, n, (nh + 2 * nkv) * hd, seed=3), torch.zeros(n, nh * hd, dtype=torch.bfloat16, device=DEV), []
-    for parts in (1, 2):
-        times.append(time_of(lambda: ops().rope_kv_write(qkv if parts == 2 else qkv[0], pos, seq, table, out, cache, nh, rot, 1e4, parts=parts)))
+    qkv, out = rnd(2, n, (nh + 2 * nkv) * hd, seed=3), torch.zeros(n, nh * hd, dtype=torch.bfloat16, device=DEV)
+    times = times_in_turn(*(lambda p=p: ops().rope_kv_write(qkv if p == 2 else qkv[0], pos, seq, table, out, cache, nh, rot, 1e4, parts=p) for p in (1, 2)))
     assert times[1] < 1.12 * times[0], times
 
 
@@ -786,10 +785,9 @@ def test_gemm_tiled_plan_knows_what_is_faster(M, N, K, gate, variant, splits):
     w = [rnd(N * K, dtype=torch.bfloat16, seed=22, scale=0.05) for _ in range(copies)]       # (N, K multiples of a tile: any values are a packed matrix)
     x, out = rnd(M, K, dtype=torch.bfloat16, seed=21), torch.empty(M, N // 2 if gate else N, dtype=torch.bfloat16, device=DEV)
     ws = torch.empty(8 * M * N, dtype=torch.float32, device=DEV)
-    times = []
-    for v, s in ((variant, splits), (0, 0)):
-        turn = iter(range(1 << 30))
-        times.append(time_of(lambda: tuned().gemm_tiled(x, w[next(turn) % copies], out, ws, swiglu_rows=N if gate else 0, variant=v, splits=s)))
+    turn = iter(range(1 << 30))
+    times = times_in_turn(*(lambda v=v, s=s: tuned().gemm_tiled(x, w[next(turn) % copies], out, ws, swiglu_rows=N if gate else 0, variant=v, splits=s)
+                            for v, s in ((variant, splits), (0, 0))))
     assert times[1] < 1.1 * times[0], times
 
 
@@ -1380,21 +1378,18 @@ def test_gemm_float_blocks_of_one_to_three_tiles_give_the_plain_kernel_s_bits(M,
 def test_gemm_float_takes_short_sums_where_it_is_faster(M, N, K):
     """Measured 0.58 to 0.84 of the plain kernel's time: sizes next to those that it leaves to that one (the test above).  They must not take
     as long as operands that always go there."""
-    w, out, times = rnd(N, K, seed=32), torch.empty(M, N, dtype=torch.float32, device=DEV), []
-    for offset in (0, 1):
-        x = torch.empty(M * K + 4, dtype=torch.float32, device=DEV)[offset:offset + M * K].view(M, K)
-        x.copy_(rnd(M, K, seed=31))
-        times.append(time_of(lambda: ops().gemm_plain(x, w, out)))
+    w, out = rnd(N, K, seed=32), torch.empty(M, N, dtype=torch.float32, device=DEV)
+    rows = [torch.empty(M * K + 4, dtype=torch.float32, device=DEV)[offset:offset + M * K].view(M, K).copy_(rnd(M, K, seed=31)) for offset in (0, 1)]
+    times = times_in_turn(*(lambda x=x: ops().gemm_plain(x, w, out) for x in rows))
     assert times[0] < 0.93 * times[1], times
 
 
 @pytest.mark.parametrize("M,N,K", [(8, 256, 16), (1000, 4096, 15)])
 def test_gemm_plain_does_no_work_behind_sums_of_up_to_16(M, N, K):
     """Such a sum takes half the products of one of 32 (measured 0.81 and 0.85 of its time, 1.0 with a step of 32 for both)."""
-    times = []
-    for k in (K, 2 * K - 1):                             # (rows that do not begin at 16 bytes; 16 k of 8 rows come here as they are)
-        x, w, out = rnd(M, k, seed=31), rnd(N, k, seed=32), torch.empty(M, N, dtype=torch.float32, device=DEV)
-        times.append(time_of(lambda: ops().gemm_plain(x, w, out)))
+    out = torch.empty(M, N, dtype=torch.float32, device=DEV)
+    pairs = [(rnd(M, k, seed=31), rnd(N, k, seed=32)) for k in (K, 2 * K - 1)]       # (rows that do not begin at 16 bytes; 16 k of 8 rows come here as they are)
+    times = times_in_turn(*(lambda x=x, w=w: ops().gemm_plain(x, w, out) for x, w in pairs))
     assert times[0] < 0.95 * times[1], times
 
 
@@ -1987,23 +1982,30 @@ def test_attn_float_is_as_precise_as_the_plain_kernel(hd, context):
     assert errors[0] < 1.05 * errors[1], errors
 
 
-def time_of(launch, times=20):
-    """Microseconds of one launch: the second fastest of five runs of a graph of ``times`` launches."""
-    launch()
-    torch.cuda.synchronize()
-    graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        for _ in range(times):
-            launch()
-    runs = []
+def times_in_turn(*launches, times=20):
+    """Microseconds of one launch of each: the second fastest of five runs of a graph of ``times`` launches, the graphs run in turn (a clock that changes
+    meanwhile changes for all of them: one behind the other, a product and itself have differed by a tenth)."""
+    graphs, runs = [], [[] for _ in launches]
+    for launch in launches:
+        launch()
+        torch.cuda.synchronize()
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1]):
+            for _ in range(times):
+                launch()
     for _ in range(5):
-        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        begin.record()
-        graph.replay()
-        end.record()
-        end.synchronize()
-        runs.append(1000 * begin.elapsed_time(end) / times)
-    return sorted(runs)[1]
+        for graph, taken in zip(graphs, runs):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            graph.replay()
+            end.record()
+            end.synchronize()
+            taken.append(1000 * begin.elapsed_time(end) / times)
+    return [sorted(taken)[1] for taken in runs]
+
+
+def time_of(launch, times=20):
+    return times_in_turn(launch, times=times)[0]
 
 
 def attn_float_times(nh, nkv, hd, seqs):
