@@ -900,7 +900,15 @@ def prefill_supported(cache, table, window: int = 0) -> bool:
 # Between 0.7 and 1.1 either is within 6 us.  For fewer rows than tiles one place was up to 27 % slower than both and up to 20 % slower than apart.  Rows that
 # keep every unit at its keys for 80 us (3,400 of a head) beside a twentieth of that work lose 2 to 6 % by the tiles' blocks among theirs.  With these lines the steps took
 # 0.66 to 1.03 of the time apart, 0.87 on average.
+#
+# Laid out for one place, nine to fifteen tiles have blocks for a part of the units and keys in one part.  A block then reads a tile's keys one behind the other, and where
+# those are many beside what a unit has of the rows (TILE_CHAIN times its keys of a head) everything waits for it: both places there.  us, one place / both / apart, by that ratio:
+#   1.3   576 tokens behind 3,500 beside 24 rows of 4,000   124 / 126 / 136    1.4   640 behind 1,000 beside 16 of 2,000   58 / 65 / 72
+#   1.8   1,024 behind 1,000 beside 16 of 2,000             69 / 75 / 82       2.4   640 behind 7,000 beside 24 of 4,000   219 / 151 / 178
+#   2.4   896 behind 7,000 beside 24 of 4,000               228 / 187 / 219    3.6   576 behind 3,500 beside 16 of 2,000   120 / 86 / 94
+#   6     prompts of 200 and 312 beside 5 rows, all but the latter at a window of 4,096   110 / 75 / 76
 ROW_KEYS = 256
+TILE_CHAIN = 2.0
 ROWS_TAKE_A_PLACE = 7 / 8
 ROWS_APART, ROWS_APART_KEYS = 20.0, 3400
 
@@ -932,6 +940,10 @@ def attention_splits(batch, n_heads: int, n_kv_heads: int, head_dim: int, window
             rows = sum([ql * (p0 + ql if p0 + ql < most else most) for ql, p0 in zip(batch.q_lens, batch.start_pos) if ql <= SHORT_PORTION]) + ROW_KEYS * n_items
             tiles = sum([-(-ql // PREFILL_TILE) * min(end, most + PREFILL_TILE) for ql, end in long])
             joined, beside = tiles_beside_rows(rows, tiles, n_heads, n_kv_heads)
+            plan = (n_tiles, n_heads, n_kv_heads, head_dim, longest)
+            if beside and attn_prefill_splits(*plan, beside) == 1 and attn_prefill_splits(*plan) > 1:
+                chain = max([min(end, most + PREFILL_TILE) for _, end in long])
+                beside = 0 if chain * DECODE_UNITS > TILE_CHAIN * rows * n_kv_heads else beside
         p_split = attn_prefill_splits(n_tiles, n_heads, n_kv_heads, head_dim, longest, beside) \
             + 64 * attn_prefill_heads(n_tiles, n_heads, n_kv_heads, head_dim, longest, beside) + 512 * joined
     if n_items and not with_items:

@@ -208,6 +208,11 @@ def test_tiles_beside_single_rows_are_laid_out_for_half_the_chip_where_the_rows_
         assert splits(1024, 3000, rows, keys)[:2] == alone(1024, 4024)
     assert splits(512, 1536, 16, 2000) == (2, 2, 1) and alone(512, 2048) == (2, 1)
     assert splits(1024, 2000, 32, 4000) == (1, 2, 1) and splits(512, 5000, 24, 2000) == (2, 2, 1)
+    # nine to fifteen tiles, which half the grid leaves whole: not where a block's keys would take longer than the rows beside it (long portions beside shorter rows)
+    for portion, behind, rows, keys in ((576, 3500, 16, 2000), (576, 7000, 24, 4000), (640, 7000, 24, 4000), (768, 7000, 24, 4000), (896, 7000, 24, 4000)):
+        assert splits(portion, behind, rows, keys) == (*alone(portion, behind + portion), 1)
+    for portion, behind, rows, keys in ((576, 1000, 24, 4000), (640, 1000, 16, 2000), (768, 1000, 16, 2000), (896, 1000, 16, 2000), (1024, 3500, 24, 4000)):
+        assert splits(portion, behind, rows, keys)[::2] == (1, 1)
     assert splits(256, 0, 64, 1500) == (*alone(256, 1500), 0) and splits(256, 0, 16, 4000)[2] == splits(128, 0, 17, 1500)[2] == splits(512, 1536, 64, 1500)[2] == 1
     assert splits(512, 0, 0, 1) == (*alone(512, 512), 0) and splits(512, 0, 4, 600, heads=(4, 2, 256))[2] == 0
     # a window bounds what both see
@@ -215,3 +220,5 @@ def test_tiles_beside_single_rows_are_laid_out_for_half_the_chip_where_the_rows_
     for rows in (1, 2, 3, 16):
         seen = [splits(512, 1536, rows, keys) for keys in range(2, 2049)]
         assert sum(a != b for a, b in zip(seen, seen[1:])) <= 1
+    seen = [splits(576, 3500, 24, keys) for keys in range(2, 8000, 7)]
+    assert sum(a != b for a, b in zip(seen, seen[1:])) == 1 and seen[0][0] == 3 and seen[-1][0] == 1
