@@ -87,8 +87,8 @@ def shared_tiles(batch, groups: int, units: int = 4):
 
 def prompt_tiles(batch, groups: int, units: int, compute_units: int):
     """``shared_tiles`` of up to ``units`` where those still give every compute unit more than one: eight share what a
-    block of four fetches too (2,048 tokens of 32 heads 171 us against 241), but the chip must not wait for a few of them
-    (1,024 tokens, 256 tiles of eight, 79 us against 73; 700 of three requests of 16 heads, 264 tiles, 40 against 49)."""
+    block of four fetches too (2,048 tokens of 32 heads 176 us against 244), but the chip must not wait for a few of them
+    (1,024 tokens, 256 tiles of eight, 80 us against 75; 1,100, 275 tiles, 86 against 96; 700 of three requests of 16 heads, 264 tiles, 62 against 76)."""
     return shared_tiles(batch, groups, units if batch.n_tokens * groups > units * compute_units else 4)
 
 
