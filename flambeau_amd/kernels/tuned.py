@@ -898,8 +898,7 @@ def prefill_supported(cache, table, window: int = 0) -> bool:
 #   1.2   the same beside 24 of 2,000                       98 / 112 / 109     1.1   the same beside 24 of 2,000            96 / 112 / 111
 #   3 to 50   one place the faster by up to 30 %            110   256 beside 64 of 1,500   86 / 86 / 82        113   128 beside 17 of 200 to 5,400   6 less than apart
 # Between 0.7 and 1.1 either is within 6 us.  For fewer rows than tiles one place was up to 27 % slower than both and up to 20 % slower than apart.  Rows that
-# keep every unit at its keys for 80 us (3,400 of a head) beside a twentieth of that work lose 2 to 6 % by the tiles' blocks among theirs.  With these lines the steps took
-# 0.66 to 1.03 of the time apart, 0.87 on average.
+# keep every unit at its keys for 80 us (3,400 of a head) beside a twentieth of that work lose 2 to 6 % by the tiles' blocks among theirs.
 #
 # Laid out for one place, nine to fifteen tiles have blocks for a part of the units and keys in one part.  A block then reads a tile's keys one behind the other, and where
 # those are many beside what a unit has of the rows (TILE_CHAIN times its keys of a head) everything waits for it: both places there.  us, one place / both / apart, by that ratio:
@@ -907,6 +906,7 @@ def prefill_supported(cache, table, window: int = 0) -> bool:
 #   1.8   1,024 behind 1,000 beside 16 of 2,000             69 / 75 / 82       2.4   640 behind 7,000 beside 24 of 4,000   219 / 151 / 178
 #   2.4   896 behind 7,000 beside 24 of 4,000               228 / 187 / 219    3.6   576 behind 3,500 beside 16 of 2,000   120 / 86 / 94
 #   6     prompts of 200 and 312 beside 5 rows, all but the latter at a window of 4,096   110 / 75 / 76
+# With these lines 256 other steps, of six layouts of heads (8 to 64 over 2 to 32 of 64 and 128), took 0.55 to 1.05 of the time apart, 0.78 on average.
 ROW_KEYS = 256
 TILE_CHAIN = 2.0
 ROWS_TAKE_A_PLACE = 7 / 8
